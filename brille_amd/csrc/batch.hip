@@ -5,14 +5,17 @@
 // adds a device array of BatchGrid (the grid's GridConst/DataConst, its error
 // record and which phase 2 its payload takes) and, per run, a device array of
 // BatchSlot (where the grid's points and outputs are, and its first work
-// item).  Work items are tiles of TB consecutive points of one grid, numbered
-// slot after slot.  k_batch is persistent: each block takes `grab` tiles at a
-// time from a device counter until none are left, finds the slot of each tile
-// by binary search, and runs the tile's two phases with that grid's tables.
-// k_batch_reset (a kernel, so that a captured graph replays it correctly)
-// clears the counter and the per-grid error records.  Both launches are
-// captured once per (precision, schedule) into a HIP graph; a run uploads the
-// slots and replays the graph.
+// item).  Work items are tiles of at most TB consecutive points of one grid,
+// numbered slot after slot, in two lists: the grids of wide rows, whose points
+// are each many units of work for a wave, and the others.  k_batch is
+// persistent: each block takes `grab` tiles at a time from its list's device
+// counter until none are left, finds the slot of each tile by binary search,
+// and runs the tile's two phases with that grid's tables.  The two lists have a
+// kernel each, side by side in the graph, so that neither carries the other's
+// registers.  k_batch_reset (a kernel, so that a captured graph replays it
+// correctly) clears the counters and the per-grid error records.  The launches
+// are captured once per (precision, schedule) into a HIP graph; a run uploads
+// the slots and replays the graph.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -37,7 +40,8 @@ enum BatchKind : int32_t {
   BK_SCALAR2 = 4,
   BK_SCALAR3 = 5,
   BK_SCALAR4 = 6,
-  BK_WIDE = 7
+  BK_WIDE = 7,
+  BK_WIDE_ATOM = 8
 };
 
 struct BatchGrid {
@@ -57,14 +61,18 @@ struct BatchSlot {
   uint64_t n;      // points of the grid
   uint64_t tile0;  // first work item of the grid
   uint32_t grid;   // index into the BatchGrid array
-  uint32_t pad;
+  uint32_t pts;    // points per tile
 };
 
+// the two work lists: 0 the narrow and general rows, 1 the wide rows
+constexpr int kLists = 2;
 struct BatchHeader {
-  unsigned long long counter;
-  uint64_t n_tiles;
-  uint32_t n_slots;
+  unsigned long long counter[kLists];
+  uint64_t n_tiles[kLists];
+  uint32_t slot0[kLists];  // first slot of the list
+  uint32_t n_slots[kLists];
   int32_t fold;  // Fold
+  int32_t pad;
 };
 
 // the specialised phase 2 a grid's payload takes inside the batch kernel
@@ -73,6 +81,7 @@ static int32_t batch_kind(const DataConst& d) {
   if (L == LAYOUT_GAMMA && d.sv == 1 && d.sc == 3) return BK_GAMMA3;
   if (L == LAYOUT_GAMMA && d.sv == 1 && d.sc == 6) return BK_GAMMA6;
   if (L == LAYOUT_SCALAR && d.sv == 1 && d.sc >= 1 && d.sc <= 4) return BK_SCALAR1 + (int32_t)d.sc - 1;
+  if (wide_by_atom(d)) return BK_WIDE_ATOM;
   if (wide_rows(d)) return BK_WIDE;
   return BK_GENERIC;
 }
@@ -99,23 +108,24 @@ __device__ __forceinline__ void batch_tile(const BatchGrid& bg, const BatchSlot&
   __syncthreads();
 }
 
-// FP32: three waves per SIMD (the wide-row branch needs the occupancy; one
-// spilled dword)
-template <typename Real, int TB>
+template <typename Real, int TB, int LIST>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 3 : 1)))
-void k_batch(const BatchGrid* grids, const BatchSlot* slots, BatchHeader* hdr, uint32_t grab) {
+void k_batch(const BatchGrid* grids, const BatchSlot* all_slots, BatchHeader* hdr, uint32_t grab) {
   using C = typename Cplx<Real>::T;
+  constexpr bool kWide = LIST == 1;
   __shared__ PointRec<Real> s_rec[TB];
-  __shared__ C s_ph[TB * 4];
+  __shared__ C s_ph[kWide ? 1 : TB * 4];
   // q (general and wide layouts) or the Gamma frames
-  __shared__ double s_q[(3 > frame_words<Real>() ? 3 : frame_words<Real>()) * TB];
-  __shared__ C s_wide[(TB / 64) * kWideMax];
+  __shared__ double s_q[(kWide || 3 > frame_words<Real>() ? 3 : frame_words<Real>()) * TB];
+  constexpr int kSlice = TileShape<LAYOUT_WIDE, kWideAtom, TB, Real>::NW;
+  __shared__ C s_wide[!kWide ? 1 : kSlice > (TB / 64) * (int)kWideMax ? kSlice : (TB / 64) * (int)kWideMax];
   __shared__ unsigned long long s_t;
-  const uint64_t n_tiles = hdr->n_tiles;
-  const uint32_t n_slots = hdr->n_slots;
+  const uint64_t n_tiles = hdr->n_tiles[LIST];
+  const uint32_t n_slots = hdr->n_slots[LIST];
+  const BatchSlot* slots = all_slots + hdr->slot0[LIST];
   const int fold = hdr->fold;
   for (;;) {
-    if (threadIdx.x == 0) s_t = atomicAdd(&hdr->counter, (unsigned long long)grab);
+    if (threadIdx.x == 0) s_t = atomicAdd(&hdr->counter[LIST], (unsigned long long)grab);
     __syncthreads();
     const uint64_t t0 = s_t;
     __syncthreads();
@@ -131,17 +141,22 @@ void k_batch(const BatchGrid* grids, const BatchSlot* slots, BatchHeader* hdr, u
       lo = __builtin_amdgcn_readfirstlane(lo);
       const BatchSlot& sl = slots[lo];
       const BatchGrid& bg = grids[sl.grid];
-      const uint64_t p0 = (t - sl.tile0) * TB;
+      const uint64_t p0 = (t - sl.tile0) * sl.pts;
       const uint64_t left = sl.n - p0;
-      const uint32_t npts = left < (uint64_t)TB ? (uint32_t)left : (uint32_t)TB;
-      switch (bg.kind) {
+      const uint32_t npts = left < (uint64_t)sl.pts ? (uint32_t)left : sl.pts;
+      if constexpr (kWide) {
+        if (bg.kind == BK_WIDE_ATOM)
+          batch_tile<Real, LAYOUT_WIDE, kWideAtom, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold);
+        else
+          batch_tile<Real, LAYOUT_WIDE, kWideAll, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold);
+        continue;
+      } else switch (bg.kind) {
         case BK_GAMMA3: batch_tile<Real, LAYOUT_GAMMA, 3, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
         case BK_GAMMA6: batch_tile<Real, LAYOUT_GAMMA, 6, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
         case BK_SCALAR1: batch_tile<Real, LAYOUT_SCALAR, 1, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
         case BK_SCALAR2: batch_tile<Real, LAYOUT_SCALAR, 2, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
         case BK_SCALAR3: batch_tile<Real, LAYOUT_SCALAR, 3, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
         case BK_SCALAR4: batch_tile<Real, LAYOUT_SCALAR, 4, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
-        case BK_WIDE: batch_tile<Real, LAYOUT_WIDE, 0, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
         default: batch_tile<Real, LAYOUT_GENERIC, 0, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
       }
     }
@@ -151,7 +166,7 @@ void k_batch(const BatchGrid* grids, const BatchSlot* slots, BatchHeader* hdr, u
 // graph-safe clear of the work counter and of every grid's error record
 __global__ void k_batch_reset(BatchHeader* hdr, const BatchGrid* grids, uint32_t n_grids) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) hdr->counter = 0ull;
+  if (i < kLists) hdr->counter[i] = 0ull;
   if (i < n_grids) {
     grids[i].err->first_bad = ~0ull;
     grids[i].err->count = 0ull;
@@ -191,6 +206,9 @@ struct brille_batch {
   uint32_t n_cu = 0;
   Schedule sched;
   hipStream_t cap_stream = nullptr;
+  // a second capture stream and events: the graph's two work lists side by side
+  hipStream_t cap_side = nullptr;
+  hipEvent_t cap_ev[2] = {};
   // streams the binned grids spread over beside the caller's (created on
   // first use, default priority), and the events that fork them from the
   // caller's stream and join them back
@@ -216,12 +234,23 @@ namespace brille_amd {
     if (e_ != hipSuccess) return fail(BRILLE_ERR_DEVICE, std::string(#expr ": ") + hipGetErrorString(e_)); \
   } while (0)
 
-template <typename Real>
+template <typename Real, int LIST>
 static void launch_batch_kernel(brille_batch* b, uint32_t tile, uint32_t blocks, uint32_t grab, hipStream_t s) {
   if (tile == 128)
-    hipLaunchKernelGGL((k_batch<Real, 128>), dim3(blocks), dim3(128), 0, s, b->d_grids, b->d_slots, b->d_hdr, grab);
+    hipLaunchKernelGGL((k_batch<Real, 128, LIST>), dim3(blocks), dim3(128), 0, s, b->d_grids, b->d_slots, b->d_hdr, grab);
   else
-    hipLaunchKernelGGL((k_batch<Real, 256>), dim3(blocks), dim3(256), 0, s, b->d_grids, b->d_slots, b->d_hdr, grab);
+    hipLaunchKernelGGL((k_batch<Real, 256, LIST>), dim3(blocks), dim3(256), 0, s, b->d_grids, b->d_slots, b->d_hdr, grab);
+}
+
+template <typename Real>
+static int launch_batch_lists(brille_batch* b, uint32_t tile, uint32_t blocks, uint32_t grab) {
+  BATCH_TRY(hipEventRecord(b->cap_ev[0], b->cap_stream));
+  BATCH_TRY(hipStreamWaitEvent(b->cap_side, b->cap_ev[0], 0));
+  launch_batch_kernel<Real, 1>(b, tile, blocks, grab, b->cap_stream);
+  launch_batch_kernel<Real, 0>(b, tile, blocks, grab, b->cap_side);
+  BATCH_TRY(hipEventRecord(b->cap_ev[1], b->cap_side));
+  BATCH_TRY(hipStreamWaitEvent(b->cap_stream, b->cap_ev[1], 0));
+  return BRILLE_OK;
 }
 
 static int graph_for(brille_batch* b, int precision, const Schedule& sc, hipGraphExec_t* out) {
@@ -236,9 +265,14 @@ static int graph_for(brille_batch* b, int precision, const Schedule& sc, hipGrap
   BATCH_TRY(hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal));
   const uint32_t ng = (uint32_t)b->grids.size();
   hipLaunchKernelGGL(k_batch_reset, dim3((ng + 63) / 64), dim3(64), 0, b->cap_stream, b->d_hdr, b->d_grids, ng);
-  if (precision == BRILLE_FP32) launch_batch_kernel<float>(b, sc.tile, blocks, sc.grab, b->cap_stream);
-  else launch_batch_kernel<double>(b, sc.tile, blocks, sc.grab, b->cap_stream);
-  BATCH_TRY(hipStreamEndCapture(b->cap_stream, &graph));
+  const int launched = precision == BRILLE_FP32 ? launch_batch_lists<float>(b, sc.tile, blocks, sc.grab)
+                                                : launch_batch_lists<double>(b, sc.tile, blocks, sc.grab);
+  const hipError_t ended = hipStreamEndCapture(b->cap_stream, &graph);
+  if (launched != BRILLE_OK) {
+    if (ended == hipSuccess) (void)hipGraphDestroy(graph);
+    return launched;
+  }
+  BATCH_TRY(ended);
   hipGraphExec_t exec;
   hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
@@ -263,25 +297,46 @@ static int stage_slots(brille_batch* b, const double* Q, const uint64_t* offsets
   if (sc.order == 1)
     std::stable_sort(order.begin(), order.end(),
                      [&](uint32_t x, uint32_t y) { return point_cost(b->grids[x]) > point_cost(b->grids[y]); });
-  std::vector<BatchSlot> slots;
-  uint64_t tiles = 0;
+  // Units of phase 2 per point: a wide row keeps a wave busy per pass of
+  // modes, a narrow one a lane per mode.  Tiles are cut so that the list's
+  // work makes about kTilesPerBlock of them per persistent block: a fixed tile
+  // of wide rows would leave a grid of few points to a few blocks.
+  const double blocks = std::max(1u, b->n_cu * sc.blocks_per_cu);
+  constexpr double kTilesPerBlock = 4.0;
+  auto units = [&](const brille_grid* G) {
+    const DataConst& d = G->d;
+    if (!wide_rows(d)) return (double)d.B / 64.0;
+    const uint32_t mpw = wide_by_atom(d) ? 64u / (d.sc / 3u) : 1u;
+    return (double)((d.B + mpw - 1) / mpw);
+  };
+  double work[kLists] = {0.0, 0.0};
   for (uint32_t g : order) {
     const uint64_t n = offsets[g + 1] - offsets[g];
-    if (n == 0 || n >= sc.binned_min) continue;
-    BatchSlot sl{};
-    sl.Q = Q + 3 * offsets[g];
-    sl.vals = vals[g];
-    sl.vecs = vecs[g];
-    sl.n = n;
-    sl.tile0 = tiles;
-    sl.grid = g;
-    slots.push_back(sl);
-    tiles += (n + sc.tile - 1) / sc.tile;
+    if (n && n < sc.binned_min) work[wide_rows(b->grids[g]->d)] += (double)n * units(b->grids[g]);
   }
+  std::vector<BatchSlot> slots;
   BatchHeader h{};
-  h.counter = 0;
-  h.n_tiles = tiles;
-  h.n_slots = (uint32_t)slots.size();
+  for (int list = 0; list < kLists; ++list) {
+    uint64_t tiles = 0;
+    h.slot0[list] = (uint32_t)slots.size();
+    for (uint32_t g : order) {
+      const uint64_t n = offsets[g + 1] - offsets[g];
+      if (n == 0 || n >= sc.binned_min || (int)wide_rows(b->grids[g]->d) != list) continue;
+      const double per = work[list] / (blocks * kTilesPerBlock) / units(b->grids[g]);
+      BatchSlot sl{};
+      sl.Q = Q + 3 * offsets[g];
+      sl.vals = vals[g];
+      sl.vecs = vecs[g];
+      sl.n = n;
+      sl.tile0 = tiles;
+      sl.grid = g;
+      sl.pts = (uint32_t)std::min<double>(sc.tile, std::max<double>(list ? 1.0 : 32.0, per));
+      slots.push_back(sl);
+      tiles += (n + sl.pts - 1) / sl.pts;
+    }
+    h.n_tiles[list] = tiles;
+    h.n_slots[list] = (uint32_t)slots.size() - h.slot0[list];
+  }
   h.fold = fold;
   if (!slots.empty())
     BATCH_TRY(hipMemcpyAsync(b->d_slots, slots.data(), slots.size() * sizeof(BatchSlot), hipMemcpyHostToDevice, s));
@@ -466,7 +521,13 @@ int brille_batch_create(brille_grid* const* grids, uint32_t n_grids, brille_batc
   if (hipMalloc(&pg, n_grids * sizeof(BatchGrid)) != hipSuccess || hipMalloc(&ps, n_grids * sizeof(BatchSlot)) != hipSuccess ||
       hipMalloc(&ph, sizeof(BatchHeader)) != hipSuccess ||
       hipMemcpy(pg, host.data(), n_grids * sizeof(BatchGrid), hipMemcpyHostToDevice) != hipSuccess ||
-      hipStreamCreateWithFlags(&b->cap_stream, hipStreamNonBlocking) != hipSuccess) {
+      hipStreamCreateWithFlags(&b->cap_stream, hipStreamNonBlocking) != hipSuccess ||
+      hipStreamCreateWithFlags(&b->cap_side, hipStreamNonBlocking) != hipSuccess ||
+      hipEventCreateWithFlags(&b->cap_ev[0], hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&b->cap_ev[1], hipEventDisableTiming) != hipSuccess) {
+    if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
+    if (b->cap_side) (void)hipStreamDestroy(b->cap_side);
+    if (b->cap_ev[0]) (void)hipEventDestroy(b->cap_ev[0]);
     if (pg) (void)hipFree(pg);
     if (ps) (void)hipFree(ps);
     if (ph) (void)hipFree(ph);
@@ -600,6 +661,9 @@ int brille_batch_destroy(brille_batch* b) {
   if (b->d_slots) (void)hipFree(b->d_slots);
   if (b->d_hdr) (void)hipFree(b->d_hdr);
   if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
+  if (b->cap_side) (void)hipStreamDestroy(b->cap_side);
+  for (hipEvent_t e : b->cap_ev)
+    if (e) (void)hipEventDestroy(e);
   for (int k = 0; k < brille_batch::kLanes; ++k) {
     if (b->lanes[k]) (void)hipStreamDestroy(b->lanes[k]);
     if (b->join[k]) (void)hipEventDestroy(b->join[k]);

@@ -377,17 +377,22 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nb) {
   return x * q + (x < r ? x : r) + i;
 }
 
-// (The FP32 wide-row sums run at two waves per SIMD, over 200 VGPRs: held
-// to three waves (168 VGPRs, some spilled) the wave-per-unit walk gained
-// 12 %, the atom-major walk lost 8 %; four waves spill too much.)
+// waves per SIMD asked of the compiler: the atom-major wide sums run best at
+// four (FP32) and two (FP64), a few registers below what it would take for
+// the antiphases of the rare points without a table block
+template <typename Real, int L, int SC>
+constexpr int sums_waves() {
+  return L == LAYOUT_WIDE && SC == kWideAtom ? (sizeof(Real) == 4 ? 4 : 2) : 1;
+}
 template <typename Real, int L, int SC, int SV, bool Prop>
-__global__ __launch_bounds__(TILE) void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
+__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(sums_waves<Real, L, SC>())))
+void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
                                                     const uint32_t* perm, uint32_t n, void* __restrict__ vals,
                                                     void* __restrict__ vecs, brille_aux_out aux,
-                                                    ErrRec* __restrict__ err, uint64_t base, uint32_t* rest,
-                                                    uint32_t* rest_n) {
+                                                    ErrRec* __restrict__ err, uint64_t base) {
   using C = typename Cplx<Real>::T;
-  using S = TileShape<L, SC, TILE, Real>;
+  constexpr int WSL = wide_bin_slots<Real>();
+  using S = TileShape<L, SC, TILE, Real, WSL>;
   __shared__ PointRec<Real> s_rec[TILE];
   // wide rows: the phase table of the node-ordered Gamma sums instead
   constexpr bool kWide = L == LAYOUT_WIDE;
@@ -409,113 +414,97 @@ __global__ __launch_bounds__(TILE) void k_bin_sums(GridConst g, DataConst d, Pro
     s_tried = 0;
     s_verified = 0;
   }
-  // wide rows, kWideAtom: the located points without a table block are
-  // listed in rest[0 .. *rest_n) (record indices) for the kWideRest launch,
-  // which takes its points from that list
-  constexpr bool kAtom = L == LAYOUT_WIDE && SC == kWideAtom;
-  constexpr bool kRest = L == LAYOUT_WIDE && SC == kWideRest;
-  if constexpr (kRest) n = min(n, *rest_n);
-  // kWideRest: a few blocks (the launch has no count of the list) walk the
-  // listed points tile by tile; every other launch has one tile per block
-  const uint32_t first_tile = kRest ? blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
-  for (uint32_t tile = first_tile; (uint64_t)tile * TILE < n; tile += gridDim.x) {
-    if (tile != first_tile) __syncthreads();  // the previous tile's records are read
-    const uint32_t tile0 = tile * TILE;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t p = tile0 + tid;
-    // wide rows: blockIdx.y picks a group of modes (gridDim.y groups; the
-    // first one reports the points' errors and aux outputs)
-    const bool lead = blockIdx.y == 0;
-    const uint32_t per_group = (d.B + gridDim.y - 1) / gridDim.y;
-    const uint32_t b_lo = blockIdx.y * per_group, b_hi = b_lo + per_group;
-    const bool want_phase = d.vec_rot == BRILLE_ROT_GAMMA && d.ec[1] > 0;
-    const uint32_t n_atoms = d.ec[1] / 3u;
-    const bool ph_in_lds = L == LAYOUT_GAMMA || (want_phase && n_atoms <= 4);
-    WideGammaLds<Real> wg;
-    if (kWide && want_phase) {
-      wg.ph = s_ph;
-      wg.rot = s_wrot;
-      wg.dst = s_wdst;
-      wg.cap = kPh;
-      wide_gamma_ops<Real, TILE>(g, d, wg);
-    }
-    __shared__ uint32_t s_wave_tab[TILE / 64];
-    if (Prop) __syncthreads();
-    const bool live = p < n;
-    SortRec sr;
-    Located P;
-    P.status = BRILLE_PT_OK;
-    P.cube = kNoCube;
-    uint32_t ridx = 0;
-    if (live) {
-      ridx = kRest ? rest[p] : (perm[p] & ~kPermPoly);
-      sr = srt[ridx];
-      P.q[0] = sr.q[0]; P.q[1] = sr.q[1]; P.q[2] = sr.q[2];
-      P.tau[0] = P.tau[1] = P.tau[2] = 0;
-      P.node = sr.node;
-      P.rot = sr.meta & 255u;
-      P.invrot = (sr.meta >> 8) & 255u;
-      P.status = (int)meta_status(sr.meta);
-      P.tet = kNoTet;
-      P.nslot = 0;
-      P.nkept = 0;
-      if (P.status == BRILLE_PT_OK) {
-        if constexpr (Prop) {
-          bool verified = false;
-          node_slots(g, P, sr.hint, pc.margin, &verified);
-          if (sr.hint != kNoTet) {
-            atomicAdd(&s_tried, 1u);
-            if (verified) atomicAdd(&s_verified, 1u);
-          }
-        } else {
-          node_slots(g, P);
-        }
-        // failed fold-ins were reported by k_bin_fold
-        if (P.status != BRILLE_PT_OK && lead) report_point(err, base + sr.index, P.status);
-        if (kAtom && lead && P.status == BRILLE_PT_OK && table_row(d, P) == kNoCube) rest[atomicAdd(rest_n, 1u)] = ridx;
-      }
-    }
-    // Stable partition of the tile: points the cube factor table serves first,
-    // so that few waves of the sums mix the two kinds of point.
-    const bool table = (L == LAYOUT_GAMMA || L == LAYOUT_SCALAR) && cube_rows<Real>(d) != nullptr;
-    const bool tab = table && live && P.status == BRILLE_PT_OK && table_row(d, P) != kNoCube;
-    const uint32_t lane = tid & 63u, wave = tid >> 6;
-    const unsigned long long bal = __ballot(tab);
-    const uint32_t rank = (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-    if (lane == 0) s_wave_tab[wave] = (uint32_t)__popcll(bal);
-    __syncthreads();
-    uint32_t before = 0, n_tab = 0;
-  #pragma unroll
-    for (uint32_t w = 0; w < TILE / 64; ++w) {
-      const uint32_t c = s_wave_tab[w];
-      before += w < wave ? c : 0u;
-      n_tab += c;
-    }
-    const uint32_t slot = tab ? before + rank : n_tab + (tid - before - rank);
-    {
-      PointRec<Real>& r = s_rec[slot];
-      r.nslot = 0;
-      if (live) {
-        s_out[slot] = sr.index;
-        if (P.status == BRILLE_PT_OK)
-          store_record<Real, L, SC>(g, d, P, r, s_ph, s_q, slot, ph_in_lds, n_atoms, !kOpFrames);
-        if (lead && !kRest) write_aux(aux, sr.index, P);
-      }
-    }
-    __syncthreads();
-    if (Prop && lead && threadIdx.x == 0 && s_tried) {
-      atomicAdd(&pc.stats[0], (unsigned long long)s_tried);
-      atomicAdd(&pc.stats[1], (unsigned long long)s_verified);
-    }
-    const uint32_t npts = n - tile0 < (uint32_t)TILE ? n - tile0 : (uint32_t)TILE;
-    // the one-lane-per-unit sums see only the points the table does not serve:
-    // fewer rows in flight keep the registers for occupancy
-    constexpr int GRP = sizeof(Real) == 4 ? 2 : 1;
-    tile_sums<Real, true, L, SC, SV, TILE, GRP>(g, d, s_rec, s_ph, s_q, s_out, 0, npts, ph_in_lds, vals, vecs, s_wide,
-                                                table, n_tab, kOpFrames ? s_frames : nullptr, true, wg, b_lo, b_hi);
-
-    if (!kRest) break;
+  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t tile0 = tile * TILE;
+  const uint32_t tid = threadIdx.x;
+  const uint32_t p = tile0 + tid;
+  // wide rows: blockIdx.y picks a group of modes (gridDim.y groups; the
+  // first one reports the points' errors and aux outputs)
+  const bool lead = blockIdx.y == 0;
+  const uint32_t per_group = (d.B + gridDim.y - 1) / gridDim.y;
+  const uint32_t b_lo = blockIdx.y * per_group, b_hi = b_lo + per_group;
+  const bool want_phase = d.vec_rot == BRILLE_ROT_GAMMA && d.ec[1] > 0;
+  const uint32_t n_atoms = d.ec[1] / 3u;
+  const bool ph_in_lds = L == LAYOUT_GAMMA || (want_phase && n_atoms <= 4);
+  WideGammaLds<Real> wg;
+  if (kWide && want_phase) {
+    wg.ph = s_ph;
+    wg.rot = s_wrot;
+    wg.dst = s_wdst;
+    wg.cap = kPh;
+    wide_gamma_ops<Real, TILE>(g, d, wg);
   }
+  __shared__ uint32_t s_wave_tab[TILE / 64];
+  if (Prop) __syncthreads();
+  const bool live = p < n;
+  SortRec sr;
+  Located P;
+  P.status = BRILLE_PT_OK;
+  P.cube = kNoCube;
+  if (live) {
+    sr = srt[perm[p] & ~kPermPoly];
+    P.q[0] = sr.q[0]; P.q[1] = sr.q[1]; P.q[2] = sr.q[2];
+    P.tau[0] = P.tau[1] = P.tau[2] = 0;
+    P.node = sr.node;
+    P.rot = sr.meta & 255u;
+    P.invrot = (sr.meta >> 8) & 255u;
+    P.status = (int)meta_status(sr.meta);
+    P.tet = kNoTet;
+    P.nslot = 0;
+    P.nkept = 0;
+    if (P.status == BRILLE_PT_OK) {
+      if constexpr (Prop) {
+        bool verified = false;
+        node_slots(g, P, sr.hint, pc.margin, &verified);
+        if (sr.hint != kNoTet) {
+          atomicAdd(&s_tried, 1u);
+          if (verified) atomicAdd(&s_verified, 1u);
+        }
+      } else {
+        node_slots(g, P);
+      }
+      // failed fold-ins were reported by k_bin_fold
+      if (P.status != BRILLE_PT_OK && lead) report_point(err, base + sr.index, P.status);
+    }
+  }
+  // Stable partition of the tile: points the cube factor table serves first,
+  // so that few waves of the sums mix the two kinds of point.
+  const bool table = (L == LAYOUT_GAMMA || L == LAYOUT_SCALAR) && cube_rows<Real>(d) != nullptr;
+  const bool tab = table && live && P.status == BRILLE_PT_OK && table_row(d, P) != kNoCube;
+  const uint32_t lane = tid & 63u, wave = tid >> 6;
+  const unsigned long long bal = __ballot(tab);
+  const uint32_t rank = (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
+  if (lane == 0) s_wave_tab[wave] = (uint32_t)__popcll(bal);
+  __syncthreads();
+  uint32_t before = 0, n_tab = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < TILE / 64; ++w) {
+    const uint32_t c = s_wave_tab[w];
+    before += w < wave ? c : 0u;
+    n_tab += c;
+  }
+  const uint32_t slot = tab ? before + rank : n_tab + (tid - before - rank);
+  {
+    PointRec<Real>& r = s_rec[slot];
+    r.nslot = 0;
+    if (live) {
+      s_out[slot] = sr.index;
+      if (P.status == BRILLE_PT_OK)
+        store_record<Real, L, SC>(g, d, P, r, s_ph, s_q, slot, ph_in_lds, n_atoms, !kOpFrames);
+      if (lead) write_aux(aux, sr.index, P);
+    }
+  }
+  __syncthreads();
+  if (Prop && lead && threadIdx.x == 0 && s_tried) {
+    atomicAdd(&pc.stats[0], (unsigned long long)s_tried);
+    atomicAdd(&pc.stats[1], (unsigned long long)s_verified);
+  }
+  const uint32_t npts = n - tile0 < (uint32_t)TILE ? n - tile0 : (uint32_t)TILE;
+  // the one-lane-per-unit sums see only the points the table does not serve:
+  // fewer rows in flight keep the registers for occupancy
+  constexpr int GRP = sizeof(Real) == 4 ? 2 : 1;
+  tile_sums<Real, true, L, SC, SV, TILE, GRP, WSL>(g, d, s_rec, s_ph, s_q, s_out, 0, npts, ph_in_lds, vals, vecs, s_wide,
+                                              table, n_tab, kOpFrames ? s_frames : nullptr, true, wg, b_lo, b_hi);
 }
 
 // The row table: thread t = (block row, mode b) phases the row of a cube's or
@@ -600,16 +589,45 @@ __global__ __launch_bounds__(256) void k_wide_factors(GridConst g, DataConst d, 
   }
 }
 
-using SumsKernel = void (*)(GridConst, DataConst, ProposalConst, const SortRec*, const uint32_t*, uint32_t, void*,
-                           void*, brille_aux_out, ErrRec*, uint64_t, uint32_t*, uint32_t*);
-
-// Gamma rows too long for one lane that the atom-major walk takes whole: the
-// derived antiphase factor table exists and there is at most one value per atom
-static bool wide_by_atom(const DataConst& d, int precision) {
-  const bool fac = precision == BRILLE_FP32 ? d.wide_fac32 != nullptr : d.wide_fac64 != nullptr;
-  return payload_layout(d) == LAYOUT_GAMMA && d.vec_rot == BRILLE_ROT_GAMMA && d.ec[1] > 0 && fac &&
-         d.sv <= d.sc / 3u;
+// The same for Gamma rows summed atom-major: a wave forms the factors of the
+// mpw modes of one pass of a block (wide_atom_antiphases, as the sums do).
+template <typename Real>
+__global__ __launch_bounds__(256) void k_wide_atom_factors(GridConst g, DataConst d, uint64_t n_cube_units,
+                                                           uint64_t n_units, typename Cplx<Real>::T* out) {
+  using C = typename Cplx<Real>::T;
+  constexpr int SL = wide_bin_slots<Real>();
+  __shared__ C s_lds[4 * wide_atom_slice<Real>(SL)];
+  const uint64_t t = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t >= n_units) return;  // wave-uniform; no block-wide barrier follows
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t na = d.sc / 3u, mpw = 64u / na, passes = (d.B + mpw - 1) / mpw;
+  const uint32_t m = lane / na, a = lane - m * na;
+  const bool cube = t < n_cube_units;
+  const uint64_t u = cube ? t : t - n_cube_units;
+  const uint64_t c = u / passes;
+  const uint32_t b = (uint32_t)(u - c * passes) * mpw + m;
+  const bool on = m < mpw && b < d.B;
+  const uint32_t ns = cube ? 8u : 4u;
+  const uint64_t trow = cube ? c * 8 * d.B : d.tab_tet_row + c * 4 * d.B;
+  C v[8][3], e[8];
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    const bool use = on && x < (int)ns;
+    const uint32_t vert = cube ? g.cube_v[8 * c + 7 - x] : g.tet_v[4 * c + (x & 3)];
+    const C* rc = reinterpret_cast<const C*>(row_at<Real>(d, vert, on ? b : 0u)) + 3u * a;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[x][i] = use ? rc[i] : Elem<C>::zero();
+  }
+  wide_atom_antiphases<Real, SL>(v[0], v, ns, na, mpw, m, e, s_lds + (threadIdx.x >> 6) * wide_atom_slice<Real>(SL));
+  if (on && a == 0) {
+#pragma unroll
+    for (int x = 0; x < 8; ++x)
+      if ((uint32_t)x < ns) out[trow + (uint64_t)x * d.B + b] = e[x];
+  }
 }
+
+using SumsKernel = void (*)(GridConst, DataConst, ProposalConst, const SortRec*, const uint32_t*, uint32_t, void*,
+                           void*, brille_aux_out, ErrRec*, uint64_t);
 
 template <typename Real>
 static SumsKernel pick_sums(const DataConst& d, bool prop) {
@@ -637,9 +655,8 @@ static SumsKernel pick_sums(const DataConst& d, bool prop) {
       default: break;
     }
   }
-  if (wide_rows(d))
-    return wide_by_atom(d, sizeof(Real) == 4 ? BRILLE_FP32 : BRILLE_FP64) ? k_bin_sums<Real, LAYOUT_WIDE, kWideAtom, 0, false>
-                                                                         : k_bin_sums<Real, LAYOUT_WIDE, kWideAll, 0, false>;
+  if (wide_by_atom(d)) return k_bin_sums<Real, LAYOUT_WIDE, kWideAtom, 0, false>;
+  if (wide_rows(d)) return k_bin_sums<Real, LAYOUT_WIDE, kWideAll, 0, false>;
   return k_bin_sums<Real, LAYOUT_GENERIC, 0, 0, false>;
 }
 
@@ -702,15 +719,22 @@ template <typename Real>
 static int build_wide_factors(brille_grid* G, hipStream_t s, typename Cplx<Real>::T** out) {
   using C = typename Cplx<Real>::T;
   const DataConst& d = G->d;
-  const uint64_t cube_units = G->n_cubes * d.B;
-  const uint64_t units = cube_units + G->n_tets * d.B;
+  const bool atom = wide_by_atom(d);
+  const uint64_t mpw = 64u / (d.sc / 3u);
+  const uint64_t per = atom ? (d.B + mpw - 1) / mpw : d.B;  // waves per block
+  const uint64_t cube_units = G->n_cubes * per;
+  const uint64_t units = cube_units + G->n_tets * per;
   void* p = nullptr;
   if (hipMalloc(&p, (G->n_cubes * 8 + G->n_tets * 4) * d.B * sizeof(C)) != hipSuccess)
     return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the wide factor table");
   G->data_allocs.push_back(p);
   C* t = static_cast<C*>(p);
-  hipLaunchKernelGGL((k_wide_factors<Real>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, G->g, d, cube_units,
-                     units, t);
+  if (atom)
+    hipLaunchKernelGGL((k_wide_atom_factors<Real>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, G->g, d,
+                       cube_units, units, t);
+  else
+    hipLaunchKernelGGL((k_wide_factors<Real>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, G->g, d, cube_units,
+                       units, t);
   if (hipGetLastError() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "wide factor table launch failed");
   *out = t;
   return BRILLE_OK;
@@ -759,22 +783,6 @@ int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s) {
   const int rc = build_cube_rows<double>(G, s, &t);
   if (rc == BRILLE_OK) d.cube_rows64 = t;
   return rc;
-}
-
-// the aux outputs of a pass that starts at point c0
-static brille_aux_out offset_aux(const brille_aux_out& x, uint64_t c0) {
-  brille_aux_out o = x;
-  if (o.ir_q) o.ir_q += 3 * c0;
-  if (o.tau) o.tau += 3 * c0;
-  if (o.rot) o.rot += c0;
-  if (o.invrot) o.invrot += c0;
-  if (o.node) o.node += c0;
-  if (o.tet) o.tet += c0;
-  if (o.n_iw) o.n_iw += c0;
-  if (o.iw_index) o.iw_index += 8 * c0;
-  if (o.iw_weight) o.iw_weight += 8 * c0;
-  if (o.status) o.status += c0;
-  return o;
 }
 
 // Buckets of at most kNodesPerBucket trellis nodes: k_bucket_perm orders each
@@ -975,9 +983,6 @@ int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStr
     if (stage_ms) (void)hipEventRecord(tev[k * 5 + j], st);
   };
   const SumsKernel sums = precision == BRILLE_FP32 ? pick_sums<float>(G->d, prop) : pick_sums<double>(G->d, prop);
-  const bool by_atom = !prop && wide_rows(G->d) && wide_by_atom(G->d, precision);
-  const SumsKernel rest_sums = precision == BRILLE_FP32 ? k_bin_sums<float, LAYOUT_WIDE, kWideRest, 0, false>
-                                                        : k_bin_sums<double, LAYOUT_WIDE, kWideRest, 0, false>;
   const size_t rs = precision == BRILLE_FP32 ? 4 : 8;
   const size_t vb = (size_t)G->d.B * G->d.sv * rs, cb = (size_t)G->d.B * G->d.sc * 2 * rs;
   const size_t lds1 = (size_t)(nb + 1) * 4;
@@ -1024,15 +1029,9 @@ int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStr
     // sums of pass k on the call stream
     mark(k, 3, s);
     const dim3 sgrid((m + TILE - 1) / TILE, sum_groups(G, m, prop));
-    if (by_atom) zero_words(b.pcount, 1, s);
     hipLaunchKernelGGL(sums, sgrid, dim3(TILE), 0, s, G->g, G->d, a.prop, b.srt, b.perm, m,
                        static_cast<char*>(a.vals) + c0 * vb, static_cast<char*>(a.vecs) + c0 * cb,
-                       offset_aux(a.aux, c0), a.err, a.base + c0, b.plist, b.pcount);
-    if (by_atom)  // the listed points without a table block: one block per CU at most
-      hipLaunchKernelGGL(rest_sums, dim3(std::min<uint32_t>(sgrid.x, std::max<uint32_t>(G->n_cu, 1)), sgrid.y),
-                         dim3(TILE), 0, s, G->g, G->d, a.prop, b.srt, b.perm, m,
-                         static_cast<char*>(a.vals) + c0 * vb, static_cast<char*>(a.vecs) + c0 * cb,
-                         offset_aux(a.aux, c0), a.err, a.base + c0, b.plist, b.pcount);
+                       offset_aux(a.aux, c0), a.err, a.base + c0);
     mark(k, 4, s);
     if (halves > 1) (void)hipEventRecord(G->bin_ev[EV_DONE + h], s);
   }

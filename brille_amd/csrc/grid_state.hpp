@@ -91,6 +91,22 @@ int check_payload_precision(const brille_grid* G, int precision);
 void launch_tile(const brille_grid* G, const LaunchArgs& a, int precision, bool fast, hipStream_t s);
 int payload_layout(const DataConst& d);
 bool wide_rows(const DataConst& d);
+bool wide_by_atom(const DataConst& d);
+// the aux outputs of a part of a call that starts at point c0
+inline brille_aux_out offset_aux(const brille_aux_out& x, uint64_t c0) {
+  brille_aux_out o = x;
+  if (o.ir_q) o.ir_q += 3 * c0;
+  if (o.tau) o.tau += 3 * c0;
+  if (o.rot) o.rot += c0;
+  if (o.invrot) o.invrot += c0;
+  if (o.node) o.node += c0;
+  if (o.tet) o.tet += c0;
+  if (o.n_iw) o.n_iw += c0;
+  if (o.iw_index) o.iw_index += 8 * c0;
+  if (o.iw_weight) o.iw_weight += 8 * c0;
+  if (o.status) o.status += c0;
+  return o;
+}
 // binned pipeline (binned.hip)
 bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel);
 int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms);

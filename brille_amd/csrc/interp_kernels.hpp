@@ -850,30 +850,38 @@ enum Layout : int {
 };
 constexpr uint32_t kWideMax = 128;  // complex elements per row the wide phase 2 handles (two per lane)
 constexpr uint32_t kWideAtoms = kWideMax / 3;  // atoms of the longest wide Gamma row
-// SC of the node-ordered wide sums (LAYOUT_WIDE): every point (kWideAll);
-// only the atom-major walk, the points without a table block listed for a
-// second launch (kWideAtom); that second launch over the listed points
-// (kWideRest)
-constexpr int kWideAll = 0, kWideAtom = 1, kWideRest = 2;
+// SC of the wide sums (LAYOUT_WIDE): rows summed a wave per (point, mode)
+// (kWideAll: scalar rows, or more values than atoms), or atom-major
+// (kWideAtom: Gamma rows of at most one value per atom)
+constexpr int kWideAll = 0, kWideAtom = 1;
 // LDS of the node-ordered wide sums' Gamma table: per-point phases of a chunk
 // of the tile's points, every atom (FP32: 4608 complex, 192 points of 24
 // atoms).  Those sums hold over 200 VGPRs, so two blocks per CU is their
 // occupancy with or without it.
 constexpr uint32_t kWidePhaseBytes = 36864;
-// the same for the atom-only sums (kWideAtom below), whose 109 VGPRs allow
-// four waves per SIMD when a block's LDS stays under 40 KB: 8 KB, 42 points
-// of 24 atoms per chunk (with 36 KB, two waves: about 12 % slower)
-constexpr uint32_t kWideAtomPhaseBytes = 8192;
-
-__device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+// the same for the atom-major sums (kWideAtom), whose registers allow four
+// waves per SIMD when a block's LDS stays under 40 KB: 34 points of 24 atoms
+// per chunk (with 36 KB, two waves: about 12 % slower)
+constexpr uint32_t kWideAtomPhaseBytes = 6656;
+// modes a wave sums at once in the atom-major walk: wide Gamma rows have at
+// least five atoms
+constexpr uint32_t kWideModesMax = 64 / 5;
+// LDS of one wave's antiphases in the atom-major walk, SL slots at a time:
+// per slot and lane the terms of the Hermitian product (one complex in FP32,
+// three in FP64), then the factors of the wave's modes
+template <typename Real>
+constexpr uint32_t wide_atom_slice(int sl) {
+  return (uint32_t)sl * (sizeof(Real) == 4 ? 64u : 192u) + (uint32_t)sl * kWideModesMax;
 }
-__device__ __forceinline__ double wave_sum_f(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+// slots at a time: the tile kernels take more (shorter chains of LDS
+// exchanges in small calls), the node-ordered sums fewer (four blocks per CU)
+template <typename Real>
+constexpr int wide_tile_slots() {
+  return sizeof(Real) == 4 ? 4 : 2;
+}
+template <typename Real>
+constexpr int wide_bin_slots() {
+  return 1;
 }
 
 // the wide factor table of a precision (antiphase of every slot row against
@@ -952,6 +960,173 @@ __device__ __forceinline__ void wide_antiphases(typename Cplx<Real>::T p0, typen
       }
 #pragma unroll
     for (int x = 0; x < NS; ++x) e[x] = antiphase_closed<Real>(re[x], im[x]);
+  }
+}
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Antiphases of the atom-major walk: lane l holds atom a = l % na of mode
+// m = l / na of the wave's mpw modes, v[x] the atom's three elements of the
+// slot-x rows and p those of the pivot row.  e[x] becomes the antiphase of the
+// lane's mode in slot x (1 from nslot on).  Every lane of the wave calls it;
+// lanes without a mode hold zeros.  One definition for the sums and for the
+// factor table, so both give the same bits.
+//
+// The terms go through LDS (SL slots at a time): one lane per (slot, mode)
+// adds them up, so a product costs a few LDS reads instead of a reduction of
+// sixteen values across the wave per mode.  FP32 adds an atom's three terms
+// in its lane and then the atoms in four interleaved sums, (s0 + s1) + (s2 +
+// s3); FP64 keeps the reference's order (src/utilities.tpp:567-577: one term
+// per element, added to the running sum element by element): where two modes
+// are degenerate their overlap is rounding noise around zero, and its
+// antiphase is then decided by the exact order of the additions.
+template <typename Real, int SL>
+__device__ __forceinline__ void wide_atom_antiphases(const typename Cplx<Real>::T* p,
+                                                     const typename Cplx<Real>::T (*v)[3], uint32_t nslot,
+                                                     uint32_t na, uint32_t mpw, uint32_t m, typename Cplx<Real>::T* e,
+                                                     typename Cplx<Real>::T* lds) {
+  using C = typename Cplx<Real>::T;
+  constexpr uint32_t T = sizeof(Real) == 4 ? 1 : 3;  // terms a lane puts down per slot
+  const uint32_t lane = threadIdx.x & 63u;
+  C* fac = lds + SL * T * 64;
+#pragma unroll
+  for (int x0 = 0; x0 < 8; x0 += SL) {
+    if ((uint32_t)x0 >= nslot) {  // wave-uniform
+#pragma unroll
+      for (int x = 0; x < SL; ++x) e[x0 + x] = C{(Real)1, (Real)0};
+      continue;
+    }
+#pragma unroll
+    for (int x = 0; x < SL; ++x) {
+      C t[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const C w = v[x0 + x][i];
+        t[i].x = p[i].x * w.x + p[i].y * w.y;
+        t[i].y = p[i].x * w.y - p[i].y * w.x;
+      }
+      if constexpr (T == 1) {
+        lds[x * 64 + lane] = Elem<C>::add(Elem<C>::add(t[0], t[1]), t[2]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) lds[(x * 3 + i) * 64 + lane] = t[i];
+      }
+    }
+    wave_lds_fence();
+    for (uint32_t k = lane; k < (uint32_t)SL * mpw; k += 64) {
+      const uint32_t x = k / mpw, mm = k - x * mpw;
+      const C* t = lds + x * T * 64 + mm * na;
+      C z = Elem<C>::zero();
+      if constexpr (T == 1) {
+        C s[4] = {z, z, z, z};
+        uint32_t a = 0;
+        for (; a + 4 <= na; a += 4)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) s[j] = Elem<C>::add(s[j], t[a + j]);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (a + j < na) s[j] = Elem<C>::add(s[j], t[a + j]);
+        z = Elem<C>::add(Elem<C>::add(s[0], s[1]), Elem<C>::add(s[2], s[3]));
+      } else {
+#pragma unroll 4
+        for (uint32_t a = 0; a < na; ++a)
+#pragma unroll
+          for (int i = 0; i < 3; ++i) z = Elem<C>::add(z, t[i * 64 + a]);
+      }
+      fac[k] = antiphase_closed<Real>(z.x, z.y);
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int x = 0; x < SL; ++x) e[x0 + x] = m < mpw ? fac[x * mpw + m] : C{(Real)1, (Real)0};
+  }
+}
+
+// The slot rows of one lane of the atom-major walk: the three elements of its
+// atom a of mode b in each slot's row (vv: value a), zeros for lanes that are
+// off, and from the fifth on for a tetrahedron, whose four slots are all
+template <typename Real>
+__device__ __forceinline__ void wide_atom_load(const DataConst& d, const PointRec<Real>& r, uint32_t b, uint32_t a,
+                                               bool on, typename Cplx<Real>::T (*v)[3], Real* vv) {
+  using C = typename Cplx<Real>::T;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    const Real* rw = row_at<Real>(d, r.idx[x], on ? b : 0u);
+    const C* rc = reinterpret_cast<const C*>(rw) + 3u * a;
+    const bool use = on && x < (int)r.nslot;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[x][i] = use ? rc[i] : Elem<C>::zero();
+    vv[x] = use && a < d.sv ? rw[2 * d.sc + a] : (Real)0;
+  }
+}
+
+// ... and those rows multiplied by their antiphases in place: factors from
+// the table for a point with a block there, else formed here (whole wave)
+template <typename Real, int SL>
+__device__ __forceinline__ void wide_atom_phase(const DataConst& d, const PointRec<Real>& r, uint32_t b, uint32_t na,
+                                                uint32_t mpw, uint32_t m, bool on, const typename Cplx<Real>::T* fac,
+                                                typename Cplx<Real>::T (*v)[3], typename Cplx<Real>::T* lds) {
+  using C = typename Cplx<Real>::T;
+  C e[8];
+  if (fac && r.trow != kNoCube) {
+#pragma unroll
+    for (int x = 0; x < 8; ++x)
+      e[x] = on && x < (int)r.nslot ? fac[r.trow + (uint32_t)x * d.B + b] : C{(Real)1, (Real)0};
+  } else {
+    C p[3] = {Elem<C>::zero(), Elem<C>::zero(), Elem<C>::zero()};
+#pragma unroll
+    for (int x = 7; x >= 0; --x)
+      if (x < (int)r.nslot && r.idx[x] == r.pivot)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) p[i] = v[x][i];
+    wide_atom_antiphases<Real, SL>(p, v, r.nslot, na, mpw, m, e, lds);
+  }
+#pragma unroll
+  for (int x = 0; x < 8; ++x)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const C el = v[x][i];
+      phase_elem<Real>(e[x], el.x, el.y, &v[x][i].x, &v[x][i].y);
+    }
+}
+
+// the weighted sums of a lane's atom from its antiphased rows
+template <typename Real>
+__device__ __forceinline__ void wide_atom_sum(const PointRec<Real>& r, const typename Cplx<Real>::T (*v)[3],
+                                              const Real* vv, typename Cplx<Real>::T* acc, Real* va) {
+  using C = typename Cplx<Real>::T;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) acc[i] = Elem<C>::zero();
+  *va = 0;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    const Real wx = r.w[x];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      acc[i].x = fma_r(wx, v[x][i].x, acc[i].x);
+      acc[i].y = fma_r(wx, v[x][i].y, acc[i].y);
+    }
+    *va = fma_r(wx, vv[x], *va);
+  }
+}
+
+// rip_gamma_complex  src/interpolator_gamma.tpp:100-114 of one atom: R times
+// the accumulated 3-vector, times the atom's phase, to the output atom
+template <typename Real>
+__device__ __forceinline__ void wide_atom_store(const typename Cplx<Real>::T* acc, const Real* R,
+                                                typename Cplx<Real>::T ph, typename Cplx<Real>::T* dst) {
+  using C = typename Cplx<Real>::T;
+  typedef Real real2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    C tt = Elem<C>::zero();
+#pragma unroll
+    for (int j = 0; j < 3; ++j) tt = Elem<C>::add(tt, Elem<C>::scale(acc[j], R[3 * i + j]));
+    const C o = cmul(ph, tt);
+    __builtin_nontemporal_store(real2{o.x, o.y}, reinterpret_cast<real2*>(dst + i));
   }
 }
 
@@ -1152,6 +1327,7 @@ struct LaunchArgs {
   ErrRec* err;
   int fold;  // Fold
   int use_proposal;
+  uint32_t tile;  // points per block of the fused kernel (at most tile_capacity)
   ProposalConst prop;
 };
 
@@ -1284,13 +1460,15 @@ __device__ inline void write_aux(const brille_aux_out& aux, uint64_t p, const Lo
 // compile-time row sizes of the specialised layouts (ignored by
 // LAYOUT_GENERIC).
 
-template <int L, int SC, int TB = TILE, typename Real = double>
+template <int L, int SC, int TB = TILE, typename Real = double, int WSL = wide_tile_slots<Real>()>
 struct TileShape {
   static constexpr int NPH = L == LAYOUT_GAMMA ? SC / 3 : (L == LAYOUT_GENERIC ? 4 : 1);  // phases per point
   // per-point side data in s_q: q (general and wide layouts) or the GammaFrame
   static constexpr int NQ = (L == LAYOUT_GENERIC || L == LAYOUT_WIDE) ? 3 * TB
                             : (L == LAYOUT_GAMMA ? frame_words<Real>() * TB : 1);
-  static constexpr int NW = L == LAYOUT_WIDE ? (TB / 64) * (int)kWideMax : 1;              // wide-row slices
+  // wide-row slices, one per wave
+  static constexpr int NW =
+      L == LAYOUT_WIDE ? (TB / 64) * (int)(SC == kWideAtom ? wide_atom_slice<Real>(WSL) : kWideMax) : 1;
 };
 
 // The row-table block of a point: cube c's eight slots at rows c * 8 * B, the
@@ -1364,7 +1542,9 @@ __device__ __forceinline__ void store_record(const GridConst& g, const DataConst
 // overrides the rows the one-pass sums keep in flight (0: their default)
 // table: the cube factor table is built; its points are the first n_coop
 // records, summed by unit_coop where the rows allow it
-template <typename Real, bool Fast, int L, int SC, int SV, int TB = TILE, int GRP = 0>
+// WSL: the slots whose antiphases the atom-major wide sums form at a time
+template <typename Real, bool Fast, int L, int SC, int SV, int TB = TILE, int GRP = 0,
+          int WSL = wide_tile_slots<Real>()>
 __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d, const PointRec<Real>* s_rec,
                                           const typename Cplx<Real>::T* s_ph, const double* s_q,
                                           const uint32_t* out_row, uint64_t row0, uint32_t npts, bool ph_in_lds,
@@ -1382,107 +1562,135 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
   if constexpr (L == LAYOUT_WIDE) {
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const bool gamma = d.vec_rot == BRILLE_ROT_GAMMA && d.ec[1] > 0;
-    C* lds = s_wide + wave * kWideMax;
-    WideCache<Real> wc;
-    const bool two = d.sc > 64;
     const bool tab = wide_factors<Real>(d) != nullptr;
-    if (!node_order && gamma && tab && d.sv <= d.sc / 3u) {
-      // Point-major, atom-major (Gamma rows with the factor table): wave w
-      // takes units w, w + TB/64, ... of (point, pass), a pass being 64 /
-      // n_atoms modes with a lane per (mode, atom) as in the node-ordered
-      // walk below; the wave keeps the point's phase, rotation rows and
-      // output atom while it stays on the point.  Points without a table
-      // block take the wave-per-unit sums for the pass's modes.
+    const uint32_t b_end = b_hi < B ? b_hi : B;
+    if constexpr (SC == kWideAtom) {
+      // Atom-major (Gamma rows of at most one value per atom): lane l takes
+      // atom a = l % na of mode l / na, so a wave sums mpw = 64 / na modes of a
+      // point at once (a "pass"), each lane its atom's three elements: the
+      // rotation needs no exchange between lanes.  Points with a block in the
+      // factor table take their antiphases there, the others form them.
+      constexpr int SL = WSL;
+      C* lds = s_wide + wave * wide_atom_slice<Real>(SL);
       const uint32_t na = d.sc / 3u, sc = d.sc, sv = d.sv;
       const uint32_t mpw = 64u / na;
       const uint32_t m = lane / na, a = lane - m * na;
-      const uint32_t passes = (B + mpw - 1) / mpw;
+      const uint32_t nmodes = b_end > b_lo ? b_end - b_lo : 0u;
+      const uint32_t passes = (nmodes + mpw - 1) / mpw;
       const C* fac = wide_factors<Real>(d);
-      uint32_t last = 0xFFFFFFFFu;
-      C ph = Elem<C>::zero();
-      Real R[9];
-      uint32_t dsta = 0;
-      for (uint32_t c = wave; c < npts * passes; c += TB / 64) {
-        const uint32_t pl = c / passes, t = c - pl * passes;
-        const PointRec<Real>& r = s_rec[pl];
-        const uint64_t row = ((out_row ? (uint64_t)out_row[pl] : row0 + pl)) * B;
-        if (r.nslot == 0 || r.trow == kNoCube) {
-          Real* ovp = vals + row * sv;
-          C* ocp = vecs + row * sc;
-          const uint32_t bend = (t + 1) * mpw < B ? (t + 1) * mpw : B;
-          for (uint32_t b = t * mpw; b < bend; ++b) {
-            if (r.nslot == 0) {
-              for (uint32_t e = lane; e < sv; e += 64) ovp[(uint64_t)b * sv + e] = 0;
-              for (uint32_t e = lane; e < sc; e += 64) ocp[(uint64_t)b * sc + e] = Elem<C>::zero();
-            } else if (two) {
-              unit_wide<Real, true>(g, d, r, s_q + 3 * pl, b, ovp, ocp, lds, gamma, cart, wc, true, tab);
-            } else {
-              unit_wide<Real, false>(g, d, r, s_q + 3 * pl, b, ovp, ocp, lds, gamma, cart, wc, true, tab);
+      auto zero_rows = [&](uint64_t row, uint32_t b) {
+        C* oc = vecs + row * sc + (uint64_t)b * sc;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) oc[3u * a + i] = Elem<C>::zero();
+        if (a < sv) vals[row * sv + (uint64_t)b * sv + a] = 0;
+      };
+      if (!node_order) {
+        // Point-major: wave w takes units w, w + TB/64, ... of (point, pass) and
+        // keeps the point's phase, rotation rows and output atom while it
+        // stays on the point.
+        uint32_t last = 0xFFFFFFFFu;
+        C ph = Elem<C>::zero();
+        Real R[9];
+        uint32_t dsta = 0;
+        for (uint32_t c = wave; c < npts * passes; c += TB / 64) {
+          const uint32_t pl = c / passes, t = c - pl * passes;
+          const PointRec<Real>& r = s_rec[pl];
+          const uint64_t row = ((out_row ? (uint64_t)out_row[pl] : row0 + pl)) * B;
+          const uint32_t b = b_lo + t * mpw + m;
+          const bool on = m < mpw && b < b_end;
+          if (r.nslot == 0) {
+            if (on) zero_rows(row, b);
+            continue;
+          }
+          C v[8][3], acc[3];
+          Real vv[8], va;
+          wide_atom_load<Real>(d, r, b, a, on, v, vv);
+          if (pl != last) {
+            last = pl;
+            if (m < mpw) {
+              ph = gamma_phase<Real>(d, s_q + 3 * pl, r.invrot, a);
+#pragma unroll
+              for (int k = 0; k < 9; ++k)
+                R[k] = cart ? (Real)d.cart_rot[9 * (uint64_t)r.invrot + k] : (Real)g.rot[9 * (uint64_t)r.invrot + k];
+              dsta = d.F0[a * d.gamma_ops + r.invrot];
             }
           }
-          continue;
+          wide_atom_phase<Real, SL>(d, r, b, na, mpw, m, on, fac, v, lds);
+          if (!on) continue;
+          wide_atom_sum<Real>(r, v, vv, acc, &va);
+          if (a < sv) __builtin_nontemporal_store(va, vals + row * sv + (uint64_t)b * sv + a);
+          wide_atom_store<Real>(acc, R, ph, vecs + row * sc + (uint64_t)b * sc + 3u * dsta);
         }
-        if (pl != last) {
-          last = pl;
-          if (m < mpw) {
-            ph = gamma_phase<Real>(d, s_q + 3 * pl, r.invrot, a);
-#pragma unroll
-            for (int k = 0; k < 9; ++k)
-              R[k] = cart ? (Real)d.cart_rot[9 * (uint64_t)r.invrot + k] : (Real)g.rot[9 * (uint64_t)r.invrot + k];
-            dsta = d.F0[a * d.gamma_ops + r.invrot];
+        return;
+      }
+      // Node-ordered: mode-major, wave w takes passes w, w + TB/64, ... and
+      // for each walks the tile's points in their node order, run by run
+      // (consecutive points of one table block, whose rows and factors are the
+      // same): the rows are loaded and antiphased once per run and stay
+      // loop-invariant over its points.  The points go in chunks whose Gamma
+      // phases the block first computes into LDS (once per point and atom
+      // instead of once per mode); the rotation rows and atom map come from
+      // per-operation LDS tables.
+      // (Staging a wave's rotated rows in LDS, to write them as one contiguous
+      // run per point instead of three 8-byte stores per lane at a permuted
+      // atom, saved no time: 64-grid batch of 1e7 points 140 -> 145 ms.)
+      const uint32_t chunk = wg.cap / na < npts ? wg.cap / na : npts;
+      for (uint32_t c0 = 0; c0 < npts; c0 += chunk) {
+        const uint32_t c1 = c0 + chunk < npts ? c0 + chunk : npts;
+        __syncthreads();  // the previous chunk's phases are read
+        for (uint32_t k = threadIdx.x; k < (c1 - c0) * na; k += TB) {
+          const uint32_t pl = c0 + k / na, ka = k - (k / na) * na;
+          const PointRec<Real>& r = s_rec[pl];
+          wg.ph[k] = r.nslot ? gamma_phase<Real>(d, s_q + 3 * pl, r.invrot, ka) : Elem<C>::zero();
+        }
+        __syncthreads();
+        for (uint32_t t = wave; t < passes; t += TB / 64) {
+          const uint32_t b = b_lo + t * mpw + m;
+          const bool on = m < mpw && b < b_end;
+          uint32_t p0 = c0;
+          while (true) {
+            while (p0 < c1 && s_rec[p0].nslot == 0) {
+              if (on) zero_rows(((out_row ? (uint64_t)out_row[p0] : row0 + p0)) * B, b);
+              ++p0;
+            }
+            if (p0 >= c1) break;
+            const PointRec<Real>& rb = s_rec[p0];
+            uint32_t p1 = p0 + 1;
+            if (rb.trow != kNoCube)
+              while (p1 < c1 && s_rec[p1].nslot != 0 && s_rec[p1].trow == rb.trow) ++p1;
+            C v[8][3];
+            Real vv[8];
+            wide_atom_load<Real>(d, rb, b, a, on, v, vv);
+            wide_atom_phase<Real, SL>(d, rb, b, na, mpw, m, on, fac, v, lds);
+            for (uint32_t pl = p0; pl < p1; ++pl) {
+              if (!on) continue;
+              const PointRec<Real>& r = s_rec[pl];
+              const uint64_t row = ((out_row ? (uint64_t)out_row[pl] : row0 + pl)) * B;
+              C acc[3];
+              Real va;
+              wide_atom_sum<Real>(r, v, vv, acc, &va);
+              if (a < sv) __builtin_nontemporal_store(va, vals + row * sv + (uint64_t)b * sv + a);
+              wide_atom_store<Real>(acc, wg.rot + 9u * r.invrot, wg.ph[(pl - c0) * na + a],
+                                    vecs + row * sc + (uint64_t)b * sc + 3u * wg.dst[r.invrot * na + a]);
+            }
+            p0 = p1;
           }
-        }
-        const uint32_t b = t * mpw + m;
-        if (m >= mpw || b >= B) continue;
-        C v[8][3];
-        Real vv[8];
-#pragma unroll
-        for (int x = 0; x < 8; ++x) {
-          const Real* rw = row_at<Real>(d, r.idx[x], b);
-          const C* rc = reinterpret_cast<const C*>(rw) + 3u * a;
-          const C e = x < (int)r.nslot ? fac[r.trow + (uint32_t)x * B + b] : C{(Real)1, (Real)0};
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            const C el = rc[i];
-            phase_elem<Real>(e, el.x, el.y, &v[x][i].x, &v[x][i].y);
-          }
-          vv[x] = a < sv ? rw[2 * sc + a] : (Real)0;
-        }
-        C acc[3] = {Elem<C>::zero(), Elem<C>::zero(), Elem<C>::zero()};
-        Real va = 0;
-#pragma unroll
-        for (int x = 0; x < 8; ++x) {
-          const Real wx = r.w[x];
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            acc[i].x = fma_r(wx, v[x][i].x, acc[i].x);
-            acc[i].y = fma_r(wx, v[x][i].y, acc[i].y);
-          }
-          va = fma_r(wx, vv[x], va);
-        }
-        if (a < sv) __builtin_nontemporal_store(va, vals + row * sv + (uint64_t)b * sv + a);
-        // rip_gamma_complex  src/interpolator_gamma.tpp:100-114, atom by atom
-        C* dst = vecs + row * sc + (uint64_t)b * sc + 3u * dsta;
-        typedef Real real2 __attribute__((ext_vector_type(2)));
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          C tt = Elem<C>::zero();
-#pragma unroll
-          for (int j = 0; j < 3; ++j) tt = Elem<C>::add(tt, Elem<C>::scale(acc[j], R[3 * i + j]));
-          const C o = cmul(ph, tt);
-          __builtin_nontemporal_store(real2{o.x, o.y}, reinterpret_cast<real2*>(dst + i));
         }
       }
       return;
     }
+    C* lds = s_wide + wave * kWideMax;
+    WideCache<Real> wc;
+    const bool two = d.sc > 64;
     if (!node_order) {
       // Point-major: wave w takes units w, w + TB/64, ... of (point, mode),
       // so it stays on a point for its share of the modes and keeps the
       // point's rotation data (a second mode in flight per wave doubled the
       // registers and made the 64-grid batch of 1e7 points slower, 466 -> 511 ms)
       uint32_t last = 0xFFFFFFFFu;
-      for (uint32_t c = wave; c < units; c += TB / 64) {
-        const uint32_t pl = c / B, b = c - pl * B;
+      const uint32_t nb = b_end > b_lo ? b_end - b_lo : 0u;
+      for (uint32_t c = wave; c < npts * nb; c += TB / 64) {
+        const uint32_t pl = c / nb, b = b_lo + (c - pl * nb);
         const PointRec<Real>& r = s_rec[pl];
         const uint64_t row = ((out_row ? (uint64_t)out_row[pl] : row0 + pl)) * B;
         Real* ov = vals + row * d.sv;
@@ -1510,117 +1718,13 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
     const bool pre = gamma && wg.ph != nullptr;
     const uint32_t na = d.sc / 3u;
     const uint32_t chunk = pre ? (wg.cap / na < npts ? wg.cap / na : npts) : npts;
-    const uint32_t b_end = b_hi < B ? b_hi : B;
-    // Atom-major (Gamma rows with the factor table and at most one value per
-    // atom): lane l takes atom a = l % na of mode l / na, so a wave sums
-    // 64 / na modes of a point at once, each lane its atom's three elements:
-    // the rotation needs no exchange between lanes.  Same per-element
-    // arithmetic as the wave-per-unit walk below, so the same bits.  Points
-    // without a table block are left to that walk.
-    // (Staging a wave's rotated rows in LDS, to write them as one contiguous
-    // run per point instead of three 8-byte stores per lane at a permuted
-    // atom, saved no time: 64-grid batch of 1e7 points 140 -> 145 ms.)
-    // kWideAtom: the caller chose it for such rows; kWideRest: no point here
-    // has a table block
-    const bool by_atom = SC == kWideAtom || (SC == kWideAll && pre && tab && d.sv <= na);
-    auto atom_walk = [&](uint32_t c0, uint32_t c1) {
-      const uint32_t mpw = 64u / na;  // modes per wave pass
-      const uint32_t m = lane / na, a = lane - m * na;
-      const uint32_t nmodes = b_end > b_lo ? b_end - b_lo : 0u;
-      const uint32_t passes = (nmodes + mpw - 1) / mpw;
-      const C* fac = wide_factors<Real>(d);
-      const uint32_t sc = d.sc, sv = d.sv;
-      // the points this walk takes: located, with a table block
-      auto taken = [&](uint32_t pl) { return s_rec[pl].nslot != 0 && s_rec[pl].trow != kNoCube; };
-      for (uint32_t t = wave; t < passes; t += TB / 64) {
-        const uint32_t b = b_lo + t * mpw + m;
-        const bool on = m < mpw && b < b_end;
-        // Runs of consecutive points of one table block: the block's rows of
-        // this lane's mode and atom are loaded and antiphased once per run,
-        // and stay loop-invariant over the run's points.
-        uint32_t p0 = c0;
-        while (true) {
-          while (p0 < c1 && !taken(p0)) {
-            // without the wave-per-unit walk the unlocated points are zeroed here
-            if (SC == kWideAtom && s_rec[p0].nslot == 0 && on) {
-              const uint64_t row = ((out_row ? (uint64_t)out_row[p0] : row0 + p0)) * B;
-              C* oc = vecs + row * sc + (uint64_t)b * sc;
-#pragma unroll
-              for (int i = 0; i < 3; ++i) oc[3u * a + i] = Elem<C>::zero();
-              if (a < sv) vals[row * sv + (uint64_t)b * sv + a] = 0;
-            }
-            ++p0;
-          }
-          if (p0 >= c1) break;
-          const uint32_t trow = s_rec[p0].trow;
-          uint32_t p1 = p0 + 1;
-          while (p1 < c1 && taken(p1) && s_rec[p1].trow == trow) ++p1;
-          C v[8][3];
-          Real vv[8];
-          {
-            const PointRec<Real>& rb = s_rec[p0];
-#pragma unroll
-            for (int x = 0; x < 8; ++x) {
-              if (on) {
-                const Real* rw = row_at<Real>(d, rb.idx[x], b);
-                const C* rc = reinterpret_cast<const C*>(rw) + 3u * a;
-                const C e = x < (int)rb.nslot ? fac[trow + (uint32_t)x * B + b] : C{(Real)1, (Real)0};
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                  const C el = rc[i];
-                  phase_elem<Real>(e, el.x, el.y, &v[x][i].x, &v[x][i].y);
-                }
-                vv[x] = a < sv ? rw[2 * sc + a] : (Real)0;
-              }
-            }
-          }
-          for (uint32_t pl = p0; pl < p1; ++pl) {
-            if (!on) continue;
-            const PointRec<Real>& r = s_rec[pl];
-            const uint64_t row = ((out_row ? (uint64_t)out_row[pl] : row0 + pl)) * B;
-            Real* ov = vals + row * sv + (uint64_t)b * sv;
-            C* oc = vecs + row * sc + (uint64_t)b * sc;
-            C acc[3] = {Elem<C>::zero(), Elem<C>::zero(), Elem<C>::zero()};
-            Real va = 0;
-#pragma unroll
-            for (int x = 0; x < 8; ++x) {
-              const Real wx = r.w[x];
-#pragma unroll
-              for (int i = 0; i < 3; ++i) {
-                acc[i].x = fma_r(wx, v[x][i].x, acc[i].x);
-                acc[i].y = fma_r(wx, v[x][i].y, acc[i].y);
-              }
-              va = fma_r(wx, vv[x], va);
-            }
-            if (a < sv) __builtin_nontemporal_store(va, ov + a);
-            // rip_gamma_complex  src/interpolator_gamma.tpp:100-114, atom by atom
-            const Real* R = wg.rot + 9u * r.invrot;
-            const C ph = wg.ph[(pl - c0) * na + a];
-            C* dst = oc + 3u * wg.dst[r.invrot * na + a];
-            typedef Real real2 __attribute__((ext_vector_type(2)));
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-              C tt = Elem<C>::zero();
-#pragma unroll
-              for (int j = 0; j < 3; ++j) tt = Elem<C>::add(tt, Elem<C>::scale(acc[j], R[3 * i + j]));
-              const C o = cmul(ph, tt);
-              __builtin_nontemporal_store(real2{o.x, o.y}, reinterpret_cast<real2*>(dst + i));
-            }
-          }
-          p0 = p1;
-        }
-      }
-    };
-    // Wave per (point, mode): wave w takes modes w, w + TB/64, ... of the
-    // block's group; with by_atom only the points the atom walk leaves.
-    auto walk = [&](auto two_tag, uint32_t c0, uint32_t c1, bool untabled_only) {
+    auto walk = [&](auto two_tag, uint32_t c0, uint32_t c1) {
       constexpr bool TWO = decltype(two_tag)::value;
       WideRows<Real, TWO> w;
       for (uint32_t b = b_lo + wave; b < b_end; b += TB / 64) {
         uint32_t cached = kNoCube;
         for (uint32_t pl = c0; pl < c1; ++pl) {
           const PointRec<Real>& r = s_rec[pl];
-          if (untabled_only && r.nslot != 0 && r.trow != kNoCube) continue;
           const uint64_t row = ((out_row ? (uint64_t)out_row[pl] : row0 + pl)) * B;
           Real* ov = vals + row * d.sv;
           C* oc = vecs + row * d.sc;
@@ -1663,14 +1767,8 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
         }
         __syncthreads();
       }
-      if (by_atom) atom_walk(c0, c1);
-      // (kWideAtom compiles without the wave-per-unit walk: 109 instead of
-      // 240 VGPRs; its points without a table block go to the kWideRest
-      // launch.  64-grid batch of 1e7 points 103 -> 87-90 ms.)
-      if constexpr (SC != kWideAtom) {
-        if (two) walk(std::true_type{}, c0, c1, by_atom);
-        else walk(std::false_type{}, c0, c1, by_atom);
-      }
+      if (two) walk(std::true_type{}, c0, c1);
+      else walk(std::false_type{}, c0, c1);
     }
     return;
   }
@@ -1762,21 +1860,30 @@ __device__ __forceinline__ void report_point(ErrRec* err, uint64_t index, int st
 // (Fast = false) is the literal restatement: exact fold-in and location,
 // atan2/sincos antiphases.
 
+// points a block's LDS holds: a wide row keeps four waves busy with few points
+constexpr uint32_t tile_capacity(int L) { return L == LAYOUT_WIDE ? 64u : (uint32_t)TILE; }
+
+// a.tile points per block (phase 1 on its first lanes, phase 2 on all 256);
+// wide rows: blockIdx.y picks a group of modes, and the first group reports
+// the points' errors and aux outputs
 template <typename Real, bool Fast, int L, int SC, int SV>
 __global__ __launch_bounds__(TILE) void k_ir_interpolate(GridConst g, DataConst d, LaunchArgs a) {
   using C = typename Cplx<Real>::T;
+  constexpr int TP = (int)tile_capacity(L);
   using S = TileShape<L, SC, TILE, Real>;
-  __shared__ PointRec<Real> s_rec[TILE];
-  __shared__ C s_ph[TILE * S::NPH];
-  __shared__ double s_q[S::NQ];
+  using P_ = TileShape<L, SC, TP, Real>;
+  __shared__ PointRec<Real> s_rec[TP];
+  __shared__ C s_ph[TP * S::NPH];
+  __shared__ double s_q[P_::NQ];
   __shared__ C s_wide[S::NW];
-  const uint64_t tile0 = (uint64_t)blockIdx.x * TILE;
+  const uint64_t tile0 = (uint64_t)blockIdx.x * a.tile;
   const uint32_t tid = threadIdx.x;
   const uint64_t p = tile0 + tid;
+  const bool lead = blockIdx.y == 0;
   const bool want_phase = d.vec_rot == BRILLE_ROT_GAMMA && d.ec[1] > 0;
   const uint32_t n_atoms = d.ec[1] / 3u;
   const bool ph_in_lds = L == LAYOUT_GAMMA || (want_phase && n_atoms <= 4);
-  {
+  if (tid < a.tile) {
     PointRec<Real>& r = s_rec[tid];
     r.nslot = 0;
     const bool live = p < a.n;
@@ -1788,15 +1895,18 @@ __global__ __launch_bounds__(TILE) void k_ir_interpolate(GridConst g, DataConst 
     }
     if (live && P.status == BRILLE_PT_OK) node_slots(g, P);
     if (live) {
-      write_aux(a.aux, p, P);
-      if (P.status != BRILLE_PT_OK) report_point(a.err, a.base + p, P.status);
-      else store_record<Real, L, SC>(g, d, P, r, s_ph, s_q, tid, ph_in_lds, n_atoms);
+      if (lead) write_aux(a.aux, p, P);
+      if (P.status == BRILLE_PT_OK) store_record<Real, L, SC>(g, d, P, r, s_ph, s_q, tid, ph_in_lds, n_atoms);
+      else if (lead) report_point(a.err, a.base + p, P.status);
     }
   }
   __syncthreads();
   const uint64_t left = a.n - tile0;
-  const uint32_t npts = left < (uint64_t)TILE ? (uint32_t)left : (uint32_t)TILE;
-  tile_sums<Real, Fast, L, SC, SV>(g, d, s_rec, s_ph, s_q, nullptr, tile0, npts, ph_in_lds, a.vals, a.vecs, s_wide);
+  const uint32_t npts = left < (uint64_t)a.tile ? (uint32_t)left : a.tile;
+  const uint32_t per_group = (d.B + gridDim.y - 1) / gridDim.y;
+  const uint32_t b_lo = blockIdx.y * per_group;
+  tile_sums<Real, Fast, L, SC, SV>(g, d, s_rec, s_ph, s_q, nullptr, tile0, npts, ph_in_lds, a.vals, a.vecs, s_wide,
+                                   false, 0, nullptr, false, {}, b_lo, b_lo + per_group);
 }
 
 }  // namespace brille_amd

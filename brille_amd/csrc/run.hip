@@ -103,6 +103,11 @@ bool wide_rows(const DataConst& d) {
   return (L == LAYOUT_GAMMA || L == LAYOUT_SCALAR) && d.sc > 12 && d.sc <= kWideMax && d.sv <= 64;
 }
 
+// wide Gamma rows of at most one value per atom: the sums go atom-major
+bool wide_by_atom(const DataConst& d) {
+  return wide_rows(d) && payload_layout(d) == LAYOUT_GAMMA && d.sv <= d.sc / 3u;
+}
+
 // The instantiated specialisations: Gamma payloads of 1-4 atoms and scalar
 // payloads of 1-4 complex elements, each with one value per mode; anything
 // else runs the general phase 2.
@@ -127,18 +132,65 @@ static TileKernel pick_tuned(const DataConst& d) {
       default: break;
     }
   }
-  if (wide_rows(d)) return k_ir_interpolate<Real, true, LAYOUT_WIDE, 0, 0>;
+  if (wide_by_atom(d)) return k_ir_interpolate<Real, true, LAYOUT_WIDE, kWideAtom, 0>;
+  if (wide_rows(d)) return k_ir_interpolate<Real, true, LAYOUT_WIDE, kWideAll, 0>;
   return k_ir_interpolate<Real, true, LAYOUT_GENERIC, 0, 0>;
 }
 
+// Points per block and mode groups of a fused launch.  A block of TILE points
+// walks them in sequence (narrow rows: TILE lanes take (point, mode) units;
+// wide rows: four waves take (point, modes) units), so a call of few points
+// gets smaller tiles.
+//   narrow rows: down to one block per CU, as long as a tile has more units
+//     than lanes (a second round of blocks repeats phase 1's latency: FP64 hex
+//     grid of 6 modes, 20 011 points: 81 us in 256-point tiles, 56 us in 64,
+//     72 us in 32);
+//   wide rows: to eight blocks per CU, which spreads the tail, as long as a
+//     block's waves have three units each (3 001 points of 72 modes: 17.8 ms in
+//     256-point tiles, 0.25 ms in single points; 3 001 points of 24 modes: 88
+//     us in single points, 50 us in fours); when single points still leave CUs
+//     idle, the modes split too, to three blocks per CU (301 points of 72
+//     modes: 64 us whole, 50 us in two groups, 68 us in six, each of which
+//     repeats phase 1).
+static void tile_split(const brille_grid* G, uint64_t n, bool fast, uint32_t* tile, uint32_t* groups) {
+  const DataConst& d = G->d;
+  const uint64_t cu = std::max<uint32_t>(G->n_cu, 1);
+  uint32_t t = TILE;
+  *groups = 1;
+  if (fast && wide_rows(d)) {
+    const uint32_t mpw = wide_by_atom(d) ? 64u / (d.sc / 3u) : 1u;
+    const uint32_t passes = (d.B + mpw - 1) / mpw;
+    t = tile_capacity(LAYOUT_WIDE);
+    while (t > 1 && (n + t - 1) / t < 8 * cu && (t >> 1) * passes >= 12) t >>= 1;
+    const uint64_t blocks = (n + t - 1) / t;
+    if (t == 1) *groups = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((d.B + 3) / 4, 3 * cu / blocks));
+  } else {
+    while (t > 32 && (n + t - 1) / t < cu && t * d.B > (uint32_t)TILE) t >>= 1;
+  }
+  *tile = t;
+}
+
 // plain: the literal FP64 restatement; tuned: fast fold-in and specialised sums
-static void launch_sel(const brille_grid* G, const LaunchArgs& a, int precision, bool fast, hipStream_t s) {
-  const uint64_t blocks = (a.n + TILE - 1) / TILE;
-  if (!blocks) return;
+static void launch_sel(const brille_grid* G, LaunchArgs a, int precision, bool fast, hipStream_t s) {
+  uint32_t groups;
+  tile_split(G, a.n, fast, &a.tile, &groups);
   TileKernel k;
   if (precision == BRILLE_FP32) k = fast ? pick_tuned<float>(G->d) : k_ir_interpolate<float, false, LAYOUT_GENERIC, 0, 0>;
   else k = fast ? pick_tuned<double>(G->d) : k_ir_interpolate<double, false, LAYOUT_GENERIC, 0, 0>;
-  hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(TILE), 0, s, G->g, G->d, a);
+  // a launch holds fewer than 2^32 threads along x
+  constexpr uint64_t kMostBlocks = (1ull << 24) - 1;
+  const size_t rs = precision == BRILLE_FP32 ? 4 : 8;
+  const uint64_t n = a.n, piece = kMostBlocks * a.tile;
+  for (uint64_t c0 = 0; c0 < n; c0 += piece) {
+    LaunchArgs c = a;
+    c.Q = a.Q + 3 * c0;
+    c.n = std::min(piece, n - c0);
+    c.base = a.base + c0;
+    c.vals = static_cast<char*>(a.vals) + c0 * G->d.B * G->d.sv * rs;
+    c.vecs = static_cast<char*>(a.vecs) + c0 * G->d.B * G->d.sc * 2 * rs;
+    c.aux = offset_aux(a.aux, c0);
+    hipLaunchKernelGGL(k, dim3((unsigned)((c.n + a.tile - 1) / a.tile), groups), dim3(TILE), 0, s, G->g, G->d, c);
+  }
 }
 
 void launch_tile(const brille_grid* G, const LaunchArgs& a, int precision, bool fast, hipStream_t s) {

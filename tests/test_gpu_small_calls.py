@@ -1,0 +1,78 @@
+"""Calls of few points: the fused kernel cuts its tiles by the call's size and
+splits the modes of wide rows, and wide Gamma rows form their antiphases
+atom by atom where no factor table holds them.
+
+Every size must give the oracle's results (FP64 within 1e-12 relative, FP32
+within 1e-5 of the scale), at the edges of the tiles and on points without a
+table block (grid vertices and cell edges, where the first slot weighs
+nothing).  Needs an MI355X.
+"""
+import numpy as np
+import pytest
+
+from brille_amd import capi
+from brille_amd import synthetic as S
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SIZES = (1, 2, 31, 33, 64, 65, 255, 257, 2049)
+
+
+def points(g, r, n):
+    """Uniform Q with every third point on a vertex or on the edge of two neighbouring vertices."""
+    Q = r.uniform(-3, 3, size=(n, 3))
+    rlu = np.asarray(g.rlu)
+    k = r.integers(0, len(rlu) - 1, size=n)
+    special = np.where(r.random((n, 1)) < 0.5, rlu[k], 0.5 * (rlu[k] + rlu[k + 1]))
+    Q[::3] = special[::3]
+    return Q
+
+
+# atoms 2 and 4 (one lane per mode), 12 (5 modes a wave), 24 (2 modes a wave)
+@pytest.mark.parametrize("spec", [3, 7, 2, 5])
+def test_every_call_size_matches_the_oracle(spec):
+    print(f"small calls: grid {spec}", flush=True)
+    sp = dict(S.batch_specs(16)[spec], v_target=600.0)
+    g = S.batch_grid(sp)
+    vals, vecs = S.batch_payload(g, sp)
+    t = dict(S.batch_layout_tables(g, sp), values=vals, vectors=vecs)
+    dev = capi.Grid(t)
+    r = np.random.default_rng(31 + spec)
+    for n in SIZES:
+        print(f"  n={n} B={sp['modes']}", flush=True)
+        Q = points(g, r, n)
+        rc, ov, oc, oaux, _ = O.ir_interpolate_at(t, Q, nthreads=8)
+        assert rc == 0
+        gv, gc, gaux = dev.ir_interpolate_at(Q, precision=capi.FP64, kernel=capi.KERNEL_TILE, aux=True)
+        for k in ("tau", "rot", "invrot", "node", "tet", "n_iw", "iw_index", "iw_weight", "ir_q"):
+            np.testing.assert_array_equal(gaux[k], oaux[k], err_msg=f"n={n} {k}")
+        assert np.max(np.abs(gv - ov)) <= 1e-12 * np.abs(ov).max(), n
+        assert np.max(np.abs(gc - oc)) <= 1e-12 * np.abs(oc).max(), n
+        fv, fc = dev.ir_interpolate_at(Q, precision=capi.FP32, kernel=capi.KERNEL_TILE)
+        assert np.max(np.abs(fv - ov)) <= 1e-5 * np.abs(ov).max(), n
+        assert np.max(np.abs(fc - oc)) <= 1e-5 * np.abs(oc).max(), n
+        for prec, (tv, tc) in ((capi.FP64, (gv, gc)), (capi.FP32, (fv, fc))):
+            bv, bc = dev.ir_interpolate_at(Q, precision=prec, kernel=capi.KERNEL_BINNED)
+            np.testing.assert_array_equal(bv, tv)
+            np.testing.assert_array_equal(bc, tc)
+            # the first binned call built the factor table: the fused kernel now reads it
+            av, ac = dev.ir_interpolate_at(Q, precision=prec, kernel=capi.KERNEL_TILE)
+            np.testing.assert_array_equal(av, tv)
+            np.testing.assert_array_equal(ac, tc)
+
+
+def test_a_failing_point_is_reported_once_by_every_split():
+    """Modes split over several blocks of one tile: only the first reports, so the count stays exact."""
+    print("small calls: errors", flush=True)
+    sp = dict(S.batch_specs(16)[5], v_target=600.0)
+    g = S.batch_grid(sp)
+    vals, vecs = S.batch_payload(g, sp)
+    dev = capi.Grid(dict(S.batch_layout_tables(g, sp), values=vals, vectors=vecs))
+    Q = np.random.default_rng(5).uniform(-3, 3, size=(5, 3))
+    Q[3] = np.nan
+    rc, v, c, aux = dev.run_device(Q, precision=capi.FP32, kernel=capi.KERNEL_TILE, check=False)
+    assert rc == 0 and list(np.nonzero(aux["status"])[0]) == [3]
+    assert np.all(v[3] == 0) and np.all(c[3] == 0) and np.all(np.isfinite(v))
+    with pytest.raises(capi.BrilleError, match="Not all points inside Brillouin zone"):
+        dev.ir_interpolate_at(Q, precision=capi.FP32, kernel=capi.KERNEL_TILE)
