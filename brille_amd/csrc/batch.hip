@@ -89,7 +89,7 @@ static int32_t batch_kind(const DataConst& d) {
 template <typename Real, int L, int SC, int SV, int TB>
 __device__ __forceinline__ void batch_tile(const BatchGrid& bg, const BatchSlot& sl, uint64_t p0, uint32_t npts,
                                            PointRec<Real>* s_rec, typename Cplx<Real>::T* s_ph, double* s_q,
-                                           typename Cplx<Real>::T* s_wide, int fold) {
+                                           typename Cplx<Real>::T* s_wide, uint32_t* s_pm, int fold) {
   const uint32_t tid = threadIdx.x;
   PointRec<Real>& r = s_rec[tid];
   r.nslot = 0;
@@ -102,9 +102,14 @@ __device__ __forceinline__ void batch_tile(const BatchGrid& bg, const BatchSlot&
     else store_record<Real, L, SC>(bg.g, bg.d, P, r, s_ph, s_q, tid, bg.ph_in_lds != 0, bg.n_atoms);
   }
   __syncthreads();
+  if (bg.d.n_keys) {
+    tile_perms<TB>(bg.d, s_rec, 0, npts, s_pm);
+    __syncthreads();
+  }
   // four rows in flight: the persistent kernel's registers are the largest of all its branches
   tile_sums<Real, true, L, SC, SV, TB, 4>(bg.g, bg.d, s_rec, s_ph, s_q, nullptr, p0, npts, bg.ph_in_lds != 0, sl.vals,
-                                         sl.vecs, s_wide);
+                                         sl.vecs, s_wide, false, 0, nullptr, false, {}, 0, ~0u,
+                                         bg.d.n_keys ? s_pm : nullptr);
   __syncthreads();
 }
 
@@ -119,6 +124,7 @@ void k_batch(const BatchGrid* grids, const BatchSlot* all_slots, BatchHeader* hd
   __shared__ double s_q[(kWide || 3 > frame_words<Real>() ? 3 : frame_words<Real>()) * TB];
   constexpr int kSlice = TileShape<LAYOUT_WIDE, kWideAtom, TB, Real>::NW;
   __shared__ C s_wide[!kWide ? 1 : kSlice > (TB / 64) * (int)kWideMax ? kSlice : (TB / 64) * (int)kWideMax];
+  __shared__ uint32_t s_pm[8 * TB];  // slot permutations of sorted members
   __shared__ unsigned long long s_t;
   const uint64_t n_tiles = hdr->n_tiles[LIST];
   const uint32_t n_slots = hdr->n_slots[LIST];
@@ -146,18 +152,18 @@ void k_batch(const BatchGrid* grids, const BatchSlot* all_slots, BatchHeader* hd
       const uint32_t npts = left < (uint64_t)sl.pts ? (uint32_t)left : sl.pts;
       if constexpr (kWide) {
         if (bg.kind == BK_WIDE_ATOM)
-          batch_tile<Real, LAYOUT_WIDE, kWideAtom, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold);
+          batch_tile<Real, LAYOUT_WIDE, kWideAtom, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold);
         else
-          batch_tile<Real, LAYOUT_WIDE, kWideAll, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold);
+          batch_tile<Real, LAYOUT_WIDE, kWideAll, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold);
         continue;
       } else switch (bg.kind) {
-        case BK_GAMMA3: batch_tile<Real, LAYOUT_GAMMA, 3, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
-        case BK_GAMMA6: batch_tile<Real, LAYOUT_GAMMA, 6, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
-        case BK_SCALAR1: batch_tile<Real, LAYOUT_SCALAR, 1, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
-        case BK_SCALAR2: batch_tile<Real, LAYOUT_SCALAR, 2, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
-        case BK_SCALAR3: batch_tile<Real, LAYOUT_SCALAR, 3, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
-        case BK_SCALAR4: batch_tile<Real, LAYOUT_SCALAR, 4, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
-        default: batch_tile<Real, LAYOUT_GENERIC, 0, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, fold); break;
+        case BK_GAMMA3: batch_tile<Real, LAYOUT_GAMMA, 3, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
+        case BK_GAMMA6: batch_tile<Real, LAYOUT_GAMMA, 6, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
+        case BK_SCALAR1: batch_tile<Real, LAYOUT_SCALAR, 1, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
+        case BK_SCALAR2: batch_tile<Real, LAYOUT_SCALAR, 2, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
+        case BK_SCALAR3: batch_tile<Real, LAYOUT_SCALAR, 3, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
+        case BK_SCALAR4: batch_tile<Real, LAYOUT_SCALAR, 4, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
+        default: batch_tile<Real, LAYOUT_GENERIC, 0, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
       }
     }
   }

@@ -500,11 +500,17 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
     atomicAdd(&pc.stats[1], (unsigned long long)s_verified);
   }
   const uint32_t npts = n - tile0 < (uint32_t)TILE ? n - tile0 : (uint32_t)TILE;
+  const uint32_t* pm = nullptr;
+  if (d.n_keys) {  // the row table's rows are permuted already
+    tile_perms<TILE>(d, s_rec, table ? n_tab : 0u, npts, s_perms);
+    __syncthreads();
+    pm = s_perms;
+  }
   // the one-lane-per-unit sums see only the points the table does not serve:
   // fewer rows in flight keep the registers for occupancy
   constexpr int GRP = sizeof(Real) == 4 ? 2 : 1;
   tile_sums<Real, true, L, SC, SV, TILE, GRP, WSL>(g, d, s_rec, s_ph, s_q, s_out, 0, npts, ph_in_lds, vals, vecs, s_wide,
-                                              table, n_tab, kOpFrames ? s_frames : nullptr, true, wg, b_lo, b_hi);
+                                              table, n_tab, kOpFrames ? s_frames : nullptr, true, wg, b_lo, b_hi, pm);
 }
 
 // The row table: thread t = (block row, mode b) phases the row of a cube's or
@@ -534,7 +540,8 @@ __global__ __launch_bounds__(256) void k_table_rows(GridConst g, DataConst d, ui
   const uint64_t stride = payload_stride<Real>(d);
   Real pr[2 * SC];
   load_row<Real, 2 * SC>(pr, base + ((uint64_t)pv * d.B + b) * stride);
-  const Real* src = base + ((uint64_t)sv * d.B + b) * stride;
+  const uint32_t bs = d.cell_perm ? perm_mode(d, d.cell_perm[t / d.B], b) : b;
+  const Real* src = base + ((uint64_t)sv * d.B + bs) * stride;
   Real row[2 * SC];
   load_row<Real, 2 * SC>(row, src);
   const typename Cplx<Real>::T e = slot_antiphase<Real, SC>(pr, row);
@@ -577,7 +584,9 @@ __global__ __launch_bounds__(256) void k_wide_factors(GridConst g, DataConst d, 
   C v0[8], v1[8], e[8];
 #pragma unroll
   for (int x = 0; x < 8; ++x) {
-    const C* rc = reinterpret_cast<const C*>(row_at<Real>(d, v[x], b));
+    const uint32_t bx =
+        d.cell_perm && (uint32_t)x < ns ? perm_mode(d, d.cell_perm[trow / d.B + x], b) : b;
+    const C* rc = reinterpret_cast<const C*>(row_at<Real>(d, v[x], bx));
     v0[x] = h0 ? rc[l] : zero;
     v1[x] = h1 ? rc[l + 64] : zero;
   }
@@ -614,7 +623,8 @@ __global__ __launch_bounds__(256) void k_wide_atom_factors(GridConst g, DataCons
   for (int x = 0; x < 8; ++x) {
     const bool use = on && x < (int)ns;
     const uint32_t vert = cube ? g.cube_v[8 * c + 7 - x] : g.tet_v[4 * c + (x & 3)];
-    const C* rc = reinterpret_cast<const C*>(row_at<Real>(d, vert, on ? b : 0u)) + 3u * a;
+    const uint32_t bx = use && d.cell_perm ? perm_mode(d, d.cell_perm[trow / d.B + x], b) : (on ? b : 0u);
+    const C* rc = reinterpret_cast<const C*>(row_at<Real>(d, vert, bx)) + 3u * a;
 #pragma unroll
     for (int i = 0; i < 3; ++i) v[x][i] = use ? rc[i] : Elem<C>::zero();
   }
@@ -697,7 +707,7 @@ static int build_cube_rows(brille_grid* G, hipStream_t s, Real** out) {
   void* p = nullptr;
   if (hipMalloc(&p, units * payload_stride_host<Real>(d) * sizeof(Real)) != hipSuccess)
     return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the cube row table");
-  G->data_allocs.push_back(p);
+  G->derived_allocs.push_back(p);
   Real* t = static_cast<Real*>(p);
   const dim3 grid((unsigned)((units + 255) / 256));
   switch (onepass_sc(d)) {
@@ -727,7 +737,7 @@ static int build_wide_factors(brille_grid* G, hipStream_t s, typename Cplx<Real>
   void* p = nullptr;
   if (hipMalloc(&p, (G->n_cubes * 8 + G->n_tets * 4) * d.B * sizeof(C)) != hipSuccess)
     return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the wide factor table");
-  G->data_allocs.push_back(p);
+  G->derived_allocs.push_back(p);
   C* t = static_cast<C*>(p);
   if (atom)
     hipLaunchKernelGGL((k_wide_atom_factors<Real>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, G->g, d,
@@ -741,19 +751,18 @@ static int build_wide_factors(brille_grid* G, hipStream_t s, typename Cplx<Real>
 }
 
 // Builds the payload's derived table of the given precision once (freed with
-// the payload): the antiphased rows (8 per cube, 4 per tetrahedron and mode)
+// the payload, or when a sort replaces the permutations it follows): the antiphased rows (8 per cube, 4 per tetrahedron and mode)
 // for the one-pass layouts, the antiphase factors alone for wide rows.  The
 // general layout, grids without cells and tables beyond kCubeRowsMax go
 // without, and their sums compute every antiphase on the fly.
 constexpr uint64_t kCubeRowsMax = (4ull << 30) - 1;  // the sums address the table with 32-bit offsets
 int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s) {
   DataConst& d = G->d;
-  if (G->n_cubes + G->n_tets == 0 || d.B == 0) return BRILLE_OK;
+  if (G->n_cubes + G->n_tets == 0 || d.B == 0 || !d.has_blocks) return BRILLE_OK;
   if (wide_rows(d)) {
     // wide rows: the antiphases only (one complex per slot row)
     const uint64_t fac_bytes = (G->n_cubes * 8 + G->n_tets * 4) * d.B * (precision == BRILLE_FP32 ? 8ull : 16ull);
     if (fac_bytes > kCubeRowsMax) return BRILLE_OK;
-    d.tab_tet_row = (uint32_t)(G->n_cubes * 8 * d.B);
     if (precision == BRILLE_FP32) {
       if (d.wide_fac32) return BRILLE_OK;
       float2* t = nullptr;
@@ -770,7 +779,6 @@ int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s) {
   if (onepass_sc(d) == 0) return BRILLE_OK;
   const uint64_t row_bytes = precision == BRILLE_FP32 ? d.stride32 * 4ull : d.stride64 * 8ull;
   if ((G->n_cubes * 8 + G->n_tets * 4) * d.B * row_bytes > kCubeRowsMax) return BRILLE_OK;
-  d.tab_tet_row = (uint32_t)(G->n_cubes * 8 * d.B);
   if (precision == BRILLE_FP32) {
     if (d.cube_rows32) return BRILLE_OK;
     float* t = nullptr;
@@ -1029,7 +1037,7 @@ int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStr
     // sums of pass k on the call stream
     mark(k, 3, s);
     const dim3 sgrid((m + TILE - 1) / TILE, sum_groups(G, m, prop));
-    hipLaunchKernelGGL(sums, sgrid, dim3(TILE), 0, s, G->g, G->d, a.prop, b.srt, b.perm, m,
+    hipLaunchKernelGGL(sums, sgrid, dim3(TILE), G->d.n_keys ? 32u * TILE : 0u, s, G->g, G->d, a.prop, b.srt, b.perm, m,
                        static_cast<char*>(a.vals) + c0 * vb, static_cast<char*>(a.vecs) + c0 * cb,
                        offset_aux(a.aux, c0), a.err, a.base + c0);
     mark(k, 4, s);

@@ -318,6 +318,7 @@ int brille_grid_destroy(brille_grid* G) {
   free_all(G->grid_allocs);
   free_all(G->data_allocs);
   free_all(G->sort_allocs);
+  free_all(G->derived_allocs);
   free_proposal(G);
   free_staging(G);
   free_binned(G);
@@ -421,6 +422,7 @@ static int grid_fill(brille_grid* G, const brille_data_desc* vals, const brille_
     }
   }
   if (perm && perm->n_keys) {
+    // (keys without a permutation are refused below: every index is out of range)
     if (!perm->keys || !perm->perm_index || (perm->n_perms && !perm->perms))
       return fail(BRILLE_ERR_INVALID_ARGUMENT, "permutation table arrays must not be null");
     for (uint64_t i = 0; i < perm->n_keys; ++i) {
@@ -433,6 +435,7 @@ static int grid_fill(brille_grid* G, const brille_data_desc* vals, const brille_
   (void)hipDeviceSynchronize();  // nothing still reads the payload that is replaced
   free_all(G->data_allocs);
   free_all(G->sort_allocs);
+  free_all(G->derived_allocs);
   G->n_perms = 0;
   ++G->fill_gen;  // the payload tables are replaced from here on (batches re-read them)
   G->filled = false;
@@ -449,6 +452,11 @@ static int grid_fill(brille_grid* G, const brille_data_desc* vals, const brille_
   d.vec_lu = vecs->length_unit;
   auto& A = G->data_allocs;
   const uint32_t used = 2 * d.sc + d.sv;
+  // every cell a block of row numbers, whether or not a derived table follows
+  // them: points of one block share their slot rows
+  const uint64_t block_rows = (G->n_cubes * 8 + G->n_tets * 4) * d.B;
+  d.has_blocks = block_rows < 0xFFFFFFFFull ? 1 : 0;
+  d.tab_tet_row = d.has_blocks ? (uint32_t)(G->n_cubes * 8 * d.B) : 0u;
   d.stride64 = row_stride(used, sizeof(double));
   d.stride32 = row_stride(used, sizeof(float));
   int rc = fill_payload(G, vals, vecs, o);
@@ -471,6 +479,7 @@ static int grid_fill(brille_grid* G, const brille_data_desc* vals, const brille_
     chk(upload(perm->perm_index, (size_t)perm->n_keys, &d.perm_index, A));
     chk(upload(perm->perms, (size_t)perm->n_perms * d.B, &d.perms, A));
     G->n_perms = perm->n_perms;
+    if (rc == BRILLE_OK) rc = install_permutations(G, A, nullptr);
   }
   if (rc != BRILLE_OK) {
     free_all(A);

@@ -97,6 +97,7 @@ struct DataConst {
   const float* cube_rows32;
   const double* cube_rows64;
   uint32_t tab_tet_row;
+  uint32_t has_blocks;  // 0: the rows of all blocks do not fit 32-bit numbers
   // Wide-row payloads instead keep only the antiphases: the factor of slot x
   // for mode b of the block at table row trow (numbered as above) at
   // trow + x * B + b (null until built).
@@ -116,7 +117,14 @@ struct DataConst {
   const uint64_t* keys;
   const uint32_t* perm_index;
   const uint32_t* perms;
+  // derived from the table (install_permutations): the first key of every
+  // vertex (V + 1 entries; null for 2^32 keys or more), and the permutation of
+  // every block slot against its block's slot-0 vertex, numbered like the row
+  // table's rows without the modes (null without block numbers)
+  const uint32_t* vkey;
+  const uint32_t* cell_perm;
 };
+constexpr uint32_t kNoPerm = 0xFFFFFFFFu;  // no key: the modes as they are
 
 // Learned tetrahedron proposal: an MLP 3 -> 128 -> 128 -> K over the
 // tetrahedra of the trellis (K = number of tetrahedra), evaluated only for the

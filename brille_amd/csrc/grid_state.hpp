@@ -27,6 +27,9 @@ struct brille_grid {
   std::vector<void*> data_allocs;
   // the permutation table brille_grid_sort built (freed by the next sort or fill)
   std::vector<void*> sort_allocs;
+  // the row and factor tables built from the payload and its permutations
+  // (freed by the next fill or sort)
+  std::vector<void*> derived_allocs;
   uint32_t n_perms = 0;  // permutations of the installed table
   bool filled = false;
   uint64_t n_vertices = 0, n_cubes = 0, n_polys = 0, n_tets = 0;
@@ -124,7 +127,10 @@ void zero_words(void* p, uint32_t n, hipStream_t s);
 // exclusive prefix sum of a[0, m) in place on stream s; part holds
 // (m + 4095) / 4096 words; m at most 2^30
 int exclusive_scan_u32(uint32_t* a, uint64_t m, uint32_t* part, hipStream_t s);
-// the cube row table of the bucketed sums, built on first use (data_allocs)
+// the lookup tables of an installed PermutationTable (d.keys and d.perm_index
+// set), kept in `allocs`
+int install_permutations(brille_grid* G, std::vector<void*>& allocs, hipStream_t s);
+// the cube row table of the bucketed sums, built on first use (derived_allocs)
 int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s);
 // the first failing point of a call as the reference's error text
 int report_point_error(const ErrRec& e, const double* Q, uint64_t n, bool host_mem);

@@ -137,18 +137,43 @@ __device__ __forceinline__ void load_row(Real* out, const Real* row) {
   }
 }
 
-// PermutationTable::safe_get with pivot iw[0]  src/permutation_table.hpp:193-198
-__device__ __forceinline__ uint32_t perm_at(const DataConst& d, uint32_t pivot, uint32_t idx, uint32_t b) {
-  if (d.n_keys == 0 || pivot == idx) return b;
-  uint64_t key = (uint64_t)pivot * d.V + idx;
-  uint64_t lo = 0, hi = d.n_keys;
+// PermutationTable::safe_get with pivot iw[0]  src/permutation_table.hpp:193-198:
+// the permutation of vertex idx against pivot (kNoPerm: none), found among
+// the pivot's own keys (a few dozen)
+__device__ __forceinline__ uint32_t perm_find(const DataConst& d, uint32_t pivot, uint32_t idx) {
+  if (pivot == idx) return kNoPerm;
+  const uint64_t key = (uint64_t)pivot * d.V + idx;
+  uint64_t lo = 0, end = d.n_keys;
+  if (d.vkey) {
+    lo = d.vkey[pivot];
+    end = d.vkey[pivot + 1];
+  }
+  uint64_t hi = end;
   while (lo < hi) {
-    uint64_t mid = (lo + hi) >> 1;
+    const uint64_t mid = (lo + hi) >> 1;
     if (d.keys[mid] < key) lo = mid + 1;
     else hi = mid;
   }
-  if (lo < d.n_keys && d.keys[lo] == key) return d.perms[(uint64_t)d.perm_index[lo] * d.B + b];
-  return b;
+  return lo < end && d.keys[lo] == key ? d.perm_index[lo] : kNoPerm;
+}
+
+// the permutation of slot x of a point: from its block when it has one
+template <typename Real>
+__device__ __forceinline__ uint32_t slot_perm(const DataConst& d, const PointRec<Real>& r, uint32_t x) {
+  if (x >= r.nslot) return kNoPerm;
+  if (r.trow != kNoCube && d.cell_perm) return d.cell_perm[r.trow / d.B + x];
+  return perm_find(d, r.pivot, r.idx[x]);
+}
+
+// the mode of a slot's row that belongs to mode b of the pivot
+__device__ __forceinline__ uint32_t perm_mode(const DataConst& d, uint32_t k, uint32_t b) {
+  // (a table has at least one permutation; no branch splits the row loads)
+  const uint32_t m = d.perms[(uint64_t)(k == kNoPerm ? 0u : k) * d.B + b];
+  return k == kNoPerm ? b : m;
+}
+// pm: the permutations of a point's slots, or null (no table)
+__device__ __forceinline__ uint32_t slot_mode(const DataConst& d, const uint32_t* pm, int x, uint32_t b) {
+  return pm ? perm_mode(d, pm[x], b) : b;
 }
 
 // ---------------------------------------------------------------------------
@@ -436,7 +461,7 @@ __device__ __forceinline__ typename Cplx<Real>::T wsum_cplx(typename Cplx<Real>:
 template <typename Real, bool Literal>
 __device__ inline void unit_generic(const GridConst& g, const DataConst& d, const PointRec<Real>& r, const double* q,
                                     uint32_t b, Real* ov, typename Cplx<Real>::T* oc,
-                                    const typename Cplx<Real>::T* phases) {
+                                    const typename Cplx<Real>::T* phases, const uint32_t* pm) {
   using C = typename Cplx<Real>::T;
   const uint32_t sv = d.sv, sc = d.sc;
   const uint32_t ns = d.ev[0], nv = d.ev[1] / 3u, nm = d.ev[2] / 9u;
@@ -449,7 +474,7 @@ __device__ inline void unit_generic(const GridConst& g, const DataConst& d, cons
   for (int x = 0; x < 8; ++x) {
     const bool use = x < nslot && r.w[x] != (Real)0;
     w[x] = use ? r.w[x] : (Real)0;
-    row[x] = use ? row_at<Real>(d, r.idx[x], perm_at(d, r.pivot, r.idx[x], b)) : prow;
+    row[x] = use ? row_at<Real>(d, r.idx[x], slot_mode(d, pm, x, b)) : prow;
     cw[x] = Elem<C>::zero();
     if (use && sc) {
       Real re, im;
@@ -552,7 +577,7 @@ __device__ inline void unit_generic(const GridConst& g, const DataConst& d, cons
 
 // ---------------------------------------------------------------------------
 // phase 2, specialised payloads with compile-time row sizes: SC complex vector
-// elements and SV scalar values per (vertex, mode), no PermutationTable.
+// elements and SV scalar values per (vertex, mode).
 //   GAMMA: the vectors are SC/3 atom 3-vectors rotating like Gamma
 //          (rip_gamma_complex  src/interpolator_gamma.tpp:100-114);
 //   otherwise the vectors are scalars (no rotation).
@@ -593,7 +618,8 @@ __device__ __forceinline__ typename Cplx<Real>::T slot_antiphase(const Real* p, 
 template <typename Real, int SC, int SV, bool GAMMA, int GRP = 0>
 __device__ __forceinline__ void unit_onepass(const DataConst& d, const PointRec<Real>& r, uint32_t b, Real* ov,
                                              typename Cplx<Real>::T* oc, const typename Cplx<Real>::T* phases,
-                                             const GammaFrame<Real>* fr, bool table = false) {
+                                             const GammaFrame<Real>* fr, bool table = false,
+                                             const uint32_t* pm = nullptr) {
   using C = typename Cplx<Real>::T;
   constexpr int NR = 2 * SC + SV;
   const Real* base = payload_rows<Real>(d);
@@ -613,6 +639,13 @@ __device__ __forceinline__ void unit_onepass(const DataConst& d, const PointRec<
   // register budget).  Unused tetrahedron slots repeat the pivot with weight 0:
   // their loads hit in cache and add exact zeros, and no branch splits the loads.
   constexpr int GR = GRP ? GRP : (sizeof(Real) == 4 ? 8 : 4);
+  uint32_t md[8];  // the row of mode b in every slot
+#pragma unroll
+  for (int x = 0; x < 8; ++x) md[x] = b;
+  if (pm && !tab) {
+#pragma unroll
+    for (int x = 0; x < 8; ++x) md[x] = perm_mode(d, pm[x], b);
+  }
 #pragma unroll
   for (int x0 = 0; x0 < 8; x0 += GR) {
     Real row[GR][NR];
@@ -629,7 +662,7 @@ __device__ __forceinline__ void unit_onepass(const DataConst& d, const PointRec<
       }
     } else {
 #pragma unroll
-      for (int x = 0; x < GR; ++x) load_row<Real, NR>(row[x], base + ((uint64_t)r.idx[x0 + x] * d.B + b) * stride);
+      for (int x = 0; x < GR; ++x) load_row<Real, NR>(row[x], base + ((uint64_t)r.idx[x0 + x] * d.B + md[x0 + x]) * stride);
 #pragma unroll
       for (int x = 0; x < GR; ++x) {
         const C e = slot_antiphase<Real, SC>(pr, row[x]);
@@ -843,9 +876,9 @@ __device__ __forceinline__ void unit_coop(const PointRec<Real>& r, const Chunk<R
 
 // Payload layouts with a specialised phase 2 (the general one handles all).
 enum Layout : int {
-  LAYOUT_GENERIC = 0,  // any elements, rotations and permutation table
-  LAYOUT_GAMMA = 1,    // scalar values; vectors = one 3-vector per atom rotating like Gamma; no permutations
-  LAYOUT_SCALAR = 2,   // scalar values and scalar vectors; no permutations
+  LAYOUT_GENERIC = 0,  // any elements and rotations
+  LAYOUT_GAMMA = 1,    // scalar values; vectors = one 3-vector per atom rotating like Gamma
+  LAYOUT_SCALAR = 2,   // scalar values and scalar vectors
   LAYOUT_WIDE = 3      // as GAMMA or SCALAR with long rows (up to kWideMax complex): one wave per (point, mode)
 };
 constexpr uint32_t kWideMax = 128;  // complex elements per row the wide phase 2 handles (two per lane)
@@ -1050,11 +1083,12 @@ __device__ __forceinline__ void wide_atom_antiphases(const typename Cplx<Real>::
 // off, and from the fifth on for a tetrahedron, whose four slots are all
 template <typename Real>
 __device__ __forceinline__ void wide_atom_load(const DataConst& d, const PointRec<Real>& r, uint32_t b, uint32_t a,
-                                               bool on, typename Cplx<Real>::T (*v)[3], Real* vv) {
+                                               bool on, typename Cplx<Real>::T (*v)[3], Real* vv,
+                                               const uint32_t* pm) {
   using C = typename Cplx<Real>::T;
 #pragma unroll
   for (int x = 0; x < 8; ++x) {
-    const Real* rw = row_at<Real>(d, r.idx[x], on ? b : 0u);
+    const Real* rw = row_at<Real>(d, r.idx[x], on ? slot_mode(d, pm, x, b) : 0u);
     const C* rc = reinterpret_cast<const C*>(rw) + 3u * a;
     const bool use = on && x < (int)r.nslot;
 #pragma unroll
@@ -1155,7 +1189,7 @@ struct WideRows {
 
 template <typename Real, bool TWO>
 __device__ __forceinline__ void wide_load(const DataConst& d, const PointRec<Real>& r, uint32_t b, bool tab,
-                                          WideRows<Real, TWO>& w) {
+                                          WideRows<Real, TWO>& w, const uint32_t* pm) {
   using C = typename Cplx<Real>::T;
   const uint32_t l = threadIdx.x & 63u;
   const uint32_t sc = d.sc, sv = d.sv, B = d.B;
@@ -1165,7 +1199,7 @@ __device__ __forceinline__ void wide_load(const DataConst& d, const PointRec<Rea
   const C* fac = wide_factors<Real>(d);
 #pragma unroll
   for (int x = 0; x < 8; ++x) {
-    const Real* row = row_at<Real>(d, r.idx[x], b);
+    const Real* row = row_at<Real>(d, r.idx[x], slot_mode(d, pm, x, b));
     const C* rc = reinterpret_cast<const C*>(row);
     w.v0[x] = h0 ? rc[l] : zero;
     if constexpr (TWO) w.v1[x] = h1 ? rc[l + 64] : zero;
@@ -1315,9 +1349,9 @@ template <typename Real, bool TWO>
 __device__ inline void unit_wide(const GridConst& g, const DataConst& d, const PointRec<Real>& r, const double* q,
                                  uint32_t b, Real* ov_point, typename Cplx<Real>::T* oc_point,
                                  typename Cplx<Real>::T* lds, bool gamma, bool cart, WideCache<Real>& wc, bool fresh,
-                                 bool table) {
+                                 bool table, const uint32_t* pm) {
   WideRows<Real, TWO> w;
-  wide_load<Real, TWO>(d, r, b, table, w);
+  wide_load<Real, TWO>(d, r, b, table, w, pm);
   wide_sum_store<Real, TWO>(g, d, r, q, b, w, ov_point, oc_point, lds, gamma, cart, wc, fresh);
 }
 
@@ -1479,6 +1513,7 @@ struct TileShape {
 // four slots of tetrahedron t at tab_tet_row + t * 4 * B; only points whose
 // antiphase pivot is slot 0 have one.
 __device__ __forceinline__ uint32_t table_row(const DataConst& d, const Located& P) {
+  if (!d.has_blocks) return kNoCube;
   if (P.cube != kNoCube) return P.cube * 8u * d.B;
   if (P.tet != kNoTet && P.nslot == 4 && P.w[0] != 0.0) return d.tab_tet_row + P.tet * 4u * d.B;
   return kNoCube;
@@ -1546,6 +1581,8 @@ __device__ __forceinline__ void store_record(const GridConst& g, const DataConst
 // overrides the rows the one-pass sums keep in flight (0: their default)
 // table: the cube factor table is built; its points are the first n_coop
 // records, summed by unit_coop where the rows allow it
+// s_pm: with a PermutationTable, eight slot permutations per record
+// (tile_perms; not read for records that the row table serves)
 // WSL: the slots whose antiphases the atom-major wide sums form at a time
 template <typename Real, bool Fast, int L, int SC, int SV, int TB = TILE, int GRP = 0,
           int WSL = wide_tile_slots<Real>()>
@@ -1555,7 +1592,8 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
                                           void* vals_, void* vecs_, typename Cplx<Real>::T* s_wide = nullptr,
                                           bool table = false, uint32_t n_coop = 0,
                                           const GammaFrame<Real>* op_frames = nullptr, bool node_order = false,
-                                          WideGammaLds<Real> wg = {}, uint32_t b_lo = 0, uint32_t b_hi = ~0u) {
+                                          WideGammaLds<Real> wg = {}, uint32_t b_lo = 0, uint32_t b_hi = ~0u,
+                                          const uint32_t* s_pm = nullptr) {
   using C = typename Cplx<Real>::T;
   constexpr int NPH = TileShape<L, SC>::NPH;
   const uint32_t B = d.B;
@@ -1563,6 +1601,7 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
   Real* vals = (Real*)vals_;
   C* vecs = (C*)vecs_;
   const bool cart = d.vec_lu == BRILLE_LU_ANGSTROM;
+  auto pm_of = [&](uint32_t pl) { return s_pm ? s_pm + 8u * pl : nullptr; };
   if constexpr (L == LAYOUT_WIDE) {
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const bool gamma = d.vec_rot == BRILLE_ROT_GAMMA && d.ec[1] > 0;
@@ -1608,7 +1647,7 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
           }
           C v[8][3], acc[3];
           Real vv[8], va;
-          wide_atom_load<Real>(d, r, b, a, on, v, vv);
+          wide_atom_load<Real>(d, r, b, a, on, v, vv, pm_of(pl));
           if (pl != last) {
             last = pl;
             if (m < mpw) {
@@ -1664,7 +1703,7 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
               while (p1 < c1 && s_rec[p1].nslot != 0 && s_rec[p1].trow == rb.trow) ++p1;
             C v[8][3];
             Real vv[8];
-            wide_atom_load<Real>(d, rb, b, a, on, v, vv);
+            wide_atom_load<Real>(d, rb, b, a, on, v, vv, pm_of(p0));
             wide_atom_phase<Real, SL>(d, rb, b, na, mpw, m, on, fac, v, lds);
             for (uint32_t pl = p0; pl < p1; ++pl) {
               if (!on) continue;
@@ -1704,8 +1743,8 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
           for (uint32_t e = lane; e < d.sc; e += 64) oc[(uint64_t)b * d.sc + e] = Elem<C>::zero();
           continue;
         }
-        if (two) unit_wide<Real, true>(g, d, r, s_q + 3 * pl, b, ov, oc, lds, gamma, cart, wc, pl != last, tab);
-        else unit_wide<Real, false>(g, d, r, s_q + 3 * pl, b, ov, oc, lds, gamma, cart, wc, pl != last, tab);
+        if (two) unit_wide<Real, true>(g, d, r, s_q + 3 * pl, b, ov, oc, lds, gamma, cart, wc, pl != last, tab, pm_of(pl));
+        else unit_wide<Real, false>(g, d, r, s_q + 3 * pl, b, ov, oc, lds, gamma, cart, wc, pl != last, tab, pm_of(pl));
         last = pl;
       }
       return;
@@ -1739,7 +1778,7 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
           }
           const bool reuse = tab && r.trow != kNoCube && r.trow == cached;
           if (!reuse) {
-            wide_load<Real, TWO>(d, r, b, tab, w);
+            wide_load<Real, TWO>(d, r, b, tab, w, pm_of(pl));
             wide_phase_rows<Real, TWO>(w);
             cached = (tab && r.trow != kNoCube) ? r.trow : kNoCube;
           }
@@ -1845,14 +1884,27 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
     }
     // with the cooperative sums, every table point went there
     if constexpr (L == LAYOUT_GAMMA) {
-      unit_onepass<Real, SC, SV, true, GRP>(d, r, b, ov, oc, s_ph + NPH * pl, frame_of(pl), table && !kCoop);
+      unit_onepass<Real, SC, SV, true, GRP>(d, r, b, ov, oc, s_ph + NPH * pl, frame_of(pl), table && !kCoop,
+                                             pm_of(pl));
     } else if constexpr (L == LAYOUT_SCALAR) {
-      unit_onepass<Real, SC, SV, false, GRP>(d, r, b, ov, oc, nullptr, nullptr, table && !kCoop);
+      unit_onepass<Real, SC, SV, false, GRP>(d, r, b, ov, oc, nullptr, nullptr, table && !kCoop,
+                                              pm_of(pl));
     } else {
-      unit_generic<Real, !Fast>(g, d, r, s_q + 3 * pl, b, ov, oc, ph_in_lds ? s_ph + NPH * pl : nullptr);
+      unit_generic<Real, !Fast>(g, d, r, s_q + 3 * pl, b, ov, oc, ph_in_lds ? s_ph + NPH * pl : nullptr, pm_of(pl));
     }
   }
 }
+
+// The permutations of the slots of records [first, npts) into LDS, a lane per
+// (record, slot): eight dependent searches in every (point, mode) lane of the
+// sums cost the general sums most of their time (500 009 points, 6 modes FP64:
+// 1.76 ms).  The caller has synchronised the records and does so again.
+template <int TB, typename Real>
+__device__ __forceinline__ void tile_perms(const DataConst& d, const PointRec<Real>* s_rec, uint32_t first,
+                                           uint32_t npts, uint32_t* s_pm) {
+  for (uint32_t k = 8 * first + threadIdx.x; k < 8 * npts; k += TB) s_pm[k] = slot_perm(d, s_rec[k >> 3], k & 7u);
+}
+extern __shared__ uint32_t s_perms[];  // of the tile kernels: 8 words per point, with a PermutationTable
 
 __device__ __forceinline__ void report_point(ErrRec* err, uint64_t index, int status) {
   atomicMin(&err->first_bad, err_key(index, status));
@@ -1909,8 +1961,12 @@ __global__ __launch_bounds__(TILE) void k_ir_interpolate(GridConst g, DataConst 
   const uint32_t npts = left < (uint64_t)a.tile ? (uint32_t)left : a.tile;
   const uint32_t per_group = (d.B + gridDim.y - 1) / gridDim.y;
   const uint32_t b_lo = blockIdx.y * per_group;
+  if (d.n_keys) {
+    tile_perms<TILE>(d, s_rec, 0, npts, s_perms);
+    __syncthreads();
+  }
   tile_sums<Real, Fast, L, SC, SV>(g, d, s_rec, s_ph, s_q, nullptr, tile0, npts, ph_in_lds, a.vals, a.vecs, s_wide,
-                                   false, 0, nullptr, false, {}, b_lo, b_lo + per_group);
+                                   false, 0, nullptr, false, {}, b_lo, b_lo + per_group, d.n_keys ? s_perms : nullptr);
 }
 
 }  // namespace brille_amd

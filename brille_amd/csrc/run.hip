@@ -88,7 +88,7 @@ using TileKernel = void (*)(GridConst, DataConst, LaunchArgs);
 // which specialised phase 2 the payload admits
 int payload_layout(const DataConst& d) {
   const bool scalar_values = d.ev[1] == 0 && d.ev[2] == 0;
-  if (d.n_keys || !scalar_values) return LAYOUT_GENERIC;
+  if (!scalar_values) return LAYOUT_GENERIC;
   if (d.ec[1] == 0 && d.ec[2] == 0) return LAYOUT_SCALAR;
   if (d.ec[0] == 0 && d.ec[2] == 0 && d.vec_rot == BRILLE_ROT_GAMMA &&
       (d.vec_lu == BRILLE_LU_REAL_LATTICE || d.vec_lu == BRILLE_LU_ANGSTROM))
@@ -189,7 +189,8 @@ static void launch_sel(const brille_grid* G, LaunchArgs a, int precision, bool f
     c.vals = static_cast<char*>(a.vals) + c0 * G->d.B * G->d.sv * rs;
     c.vecs = static_cast<char*>(a.vecs) + c0 * G->d.B * G->d.sc * 2 * rs;
     c.aux = offset_aux(a.aux, c0);
-    hipLaunchKernelGGL(k, dim3((unsigned)((c.n + a.tile - 1) / a.tile), groups), dim3(TILE), 0, s, G->g, G->d, c);
+    hipLaunchKernelGGL(k, dim3((unsigned)((c.n + a.tile - 1) / a.tile), groups), dim3(TILE), G->d.n_keys ? 32u * a.tile : 0u, s,
+                       G->g, G->d, c);
   }
 }
 

@@ -591,6 +591,34 @@ __global__ void k_identity_perm(uint32_t* perms, uint32_t B) {
   for (uint32_t q = threadIdx.x; q < B; q += blockDim.x) perms[q] = q;
 }
 
+// vkey[i]: the first key of vertex i (keys sorted, i * V + j)
+__global__ __launch_bounds__(256) void k_vertex_keys(uint64_t V, const uint64_t* __restrict__ keys, uint64_t n_keys,
+                                                     uint32_t* __restrict__ vkey) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > V) return;
+  uint64_t lo = 0, hi = n_keys;
+  while (lo < hi) {
+    const uint64_t mid = (lo + hi) >> 1;
+    if (keys[mid] < i * V) lo = mid + 1;
+    else hi = mid;
+  }
+  vkey[i] = (uint32_t)lo;
+}
+
+// out[t]: the permutation of block slot t against its block's slot-0 vertex
+__global__ __launch_bounds__(256) void k_cell_perms(GridConst g, DataConst d, uint64_t n_cube_slots, uint64_t n_slots,
+                                                    uint32_t* __restrict__ out) {
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n_slots) return;
+  if (t < n_cube_slots) {
+    const uint32_t* v = g.cube_v + 8 * (t >> 3);
+    out[t] = perm_find(d, v[7], v[7 - (int)(t & 7u)]);
+  } else {
+    const uint32_t* v = g.tet_v + 4 * ((t - n_cube_slots) >> 2);
+    out[t] = perm_find(d, v[0], v[(t - n_cube_slots) & 3u]);
+  }
+}
+
 struct DevBuf {
   std::vector<void*> held;
   ~DevBuf() {
@@ -609,6 +637,35 @@ struct DevBuf {
 };
 
 }  // namespace
+
+int install_permutations(brille_grid* G, std::vector<void*>& allocs, hipStream_t s) {
+  DataConst& d = G->d;
+  d.vkey = nullptr;
+  d.cell_perm = nullptr;
+  if (d.n_keys == 0) return BRILLE_OK;
+  void* p = nullptr;
+  if (d.n_keys < 0xFFFFFFFFull) {
+    if (hipMalloc(&p, (d.V + 1) * sizeof(uint32_t)) != hipSuccess)
+      return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the permutation lookup");
+    allocs.push_back(p);
+    uint32_t* vkey = static_cast<uint32_t*>(p);
+    hipLaunchKernelGGL(k_vertex_keys, dim3((unsigned)((d.V + 256) / 256)), dim3(256), 0, s, d.V, d.keys, d.n_keys, vkey);
+    d.vkey = vkey;
+  }
+  const uint64_t cubes = 8 * G->n_cubes, slots = cubes + 4 * G->n_tets;
+  if (d.has_blocks && slots) {
+    if (hipMalloc(&p, slots * sizeof(uint32_t)) != hipSuccess)
+      return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the permutation lookup");
+    allocs.push_back(p);
+    uint32_t* cell = static_cast<uint32_t*>(p);
+    hipLaunchKernelGGL(k_cell_perms, dim3((unsigned)((slots + 255) / 256)), dim3(256), 0, s, G->g, d, cubes, slots, cell);
+    d.cell_perm = cell;
+  }
+  if (hipGetLastError() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "permutation lookup launch failed");
+  // later calls read the lookup from any stream
+  if (hipStreamSynchronize(s) != hipSuccess) return fail(BRILLE_ERR_DEVICE, "permutation lookup failed");
+  return BRILLE_OK;
+}
 }  // namespace brille_amd
 
 using namespace brille_amd;
@@ -764,11 +821,14 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   const uint32_t n_perms = 1 + 2 * n_moved;
   uint32_t* perms_fit = perms_out;
   // install: the previous sorted table goes (after the work still queued on
-  // the device that may read it), a fill-given one stays in the payload
+  // the device that may read it), and the tables derived from the payload and
+  // the permutations with it; a fill-given table stays in the payload
   // allocations until the next fill
   (void)hipDeviceSynchronize();
-  for (void* p : G->sort_allocs) (void)hipFree(p);
-  G->sort_allocs.clear();
+  for (std::vector<void*>* old : {&G->sort_allocs, &G->derived_allocs}) {
+    for (void* p : *old) (void)hipFree(p);
+    old->clear();
+  }
   for (void* p : {(void*)keys, (void*)pidx, (void*)perms_fit}) {
     buf.release(p);
     G->sort_allocs.push_back(p);
@@ -777,15 +837,15 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   d.keys = keys;
   d.perm_index = pidx;
   d.perms = perms_fit;
+  d.vkey = nullptr;
+  d.cell_perm = nullptr;
   G->n_perms = n_perms;
-  // the bucketed row tables hold unpermuted rows; with a table the general
-  // sums run and never read them
   d.cube_rows32 = nullptr;
   d.cube_rows64 = nullptr;
   d.wide_fac32 = nullptr;
   d.wide_fac64 = nullptr;
   ++G->fill_gen;
-  return BRILLE_OK;
+  return install_permutations(G, G->sort_allocs, s);
 }
 
 extern "C" int brille_grid_permutations(const brille_grid* G, uint64_t* n_keys, uint32_t* n_perms, uint64_t* keys,

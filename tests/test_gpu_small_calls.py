@@ -7,11 +7,14 @@ within 1e-5 of the scale), at the edges of the tiles and on points without a
 table block (grid vertices and cell edges, where the first slot weighs
 nothing).  Needs an MI355X.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from brille_amd import capi
 from brille_amd import synthetic as S
+from conftest import CUBE, POLY, hand_trellis
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -76,3 +79,30 @@ def test_a_failing_point_is_reported_once_by_every_split():
     assert np.all(v[3] == 0) and np.all(c[3] == 0) and np.all(np.isfinite(v))
     with pytest.raises(capi.BrilleError, match="Not all points inside Brillouin zone"):
         dev.ir_interpolate_at(Q, precision=capi.FP32, kernel=capi.KERNEL_TILE)
+
+
+def test_wide_rows_of_neighbouring_cells_without_a_table():
+    """A cube and the first tetrahedron of the node beside it, summed one after the other in node
+    order on a handle that never built its factor table: each keeps its own rows."""
+    print("small calls: neighbouring cells", flush=True)
+    corner = [(1, 0, 0), (2, 0, 0), (1, 1, 0), (1, 0, 1)]
+    t = hand_trellis({(0, 0, 0): CUBE, (1, 0, 0): POLY}, {(1, 0, 0): [corner]})
+    V, A, B, G = len(t["vertices"]), 5, 3, len(np.asarray(t["inverse_index"]))
+    r = np.random.default_rng(8)
+    t.update(values=r.normal(size=(V, B, 1)), values_elements=[1, 0, 0], branches=B,
+             vectors=r.normal(size=(V, B, 3 * A)) + 1j * r.normal(size=(V, B, 3 * A)), vectors_elements=[0, 3 * A, 0],
+             vectors_rotates_like=2, vectors_length_unit=3,
+             gamma_F0=np.repeat(np.arange(A, dtype=np.uint32)[:, None], G, 1),
+             gamma_vector_index=np.zeros((A, G), np.uint32), gamma_vectors=np.zeros((1, 3)),
+             gamma_cart_rotations=np.tile(np.eye(3).ravel(), (G, 1)))
+    Q = np.vstack([r.uniform(0.1, 0.9, size=(40, 3)), [1.05, 0.05, 0.05] + r.uniform(0, 0.25, size=(40, 3))])
+    rc, ov, oc, _, _ = O.ir_interpolate_at(t, Q, no_move=True)
+    assert rc == 0
+    dev = capi.Grid(t)
+    n = len(Q)
+    dQ, dv, dc = (capi.DeviceArray.from_host(Q), capi.DeviceArray((n, B, 1), np.float64),
+                  capi.DeviceArray((n, B, 3 * A), np.complex128))
+    o = capi.RunOpts(1, capi.FP64, 0, capi.MEM_DEVICE, capi.KERNEL_BINNED, 1)
+    capi.check(capi.lib().brille_ir_interpolate_at_noalloc(dev.h, dQ.ptr, n, C.byref(o), dv.ptr, dc.ptr, None, None))
+    assert np.max(np.abs(dv.to_host() - ov)) <= 1e-12 * np.abs(ov).max()
+    assert np.max(np.abs(dc.to_host() - oc.reshape(n, B, -1))) <= 1e-12 * np.abs(oc).max()
