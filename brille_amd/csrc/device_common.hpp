@@ -71,6 +71,13 @@ struct GridConst {
   const double* tet_vol;
   const double* verts;
   uint64_t n_nodes;
+  // 1: every cube's vertices share vertex 0's and 7's coordinates exactly
+  uint32_t cubes_aligned;
+  uint32_t pad2;
+  // n_tets x 16 (null: not made): weight j of a point x is about f[4j] x0 +
+  // f[4j+1] x1 + f[4j+2] x2 + f[4j+3]; all zero for a tetrahedron whose forms
+  // could be wrong by more than a tenth of kBarySkip
+  const float* tet_bary;
 };
 
 // Interpolation payload of one grid.

@@ -141,15 +141,16 @@ BRILLE_HD uint32_t find_bin_scan(const double* edges, uint32_t n, double x) {
 }
 
 // the same answer from O(1) arithmetic: guess floor((x - k0)/step) and move
-// to the first stored knot > x, exactly as the scan defines it
+// to the first stored knot > x, exactly as the scan defines it.  (Knot counts
+// fit 32 bits with room, and so does the clamped guess.)
 BRILLE_HD uint32_t find_bin_fast(const double* edges, uint32_t n, double lo, double inv_step, double x) {
+  const double f = fmin(fmax((x - lo) * inv_step, 0.0), (double)(n - 1));  // NaN: 0
+  int32_t d = (int32_t)f + 1;  // candidate index of the first knot > x, in [1, n]
+  const double below = edges[d - 1], above = edges[d < (int32_t)n ? d : (int32_t)n - 1];
+  if (below <= x && (d == (int32_t)n || above > x)) return (uint32_t)(d - 1);
   if (!(x >= edges[0])) return find_bin_scan(edges, n, x);  // NaN or below the first knot
-  double f = fmin((x - lo) * inv_step, (double)n);
-  int64_t d = (int64_t)f + 1;  // candidate index of the first knot > x
-  if (d < 1) d = 1;
-  if (d > (int64_t)n) d = n;
   while (d > 0 && edges[d - 1] > x) --d;
-  while (d < (int64_t)n && !(edges[d] > x)) ++d;
+  while (d < (int32_t)n && !(edges[d] > x)) ++d;
   return d > 0 ? (uint32_t)(d - 1) : 0u;
 }
 
@@ -214,6 +215,12 @@ BRILLE_HD bool node_subscript(const GridConst& g, const double* x, uint64_t* nod
   return false;
 }
 
+// the sides of a cube's vertices along x, y and z: 0 where they share vertex
+// 0's coordinate, 1 where vertex 7's (000, 100, 110, 010, 101, 001, 011, 111)
+constexpr bool kCubeX[8] = {0, 1, 1, 0, 1, 0, 0, 1};
+constexpr bool kCubeY[8] = {0, 0, 1, 1, 0, 0, 1, 1};
+constexpr bool kCubeZ[8] = {0, 0, 0, 0, 1, 1, 1, 1};
+
 // CubeNode::indices_weights  src/trellis_node.hpp:132-149, in fixed slots:
 // slot i holds vertex 7-i and its weight.  A slot the reference drops (weight
 // not > 0) keeps weight 0, so the non-zero slots in slot order are exactly the
@@ -228,6 +235,28 @@ BRILLE_HD void cube_slots(const GridConst& g, uint32_t c, const double* x, uint3
   double node_volume = 1.0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) node_volume *= fabs(v0[k] - v7[k]);
+  if (g.cubes_aligned) {
+    // every vertex's coordinates are, bit for bit, those of vertex 0 or 7
+    // (checked when the grid was made): two gathers instead of eight, and the
+    // same products from the six distances
+    double a[3], b[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      a[k] = fabs(x[k] - v0[k]);
+      b[k] = fabs(x[k] - v7[k]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      double p = 1.0;
+      p *= kCubeX[i] ? b[0] : a[0];
+      p *= kCubeY[i] ? b[1] : a[1];
+      p *= kCubeZ[i] ? b[2] : a[2];
+      const double wi = p / node_volume;
+      idx[i] = v[7 - i];
+      w[i] = cmp_gt(wi, 0.0, tdef) ? wi : 0.0;
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const double* vv = g.verts + 3 * (uint64_t)v[i];
@@ -293,11 +322,34 @@ BRILLE_HD void tet_slots(const GridConst& g, uint64_t t, const double* ww, uint3
   }
 }
 
+constexpr float kBarySkip = 1e-2f;
+
 // PolyNode::indices_weights, should_contain=true  src/trellis_node.hpp:275-308.
 // Fills slots 0..3 and returns the tetrahedron used (kNoTet: node has none).
 BRILLE_HD uint32_t poly_slots(const GridConst& g, uint32_t p, const double* x, uint32_t* idx, double* w, Tol tdef) {
   const uint32_t t0 = g.poly_off[p], t1 = g.poly_off[p + 1];
   double ww[4];
+  if (g.tet_bary) {
+    // A first look through the node's tetrahedra with FP32 barycentric forms:
+    // one whose smallest weight is below -kBarySkip (far beyond the forms'
+    // error) fails the exact containment test and is passed over without its
+    // circumsphere, vertices and determinants.  The first of the others that
+    // passes the exact test is the first of all that does; when none passes,
+    // the literal loop below finds the reference's fallback.
+    const float xf[3] = {(float)x[0], (float)x[1], (float)x[2]};
+    for (uint32_t t = t0; t < t1; ++t) {
+      const float* f = g.tet_bary + 16 * (uint64_t)t;
+      float m = 1.0f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        m = fminf(m, fmaf(f[4 * j], xf[0], fmaf(f[4 * j + 1], xf[1], fmaf(f[4 * j + 2], xf[2], f[4 * j + 3]))));
+      if (m < -kBarySkip) continue;
+      if (tet_contains(g, t, x, ww, true, tdef) >= 0.) {
+        tet_slots(g, t, ww, idx, w, tdef);
+        return t;
+      }
+    }
+  }
   double best = 0.0;
   uint32_t best_t = t0;
   for (uint32_t t = t0; t < t1; ++t) {

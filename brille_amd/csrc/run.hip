@@ -410,6 +410,109 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
   return BRILLE_OK;
 }
 
+// *differ gets a bit for every cube whose vertices do not all have exactly
+// vertex 0's or vertex 7's coordinate along each axis, in CubeNode order
+__global__ __launch_bounds__(256) void k_cube_corners(GridConst g, uint64_t n_cubes, uint32_t* differ) {
+  const uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= n_cubes) return;
+  const uint32_t* v = g.cube_v + 8 * c;
+  const double* v0 = g.verts + 3 * (uint64_t)v[0];
+  const double* v7 = g.verts + 3 * (uint64_t)v[7];
+  bool same = true;
+#pragma unroll
+  for (int i = 1; i < 7; ++i) {
+    const double* p = g.verts + 3 * (uint64_t)v[i];
+    same = same && __double_as_longlong(p[0]) == __double_as_longlong(kCubeX[i] ? v7[0] : v0[0]) &&
+           __double_as_longlong(p[1]) == __double_as_longlong(kCubeY[i] ? v7[1] : v0[1]) &&
+           __double_as_longlong(p[2]) == __double_as_longlong(kCubeZ[i] ? v7[2] : v0[2]);
+  }
+  if (!same) atomicOr(differ, 1u);
+}
+
+// FP32 affine forms of the barycentric weights of every tetrahedron (16 floats
+// each, see GridConst::tet_bary).  The forms are rounded to FP32 and evaluated
+// with x rounded to FP32 and three fused multiply-adds, an error of at most
+// about 8 x 2^-24 (|f| . reach + |c|) for points within `reach` of the origin;
+// a tetrahedron where that exceeds a tenth of kBarySkip, or that is so flat
+// that the exact weights themselves could lose that much, gets zeros.
+__global__ __launch_bounds__(256) void k_tet_bary(GridConst g, uint64_t n_tets, double reach, float* out) {
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n_tets) return;
+  double p[4][3];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) p[j][k] = g.verts[3 * (uint64_t)g.tet_v[4 * t + j] + k];
+  constexpr double kMost = 0.1 * kBarySkip;
+  const double vol6 = 6.0 * g.tet_vol[t];
+  bool fine = 512.0 * DBL_EPSILON * reach * reach * reach < kMost * vol6;
+  float f[16];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    // weight j (pseudo_orient3d with x in place of vertex j, over vol6) vanishes
+    // on the opposite face and is 1 at vertex j: its slope is the face's
+    // normal over the height
+    const double *a = p[(j + 1) & 3], *b = p[(j + 2) & 3], *c = p[(j + 3) & 3];
+    double u[3], v[3], w[3], n[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      u[k] = b[k] - a[k];
+      v[k] = c[k] - a[k];
+      w[k] = p[j][k] - a[k];
+    }
+    n[0] = u[1] * v[2] - u[2] * v[1];
+    n[1] = u[2] * v[0] - u[0] * v[2];
+    n[2] = u[0] * v[1] - u[1] * v[0];
+    const double h = n[0] * w[0] + n[1] * w[1] + n[2] * w[2];  // +-6 V
+    double off = 0, err = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      n[k] /= h;
+      off -= n[k] * a[k];
+      err += fabs(n[k]) * reach;
+      f[4 * j + k] = (float)n[k];
+    }
+    f[4 * j + 3] = (float)off;
+    // |h| is 6 V by either formula, or the forms are not the exact test's weights
+    fine = fine && fabs(fabs(h) - vol6) < 1e-6 * vol6 && 8.0 * 5.9604644775390625e-08 * (err + fabs(off)) < kMost;
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) out[16 * t + k] = fine ? f[k] : 0.0f;
+}
+
+// the location tables derived from the cells: GridConst::cubes_aligned, tet_bary
+static int build_cell_tables(const brille_grid_desc* d, brille_grid* G) {
+  GridConst& g = G->g;
+  g.cubes_aligned = 0;
+  g.tet_bary = nullptr;
+  if (d->n_cubes) {
+    void* flag = nullptr;
+    uint32_t differ = 1;
+    if (hipMalloc(&flag, sizeof(differ)) != hipSuccess) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed");
+    G->grid_allocs.push_back(flag);
+    zero_words(flag, 1, nullptr);
+    hipLaunchKernelGGL(k_cube_corners, dim3((unsigned)((d->n_cubes + 255) / 256)), dim3(256), 0, nullptr, g, d->n_cubes,
+                       static_cast<uint32_t*>(flag));
+    if (hipMemcpy(&differ, flag, sizeof(differ), hipMemcpyDeviceToHost) != hipSuccess)
+      return fail(BRILLE_ERR_DEVICE, "checking the cubes failed");
+    g.cubes_aligned = differ ? 0 : 1;
+  }
+  if (d->n_tets) {
+    double reach = 0;
+    for (int k = 0; k < 3; ++k)
+      if (d->n_knots[k])
+        reach = std::max(reach, std::max(std::abs(d->knots[k][0]), std::abs(d->knots[k][d->n_knots[k] - 1])));
+    void* forms = nullptr;
+    if (hipMalloc(&forms, 16 * d->n_tets * sizeof(float)) != hipSuccess) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed");
+    G->grid_allocs.push_back(forms);
+    hipLaunchKernelGGL(k_tet_bary, dim3((unsigned)((d->n_tets + 255) / 256)), dim3(256), 0, nullptr, g, d->n_tets, reach,
+                       static_cast<float*>(forms));
+    if (hipDeviceSynchronize() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "making the tetrahedron forms failed");
+    g.tet_bary = static_cast<const float*>(forms);
+  }
+  return BRILLE_OK;
+}
+
 // Affine forms of the zone-face orientation tests and the seed orbit of the
 // wedge (see fast_fold.hpp).  pseudo_orient3d(a,b,c,x) in a lattice with
 // reciprocal volume V equals V det[a-x, b-x, c-x] on the components, i.e.
@@ -437,7 +540,7 @@ int build_fast_tables(const brille_grid_desc* d, brille_grid* G) {
   } else {
     g.has_seed = 0;
   }
-  return BRILLE_OK;
+  return build_cell_tables(d, G);
 }
 
 

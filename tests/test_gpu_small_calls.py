@@ -14,7 +14,7 @@ import pytest
 
 from brille_amd import capi
 from brille_amd import synthetic as S
-from conftest import CUBE, POLY, hand_trellis
+from conftest import CUBE, POLY, hand_trellis, tet_record
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -106,3 +106,40 @@ def test_wide_rows_of_neighbouring_cells_without_a_table():
     capi.check(capi.lib().brille_ir_interpolate_at_noalloc(dev.h, dQ.ptr, n, C.byref(o), dv.ptr, dc.ptr, None, None))
     assert np.max(np.abs(dv.to_host() - ov)) <= 1e-12 * np.abs(ov).max()
     assert np.max(np.abs(dc.to_host() - oc.reshape(n, B, -1))) <= 1e-12 * np.abs(oc).max()
+
+
+@pytest.mark.parametrize("height", [0.3, 1e-2, 1e-4, 1e-7, 1e-11])
+def test_flat_tetrahedra_are_located_like_the_oracle(height):
+    """A tetrahedron split by a point `height` above its base: the FP32 forms that pass over the
+    node's other tetrahedra must not pass over a flat one that holds the point."""
+    print(f"small calls: flat tetrahedra {height}", flush=True)
+    a, b, c, d, e = (0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 1)
+    t = hand_trellis({(0, 0, 0): POLY}, {(0, 0, 0): [(e, b, c, d), (a, b, c, e), (a, c, d, e), (a, d, b, e)]})
+    # vertex e moves to `height` above the middle of face b, c, d
+    apex = np.array([1.0, 1.0, 1.0]) * (1 / 3 - height)
+    vid = int(np.nonzero((t["vertices"] == e).all(1))[0][0])
+    t["vertices"] = np.array(t["vertices"])
+    t["vertices"][vid] = apex
+    rec = [tet_record(t["vertices"][v]) for v in t["tet_vertices"]]
+    tv = np.array(t["tet_vertices"])
+    for k, v in enumerate(tv):  # the moved apex can turn a tetrahedron over
+        p = t["vertices"][v]
+        if np.linalg.det(p[:3] - p[3]) < 0:
+            tv[k] = v[[0, 1, 3, 2]]
+    t["tet_vertices"] = tv
+    t["tet_circumsphere"] = np.array([np.append(x[0][:3], x[0][3]) for x in rec])
+    t["tet_volume"] = np.array([x[1] for x in rec])
+    t["values"] = np.array(t["vertices"])[:, None, :].copy()
+    r = np.random.default_rng(4)
+    w = r.dirichlet(np.ones(4), size=600)
+    Q = w @ np.array([a, b, c, d], float)
+    w2 = r.dirichlet(np.ones(4), size=600)
+    Q = np.vstack([Q, w2 @ np.array([apex, b, c, d], float)])  # inside the flat one
+    rc, ov, _, oaux, _ = O.ir_interpolate_at(t, Q, no_move=True)
+    assert rc == 0
+    dev = capi.Grid(t)
+    for kernel in (capi.KERNEL_TILE, capi.KERNEL_BINNED):
+        gv, _, gaux = dev.ir_interpolate_at(Q, no_move=True, kernel=kernel, aux=dict(tau=False))
+        for k in ("node", "tet", "n_iw", "iw_index", "iw_weight"):
+            np.testing.assert_array_equal(gaux[k], oaux[k], err_msg=f"{kernel} {k}")
+        np.testing.assert_allclose(gv, ov, atol=1e-12)
