@@ -848,6 +848,14 @@ static void free_work_space(brille_grid* G) {
   G->bin_ws_bytes = 0;
 }
 
+int ensure_work_space(brille_grid* G, uint64_t bytes) {
+  if (G->bin_ws_bytes >= bytes) return BRILLE_OK;
+  free_work_space(G);
+  if (hipMalloc(&G->bin_ws, bytes) != hipSuccess) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the work space");
+  G->bin_ws_bytes = bytes;
+  return BRILLE_OK;
+}
+
 void free_binned(brille_grid* G) {
   free_work_space(G);
   for (auto& e : G->bin_ev) {
@@ -935,11 +943,7 @@ int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_
   const uint64_t passes = (a.n + chunk - 1) / chunk;
   const int halves = passes > 1 ? 2 : 1;
   const uint64_t need = binned_pass_bytes(G, chunk) * (uint64_t)halves;
-  if (G->bin_ws_bytes < need) {
-    free_work_space(G);
-    if (hipMalloc(&G->bin_ws, need) != hipSuccess) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the binned work space");
-    G->bin_ws_bytes = need;
-  }
+  if (int rc = ensure_work_space(G, need); rc != BRILLE_OK) return rc;
   if (halves > 1)
     if (int rc = ensure_side_stream(G); rc != BRILLE_OK) return rc;
   return run_binned_passes(G, a, precision, s, stage_ms, G->bin_ws, chunk, halves);

@@ -38,7 +38,7 @@ struct brille_grid {
   // staging buffers for host-memory calls
   void* stage = nullptr;
   size_t stage_bytes = 0;
-  // work space of the binned pipeline (grown on demand, kept)
+  // work space of the binned pipeline and the sort (grown on demand, kept)
   void* bin_ws = nullptr;
   size_t bin_ws_bytes = 0;
   // side stream of the binned pipeline (preparation of the next pass) and its
@@ -120,6 +120,9 @@ int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStr
 // bytes of one pass's buffers, and the largest pass whose buffers fit `bytes` (0: none)
 uint64_t binned_pass_bytes(const brille_grid* G, uint64_t chunk);
 uint64_t binned_pass_for(const brille_grid* G, uint64_t bytes);
+// at least `bytes` of the handle's work space; what it held is lost when it
+// grows (the free waits for the device)
+int ensure_work_space(brille_grid* G, uint64_t bytes);
 void free_binned(brille_grid* G);
 // clears n 32-bit words on stream s with a kernel (no memset node, so that a
 // caller may capture the call in a graph)

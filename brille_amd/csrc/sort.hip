@@ -6,15 +6,19 @@
 //    as per-vertex neighbour lists: count, scan, place, then sort and
 //    de-duplicate each list (a vertex has a few dozen entries).  The keys
 //    i * V + j come out sorted, i major.
-// 2. One wave per pair i < j: the B x B cost matrix of the pair
-//    (DualInterpolator::cost_matrix, src/interpolatordual.hpp:384-396, with
-//    Interpolator::add_cost, src/interpolator_cost.tpp:21-58), one entry per
-//    lane at a time in the reference's element order, then the exact linear
-//    assignment by successive shortest augmenting paths with the columns
-//    spread over the lanes (the LDS holds the potentials, the Dijkstra
-//    distances and the matching).  The assignment goes to key (i, j), its
-//    inverse to (j, i) (src/interpolatordual.hpp:422-432); identity
-//    assignments share permutation 0.
+// 2. The easy pairs, in one kernel (k_pair_easy): when the least cost of every
+//    row of the pair's B x B cost matrix (DualInterpolator::cost_matrix,
+//    src/interpolatordual.hpp:384-396) lies in a column of its own and leads
+//    its row by more than rounding, that column-per-row assignment is the
+//    optimum.  The matrix is never stored.
+// 3. The other pairs, listed: their cost matrices entry by entry in the
+//    reference's element order (Interpolator::add_cost,
+//    src/interpolator_cost.tpp:21-58), the same row-minimum test on the exact
+//    costs, then the exact linear assignment by successive shortest augmenting
+//    paths, one wave per pair with the columns spread over the lanes (the LDS
+//    holds the potentials, the Dijkstra distances and the matching).
+// The assignment goes to key (i, j), its inverse to (j, i)
+// (src/interpolatordual.hpp:422-432); identity assignments share permutation 0.
 #include <algorithm>
 #include <vector>
 
@@ -59,58 +63,114 @@ __global__ __launch_bounds__(256) void k_pair_emit(const uint32_t* cube_v, uint6
   }
 }
 
-// each vertex's list sorted and de-duplicated in place; uniq[v] = its length
+// Each vertex's list sorted and de-duplicated in place, one wave per vertex;
+// uniq[v] = its length, fwd[v] = its entries beyond v.  Lists of up to kListMax
+// entries go through the wave's LDS slice (a bitonic sort over the next power
+// of two: an insertion sort by one thread in memory took 1.1 ms for the 121 200
+// lists of the hexagonal grid of 318 472 nodes, this 0.06 ms); longer ones are
+// sorted by one lane.
+constexpr uint32_t kListMax = 512;
 __global__ __launch_bounds__(256) void k_pair_unique(uint64_t V, const uint32_t* __restrict__ off,
                                                      const uint32_t* __restrict__ cnt, uint32_t* __restrict__ adj,
-                                                     uint32_t* __restrict__ uniq) {
-  const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= V) return;
+                                                     uint32_t* __restrict__ uniq, uint32_t* __restrict__ fwd) {
+  __shared__ uint32_t s_list[4][kListMax];
+  const uint64_t v = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (v >= V) return;  // wave-uniform; no block-wide barrier follows
+  const uint32_t lane = threadIdx.x & 63u;
   uint32_t* a = adj + off[v];
   const uint32_t n = cnt[v];
-  for (uint32_t i = 1; i < n; ++i) {
-    const uint32_t x = a[i];
-    uint32_t j = i;
-    while (j > 0 && a[j - 1] > x) {
-      a[j] = a[j - 1];
-      --j;
+  uint32_t m = 0, beyond = 0;
+  if (n <= kListMax) {
+    uint32_t* l = s_list[threadIdx.x >> 6];
+    uint32_t size = 64;
+    while (size < n) size <<= 1;
+    for (uint32_t i = lane; i < size; i += 64) l[i] = i < n ? a[i] : 0xFFFFFFFFu;
+    wave_lds_fence();
+    for (uint32_t k = 2; k <= size; k <<= 1)
+      for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+        for (uint32_t i = lane; i < size; i += 64) {
+          const uint32_t o = i ^ j;
+          if (o > i) {
+            const uint32_t x = l[i], y = l[o];
+            if ((x > y) == ((i & k) == 0)) {
+              l[i] = y;
+              l[o] = x;
+            }
+          }
+        }
+        wave_lds_fence();
+      }
+    for (uint32_t i0 = 0; i0 < n; i0 += 64) {
+      const uint32_t i = i0 + lane;
+      const uint32_t x = i < n ? l[i] : 0u;
+      const bool keep = i < n && (i == 0 || l[i - 1] != x);
+      const unsigned long long mask = __ballot(keep);
+      if (keep) a[m + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = x;
+      m += (uint32_t)__popcll(mask);
+      beyond += (uint32_t)__popcll(__ballot(keep && x > (uint32_t)v));
     }
-    a[j] = x;
+  } else if (lane == 0) {
+    for (uint32_t i = 1; i < n; ++i) {
+      const uint32_t x = a[i];
+      uint32_t j = i;
+      while (j > 0 && a[j - 1] > x) {
+        a[j] = a[j - 1];
+        --j;
+      }
+      a[j] = x;
+    }
+    for (uint32_t i = 0; i < n; ++i)
+      if (m == 0 || a[i] != a[m - 1]) {
+        a[m++] = a[i];
+        beyond += a[m - 1] > (uint32_t)v ? 1u : 0u;
+      }
   }
-  uint32_t m = 0;
-  for (uint32_t i = 0; i < n; ++i)
-    if (m == 0 || a[i] != a[m - 1]) a[m++] = a[i];
-  uniq[v] = m;
+  if (lane == 0) {
+    uniq[v] = m;
+    fwd[v] = beyond;
+  }
 }
 
-// keys i * V + j in list order, and the neighbour j of each key
+// One wave per vertex: its keys i * V + j in list order, the neighbour j of
+// each key, and its forward pairs (j > i, the end of the sorted list) with
+// the key each came from.
 __global__ __launch_bounds__(256) void k_pair_keys(uint64_t V, const uint32_t* __restrict__ off,
-                                                   const uint32_t* __restrict__ adj, const uint32_t* __restrict__ uniq,
-                                                   const uint32_t* __restrict__ koff, uint64_t* __restrict__ keys,
-                                                   uint32_t* __restrict__ nbr) {
-  const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                                   const uint32_t* __restrict__ adj, const uint32_t* __restrict__ koff,
+                                                   const uint32_t* __restrict__ poff, uint64_t* __restrict__ keys,
+                                                   uint32_t* __restrict__ nbr, uint32_t* __restrict__ pi,
+                                                   uint32_t* __restrict__ pj, uint32_t* __restrict__ pk) {
+  const uint64_t v = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (v >= V) return;
   const uint32_t* a = adj + off[v];
-  for (uint32_t k = 0; k < uniq[v]; ++k) {
-    keys[koff[v] + k] = v * V + a[k];
-    nbr[koff[v] + k] = a[k];
+  const uint32_t k0 = koff[v], n = koff[v + 1] - k0, p0 = poff[v], nf = poff[v + 1] - p0;
+  for (uint32_t k = threadIdx.x & 63u; k < n; k += 64) {
+    const uint32_t j = a[k];
+    keys[k0 + k] = v * V + j;
+    nbr[k0 + k] = j;
+    if (k >= n - nf) {
+      const uint32_t p = p0 + (k - (n - nf));
+      pi[p] = (uint32_t)v;
+      pj[p] = j;
+      pk[p] = k0 + k;
+    }
   }
 }
 
-// rev[k]: the position of key (j, i) for key k = (i, j) (the lists are
-// symmetric), by binary search in j's list; one thread per key
-__global__ __launch_bounds__(256) void k_pair_rev(uint64_t V, uint64_t n_keys, const uint64_t* __restrict__ keys,
-                                                  const uint32_t* __restrict__ nbr, const uint32_t* __restrict__ koff,
-                                                  uint32_t* __restrict__ rev) {
-  const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n_keys) return;
-  const uint32_t i = (uint32_t)(keys[k] / V), j = nbr[k];
+// rev[p]: the position of key (j, i) for the forward pair p = (i, j) (the
+// lists are symmetric), by binary search in j's list
+__global__ __launch_bounds__(256) void k_pair_rev(uint64_t n_pairs, const uint32_t* __restrict__ pi,
+                                                  const uint32_t* __restrict__ pj, const uint32_t* __restrict__ nbr,
+                                                  const uint32_t* __restrict__ koff, uint32_t* __restrict__ rev) {
+  const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n_pairs) return;
+  const uint32_t i = pi[p], j = pj[p];
   uint32_t lo = koff[j], hi = koff[j + 1];
   while (lo < hi) {
     const uint32_t mid = (lo + hi) >> 1;
     if (nbr[mid] < i) lo = mid + 1;
     else hi = mid;
   }
-  rev[k] = (lo < koff[j + 1] && nbr[lo] == i) ? lo : 0xFFFFFFFFu;
+  rev[p] = (lo < koff[j + 1] && nbr[lo] == i) ? lo : 0xFFFFFFFFu;
 }
 
 // ---- costs ----------------------------------------------------------------
@@ -314,66 +374,135 @@ __device__ __forceinline__ void wave_argmin(double& v, uint32_t& j) {
   }
 }
 
-// forward pairs (i < j) per vertex: count, then (after a scan) the pair's
-// vertices and key index, in key order
-__global__ __launch_bounds__(256) void k_pair_fwd(uint64_t V, const uint32_t* __restrict__ koff,
-                                                  const uint32_t* __restrict__ nbr, const uint32_t* __restrict__ poff,
-                                                  uint32_t* __restrict__ cnt, uint32_t* __restrict__ pi,
-                                                  uint32_t* __restrict__ pj, uint32_t* __restrict__ pk) {
-  const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= V) return;
-  uint32_t m = 0;
-  for (uint32_t k = koff[v]; k < koff[v + 1]; ++k) {
-    const uint32_t j = nbr[k];
-    if (j <= (uint32_t)v) continue;
-    if (poff) {
-      pi[poff[v] + m] = (uint32_t)v;
-      pj[poff[v] + m] = j;
-      pk[poff[v] + m] = k;
+// The easy pairs, a lane per (pair, mode a of the first vertex): the lane walks
+// the second vertex's modes and keeps the least cost of its row and the runner-
+// up.  For Gamma-like vectors (SC complex vector elements, the default cost
+// sin^2 of the Hermitian angle) the cost needs no phase and no angle:
+// sin^2 = 1 - |a.b|^2 / (|a|^2 |b|^2), some eighty operations against seven
+// hundred, whose value agrees with the literal one to rounding (~1e-14 of the
+// terms); a row whose lead is within kLead of that scale, a norm near zero, or a
+// value that is not finite sends the pair to the literal costs.  Memory: the rows
+// alone (one wave reads each pair's from the cache); 1.4e6 pairs of 6 modes,
+// FP64: 4.1 ms for the stored matrices and their row minima, 0.3 ms here.
+// asg[p * B + a]: the column of row a; hard[p], moved[p]: 0 or 1.
+constexpr double kLead = 1e-9;
+template <typename Real, int SC>
+__global__ __launch_bounds__(256) void k_pair_easy(CostArgs c, const Real* __restrict__ rows,
+                                                   const uint32_t* __restrict__ pi, const uint32_t* __restrict__ pj,
+                                                   const uint32_t* __restrict__ rev, uint64_t n_pairs,
+                                                   uint16_t* __restrict__ asg, uint32_t* __restrict__ hard,
+                                                   uint32_t* __restrict__ moved) {
+  __shared__ uint32_t s_col[256], s_flag[256];  // column of each row; per pair: bit 0 hard, bit 1 moved
+  const uint32_t B = c.B, per = 256 / B, tid = threadIdx.x;
+  const uint32_t lp = tid / B, a = tid - lp * B;
+  const uint64_t p = (uint64_t)blockIdx.x * per + lp;
+  const bool on = lp < per && p < n_pairs;
+  s_flag[tid] = 0;
+  __syncthreads();
+  uint32_t col = 0;
+  if (on) {
+    const Real* ra = rows + ((uint64_t)pi[p] * B + a) * c.stride;
+    const Real* rb = rows + (uint64_t)pj[p] * B * c.stride;
+    double x[2 * SC], aa = 0;
+#pragma unroll
+    for (int k = 0; k < 2 * SC; ++k) {
+      x[k] = (double)ra[k];
+      aa += x[k] * x[k];
     }
-    ++m;
+    double best = __builtin_huge_val(), second = __builtin_huge_val();
+    bool fine = true;
+    for (uint32_t b = 0; b < B; ++b, rb += c.stride) {
+      double s = 0, hr = 0, hi = 0, bb = 0;
+      for (uint32_t z = 0; z < c.ev[0]; ++z) s += fabs((double)ra[2 * SC + z] - (double)rb[2 * SC + z]);
+#pragma unroll
+      for (int k = 0; k < SC; ++k) {
+        const double br = (double)rb[2 * k], bi = (double)rb[2 * k + 1];
+        hr += x[2 * k] * br + x[2 * k + 1] * bi;
+        hi += x[2 * k] * bi - x[2 * k + 1] * br;
+        bb += br * br + bi * bi;
+      }
+      const double cost = c.vw[0] * s + c.cw[1] * (1.0 - (hr * hr + hi * hi) / (aa * bb));
+      fine = fine && aa * bb > 1e-280 && fabs(cost) < 1e300;  // false for NaN
+      if (cost < best) {
+        second = best;
+        best = cost;
+        col = b;
+      } else if (cost < second) {
+        second = cost;
+      }
+    }
+    if (!(fine && second - best > kLead * (fabs(c.cw[1]) + fabs(best)))) atomicOr(&s_flag[lp], 1u);
+    if (col != a) atomicOr(&s_flag[lp], 2u);
   }
-  if (!poff) cnt[v] = m;
+  s_col[tid] = col;
+  __syncthreads();
+  if (on) {
+    for (uint32_t k = 0; k < a; ++k)
+      if (s_col[tid - a + k] == col) {
+        atomicOr(&s_flag[lp], 1u);
+        break;
+      }
+    asg[p * B + a] = (uint16_t)col;
+  }
+  __syncthreads();
+  if (on && a == 0) {
+    const uint32_t f = s_flag[lp];
+    const bool h = (f & 1u) || rev[p] == 0xFFFFFFFFu;
+    hard[p] = h ? 1u : 0u;
+    moved[p] = !h && (f & 2u) ? 1u : 0u;
+  }
 }
 
-// The cost matrices of pairs [p0, p0 + np): one lane per entry (pair, a, b),
-// so every lane of every wave computes (B x B entries per pair).
+__global__ __launch_bounds__(256) void k_fill_words(uint32_t* __restrict__ a, uint64_t n, uint32_t v) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) a[i] = v;
+}
+
+// list[off[p]] = p for the flagged pairs (off: exclusive scan of the flags)
+__global__ __launch_bounds__(256) void k_pair_list(uint64_t n_pairs, const uint32_t* __restrict__ off,
+                                                   uint32_t* __restrict__ list) {
+  const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < n_pairs && off[p + 1] != off[p]) list[off[p]] = (uint32_t)p;
+}
+
+// The cost matrices of the listed pairs [h0, h0 + nh): one lane per entry
+// (pair, a, b), so every lane of every wave computes (B x B entries per pair).
 template <typename Real>
 __global__ __launch_bounds__(256) void k_pair_costs(CostArgs c, const Real* rows, const uint32_t* __restrict__ pi,
-                                                    const uint32_t* __restrict__ pj, uint64_t p0, uint64_t np,
-                                                    double* __restrict__ C, uint32_t* __restrict__ bad) {
+                                                    const uint32_t* __restrict__ pj, const uint32_t* __restrict__ list,
+                                                    uint64_t h0, uint64_t nh, double* __restrict__ C,
+                                                    uint32_t* __restrict__ bad) {
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t B = c.B, BB = B * B;
-  if (t >= np * BB) return;
-  const uint64_t p = t / BB;
-  const uint32_t e = (uint32_t)(t - p * BB);
+  if (t >= nh * BB) return;
+  const uint64_t q = t / BB;
+  const uint32_t e = (uint32_t)(t - q * BB);
   const uint32_t a = e / B, b = e - a * B;
-  const uint64_t i = pi[p0 + p], j = pj[p0 + p];
+  const uint32_t p = list[h0 + q];
+  const uint64_t i = pi[p], j = pj[p];
   bool ok = true;
   C[t] = pair_cost(c, rows + (i * B + a) * c.stride, rows + (j * B + b) * c.stride, ok);
   if (!ok) atomicOr(bad, 1u);
 }
 
-// The easy pairs first, one thread each: when the first minimum of every row
-// of the cost matrix lies in a different column, that column-per-row
-// assignment is the optimum and is exactly what the augmenting-path solver
-// below returns (each row's search then ends at its first minimum, a free
-// column).  Such pairs are written here; the others are flagged (hard[q] = 1)
-// for the full solver.  Matrices of more than 64 columns all go to the solver.
-__global__ __launch_bounds__(256) void k_pair_fast(const double* __restrict__ Cg, uint32_t B, uint64_t p0, uint64_t np,
-                                                   const uint32_t* __restrict__ pk, const uint32_t* __restrict__ rev,
-                                                   uint32_t* __restrict__ perm_index, uint32_t* __restrict__ perms,
-                                                   uint32_t* __restrict__ hard) {
+// The row minima of the stored matrices, one thread per listed pair: when the
+// first minimum of every row lies in a different column, that assignment is
+// exactly what the augmenting-path solver below returns (each row's search
+// then ends at its first minimum, a free column).  The others stay in todo (todo[q] =
+// 1) for the solver.  Matrices of more than 64 columns all go to the solver.
+__global__ __launch_bounds__(256) void k_pair_fast(const double* __restrict__ Cg, uint32_t B,
+                                                   const uint32_t* __restrict__ list, uint64_t h0, uint64_t nh,
+                                                   const uint32_t* __restrict__ rev, uint16_t* __restrict__ asg,
+                                                   uint32_t* __restrict__ moved, uint32_t* __restrict__ todo) {
   const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= np) return;
-  if (B > 64) {
-    hard[q] = 1;
-    return;
-  }
+  if (q >= nh) return;
+  const uint64_t p = list[h0 + q];
+  todo[q] = 1;
+  if (B > 64 || rev[p] == 0xFFFFFFFFu) return;
   const double* C = Cg + q * B * B;
   unsigned long long taken = 0;
-  bool moved = false, ok = true;
-  for (uint32_t a = 0; a < B && ok; ++a) {
+  bool shift = false;
+  for (uint32_t a = 0; a < B; ++a) {
     double best = __builtin_huge_val();
     uint32_t bc = 0xFFFFFFFFu;
     for (uint32_t b = 0; b < B; ++b) {
@@ -383,58 +512,26 @@ __global__ __launch_bounds__(256) void k_pair_fast(const double* __restrict__ Cg
         bc = b;
       }
     }
-    if (bc == 0xFFFFFFFFu || (taken >> bc) & 1ull) ok = false;
-    else taken |= 1ull << bc;
-    moved = moved || bc != a;
+    if (bc == 0xFFFFFFFFu || (taken >> bc) & 1ull) return;
+    taken |= 1ull << bc;
+    shift = shift || bc != a;
+    asg[p * B + a] = (uint16_t)bc;
   }
-  const uint32_t k = pk[p0 + q], rv = rev[k];
-  if (!ok || rv == 0xFFFFFFFFu) {
-    hard[q] = 1;
-    return;
-  }
-  hard[q] = 0;
-  if (!moved) {
-    perm_index[k] = 0;
-    perm_index[rv] = 0;
-    return;
-  }
-  const uint32_t slot = (uint32_t)(1 + 2 * (p0 + q));
-  for (uint32_t a = 0; a < B; ++a) {
-    double best = __builtin_huge_val();
-    uint32_t bc = 0;
-    for (uint32_t b = 0; b < B; ++b) {
-      const double c = C[(uint64_t)a * B + b];
-      if (c < best) {
-        best = c;
-        bc = b;
-      }
-    }
-    perms[(uint64_t)slot * B + a] = bc;          // row: column of row a
-    perms[(uint64_t)(slot + 1) * B + bc] = a;    // inverse
-  }
-  perm_index[k] = slot;
-  perm_index[rv] = slot + 1;
+  todo[q] = 0;
+  moved[p] = shift ? 1u : 0u;
 }
 
-// list[h] = q for the flagged pairs (scan of the flags in `off`)
-__global__ __launch_bounds__(256) void k_pair_hard_list(uint64_t np, const uint32_t* __restrict__ hard,
-                                                        const uint32_t* __restrict__ off, uint32_t* __restrict__ list) {
-  const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < np && hard[q]) list[off[q]] = (uint32_t)q;
-}
-
-// One wave per pair of [p0, p0 + np) (grid-stride): the exact assignment of
-// its cost matrix (copied to LDS when it fits, read from C otherwise).  LDS:
-// potentials u, v, distances minv ((B + 1) doubles each), matching p,
-// predecessors way, scanned flags ((B + 1) words each), the assignment and
-// its inverse (B words each), then the matrix.
-__global__ __launch_bounds__(SORT_BLOCK) void k_pair_lap(const double* __restrict__ Cg, uint32_t B, uint64_t p0,
-                                                         const uint32_t* __restrict__ list,
-                                                         const uint32_t* __restrict__ list_n, int cost_in_lds,
-                                                         const uint32_t* __restrict__ pk,
+// One wave per listed pair of [h0, h0 + nh) still to do (grid-stride): the exact
+// assignment of its cost matrix (copied to LDS when it fits, read from C
+// otherwise).  LDS: potentials u, v, distances minv ((B + 1) doubles each),
+// matching p, predecessors way and scanned flags ((B + 1) words each), then the
+// matrix.
+__global__ __launch_bounds__(SORT_BLOCK) void k_pair_lap(const double* __restrict__ Cg, uint32_t B,
+                                                         const uint32_t* __restrict__ list, uint64_t h0, uint64_t nh,
+                                                         const uint32_t* __restrict__ todo, int cost_in_lds,
                                                          const uint32_t* __restrict__ rev,
-                                                         uint32_t* __restrict__ perm_index,
-                                                         uint32_t* __restrict__ perms, uint32_t* __restrict__ bad) {
+                                                         uint16_t* __restrict__ asg, uint32_t* __restrict__ moved,
+                                                         uint32_t* __restrict__ bad) {
   extern __shared__ double lds[];
   const uint32_t lane = threadIdx.x;
   double* u = lds;
@@ -443,22 +540,18 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_pair_lap(const double* __restric
   int32_t* p = reinterpret_cast<int32_t*>(minv + (B + 1));
   int32_t* way = p + (B + 1);
   int32_t* used = way + (B + 1);
-  uint32_t* rowv = reinterpret_cast<uint32_t*>(used + (B + 1));
-  uint32_t* colv = rowv + B;
-  double* Cl = lds + 3 * (B + 1) + (3 * (B + 1) + 2 * B + 1) / 2;
+  double* Cl = lds + 3 * (B + 1) + (3 * (B + 1) + 1) / 2;
   const double INF = __builtin_huge_val();
   const uint32_t BB = B * B;
-  const uint64_t n_list = *list_n;
-  for (uint64_t h = blockIdx.x; h < n_list; h += gridDim.x) {
-    const uint64_t q0 = list[h];
+  for (uint64_t q0 = blockIdx.x; q0 < nh; q0 += gridDim.x) {
+    if (!todo[q0]) continue;
     const double* C = Cg + q0 * BB;
     if (cost_in_lds) {
       for (uint32_t e = lane; e < BB; e += SORT_BLOCK) Cl[e] = C[e];
       C = Cl;
     }
-    const uint32_t k = pk[p0 + q0];
-    const uint32_t rv = rev[k];
-    const bool has_rev = rv != 0xFFFFFFFFu;  // always, the lists being symmetric
+    const uint64_t pair = list[h0 + q0];
+    const bool has_rev = rev[pair] != 0xFFFFFFFFu;  // always, the lists being symmetric
     for (uint32_t q = lane; q <= B; q += SORT_BLOCK) {
       u[q] = 0;
       v[q] = 0;
@@ -526,65 +619,44 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_pair_lap(const double* __restric
     if (stuck || !has_rev) {
       if (lane == 0) {
         atomicOr(bad, 1u);
-        perm_index[k] = 0;
-        if (has_rev) perm_index[rv] = 0;
+        moved[pair] = 0;
       }
       __syncthreads();
       continue;
     }
-    bool moved = false;
+    bool shift = false;
     for (uint32_t q = 1 + lane; q <= B; q += SORT_BLOCK) {
-      rowv[p[q] - 1] = q - 1;
-      colv[q - 1] = (uint32_t)(p[q] - 1);
-      moved = moved || (uint32_t)(p[q] - 1) != q - 1;
+      asg[pair * B + (uint32_t)(p[q] - 1)] = (uint16_t)(q - 1);
+      shift = shift || (uint32_t)(p[q] - 1) != q - 1;
     }
-    moved = __any(moved);
-    __syncthreads();
-    if (!moved) {
-      if (lane == 0) {
-        perm_index[k] = 0;
-        perm_index[rv] = 0;
-      }
-    } else {
-      // fixed slots per pair (a counter shared by every pair serialised the
-      // kernel on one address); the table is compacted afterwards
-      const uint32_t slot = (uint32_t)(1 + 2 * (p0 + q0));
-      for (uint32_t q = lane; q < B; q += SORT_BLOCK) {
-        perms[(uint64_t)slot * B + q] = rowv[q];
-        perms[(uint64_t)(slot + 1) * B + q] = colv[q];
-      }
-      if (lane == 0) {
-        perm_index[k] = slot;
-        perm_index[rv] = slot + 1;
-      }
-    }
+    shift = __any(shift);
+    if (lane == 0) moved[pair] = shift ? 1u : 0u;
     __syncthreads();  // the LDS is reused by the next pair
   }
 }
 
-// compaction of the table: moved[p] = 1 for pairs whose assignment is not
-// the identity, then (after a scan) their two permutations move from slots
-// 1 + 2p to 1 + 2 scan[p] and both keys are re-pointed
-__global__ __launch_bounds__(256) void k_perm_moved(uint64_t np, const uint32_t* __restrict__ pk,
-                                                    const uint32_t* __restrict__ perm_index,
-                                                    uint32_t* __restrict__ moved) {
-  const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < np) moved[p] = perm_index[pk[p]] != 0u ? 1u : 0u;
-}
-__global__ __launch_bounds__(256) void k_perm_compact(uint64_t np, uint32_t B, const uint32_t* __restrict__ pk,
-                                                      const uint32_t* __restrict__ rev,
-                                                      const uint32_t* __restrict__ scan,
-                                                      uint32_t* __restrict__ perm_index,
-                                                      const uint32_t* __restrict__ perms,
-                                                      uint32_t* __restrict__ out) {
-  const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= np) return;
-  const uint32_t k = pk[p];
-  if (perm_index[k] == 0u) return;
-  const uint64_t from = 1 + 2 * p, to = 1 + 2 * (uint64_t)scan[p];
-  for (uint32_t q = 0; q < 2 * B; ++q) out[to * B + q] = perms[from * B + q];
-  perm_index[k] = (uint32_t)to;
-  perm_index[rev[k]] = (uint32_t)to + 1;
+// The table: pair p's assignment and its inverse at permutations 1 + 2 off[p]
+// and the next (off: exclusive scan of the moved flags), a lane per (pair, row);
+// both keys point there, or to permutation 0 where nothing moved.
+__global__ __launch_bounds__(256) void k_perm_write(uint64_t n_pairs, uint32_t B, const uint16_t* __restrict__ asg,
+                                                    const uint32_t* __restrict__ off, const uint32_t* __restrict__ pk,
+                                                    const uint32_t* __restrict__ rev,
+                                                    uint32_t* __restrict__ perm_index, uint32_t* __restrict__ perms) {
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint64_t p = t / B;
+  if (p >= n_pairs) return;
+  const uint32_t a = (uint32_t)(t - p * B);
+  const bool shift = off[p + 1] != off[p];
+  const uint64_t slot = shift ? 1 + 2 * (uint64_t)off[p] : 0;
+  if (shift) {
+    const uint32_t b = asg[t];
+    perms[slot * B + a] = b;
+    perms[(slot + 1) * B + b] = a;
+  }
+  if (a == 0) {
+    perm_index[pk[p]] = (uint32_t)slot;
+    if (rev[p] != 0xFFFFFFFFu) perm_index[rev[p]] = shift ? (uint32_t)slot + 1 : 0u;
+  }
 }
 
 __global__ void k_identity_perm(uint32_t* perms, uint32_t B) {
@@ -638,6 +710,28 @@ struct DevBuf {
 
 }  // namespace
 
+// launches k_pair_easy where the payload and the cost kinds allow it (false: no)
+static bool launch_easy(const brille_grid* G, const CostArgs& c, const uint32_t* pi, const uint32_t* pj,
+                        const uint32_t* rev, uint64_t n_pairs, uint16_t* asg, uint32_t* hard, uint32_t* moved,
+                        hipStream_t s) {
+  const DataConst& d = G->d;
+  const bool vectors = c.ec[0] == 0 && c.ec[2] == 0 && (c.cv < 1 || c.cv > 4);
+  if (d.B > 64 || c.ev[1] || c.ev[2] || !vectors) return false;
+  const unsigned blocks = (unsigned)((n_pairs + 256 / d.B - 1) / (256 / d.B));
+  auto go = [&](auto k64, auto k32) {
+    if (d.rows64) hipLaunchKernelGGL(k64, dim3(blocks), dim3(256), 0, s, c, d.rows64, pi, pj, rev, n_pairs, asg, hard, moved);
+    else hipLaunchKernelGGL(k32, dim3(blocks), dim3(256), 0, s, c, d.rows32, pi, pj, rev, n_pairs, asg, hard, moved);
+    return true;
+  };
+  switch (c.sc) {
+    case 3: return go(k_pair_easy<double, 3>, k_pair_easy<float, 3>);
+    case 6: return go(k_pair_easy<double, 6>, k_pair_easy<float, 6>);
+    case 9: return go(k_pair_easy<double, 9>, k_pair_easy<float, 9>);
+    case 12: return go(k_pair_easy<double, 12>, k_pair_easy<float, 12>);
+    default: return false;
+  }
+}
+
 int install_permutations(brille_grid* G, std::vector<void*>& allocs, hipStream_t s) {
   DataConst& d = G->d;
   d.vkey = nullptr;
@@ -684,53 +778,64 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   if (d.V > 0xFFFFFFFFull) return fail(BRILLE_ERR_UNSUPPORTED, "sorting supports at most 2^32 - 1 vertices");
   const uint64_t V = d.V;
   const hipStream_t s = 0;
+  // earlier work may still use the handle's work space and the tables replaced
+  // below
+  if (hipDeviceSynchronize() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "device error before sorting");
   DevBuf buf;
   const uint64_t units = 8 * G->n_cubes + 4 * G->n_tets;
+  const uint64_t most = 56 * G->n_cubes + 12 * G->n_tets;  // ordered pairs emitted, at most
+  if (most > 0xFFFFFFFFull) return fail(BRILLE_ERR_UNSUPPORTED, "sorting supports at most 2^32 - 1 vertex pairs");
   const uint64_t scan_words = (V + 1 + 4095) / 4096 + 1;
-  uint32_t* cnt = buf.get<uint32_t>(V + 1);
-  uint32_t* off = buf.get<uint32_t>(V + 1);
-  uint32_t* part = buf.get<uint32_t>(scan_words);
-  if (!cnt || !off || !part) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the sort work space");
-  zero_words(cnt, (uint32_t)(V + 1), s);
-  const unsigned ub = (unsigned)((units + 255) / 256), vb = (unsigned)((V + 255) / 256);
+  // lists, offsets and scans in one allocation
+  uint32_t* ws0 = buf.get<uint32_t>(5 * (V + 1) + scan_words + 4 + most);
+  if (!ws0) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the sort work space");
+  uint32_t* cnt = ws0;
+  uint32_t* off = cnt + (V + 1);
+  uint32_t* koff = off + (V + 1);
+  uint32_t* poff = koff + (V + 1);
+  uint32_t* cursor = poff + (V + 1);
+  uint32_t* part = cursor + (V + 1);
+  uint32_t* counter = part + scan_words;
+  uint32_t* adj = counter + 4;
+  zero_words(ws0, (uint32_t)(5 * (V + 1) + scan_words + 4), s);
+  const unsigned ub = (unsigned)((units + 255) / 256), wb = (unsigned)((V + 3) / 4);
   if (units) hipLaunchKernelGGL(k_pair_emit<0>, dim3(ub), dim3(256), 0, s, G->g.cube_v, G->n_cubes, G->g.tet_v, G->n_tets, cnt, off, nullptr);
   if (hipMemcpyAsync(off, cnt, (V + 1) * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
     return fail(BRILLE_ERR_DEVICE, "hipMemcpyAsync failed");
   if (int rc = exclusive_scan_u32(off, V + 1, part, s); rc != BRILLE_OK) return rc;
-  uint32_t total = 0;
-  if (hipMemcpyAsync(&total, off + V, 4, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
-    return fail(BRILLE_ERR_DEVICE, "reading the pair count failed");
-  uint32_t* adj = buf.get<uint32_t>(total);
-  uint32_t* uniq = buf.get<uint32_t>(V + 1);
-  uint32_t* koff = buf.get<uint32_t>(V + 1);
-  if (!adj || !uniq || !koff) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the sort work space");
-  zero_words(cnt, (uint32_t)(V + 1), s);
-  if (units) hipLaunchKernelGGL(k_pair_emit<1>, dim3(ub), dim3(256), 0, s, G->g.cube_v, G->n_cubes, G->g.tet_v, G->n_tets, cnt, off, adj);
-  zero_words(uniq, (uint32_t)(V + 1), s);
-  hipLaunchKernelGGL(k_pair_unique, dim3(vb), dim3(256), 0, s, V, off, cnt, adj, uniq);
-  if (hipMemcpyAsync(koff, uniq, (V + 1) * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
-    return fail(BRILLE_ERR_DEVICE, "hipMemcpyAsync failed");
+  if (units) hipLaunchKernelGGL(k_pair_emit<1>, dim3(ub), dim3(256), 0, s, G->g.cube_v, G->n_cubes, G->g.tet_v, G->n_tets, cursor, off, adj);
+  hipLaunchKernelGGL(k_pair_unique, dim3(wb), dim3(256), 0, s, V, off, cnt, adj, koff, poff);
   if (int rc = exclusive_scan_u32(koff, V + 1, part, s); rc != BRILLE_OK) return rc;
-  uint32_t nk32 = 0;
-  if (hipMemcpyAsync(&nk32, koff + V, 4, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
-    return fail(BRILLE_ERR_DEVICE, "reading the key count failed");
-  const uint64_t n_keys = nk32;
-  // the new table: keys, per-key permutation index, permutations (at most
-  // one per key plus the identity; trimmed below)
+  if (int rc = exclusive_scan_u32(poff, V + 1, part, s); rc != BRILLE_OK) return rc;
+  uint32_t n32[2] = {0, 0};
+  if (hipMemcpyAsync(&n32[0], koff + V, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+      hipMemcpyAsync(&n32[1], poff + V, 4, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
+    return fail(BRILLE_ERR_DEVICE, "reading the pair counts failed");
+  const uint64_t n_keys = n32[0], n_pairs = n32[1];
+  // the new table: keys and per-key permutation index here, the permutations
+  // once their number is known
   uint64_t* keys = buf.get<uint64_t>(n_keys);
-  uint32_t* nbr = buf.get<uint32_t>(n_keys);
   uint32_t* pidx = buf.get<uint32_t>(n_keys);
-  uint32_t* perms = buf.get<uint32_t>((n_keys + 1) * (uint64_t)d.B);
-  uint32_t* counter = buf.get<uint32_t>(2);
-  if (!keys || !nbr || !pidx || !perms || !counter) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the permutation table");
-  hipLaunchKernelGGL(k_pair_keys, dim3(vb), dim3(256), 0, s, V, off, adj, uniq, koff, keys, nbr);
-  uint32_t* rev = buf.get<uint32_t>(n_keys);
-  if (!rev) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the sort work space");
-  if (n_keys)
-    hipLaunchKernelGGL(k_pair_rev, dim3((unsigned)((n_keys + 255) / 256)), dim3(256), 0, s, V, n_keys, keys, nbr, koff,
-                       rev);
-  hipLaunchKernelGGL(k_identity_perm, dim3(1), dim3(256), 0, s, perms, d.B);
-  zero_words(counter, 2, s);
+  if (!keys || !pidx) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the permutation table");
+  // the rest of the work space is the binned pipeline's, grown when it is
+  // smaller (its calls and this one hold the handle's lock in turn, and the
+  // device was synchronised above): allocating and freeing as much anew took a
+  // third of a sort of 1.4e6 pairs
+  const uint64_t hwords = (n_pairs + 1 + 4095) / 4096 + 1;
+  const uint64_t words = n_keys + 4 * n_pairs + 3 * (n_pairs + 1) + hwords;
+  const uint64_t ws_bytes = words * 4 + n_pairs * d.B * 2 + 16;
+  if (int rc = ensure_work_space(G, ws_bytes); rc != BRILLE_OK) return rc;
+  uint32_t* nbr = static_cast<uint32_t*>(G->bin_ws);
+  uint32_t* pi = nbr + n_keys;
+  uint32_t* pj = pi + n_pairs;
+  uint32_t* pk = pj + n_pairs;
+  uint32_t* rev = pk + n_pairs;
+  uint32_t* hard = rev + n_pairs;          // flags, then their exclusive scan
+  uint32_t* moved = hard + (n_pairs + 1);  // flags, then their exclusive scan
+  uint32_t* keep = moved + (n_pairs + 1);  // the moved flags, kept while hard pairs are left
+  uint32_t* hpart = keep + (n_pairs + 1);
+  uint16_t* asg = reinterpret_cast<uint16_t*>(hpart + hwords);
+  hipLaunchKernelGGL(k_pair_keys, dim3(wb), dim3(256), 0, s, V, off, adj, koff, poff, keys, nbr, pi, pj, pk);
   CostArgs ca{};
   ca.B = d.B;
   ca.sv = d.sv;
@@ -746,85 +851,76 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   ca.cs = cc.scalar_cost;
   ca.cv = cc.vector_cost;
   ca.stride = d.rows64 ? d.stride64 : d.stride32;
-  // the forward pairs (i < j) in key order
-  uint32_t* fcnt = buf.get<uint32_t>(V + 1);
-  if (!fcnt) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the sort work space");
-  zero_words(fcnt, (uint32_t)(V + 1), s);
-  hipLaunchKernelGGL(k_pair_fwd, dim3(vb), dim3(256), 0, s, V, koff, nbr, (const uint32_t*)nullptr, fcnt,
-                     (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr);
-  if (int rc = exclusive_scan_u32(fcnt, V + 1, part, s); rc != BRILLE_OK) return rc;
-  uint32_t np32 = 0;
-  if (hipMemcpyAsync(&np32, fcnt + V, 4, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
-    return fail(BRILLE_ERR_DEVICE, "reading the pair count failed");
-  const uint64_t n_pairs = np32;
-  uint32_t* pi = buf.get<uint32_t>(n_pairs);
-  uint32_t* pj = buf.get<uint32_t>(n_pairs);
-  uint32_t* pk = buf.get<uint32_t>(n_pairs);
-  if (!pi || !pj || !pk) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the sort work space");
-  hipLaunchKernelGGL(k_pair_fwd, dim3(vb), dim3(256), 0, s, V, koff, nbr, (const uint32_t*)fcnt, (uint32_t*)nullptr,
-                     pi, pj, pk);
-  // pairs in chunks whose cost matrices take at most 512 MB
-  const uint64_t BB = (uint64_t)d.B * d.B;
-  const uint64_t chunk = std::max<uint64_t>(1, std::min<uint64_t>(n_pairs, (512ull << 20) / (BB * 8)));
-  double* cost = buf.get<double>(std::max<uint64_t>(chunk, 1) * BB);
-  uint32_t* hard = buf.get<uint32_t>(chunk + 1);
-  uint32_t* hoff = buf.get<uint32_t>(chunk + 1);
-  uint32_t* hpart = buf.get<uint32_t>((chunk + 1 + 4095) / 4096 + 1);
-  uint32_t* hlist = buf.get<uint32_t>(chunk);
-  if (!cost || !hard || !hoff || !hpart || !hlist) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the cost matrices");
-  const size_t lds_state = 3 * (d.B + 1) * sizeof(double) + ((3 * (d.B + 1) + 2 * d.B + 1) / 2) * sizeof(double);
-  const int cost_in_lds = lds_state + BB * sizeof(double) <= 48 * 1024 ? 1 : 0;
-  const size_t lds = lds_state + (cost_in_lds ? BB * sizeof(double) : 0);
-  const unsigned lap_blocks = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(chunk, (uint64_t)std::max(G->n_cu, 1u) * 32));
-  for (uint64_t p0 = 0; p0 < n_pairs; p0 += chunk) {
-    const uint64_t np = std::min<uint64_t>(chunk, n_pairs - p0);
-    const unsigned cb = (unsigned)((np * BB + 255) / 256);
-    if (d.rows64)
-      hipLaunchKernelGGL(k_pair_costs<double>, dim3(cb), dim3(256), 0, s, ca, d.rows64, pi, pj, p0, np, cost, counter + 1);
-    else
-      hipLaunchKernelGGL(k_pair_costs<float>, dim3(cb), dim3(256), 0, s, ca, d.rows32, pi, pj, p0, np, cost, counter + 1);
-    const unsigned qb = (unsigned)((np + 255) / 256);
-    hipLaunchKernelGGL(k_pair_fast, dim3(qb), dim3(256), 0, s, (const double*)cost, d.B, p0, np, pk, rev, pidx, perms,
-                       hard);
-    // offsets of the flagged pairs (flags kept for the listing)
-    if (hipMemcpyAsync(hoff, hard, np * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
-      return fail(BRILLE_ERR_DEVICE, "hipMemcpyAsync failed");
-    zero_words(hoff + np, 1, s);
-    if (int rc = exclusive_scan_u32(hoff, np + 1, hpart, s); rc != BRILLE_OK) return rc;
-    hipLaunchKernelGGL(k_pair_hard_list, dim3(qb), dim3(256), 0, s, np, hard, hoff, hlist);
-    hipLaunchKernelGGL(k_pair_lap, dim3(lap_blocks), dim3(SORT_BLOCK), lds, s, (const double*)cost, d.B, p0,
-                       (const uint32_t*)hlist, (const uint32_t*)(hoff + np), cost_in_lds, pk, rev, pidx, perms,
-                       counter + 1);
-  }
-  // compact: the non-identity pairs' permutations, in pair order
-  uint32_t* moved = buf.get<uint32_t>(n_pairs + 1);
-  uint32_t* ppart = buf.get<uint32_t>((n_pairs + 1 + 4095) / 4096 + 1);
-  if (!moved || !ppart) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the sort work space");
-  zero_words(moved, (uint32_t)(n_pairs + 1), s);
   const unsigned pb = (unsigned)((n_pairs + 255) / 256);
-  if (n_pairs) hipLaunchKernelGGL(k_perm_moved, dim3(pb), dim3(256), 0, s, n_pairs, pk, pidx, moved);
-  if (int rc = exclusive_scan_u32(moved, n_pairs + 1, ppart, s); rc != BRILLE_OK) return rc;
-  uint32_t n_moved = 0;
-  if (hipMemcpyAsync(&n_moved, moved + n_pairs, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess)
-    return fail(BRILLE_ERR_DEVICE, "sort failed");
-  uint32_t* perms_out = buf.get<uint32_t>((1 + 2 * (uint64_t)n_moved) * d.B);
-  if (!perms_out) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the permutation table");
-  hipLaunchKernelGGL(k_identity_perm, dim3(1), dim3(256), 0, s, perms_out, d.B);
-  if (n_pairs) hipLaunchKernelGGL(k_perm_compact, dim3(pb), dim3(256), 0, s, n_pairs, d.B, pk, rev, moved, pidx,
-                                  perms, perms_out);
+  uint32_t n_hard = 0, n_moved = 0;
+  // exclusive scan of n_pairs flags (one word more: the total)
+  auto scan_flags = [&](uint32_t* a) {
+    zero_words(a + n_pairs, 1, s);
+    return exclusive_scan_u32(a, n_pairs + 1, hpart, s);
+  };
+  if (n_pairs) {
+    hipLaunchKernelGGL(k_pair_rev, dim3(pb), dim3(256), 0, s, n_pairs, pi, pj, nbr, koff, rev);
+    const bool easy = launch_easy(G, ca, pi, pj, rev, n_pairs, asg, hard, keep, s);
+    if (!easy) {
+      hipLaunchKernelGGL(k_fill_words, dim3(pb), dim3(256), 0, s, hard, n_pairs, 1u);
+      hipLaunchKernelGGL(k_fill_words, dim3(pb), dim3(256), 0, s, keep, n_pairs, 0u);
+    }
+    if (int rc = scan_flags(hard); rc != BRILLE_OK) return rc;
+    auto scan_moved = [&]() -> int {
+      if (hipMemcpyAsync(moved, keep, n_pairs * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
+        return fail(BRILLE_ERR_DEVICE, "hipMemcpyAsync failed");
+      if (int rc = scan_flags(moved); rc != BRILLE_OK) return rc;
+      if (hipMemcpyAsync(&n_moved, moved + n_pairs, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+          hipMemcpyAsync(&n_hard, hard + n_pairs, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+          hipStreamSynchronize(s) != hipSuccess)
+        return fail(BRILLE_ERR_DEVICE, "sort failed");
+      return BRILLE_OK;
+    };
+    if (int rc = scan_moved(); rc != BRILLE_OK) return rc;
+    if (n_hard) {
+      // listed pairs in chunks whose cost matrices take at most 512 MB
+      const uint64_t BB = (uint64_t)d.B * d.B;
+      const uint64_t chunk = std::max<uint64_t>(1, std::min<uint64_t>(n_hard, (512ull << 20) / (BB * 8)));
+      double* cost = buf.get<double>(chunk * BB);
+      uint32_t* list = buf.get<uint32_t>(n_hard);
+      uint32_t* todo = buf.get<uint32_t>(chunk);
+      if (!cost || !list || !todo) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the cost matrices");
+      hipLaunchKernelGGL(k_pair_list, dim3(pb), dim3(256), 0, s, n_pairs, hard, list);
+      const size_t lds_state = 3 * (d.B + 1) * sizeof(double) + ((3 * (d.B + 1) + 1) / 2) * sizeof(double);
+      const int cost_in_lds = lds_state + BB * sizeof(double) <= 48 * 1024 ? 1 : 0;
+      const size_t lds = lds_state + (cost_in_lds ? BB * sizeof(double) : 0);
+      const unsigned lap_blocks = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(chunk, (uint64_t)std::max(G->n_cu, 1u) * 32));
+      for (uint64_t h0 = 0; h0 < n_hard; h0 += chunk) {
+        const uint64_t nh = std::min<uint64_t>(chunk, n_hard - h0);
+        const unsigned cb = (unsigned)((nh * BB + 255) / 256), qb = (unsigned)((nh + 255) / 256);
+        if (d.rows64)
+          hipLaunchKernelGGL(k_pair_costs<double>, dim3(cb), dim3(256), 0, s, ca, d.rows64, pi, pj, list, h0, nh, cost, counter + 1);
+        else
+          hipLaunchKernelGGL(k_pair_costs<float>, dim3(cb), dim3(256), 0, s, ca, d.rows32, pi, pj, list, h0, nh, cost, counter + 1);
+        hipLaunchKernelGGL(k_pair_fast, dim3(qb), dim3(256), 0, s, (const double*)cost, d.B, list, h0, nh, rev, asg, keep,
+                           todo);
+        hipLaunchKernelGGL(k_pair_lap, dim3(lap_blocks), dim3(SORT_BLOCK), lds, s, (const double*)cost, d.B, list, h0, nh,
+                           todo, cost_in_lds, rev, asg, keep, counter + 1);
+      }
+      if (int rc = scan_moved(); rc != BRILLE_OK) return rc;
+    }
+  }
+  const uint32_t n_perms = 1 + 2 * n_moved;
+  uint32_t* perms_fit = buf.get<uint32_t>((uint64_t)n_perms * d.B);
+  if (!perms_fit) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the permutation table");
+  hipLaunchKernelGGL(k_identity_perm, dim3(1), dim3(256), 0, s, perms_fit, d.B);
+  if (n_pairs)
+    hipLaunchKernelGGL(k_perm_write, dim3((unsigned)((n_pairs * d.B + 255) / 256)), dim3(256), 0, s, n_pairs, d.B, asg,
+                       moved, pk, rev, pidx, perms_fit);
   if (hipGetLastError() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "sort launch failed");
   uint32_t hc[2] = {0, 0};
   if (hipMemcpyAsync(hc, counter, 8, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
     return fail(BRILLE_ERR_DEVICE, "sort failed");
   if (hc[1]) return fail(BRILLE_ERR_NUMERIC, "Complex Hermitian angle cos(theta) > 1 while sorting");
-  const uint32_t n_perms = 1 + 2 * n_moved;
-  uint32_t* perms_fit = perms_out;
-  // install: the previous sorted table goes (after the work still queued on
-  // the device that may read it), and the tables derived from the payload and
-  // the permutations with it; a fill-given table stays in the payload
-  // allocations until the next fill
-  (void)hipDeviceSynchronize();
+  // install: the previous sorted table goes, and the tables derived from the
+  // payload and the permutations with it (the calls queued before this one have
+  // ended, and others wait for the handle's lock); a fill-given table stays in
+  // the payload allocations until the next fill
   for (std::vector<void*>* old : {&G->sort_allocs, &G->derived_allocs}) {
     for (void* p : *old) (void)hipFree(p);
     old->clear();

@@ -10,6 +10,7 @@ import pytest
 from brille_amd import capi
 from brille_amd import synthetic as S
 from oracle import oracle as O
+from test_gpu_sort import device_table, oracle_table
 
 pytestmark = pytest.mark.gpu
 
@@ -124,3 +125,55 @@ def test_a_batch_follows_a_member_sorted_after_its_first_run():
             tv, tc = d.ir_interpolate_at(Q, precision=prec, kernel=capi.KERNEL_TILE)
             np.testing.assert_array_equal(v.to_host(), tv.reshape(v.shape))
             np.testing.assert_array_equal(c.to_host(), tc.reshape(c.shape))
+
+
+@pytest.mark.parametrize("kind,spread", [("a2", 1e-10), ("a4", 1e-11), ("a2", 1e-6)])
+def test_sort_of_near_ties_takes_the_exact_costs(kind, spread):
+    """At some vertices two modes' vectors differ by `spread`: below the lead the one-kernel
+    assignment asks for, such pairs go to the stored cost matrices and the solver; the table stays
+    the oracle's.  No two such vertices share a cell: two near-equal modes on both sides swap at a
+    cost of spread squared, a tie; and values that differ alone tie too, two absolute differences
+    summed crosswise being the same sum."""
+    print(f"sort near ties: {kind} {spread}", flush=True)
+    t, _ = small_tables(kind)
+    r = np.random.default_rng(12)
+    vals, vecs = np.array(t["values"]), np.array(t["vectors"])
+    B = vals.shape[1]
+    near = O.sort_keys(t)
+    near = np.stack([near // len(vals), near % len(vals)], 1).astype(np.int64)
+    free = np.ones(len(vals), bool)
+    for v in r.permutation(len(vals)):
+        if not free[v]:
+            continue
+        free[near[near[:, 0] == v, 1]] = False
+        a, b = r.choice(B, 2, replace=False)
+        vals[v, b] = vals[v, a]
+        vecs[v, b] = vecs[v, a] + spread * (r.normal(size=vecs.shape[2]) + 1j * r.normal(size=vecs.shape[2]))
+    t["values"], t["vectors"] = vals, vecs
+    keys, perms = oracle_table(t, nthreads=8)
+    dev = capi.Grid(t)
+    dev.sort()
+    gk, gp = device_table(dev)
+    np.testing.assert_array_equal(gk, keys)
+    np.testing.assert_array_equal(gp, perms)
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, 1e200, 0.0])
+def test_sort_of_values_beyond_the_cheap_costs(value):
+    """A NaN or an overflowing vector reaches the literal costs, which report it; zero norms are sorted."""
+    print(f"sort of {value}", flush=True)
+    t, _ = small_tables("a2")
+    t["vectors"] = np.array(t["vectors"])
+    t["vectors"][7, 2] = value
+    dev = capi.Grid(t)
+    if value == 0.0:
+        dev.sort()
+        keys, perms = oracle_table(t, nthreads=8)
+        gk, gp = device_table(dev)
+        np.testing.assert_array_equal(gk, keys)
+        np.testing.assert_array_equal(gp, perms)
+    else:
+        with pytest.raises(capi.BrilleError):
+            dev.sort()
+        # the grid stays usable without a table
+        assert len(dev.permutations()[0]) == 0
