@@ -379,17 +379,22 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nb) {
 
 // waves per SIMD asked of the compiler: the atom-major wide sums run best at
 // four (FP32) and two (FP64), a few registers below what it would take for
-// the antiphases of the rare points without a table block
+// the antiphases of the rare points without a table block, and so do the narrow
+// Gamma sums, whose one-lane-per-unit sums of those points would take up to
+// twice the registers of the rest.  (Two atoms FP64 at three waves: 112 bytes
+// of scratch in the walk, 3 000 017 points 1.03 -> 1.92 ms.)
 template <typename Real, int L, int SC>
 constexpr int sums_waves() {
-  return L == LAYOUT_WIDE && SC == kWideAtom ? (sizeof(Real) == 4 ? 4 : 2) : 1;
+  if (L == LAYOUT_WIDE && SC == kWideAtom) return sizeof(Real) == 4 ? 4 : 2;
+  if (L == LAYOUT_GAMMA) return sizeof(Real) == 4 ? 4 : 2;
+  return 1;
 }
 template <typename Real, int L, int SC, int SV, bool Prop>
 __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(sums_waves<Real, L, SC>())))
 void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
                                                     const uint32_t* perm, uint32_t n, void* __restrict__ vals,
                                                     void* __restrict__ vecs, brille_aux_out aux,
-                                                    ErrRec* __restrict__ err, uint64_t base) {
+                                                    ErrRec* __restrict__ err, uint64_t base, uint32_t tile_pts) {
   using C = typename Cplx<Real>::T;
   constexpr int WSL = wide_bin_slots<Real>();
   using S = TileShape<L, SC, TILE, Real, WSL>;
@@ -408,20 +413,28 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
   __shared__ GammaFrame<Real> s_frames[kOpFrames ? kMaxOps : 1];
   if (kOpFrames && threadIdx.x < g.G) fill_frame<Real, SC>(g, d, threadIdx.x, s_frames[threadIdx.x]);
   __shared__ uint32_t s_out[TILE];
-  __shared__ C s_wide[S::NW];
+  // wide rows' slices, or the atom lanes' records
+  constexpr uint32_t kWalk = kOpFrames ? TILE / 64 * walk_slice<Real>() / sizeof(C) : 1;
+  __shared__ __attribute__((aligned(16))) C s_wide[(uint32_t)S::NW > kWalk ? S::NW : kWalk];
   __shared__ uint32_t s_tried, s_verified;
   if (Prop && threadIdx.x == 0) {
     s_tried = 0;
     s_verified = 0;
   }
-  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  const uint32_t tile0 = tile * TILE;
+  // wide rows take fewer points per block in passes of few points (tile_pts of
+  // the TILE a block's LDS holds); the others always TILE
+  const uint32_t tile_n = kWide ? tile_pts : (uint32_t)TILE;
+  const uint32_t tile0 = xcd_tile(blockIdx.x, gridDim.x) * tile_n;
   const uint32_t tid = threadIdx.x;
   const uint32_t p = tile0 + tid;
   // wide rows: blockIdx.y picks a group of modes (gridDim.y groups; the
   // first one reports the points' errors and aux outputs)
   const bool lead = blockIdx.y == 0;
-  const uint32_t per_group = (d.B + gridDim.y - 1) / gridDim.y;
+  uint32_t per_group = (d.B + gridDim.y - 1) / gridDim.y;
+  if (L == LAYOUT_WIDE && SC == kWideAtom) {  // whole passes of the atom-major walk
+    const uint32_t mpw = 64u / (d.sc / 3u);
+    per_group = (per_group + mpw - 1) / mpw * mpw;
+  }
   const uint32_t b_lo = blockIdx.y * per_group, b_hi = b_lo + per_group;
   const bool want_phase = d.vec_rot == BRILLE_ROT_GAMMA && d.ec[1] > 0;
   const uint32_t n_atoms = d.ec[1] / 3u;
@@ -436,7 +449,7 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
   }
   __shared__ uint32_t s_wave_tab[TILE / 64];
   if (Prop) __syncthreads();
-  const bool live = p < n;
+  const bool live = tid < tile_n && p < n;
   SortRec sr;
   Located P;
   P.status = BRILLE_PT_OK;
@@ -469,7 +482,8 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
   }
   // Stable partition of the tile: points the cube factor table serves first,
   // so that few waves of the sums mix the two kinds of point.
-  const bool table = (L == LAYOUT_GAMMA || L == LAYOUT_SCALAR) && cube_rows<Real>(d) != nullptr;
+  // (a GammaTable that is not one to one keeps to the sums of one lane per unit)
+  const bool table = ((L == LAYOUT_GAMMA && d.gamma_maps) || L == LAYOUT_SCALAR) && cube_rows<Real>(d) != nullptr;
   const bool tab = table && live && P.status == BRILLE_PT_OK && table_row(d, P) != kNoCube;
   const uint32_t lane = tid & 63u, wave = tid >> 6;
   const unsigned long long bal = __ballot(tab);
@@ -499,10 +513,10 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
     atomicAdd(&pc.stats[0], (unsigned long long)s_tried);
     atomicAdd(&pc.stats[1], (unsigned long long)s_verified);
   }
-  const uint32_t npts = n - tile0 < (uint32_t)TILE ? n - tile0 : (uint32_t)TILE;
+  const uint32_t npts = n - tile0 < tile_n ? n - tile0 : tile_n;
   const uint32_t* pm = nullptr;
   if (d.n_keys) {  // the row table's rows are permuted already
-    tile_perms<TILE>(d, s_rec, table ? n_tab : 0u, npts, s_perms);
+    tile_perms<TILE>(d, s_rec, n_tab, npts, s_perms);
     __syncthreads();
     pm = s_perms;
   }
@@ -637,7 +651,7 @@ __global__ __launch_bounds__(256) void k_wide_atom_factors(GridConst g, DataCons
 }
 
 using SumsKernel = void (*)(GridConst, DataConst, ProposalConst, const SortRec*, const uint32_t*, uint32_t, void*,
-                           void*, brille_aux_out, ErrRec*, uint64_t);
+                           void*, brille_aux_out, ErrRec*, uint64_t, uint32_t);
 
 template <typename Real>
 static SumsKernel pick_sums(const DataConst& d, bool prop) {
@@ -670,19 +684,26 @@ static SumsKernel pick_sums(const DataConst& d, bool prop) {
   return k_bin_sums<Real, LAYOUT_GENERIC, 0, 0, false>;
 }
 
-// Mode groups of the sums of a pass of m points (blockIdx.y): wide rows put
-// a tile's modes in sequence on its four waves, so a pass of few tiles would
-// leave most CUs idle; its modes are split over up to B / 4 blocks per tile
-// until the pass has about eight blocks per CU (each group repeats phase 1,
-// a few FP64 predicates per point).  Other kernels pick_sums selects (the
-// proposal's among them): one group.
-static uint32_t sum_groups(const brille_grid* G, uint32_t m, bool prop) {
-  if (prop || !wide_rows(G->d)) return 1;
-  const uint32_t tiles = (m + TILE - 1) / TILE;
-  const uint32_t want = 8u * std::max<uint32_t>(G->n_cu, 1);
-  const uint32_t max_groups = std::max<uint32_t>((G->d.B + 3) / 4, 1);
-  const uint32_t g = (want + tiles - 1) / std::max<uint32_t>(tiles, 1);
-  return std::max<uint32_t>(1, std::min(g, max_groups));
+// Points per block and mode groups (blockIdx.y) of the sums of a pass of m
+// points.  Wide rows put a tile's modes in sequence on its four waves, so a
+// pass of few points would leave most CUs idle: its tiles shrink until the
+// pass has about eight blocks per CU or kLeastWideTile points are left (below
+// that the runs of one table block are cut), then the modes split over blocks
+// (each group repeats phase 1 and its points' Gamma phases).  3001 points of 72
+// modes FP32: 0.68 ms in 256-point tiles of 18 groups, kept below.  Other
+// kernels pick_sums selects (the proposal's among them): TILE points, one group.
+constexpr uint32_t kLeastWideTile = 32;
+static void sum_split(const brille_grid* G, uint32_t m, bool prop, uint32_t* tile, uint32_t* groups) {
+  *tile = TILE;
+  *groups = 1;
+  const DataConst& d = G->d;
+  if (prop || !wide_rows(d)) return;
+  const uint64_t want = 8ull * std::max<uint32_t>(G->n_cu, 1);
+  while (*tile > kLeastWideTile && (m + *tile - 1) / *tile < want) *tile >>= 1;
+  const uint64_t tiles = std::max<uint64_t>((m + *tile - 1) / *tile, 1);
+  const uint32_t mpw = wide_by_atom(d) ? 64u / (d.sc / 3u) : 4u;
+  const uint32_t most = std::max<uint32_t>((d.B + mpw - 1) / mpw, 1);
+  *groups = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want / tiles, most));
 }
 
 // SC of the one-pass sums kernel pick_sums selects, or 0 for the general ones
@@ -798,16 +819,42 @@ int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s) {
 // few enough that a bucketing block (BIN_SPAN points) puts runs of records
 // into each: the scatter writes a block's records of one bucket as one run,
 // and short runs cost partial-line writes.  Config 4 at 1e8 Q: 1024 nodes per
-// bucket 26.7 ms, 2048 26.6 ms, 4096 25.9 ms per call.
+// bucket 26.7 ms, 2048 26.6 ms, 4096 25.9 ms per call.  A grid of few nodes
+// still gets kMinBuckets of them (at most one per node): k_bucket_perm runs a
+// block per bucket, and sixteen blocks left the chip idle (1e7 points of a
+// 360-node grid: bucketing 1.24 ms with 16).
 constexpr uint32_t kNodesPerBucket = kPermNodes;
+constexpr uint32_t kMinBuckets = 256;
 static uint32_t bucket_count(const brille_grid* G) {
   const uint64_t n_nodes = std::max<uint64_t>(G->g.n_nodes, 1);
-  uint32_t nb = 16;
+  uint32_t nb = kMinBuckets;
   while (nb < 2048 && (uint64_t)nb * kNodesPerBucket < n_nodes) nb <<= 1;
   return (uint32_t)std::min<uint64_t>(nb, n_nodes);
 }
 
-bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel) {
+// the derived table of a precision exists (or the payload has none)
+static bool has_table(const DataConst& d, int precision) {
+  if (wide_rows(d)) return precision == BRILLE_FP32 ? d.wide_fac32 != nullptr : d.wide_fac64 != nullptr;
+  if (onepass_sc(d) == 0) return true;
+  return precision == BRILLE_FP32 ? d.cube_rows32 != nullptr : d.cube_rows64 != nullptr;
+}
+
+// AUTO's choice between the fused tile kernel and the binned pipeline, on the
+// complex elements summed (n B sc) of Gamma rows.  The pipeline's fixed cost is
+// nine launches; its sums read antiphased rows and reuse them over a node's
+// points.  Measured with the tables built, tile against binned (us):
+//   2 atoms FP32: 300 007 points 140 / 160, 600 011 256 / 218 (46 MB payload
+//     330 / 328); FP64: 100 003 128 / 125, 200 003 239 / 160 (93 MB: 299 / 286)
+//   4 atoms FP32: 60 013 138 / 150, 100 003 235 / 152; FP64: 60 013 157 / 155
+//   8 atoms FP32: 10 007 128 / 126, 30 001 277 / 168; FP64: 3001 97 / 120
+//   24 atoms FP32: 3001 266 / 272, 10 001 799 / 547; FP64: 1001 290 / 226
+// A first call also builds the table, whose rows it would mostly compute for
+// itself anyway once there is a point for every four cells; a call that may
+// not build it (`build` false) is binned from the size where node order alone
+// pays.  Scalar rows are so short that bucketing them costs more than it saves
+// (6 modes, 556 830 vertices, 1 000 003 points: 274 / 370) until the payload
+// is far beyond the caches.
+bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool build) {
   if (kernel == BRILLE_KERNEL_PLAIN || kernel == BRILLE_KERNEL_TILE) return false;
   const brille_aux_out& x = a.aux;
   // the records carry no tau; the sums keep a Gamma frame per point-group
@@ -816,10 +863,25 @@ bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel) {
   if (a.use_proposal || kernel == BRILLE_KERNEL_BINNED) return true;
   if (x.ir_q || x.rot || x.invrot || x.node || x.tet || x.n_iw || x.iw_index || x.iw_weight || x.status)
     return false;
-  // automatic: large calls on payloads that do not fit the L2 of one XCD
   const DataConst& d = G->d;
   const uint64_t payload = (uint64_t)d.V * d.B * d.stride32 * 4;
-  return a.n >= (1ull << 18) && payload > (8ull << 20);
+  const bool scalars = payload_layout(d) == LAYOUT_SCALAR && !wide_rows(d);
+  // large calls on payloads that do not fit the L2 of one XCD
+  if (a.n >= (1ull << 18) && payload > (scalars ? 512ull << 20 : 8ull << 20)) return true;
+  if (payload_layout(d) != LAYOUT_GAMMA || !(wide_rows(d) || onepass_sc(d))) return false;
+  if (!has_table(d, precision) && !(build && 4 * a.n >= G->n_cubes + G->n_tets / 2)) return false;
+  const uint64_t work = a.n * d.B * d.sc;
+  if (wide_rows(d)) return work >= (precision == BRILLE_FP32 ? 20000000ull : 4000000ull);
+  return work >= (precision == BRILLE_FP32 ? 13000000ull : 7000000ull);
+}
+
+// whether a binned call of n points would allocate or build nothing, so that
+// it can be captured in a graph
+bool binned_ready(const brille_grid* G, uint64_t n, int precision) {
+  const uint64_t chunk = std::min<uint64_t>(n, BIN_CHUNK);
+  const int halves = n > chunk ? 2 : 1;
+  return has_table(G->d, precision) && G->bin_ws_bytes >= binned_pass_bytes(G, chunk) * (uint64_t)halves &&
+         (halves == 1 || G->bin_side);
 }
 
 __global__ void k_zero_words(uint32_t* p, uint32_t n) {
@@ -1040,10 +1102,12 @@ int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStr
     }
     // sums of pass k on the call stream
     mark(k, 3, s);
-    const dim3 sgrid((m + TILE - 1) / TILE, sum_groups(G, m, prop));
+    uint32_t tile_pts, groups;
+    sum_split(G, m, prop, &tile_pts, &groups);
+    const dim3 sgrid((m + tile_pts - 1) / tile_pts, groups);
     hipLaunchKernelGGL(sums, sgrid, dim3(TILE), G->d.n_keys ? 32u * TILE : 0u, s, G->g, G->d, a.prop, b.srt, b.perm, m,
                        static_cast<char*>(a.vals) + c0 * vb, static_cast<char*>(a.vecs) + c0 * cb,
-                       offset_aux(a.aux, c0), a.err, a.base + c0);
+                       offset_aux(a.aux, c0), a.err, a.base + c0, tile_pts);
     mark(k, 4, s);
     if (halves > 1) (void)hipEventRecord(G->bin_ev[EV_DONE + h], s);
   }

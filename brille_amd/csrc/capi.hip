@@ -464,6 +464,13 @@ static int grid_fill(brille_grid* G, const brille_data_desc* vals, const brille_
   if (gamma) {
     d.n_atoms = gamma->n_atoms;
     d.gamma_ops = gamma->n_ops;
+    d.gamma_maps = 1;
+    for (uint32_t op = 0; op < gamma->n_ops && d.gamma_maps; ++op) {
+      std::vector<bool> seen(gamma->n_atoms, false);
+      for (uint32_t a = 0; a < gamma->n_atoms; ++a) seen[gamma->F0[(size_t)a * gamma->n_ops + op]] = true;
+      for (uint32_t a = 0; a < gamma->n_atoms; ++a)
+        if (!seen[a]) d.gamma_maps = 0;
+    }
     chk(upload(gamma->F0, (size_t)gamma->n_atoms * gamma->n_ops, &d.F0, A));
     chk(upload(gamma->vector_index, (size_t)gamma->n_atoms * gamma->n_ops, &d.vidx, A));
     chk(upload(gamma->vectors, 3 * (size_t)gamma->n_vectors, &d.gvec, A));

@@ -113,6 +113,7 @@ struct DataConst {
   // GammaTable
   uint32_t n_atoms, gamma_ops;
   const uint32_t* F0;
+  uint32_t gamma_maps;  // 1: every operation maps the atoms one to one
   const uint32_t* vidx;
   const double* gvec;
   // gvec[vidx[k * gamma_ops + op]] for every (atom k, op), 3 doubles each:

@@ -111,7 +111,9 @@ inline brille_aux_out offset_aux(const brille_aux_out& x, uint64_t c0) {
   return o;
 }
 // binned pipeline (binned.hip)
-bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel);
+// (build: the call may build the derived table)
+bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool build = true);
+bool binned_ready(const brille_grid* G, uint64_t n, int precision);
 int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms);
 // the pipeline on a given work space: passes of `chunk` points, `halves` = 2
 // overlaps preparation and sums (grid side stream), 1 runs all on `s`

@@ -614,20 +614,16 @@ __device__ __forceinline__ typename Cplx<Real>::T slot_antiphase(const Real* p, 
 // product rounded first and the weight applied with one fused multiply-add:
 // the cube row table stores the rounded products, so points summed from the
 // table and points summed on the fly get the same bits.
-// table: antiphased rows from the cube row table for the points it serves
 template <typename Real, int SC, int SV, bool GAMMA, int GRP = 0>
 __device__ __forceinline__ void unit_onepass(const DataConst& d, const PointRec<Real>& r, uint32_t b, Real* ov,
                                              typename Cplx<Real>::T* oc, const typename Cplx<Real>::T* phases,
-                                             const GammaFrame<Real>* fr, bool table = false,
-                                             const uint32_t* pm = nullptr) {
+                                             const GammaFrame<Real>* fr, const uint32_t* pm) {
   using C = typename Cplx<Real>::T;
   constexpr int NR = 2 * SC + SV;
   const Real* base = payload_rows<Real>(d);
   const uint64_t stride = payload_stride<Real>(d);
-  // only cube points with the pivot in slot 0 have rows in the table
-  const bool tab = table && r.trow != kNoCube;
   Real pr[2 * SC];
-  if (!tab) load_row<Real, 2 * SC>(pr, base + ((uint64_t)r.pivot * d.B + b) * stride);
+  load_row<Real, 2 * SC>(pr, base + ((uint64_t)r.pivot * d.B + b) * stride);
   Real acc[2 * SC];
   Real vacc[SV];
 #pragma unroll
@@ -642,34 +638,21 @@ __device__ __forceinline__ void unit_onepass(const DataConst& d, const PointRec<
   uint32_t md[8];  // the row of mode b in every slot
 #pragma unroll
   for (int x = 0; x < 8; ++x) md[x] = b;
-  if (pm && !tab) {
+  if (pm) {
 #pragma unroll
     for (int x = 0; x < 8; ++x) md[x] = perm_mode(d, pm[x], b);
   }
 #pragma unroll
   for (int x0 = 0; x0 < 8; x0 += GR) {
     Real row[GR][NR];
-    if (tab) {
 #pragma unroll
-      for (int x = 0; x < GR; ++x) {
-        // a tetrahedron's block has four slots; the others weigh 0
-        if (x0 + x < r.nslot) {
-          load_row<Real, NR>(row[x], table_row_at<Real>(d, r.trow, x0 + x, b));
-        } else {
+    for (int x = 0; x < GR; ++x) load_row<Real, NR>(row[x], base + ((uint64_t)r.idx[x0 + x] * d.B + md[x0 + x]) * stride);
 #pragma unroll
-          for (int k = 0; k < NR; ++k) row[x][k] = 0;
-        }
-      }
-    } else {
+    for (int x = 0; x < GR; ++x) {
+      const C e = slot_antiphase<Real, SC>(pr, row[x]);
 #pragma unroll
-      for (int x = 0; x < GR; ++x) load_row<Real, NR>(row[x], base + ((uint64_t)r.idx[x0 + x] * d.B + md[x0 + x]) * stride);
-#pragma unroll
-      for (int x = 0; x < GR; ++x) {
-        const C e = slot_antiphase<Real, SC>(pr, row[x]);
-#pragma unroll
-        for (int k = 0; k < SC; ++k)
-          phase_elem<Real>(e, row[x][2 * k], row[x][2 * k + 1], &row[x][2 * k], &row[x][2 * k + 1]);
-      }
+      for (int k = 0; k < SC; ++k)
+        phase_elem<Real>(e, row[x][2 * k], row[x][2 * k + 1], &row[x][2 * k], &row[x][2 * k + 1]);
     }
 #pragma unroll
     for (int x = 0; x < GR; ++x) {
@@ -705,7 +688,7 @@ __device__ __forceinline__ void unit_onepass(const DataConst& d, const PointRec<
 }
 
 // ---------------------------------------------------------------------------
-// Cooperative one-pass sums for the points the cube row table serves: G lanes
+// Cooperative one-pass sums of scalar rows for the points the cube row table serves: G lanes
 // per (point, mode) unit, lane q reading the 16-byte chunk q of each of the
 // unit's eight antiphased rows.  A cube's rows for one slot lie mode after
 // mode, so one wave load brings whole rows from a few cache lines instead of a
@@ -721,48 +704,6 @@ constexpr int coop_lanes() {
   int p = 16;
   while (p < bytes) p <<= 1;
   return p / 16;
-}
-
-// the value of lane SRC of this lane's aligned group of G lanes
-template <int G, int SRC>
-__device__ __forceinline__ int grp_bcast_i(int v) {
-  static_assert(G == 2 || G == 4 || G == 8, "groups of 2, 4 or 8 lanes");
-  static_assert(SRC >= 0 && SRC < G, "source lane inside the group");
-  if constexpr (G == 4) {
-    return __builtin_amdgcn_mov_dpp(v, SRC * 0x55, 0xF, 0xF, false);
-  } else if constexpr (G == 2) {
-    return __builtin_amdgcn_mov_dpp(v, SRC | (SRC << 2) | ((2 + SRC) << 4) | ((2 + SRC) << 6), 0xF, 0xF, false);
-  } else {
-    // ds_swizzle bit mode: source lane = (lane & 0x18) | SRC within each half wave
-    return __builtin_amdgcn_ds_swizzle(v, 0x18 | (SRC << 5));
-  }
-}
-template <int G, int SRC>
-__device__ __forceinline__ float grp_bcast(float v) {
-  return __int_as_float(grp_bcast_i<G, SRC>(__float_as_int(v)));
-}
-template <int G, int SRC>
-__device__ __forceinline__ double grp_bcast(double v) {
-  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-  const int lo = grp_bcast_i<G, SRC>((int)(uint32_t)u);
-  const int hi = grp_bcast_i<G, SRC>((int)(uint32_t)(u >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo));
-}
-
-// complex element M of the group's accumulator (lane M / CPL, pair M % CPL)
-template <typename Real, int G, int CPL, int M>
-__device__ __forceinline__ typename Cplx<Real>::T grp_elem(const Real* acc) {
-  typename Cplx<Real>::T e;
-  e.x = grp_bcast<G, (M / CPL) % G>(acc[2 * (M % CPL)]);
-  e.y = grp_bcast<G, (M / CPL) % G>(acc[2 * (M % CPL) + 1]);
-  return e;
-}
-template <typename Real, int G, int CPL, int SC, int M = 0>
-__device__ __forceinline__ void grp_gather(const Real* acc, typename Cplx<Real>::T* all) {
-  if constexpr (M < SC) {
-    all[M] = grp_elem<Real, G, CPL, M>(acc);
-    grp_gather<Real, G, CPL, SC, M + 1>(acc, all);
-  }
 }
 
 // one lane's 16-byte chunk of a row
@@ -793,10 +734,9 @@ __device__ __forceinline__ void coop_load(const DataConst& d, const PointRec<Rea
 }
 
 // the weighted sum of a unit's chunks and the unit's outputs (see coop_load)
-template <typename Real, int SC, int SV, bool GAMMA, int G>
+template <typename Real, int SC, int SV>
 __device__ __forceinline__ void unit_coop(const PointRec<Real>& r, const Chunk<Real>* rows, uint32_t q, Real* ov,
-                                          typename Cplx<Real>::T* oc, const typename Cplx<Real>::T* phases,
-                                          const GammaFrame<Real>* fr) {
+                                          typename Cplx<Real>::T* oc) {
   using C = typename Cplx<Real>::T;
   constexpr int CPL = 8 / (int)sizeof(Real);  // complex pairs per 16-byte chunk
   Real acc[2 * CPL];
@@ -818,60 +758,20 @@ __device__ __forceinline__ void unit_coop(const PointRec<Real>& r, const Chunk<R
     if (vi >= 0 && vi < SV) ov[vi] = acc[2 * h];
     if (vi >= 0 && vi + 1 < SV) ov[vi + 1] = acc[2 * h + 1];
   }
-  C out[CPL];
-  bool put[CPL];
-  if constexpr (GAMMA) {
-    C all[SC];
-    grp_gather<Real, G, CPL, SC>(acc, all);
-#pragma unroll
-    for (int h = 0; h < CPL; ++h) {
-      const uint32_t m = q * CPL + h;
-      out[h] = all[0];
-      // output element m: component j of output atom m / 3, taken from the
-      // source atom a the GammaTable maps there (none: unit_onepass leaves the
-      // element unwritten too)
-      const uint32_t oa = m / 3u, j = m - 3u * oa;
-      const uint32_t a = m < (uint32_t)SC ? fr->from[oa < 4u ? oa : 0u] : 255u;
-      put[h] = a != 255u;
-      if (!put[h]) continue;
-      C v[3];
-      v[0] = v[1] = v[2] = all[0];
-#pragma unroll
-      for (int s = 0; s < SC / 3; ++s) {
-        if ((uint32_t)s == a) {
-          v[0] = all[3 * s];
-          v[1] = all[3 * s + 1];
-          v[2] = all[3 * s + 2];
-        }
-      }
-      const Real* R = fr->R + 3 * j;
-      C t = Elem<C>::zero();
-#pragma unroll
-      for (int k = 0; k < 3; ++k) t = Elem<C>::add(t, Elem<C>::scale(v[k], R[k]));
-      out[h] = cmul(phases[a], t);
-    }
-  } else {
-#pragma unroll
-    for (int h = 0; h < CPL; ++h) {
-      out[h] = C{acc[2 * h], acc[2 * h + 1]};
-      put[h] = q * CPL + h < (uint32_t)SC;
-    }
-  }
-  // the lane's elements in one 16-byte store where they are whole and aligned;
-  // nontemporal, since a point's vectors are whole 16-byte pieces from
-  // neighbouring lanes, not read again (plain stores here cost the sums 10 %)
+  // the lane's elements in one 16-byte store where they are whole and aligned
   C* dst = oc + q * CPL;
   if constexpr (CPL == 2) {
-    if (put[0] && put[1] && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
+    if (q * CPL + 1 < (uint32_t)SC && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
       typedef Real real4 __attribute__((ext_vector_type(4)));
-      __builtin_nontemporal_store(real4{out[0].x, out[0].y, out[1].x, out[1].y}, reinterpret_cast<real4*>(dst));
+      __builtin_nontemporal_store(real4{acc[0], acc[1], acc[2], acc[3]}, reinterpret_cast<real4*>(dst));
       return;
     }
   }
   typedef Real real2 __attribute__((ext_vector_type(2)));
 #pragma unroll
   for (int h = 0; h < CPL; ++h)
-    if (put[h]) __builtin_nontemporal_store(real2{out[h].x, out[h].y}, reinterpret_cast<real2*>(dst + h));
+    if (q * CPL + h < (uint32_t)SC)
+      __builtin_nontemporal_store(real2{acc[2 * h], acc[2 * h + 1]}, reinterpret_cast<real2*>(dst + h));
 }
 
 // Payload layouts with a specialised phase 2 (the general one handles all).
@@ -1165,6 +1065,105 @@ __device__ __forceinline__ void wide_atom_store(const typename Cplx<Real>::T* ac
     for (int j = 0; j < 3; ++j) tt = Elem<C>::add(tt, Elem<C>::scale(acc[j], R[3 * i + j]));
     const C o = cmul(ph, tt);
     *reinterpret_cast<real2*>(dst + i) = real2{o.x, o.y};
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Atom lanes: the node-ordered sums of narrow Gamma rows (SC / 3 atoms) for the
+// records the row table serves, the first n of a tile.  A lane takes (point
+// slot, mode, atom): S point slots of a wave each walk their own run of
+// consecutive points and keep their block's antiphased rows in registers, so a
+// lane rotates its own atom with no exchange between lanes, and a wave of two
+// atoms and six modes sums five points at once.  Every element gets
+// unit_onepass's arithmetic in the same order.  (Lane groups sharing a row's
+// 16-byte chunks instead spent more on gathering the atoms' elements across
+// lanes than on the sums.)
+// The rotated elements of an iteration's points go through the wave's LDS
+// slice, so that the wave writes each record's 16-byte pieces as one run.
+template <typename Real>
+constexpr uint32_t walk_slice() {  // bytes per wave: 64 lanes of three elements
+  return 64 * 3 * 2 * (uint32_t)sizeof(Real);
+}
+template <typename Real, int SC, int SV, int TB>
+__device__ __forceinline__ void gamma_walk(const DataConst& d, const PointRec<Real>* s_rec,
+                                           const typename Cplx<Real>::T* s_ph, const GammaFrame<Real>* frames,
+                                           const uint32_t* out_row, uint32_t n, Real* vals,
+                                           typename Cplx<Real>::T* vecs, char* slice) {
+  using C = typename Cplx<Real>::T;
+  constexpr uint32_t NA = SC / 3;
+  static_assert(SV <= (int)NA, "a lane per value");
+  const uint32_t B = d.B, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t mb = B < 64u / NA ? B : 64u / NA;  // modes at once
+  const uint32_t S = 64u / (mb * NA);               // point slots
+  const uint32_t s = lane / (mb * NA), rem = lane - s * mb * NA, bl = rem / NA, a = rem - bl * NA;
+  const uint32_t share = (n + TB / 64 - 1) / (TB / 64);
+  const uint32_t w0 = wave * share < n ? wave * share : n, w1 = w0 + share < n ? w0 + share : n;
+  const uint32_t run = (w1 - w0 + S - 1) / S;
+  const uint32_t p0 = w0 + s * run;
+  const uint32_t p1 = p0 + run < w1 ? p0 + run : w1;
+  const uint32_t stride = payload_stride<Real>(d);
+  C* sv_vec = reinterpret_cast<C*>(slice);
+  typedef uint32_t piece_t __attribute__((ext_vector_type(4)));
+  typedef uint32_t half_t __attribute__((ext_vector_type(2)));
+  for (uint32_t b0 = 0; b0 < B; b0 += mb) {
+    const uint32_t nb = B - b0 < mb ? B - b0 : mb;
+    const uint32_t b = b0 + bl;
+    const bool on = s < S && b < B;
+    // a record's share of this round: nb rows of SC elements, in 16-byte
+    // pieces where every record's start and length allow it, else 8
+    const uint32_t bytes = nb * SC * (uint32_t)sizeof(C);
+    const bool wide = sizeof(Real) == 8 || ((((uintptr_t)vecs | (B * SC * sizeof(C)) | (b0 * SC * sizeof(C)) | bytes) & 15u) == 0);
+    const uint32_t sh = wide ? 4u : 3u, per = bytes >> sh, pieces = S * per;
+    uint32_t cached = kNoCube;
+    C v[8][3];
+    Real vv[8];
+    for (uint32_t it = 0; it < run; ++it) {
+      const uint32_t pl = p0 + it;
+      if (on && pl < p1) {
+        const PointRec<Real>& r = s_rec[pl];
+        if (r.trow != cached) {
+          cached = r.trow;
+          const Real* base = cube_rows<Real>(d) + ((uint64_t)cached + b) * stride;
+#pragma unroll
+          for (int x = 0; x < 8; ++x) {
+            const Real* row = base + (uint64_t)x * B * stride;
+            const bool use = x < 4 || r.nslot == 8;  // a tetrahedron's block has four slots
+            const C* rc = reinterpret_cast<const C*>(row) + 3u * a;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) v[x][i] = use ? rc[i] : Elem<C>::zero();
+            vv[x] = use && a < (uint32_t)SV ? row[2 * SC + a] : (Real)0;
+          }
+        }
+        C acc[3];
+        Real va;
+        wide_atom_sum<Real>(r, v, vv, acc, &va);
+        const GammaFrame<Real>& f = frames[r.invrot];
+        const C ph = s_ph[NA * pl + a];
+        C* dst = sv_vec + (s * nb + bl) * SC + 3u * f.to[a];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          C tt = Elem<C>::zero();
+#pragma unroll
+          for (int k = 0; k < 3; ++k) tt = Elem<C>::add(tt, Elem<C>::scale(acc[k], f.R[3 * i + k]));
+          dst[i] = cmul(ph, tt);
+        }
+        if (a < (uint32_t)SV) vals[((uint64_t)out_row[pl] * B + b) * SV + a] = va;
+      }
+      wave_lds_fence();
+      for (uint32_t c = lane; c < pieces; c += 64) {
+        const uint32_t ps = c / per, q = c - ps * per;
+        const uint32_t pp0 = w0 + ps * run, pp = pp0 + it;
+        if (pp < w1 && it < run) {
+          char* out = reinterpret_cast<char*>(vecs + ((uint64_t)out_row[pp] * B + b0) * SC) + (q << sh);
+          if (wide)
+            __builtin_nontemporal_store(*reinterpret_cast<const piece_t*>(slice + ((uint64_t)c << 4)),
+                                        reinterpret_cast<piece_t*>(out));
+          else
+            *reinterpret_cast<half_t*>(out) = *reinterpret_cast<const half_t*>(slice + ((uint64_t)c << 3));
+        }
+      }
+      wave_lds_fence();
+    }
   }
 }
 
@@ -1687,20 +1686,25 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
           wg.ph[k] = r.nslot ? gamma_phase<Real>(d, s_q + 3 * pl, r.invrot, ka) : Elem<C>::zero();
         }
         __syncthreads();
-        for (uint32_t t = wave; t < passes; t += TB / 64) {
+        // fewer passes than waves: the chunk's points split too
+        const uint32_t parts = passes < TB / 64 ? TB / 64 / passes : 1u;
+        const uint32_t part_n = (c1 - c0 + parts - 1) / parts;
+        for (uint32_t u = wave; u < passes * parts; u += TB / 64) {
+          const uint32_t part = u / passes, t = u - part * passes;
           const uint32_t b = b_lo + t * mpw + m;
           const bool on = m < mpw && b < b_end;
-          uint32_t p0 = c0;
+          uint32_t p0 = c0 + part * part_n;
+          const uint32_t pe = p0 + part_n < c1 ? p0 + part_n : c1;
           while (true) {
-            while (p0 < c1 && s_rec[p0].nslot == 0) {
+            while (p0 < pe && s_rec[p0].nslot == 0) {
               if (on) zero_rows(((out_row ? (uint64_t)out_row[p0] : row0 + p0)) * B, b);
               ++p0;
             }
-            if (p0 >= c1) break;
+            if (p0 >= pe) break;
             const PointRec<Real>& rb = s_rec[p0];
             uint32_t p1 = p0 + 1;
             if (rb.trow != kNoCube)
-              while (p1 < c1 && s_rec[p1].nslot != 0 && s_rec[p1].trow == rb.trow) ++p1;
+              while (p1 < pe && s_rec[p1].nslot != 0 && s_rec[p1].trow == rb.trow) ++p1;
             C v[8][3];
             Real vv[8];
             wide_atom_load<Real>(d, rb, b, a, on, v, vv, pm_of(p0));
@@ -1819,7 +1823,15 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
   const GammaFrame<Real>* frames = reinterpret_cast<const GammaFrame<Real>*>(s_q);
   auto frame_of = [&](uint32_t pl) { return op_frames ? op_frames + s_rec[pl].invrot : frames + pl; };
   uint32_t u0 = 0;
-  constexpr bool kCoop = (L == LAYOUT_GAMMA || L == LAYOUT_SCALAR) && coop_lanes<Real, SC, SV>() > 1;
+  if constexpr (L == LAYOUT_GAMMA) {
+    // (out_row and op_frames: the node-ordered sums)
+    if (table && out_row && op_frames) {
+      gamma_walk<Real, SC, SV, TB>(d, s_rec, s_ph, op_frames, out_row, n_coop, vals, vecs,
+                                   reinterpret_cast<char*>(s_wide) + (threadIdx.x >> 6) * walk_slice<Real>());
+      u0 = n_coop * B;
+    }
+  }
+  constexpr bool kCoop = L == LAYOUT_SCALAR && coop_lanes<Real, SC, SV>() > 1;
   if constexpr (kCoop) {
     constexpr uint32_t G = coop_lanes<Real, SC, SV>();
     if (table) {
@@ -1845,8 +1857,7 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
             cached = r.trow;
           }
           const uint64_t row = ((out_row ? (uint64_t)out_row[pl] : row0 + pl)) * B + b;
-          unit_coop<Real, SC, SV, L == LAYOUT_GAMMA, (int)G>(r, rows, q, vals + row * d.sv, vecs + row * d.sc,
-                                                             s_ph + NPH * pl, frame_of(pl));
+          unit_coop<Real, SC, SV>(r, rows, q, vals + row * d.sv, vecs + row * d.sc);
         }
       } else {
         constexpr uint32_t STEP = NG;  // units per block and iteration
@@ -1858,8 +1869,7 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
           const PointRec<Real>& r = s_rec[pl];
           const uint64_t row = ((out_row ? (uint64_t)out_row[pl] : row0 + pl)) * B + b;
           coop_load<Real>(d, r, (r.trow + b) * rb + q * 16u, slot_bytes, rows);
-          unit_coop<Real, SC, SV, L == LAYOUT_GAMMA, (int)G>(r, rows, q, vals + row * d.sv, vecs + row * d.sc,
-                                                             s_ph + NPH * pl, frame_of(pl));
+          unit_coop<Real, SC, SV>(r, rows, q, vals + row * d.sv, vecs + row * d.sc);
           b += sb;
           pl += sp;
           if (b >= B) {
@@ -1882,13 +1892,10 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
       for (uint32_t e = 0; e < d.sc; ++e) oc[e] = Elem<C>::zero();
       continue;
     }
-    // with the cooperative sums, every table point went there
     if constexpr (L == LAYOUT_GAMMA) {
-      unit_onepass<Real, SC, SV, true, GRP>(d, r, b, ov, oc, s_ph + NPH * pl, frame_of(pl), table && !kCoop,
-                                             pm_of(pl));
+      unit_onepass<Real, SC, SV, true, GRP>(d, r, b, ov, oc, s_ph + NPH * pl, frame_of(pl), pm_of(pl));
     } else if constexpr (L == LAYOUT_SCALAR) {
-      unit_onepass<Real, SC, SV, false, GRP>(d, r, b, ov, oc, nullptr, nullptr, table && !kCoop,
-                                              pm_of(pl));
+      unit_onepass<Real, SC, SV, false, GRP>(d, r, b, ov, oc, nullptr, nullptr, pm_of(pl));
     } else {
       unit_generic<Real, !Fast>(g, d, r, s_q + 3 * pl, b, ov, oc, ph_in_lds ? s_ph + NPH * pl : nullptr, pm_of(pl));
     }

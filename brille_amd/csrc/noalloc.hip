@@ -105,7 +105,7 @@ extern "C" int brille_ir_interpolate_at_noalloc(brille_grid* G, const double* Q,
   a.use_proposal = o.use_proposal;
   a.prop = G->prop;
   const bool fast = o.kernel != BRILLE_KERNEL_PLAIN;
-  const bool binned = fast && binned_applies(G, a, o.kernel);
+  const bool binned = fast && binned_applies(G, a, o.kernel, o.precision, false);
   uint64_t chunk = 0;
   if (binned) {
     chunk = binned_pass_for(G, ws_bytes);

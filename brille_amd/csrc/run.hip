@@ -198,10 +198,19 @@ void launch_tile(const brille_grid* G, const LaunchArgs& a, int precision, bool 
   launch_sel(G, a, precision, fast, s);
 }
 
+// an AUTO call under graph capture stays with the fused kernel until an earlier
+// binned call has left the work space and the tables it would need
+static bool must_not_allocate(const brille_grid* G, const LaunchArgs& a, const brille_run_opts& o, hipStream_t s) {
+  if (o.kernel == BRILLE_KERNEL_BINNED || a.use_proposal || !s || binned_ready(G, a.n, o.precision)) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 // every kernel of one call on device buffers
 static int dispatch(brille_grid* G, const LaunchArgs& a, const brille_run_opts& o, hipStream_t s) {
   const bool fast = o.kernel != BRILLE_KERNEL_PLAIN;
-  if (fast && binned_applies(G, a, o.kernel)) return launch_binned(G, a, o.precision, s, nullptr);
+  if (fast && binned_applies(G, a, o.kernel, o.precision) && !(must_not_allocate(G, a, o, s)))
+    return launch_binned(G, a, o.precision, s, nullptr);
   launch_sel(G, a, o.precision, fast, s);
   return BRILLE_OK;
 }
@@ -291,7 +300,7 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
     if (times) {
       std::memset(times, 0, sizeof(*times));
       const uint32_t it_n = std::max(iters, 1u);
-      if (fast && binned_applies(G, a, opts.kernel)) {
+      if (fast && binned_applies(G, a, opts.kernel, opts.precision)) {
         // stages from events on the streams that ran them; the call from
         // events on `s` around all of it
         float st[3] = {0.f, 0.f, 0.f};

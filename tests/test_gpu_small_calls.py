@@ -143,3 +143,74 @@ def test_flat_tetrahedra_are_located_like_the_oracle(height):
         for k in ("node", "tet", "n_iw", "iw_index", "iw_weight"):
             np.testing.assert_array_equal(gaux[k], oaux[k], err_msg=f"{kernel} {k}")
         np.testing.assert_allclose(gv, ov, atol=1e-12)
+
+
+def device_call(dev, Q, precision, kernel, stream=None, out=None):
+    n = len(Q)
+    vs, cs = dev.out_shapes(n)
+    f32 = precision == capi.FP32
+    dQ = capi.DeviceArray.from_host(Q)
+    dv, dc = out or (capi.DeviceArray(vs, np.float32 if f32 else np.float64),
+                     capi.DeviceArray(cs, np.complex64 if f32 else np.complex128))
+    o = capi.RunOpts(0, precision, 0, capi.MEM_DEVICE, kernel, 0 if stream else 1)
+    capi.check(capi.lib().brille_ir_interpolate_at(dev.h, dQ.ptr, n, C.byref(o), dv.ptr, dc.ptr, None, stream))
+    return dQ, dv, dc
+
+
+@pytest.mark.parametrize("spec,precision,sizes", [
+    (3, capi.FP32, (361_000, 361_200)), (3, capi.FP64, (194_000, 194_500)),
+    (7, capi.FP32, (90_000, 90_300)), (7, capi.FP64, (48_500, 48_700)),
+    (2, capi.FP32, (15_400, 15_500)), (5, capi.FP64, (770, 780)), (5, capi.FP32, (3_800, 3_900))])
+def test_auto_agrees_with_the_fused_kernel_across_its_line(spec, precision, sizes):
+    """The sizes on both sides of AUTO's choice between the fused kernel and the binned pipeline."""
+    print(f"auto line: grid {spec} {precision}", flush=True)
+    sp = dict(S.batch_specs(16)[spec], v_target=600.0)
+    g = S.batch_grid(sp)
+    vals, vecs = S.batch_payload(g, sp)
+    dev = capi.Grid(dict(S.batch_layout_tables(g, sp), values=vals, vectors=vecs))
+    r = np.random.default_rng(2)
+    for n in sizes:
+        Q = points(g, r, n)
+        tile = device_call(dev, Q, precision, capi.KERNEL_TILE)
+        auto = device_call(dev, Q, precision, capi.KERNEL_AUTO)
+        for a, b in zip(tile[1:], auto[1:]):
+            np.testing.assert_array_equal(a.to_host(), b.to_host())
+
+
+def test_an_auto_call_can_be_captured_first_and_after_a_binned_call():
+    """Under capture nothing may be allocated: the first call of a handle stays with the fused
+    kernel, one after an eager call of the same size takes the pipeline; both replay."""
+    print("auto under capture", flush=True)
+    lib = capi.lib()
+    maps = open("/proc/self/maps").read().split()
+    hip = C.CDLL(next(m for m in maps if "libamdhip64" in m))  # the runtime the library itself uses
+    sp = dict(S.batch_specs(16)[7], v_target=600.0)
+    g = S.batch_grid(sp)
+    vals, vecs = S.batch_payload(g, sp)
+    t = dict(S.batch_layout_tables(g, sp), values=vals, vectors=vecs)
+    Q = points(g, np.random.default_rng(3), 120_000)
+    want = device_call(capi.Grid(t), Q, capi.FP32, capi.KERNEL_TILE)
+    for warm in (False, True):
+        dev = capi.Grid(t)
+        keep = device_call(dev, Q, capi.FP32, capi.KERNEL_AUTO if warm else capi.KERNEL_TILE)
+        side, graph, replay = C.c_void_p(), C.c_void_p(), C.c_void_p()
+        capi.check(lib.brille_stream_create(C.byref(side)))
+        capi.check(lib.brille_device_sync())
+        assert hip.hipStreamBeginCapture(side, 1) == 0  # thread-local mode
+        o = capi.RunOpts(0, capi.FP32, 0, capi.MEM_DEVICE, capi.KERNEL_AUTO, 0)
+        rc = lib.brille_ir_interpolate_at(dev.h, keep[0].ptr, len(Q), C.byref(o), keep[1].ptr, keep[2].ptr, None, side)
+        assert hip.hipStreamEndCapture(side, C.byref(graph)) == 0
+        capi.check(rc)
+        assert hip.hipGraphInstantiate(C.byref(replay), graph, None, None, C.c_size_t(0)) == 0
+        for _ in range(3):
+            # eager work and clobbered outputs between the replays
+            device_call(dev, Q[:500], capi.FP32, capi.KERNEL_TILE)
+            for x in keep[1:]:
+                junk = np.full(x.shape, 7, x.dtype)
+                capi.check(lib.brille_memcpy_h2d(x.ptr, junk.ctypes.data_as(C.c_void_p), x.nbytes))
+            assert hip.hipGraphLaunch(replay, side) == 0
+            capi.check(lib.brille_stream_sync(side))
+            for a, b in zip(want[1:], keep[1:]):
+                np.testing.assert_array_equal(a.to_host(), b.to_host())
+        assert hip.hipGraphExecDestroy(replay) == 0 and hip.hipGraphDestroy(graph) == 0
+        capi.check(lib.brille_stream_destroy(side))
