@@ -377,6 +377,11 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nb) {
   return x * q + (x < r ? x : r) + i;
 }
 
+// points a block of the sums holds: the atom-major wide sums run as fast with 64
+// as with 128 or 256 (24 atoms, 300 007 points of 72 modes FP32 5.2 ms), which
+// leaves the LDS to the records being assembled
+constexpr uint32_t sums_points(int L, int SC) { return L == LAYOUT_WIDE && SC == kWideAtom ? 64u : (uint32_t)TILE; }
+
 // waves per SIMD asked of the compiler: the atom-major wide sums run best at
 // four (FP32) and two (FP64), a few registers below what it would take for
 // the antiphases of the rare points without a table block, and so do the narrow
@@ -398,9 +403,10 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
   using C = typename Cplx<Real>::T;
   constexpr int WSL = wide_bin_slots<Real>();
   using S = TileShape<L, SC, TILE, Real, WSL>;
-  __shared__ PointRec<Real> s_rec[TILE];
-  // wide rows: the phase table of the node-ordered Gamma sums instead
   constexpr bool kWide = L == LAYOUT_WIDE;
+  constexpr uint32_t TP = sums_points(L, SC);
+  __shared__ PointRec<Real> s_rec[TP];
+  // wide rows: the phase table of the node-ordered Gamma sums instead
   constexpr uint32_t kPh =
       kWide ? (SC == kWideAtom ? kWideAtomPhaseBytes : kWidePhaseBytes) / sizeof(C) : TILE * S::NPH;
   __shared__ C s_ph[kPh];
@@ -409,12 +415,15 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
   // Gamma layout: one frame per point-group operation instead of one per
   // point (12 KB less LDS in FP32, 20 KB in FP64)
   constexpr bool kOpFrames = L == LAYOUT_GAMMA;
-  __shared__ double s_q[kOpFrames ? 1 : S::NQ];
+  __shared__ double s_q[kWide ? S::NQ / TILE * TP : kOpFrames ? 1 : S::NQ];
   __shared__ GammaFrame<Real> s_frames[kOpFrames ? kMaxOps : 1];
   if (kOpFrames && threadIdx.x < g.G) fill_frame<Real, SC>(g, d, threadIdx.x, s_frames[threadIdx.x]);
-  __shared__ uint32_t s_out[TILE];
+  __shared__ uint32_t s_out[TP];
   // wide rows' slices, or the atom lanes' records
-  constexpr uint32_t kWalk = kOpFrames ? TILE / 64 * walk_slice<Real>() / sizeof(C) : 1;
+  constexpr bool kAtoms = kWide && SC == kWideAtom;
+  constexpr uint32_t kWalk = kOpFrames ? TILE / 64 * walk_slice<Real>() / sizeof(C)
+                             : kAtoms  ? TILE / 64 * wide_walk_slice<Real>(WSL)
+                                       : 1;
   __shared__ __attribute__((aligned(16))) C s_wide[(uint32_t)S::NW > kWalk ? S::NW : kWalk];
   __shared__ uint32_t s_tried, s_verified;
   if (Prop && threadIdx.x == 0) {
@@ -422,8 +431,8 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
     s_verified = 0;
   }
   // wide rows take fewer points per block in passes of few points (tile_pts of
-  // the TILE a block's LDS holds); the others always TILE
-  const uint32_t tile_n = kWide ? tile_pts : (uint32_t)TILE;
+  // the TP a block's LDS holds); the others always TP
+  const uint32_t tile_n = kWide ? tile_pts : TP;
   const uint32_t tile0 = xcd_tile(blockIdx.x, gridDim.x) * tile_n;
   const uint32_t tid = threadIdx.x;
   const uint32_t p = tile0 + tid;
@@ -432,7 +441,7 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
   const bool lead = blockIdx.y == 0;
   uint32_t per_group = (d.B + gridDim.y - 1) / gridDim.y;
   if (L == LAYOUT_WIDE && SC == kWideAtom) {  // whole passes of the atom-major walk
-    const uint32_t mpw = 64u / (d.sc / 3u);
+    const uint32_t mpw = wide_pass_modes(d.sc, sizeof(C));
     per_group = (per_group + mpw - 1) / mpw * mpw;
   }
   const uint32_t b_lo = blockIdx.y * per_group, b_hi = b_lo + per_group;
@@ -498,7 +507,7 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
     n_tab += c;
   }
   const uint32_t slot = tab ? before + rank : n_tab + (tid - before - rank);
-  {
+  if (tid < TP) {
     PointRec<Real>& r = s_rec[slot];
     r.nslot = 0;
     if (live) {
@@ -689,21 +698,35 @@ static SumsKernel pick_sums(const DataConst& d, bool prop) {
 // pass of few points would leave most CUs idle: its tiles shrink until the
 // pass has about eight blocks per CU or kLeastWideTile points are left (below
 // that the runs of one table block are cut), then the modes split over blocks
-// (each group repeats phase 1 and its points' Gamma phases).  3001 points of 72
-// modes FP32: 0.68 ms in 256-point tiles of 18 groups, kept below.  Other
-// kernels pick_sums selects (the proposal's among them): TILE points, one group.
+// (each group repeats phase 1 and its points' Gamma phases).  The atom-major
+// sums take eight mode passes per block, two per wave, however many the points:
+// blocks of a whole tile's modes ran for milliseconds, four at a time on a CU,
+// and left most of them idle at the end (72 modes FP32, 300 007 points: all 36
+// passes in a block 6.6 ms, 16 5.4, 8 5.1, 6 (two of four waves idle in the
+// second round) 5.8, 4 5.1, 2 5.6); fewer where even these leave under ten
+// blocks per CU (10 001 points: eight 0.50 ms, four 0.47; 3 001: eight 0.30,
+// two 0.26).  Other kernels pick_sums selects (the proposal's among them): TILE
+// points, one group.
 constexpr uint32_t kLeastWideTile = 32;
-static void sum_split(const brille_grid* G, uint32_t m, bool prop, uint32_t* tile, uint32_t* groups) {
+static void sum_split(const brille_grid* G, uint32_t m, bool prop, int precision, uint32_t* tile, uint32_t* groups) {
   *tile = TILE;
   *groups = 1;
   const DataConst& d = G->d;
   if (prop || !wide_rows(d)) return;
+  const bool atoms = wide_by_atom(d);
+  if (atoms) *tile = sums_points(LAYOUT_WIDE, kWideAtom);
   const uint64_t want = 8ull * std::max<uint32_t>(G->n_cu, 1);
   while (*tile > kLeastWideTile && (m + *tile - 1) / *tile < want) *tile >>= 1;
   const uint64_t tiles = std::max<uint64_t>((m + *tile - 1) / *tile, 1);
-  const uint32_t mpw = wide_by_atom(d) ? 64u / (d.sc / 3u) : 4u;
-  const uint32_t most = std::max<uint32_t>((d.B + mpw - 1) / mpw, 1);
-  *groups = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want / tiles, most));
+  if (!atoms) {
+    *groups = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want / tiles, (d.B + 3) / 4));
+    return;
+  }
+  const uint32_t mpw = wide_pass_modes(d.sc, precision == BRILLE_FP32 ? 8u : 16u);
+  const uint32_t passes = (d.B + mpw - 1) / mpw;
+  uint32_t per = 8;
+  while (per > 2 && tiles * ((passes + per - 1) / per) < 5 * want / 4) per >>= 1;
+  *groups = std::max<uint32_t>((passes + per - 1) / per, 1);
 }
 
 // SC of the one-pass sums kernel pick_sums selects, or 0 for the general ones
@@ -1103,7 +1126,7 @@ int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStr
     // sums of pass k on the call stream
     mark(k, 3, s);
     uint32_t tile_pts, groups;
-    sum_split(G, m, prop, &tile_pts, &groups);
+    sum_split(G, m, prop, precision, &tile_pts, &groups);
     const dim3 sgrid((m + tile_pts - 1) / tile_pts, groups);
     hipLaunchKernelGGL(sums, sgrid, dim3(TILE), G->d.n_keys ? 32u * TILE : 0u, s, G->g, G->d, a.prop, b.srt, b.perm, m,
                        static_cast<char*>(a.vals) + c0 * vb, static_cast<char*>(a.vecs) + c0 * cb,

@@ -806,6 +806,22 @@ template <typename Real>
 constexpr uint32_t wide_atom_slice(int sl) {
   return (uint32_t)sl * (sizeof(Real) == 4 ? 64u : 192u) + (uint32_t)sl * kWideModesMax;
 }
+// the node-ordered sums also assemble a point's records there (64 lanes of
+// three elements) before they are written as one run
+template <typename Real>
+constexpr uint32_t wide_walk_slice(int sl) {
+  return wide_atom_slice<Real>(sl) > 192u ? wide_atom_slice<Real>(sl) : 192u;
+}
+// modes of a pass of the atom-major walk: as many as the wave's lanes hold, or
+// up to a quarter fewer where their rows then end on a 64-byte granule (a
+// granule two passes share is written in halves: 12 atoms FP32, four modes
+// instead of five)
+__host__ __device__ inline uint32_t wide_pass_modes(uint32_t sc, uint32_t elem_bytes) {
+  const uint32_t most = 64u / (sc / 3u);
+  for (uint32_t k = most; 4 * k >= 3 * most && k > 0; --k)
+    if (k * sc * elem_bytes % 64u == 0) return k;
+  return most;
+}
 // slots at a time: the tile kernels take more (shorter chains of LDS
 // exchanges in small calls), the node-ordered sums fewer (four blocks per CU)
 template <typename Real>
@@ -1027,6 +1043,9 @@ __device__ __forceinline__ void wide_atom_phase(const DataConst& d, const PointR
     }
 }
 
+// a value all lanes of the wave hold alike, as a scalar
+__device__ __forceinline__ uint32_t uniform(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
+
 // the weighted sums of a lane's atom from its antiphased rows
 template <typename Real>
 __device__ __forceinline__ void wide_atom_sum(const PointRec<Real>& r, const typename Cplx<Real>::T (*v)[3],
@@ -1048,27 +1067,54 @@ __device__ __forceinline__ void wide_atom_sum(const PointRec<Real>& r, const typ
 }
 
 // rip_gamma_complex  src/interpolator_gamma.tpp:100-114 of one atom: R times
-// the accumulated 3-vector, times the atom's phase, to the output atom.  Plain
-// stores: a wave's three stores of 8 or 16 bytes per lane fill whole lines
-// between them, which the L2 merges; nontemporal ones went out as partial
-// lines (node-ordered sums, 300 007 points: 36 modes FP64 6.8 -> 1.8 ms, 72
-// modes FP32 7.8 -> 7.2 ms).
-template <typename Real>
-__device__ __forceinline__ void wide_atom_store(const typename Cplx<Real>::T* acc, const Real* R,
-                                                typename Cplx<Real>::T ph, typename Cplx<Real>::T* dst) {
+// the accumulated 3-vector, times the atom's phase
+template <typename Real, bool Fma>
+__device__ __forceinline__ void wide_atom_rotate(const typename Cplx<Real>::T* acc, const Real* R,
+                                                 typename Cplx<Real>::T ph, typename Cplx<Real>::T* out) {
   using C = typename Cplx<Real>::T;
-  typedef Real real2 __attribute__((ext_vector_type(2)));
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     C tt = Elem<C>::zero();
+    if constexpr (Fma) {
 #pragma unroll
-    for (int j = 0; j < 3; ++j) tt = Elem<C>::add(tt, Elem<C>::scale(acc[j], R[3 * i + j]));
-    const C o = cmul(ph, tt);
-    *reinterpret_cast<real2*>(dst + i) = real2{o.x, o.y};
+      for (int j = 0; j < 3; ++j) {
+        tt.x = j ? fma_r(acc[j].x, R[3 * i + j], tt.x) : acc[j].x * R[3 * i];
+        tt.y = j ? fma_r(acc[j].y, R[3 * i + j], tt.y) : acc[j].y * R[3 * i];
+      }
+      out[i] = C{fma_r(ph.x, tt.x, -(ph.y * tt.y)), fma_r(ph.x, tt.y, ph.y * tt.x)};
+    } else {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) tt = Elem<C>::add(tt, Elem<C>::scale(acc[j], R[3 * i + j]));
+      out[i] = cmul(ph, tt);
+    }
   }
 }
 
+// ... straight to the output atom (the point-major sums).  Plain stores: a
+// wave's three stores of 8 or 16 bytes per lane fill whole lines between them,
+// which the L2 merges; nontemporal ones went out as partial lines.
+template <typename Real>
+__device__ __forceinline__ void wide_atom_store(const typename Cplx<Real>::T* acc, const Real* R,
+                                                typename Cplx<Real>::T ph, typename Cplx<Real>::T* dst) {
+  typename Cplx<Real>::T o[3];
+  wide_atom_rotate<Real, true>(acc, R, ph, o);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) dst[i] = o[i];
+}
+
 // ---------------------------------------------------------------------------
+// Bytes an LDS slice holds of one record, written by the wave as one run: a
+// lane per 16-byte piece where the record's start and length allow it, else 8.
+// Nontemporal 16-byte pieces: a run covers whole 64-byte granules but for its
+// ends, and half-written granules are what scattered records cost (2^24 random
+// records of 320 bytes 4.7 TB/s, of 288 bytes 2.5 TB/s).
+typedef uint32_t piece16 __attribute__((ext_vector_type(4)));
+typedef uint32_t piece8 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void put_piece(char* out, const char* from, bool wide) {
+  if (wide) __builtin_nontemporal_store(*reinterpret_cast<const piece16*>(from), reinterpret_cast<piece16*>(out));
+  else *reinterpret_cast<piece8*>(out) = *reinterpret_cast<const piece8*>(from);
+}
+
 // Atom lanes: the node-ordered sums of narrow Gamma rows (SC / 3 atoms) for the
 // records the row table serves, the first n of a tile.  A lane takes (point
 // slot, mode, atom): S point slots of a wave each walk their own run of
@@ -1103,8 +1149,6 @@ __device__ __forceinline__ void gamma_walk(const DataConst& d, const PointRec<Re
   const uint32_t p1 = p0 + run < w1 ? p0 + run : w1;
   const uint32_t stride = payload_stride<Real>(d);
   C* sv_vec = reinterpret_cast<C*>(slice);
-  typedef uint32_t piece_t __attribute__((ext_vector_type(4)));
-  typedef uint32_t half_t __attribute__((ext_vector_type(2)));
   for (uint32_t b0 = 0; b0 < B; b0 += mb) {
     const uint32_t nb = B - b0 < mb ? B - b0 : mb;
     const uint32_t b = b0 + bl;
@@ -1139,14 +1183,7 @@ __device__ __forceinline__ void gamma_walk(const DataConst& d, const PointRec<Re
         wide_atom_sum<Real>(r, v, vv, acc, &va);
         const GammaFrame<Real>& f = frames[r.invrot];
         const C ph = s_ph[NA * pl + a];
-        C* dst = sv_vec + (s * nb + bl) * SC + 3u * f.to[a];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          C tt = Elem<C>::zero();
-#pragma unroll
-          for (int k = 0; k < 3; ++k) tt = Elem<C>::add(tt, Elem<C>::scale(acc[k], f.R[3 * i + k]));
-          dst[i] = cmul(ph, tt);
-        }
+        wide_atom_rotate<Real, false>(acc, f.R, ph, sv_vec + (s * nb + bl) * SC + 3u * f.to[a]);
         if (a < (uint32_t)SV) vals[((uint64_t)out_row[pl] * B + b) * SV + a] = va;
       }
       wave_lds_fence();
@@ -1155,11 +1192,7 @@ __device__ __forceinline__ void gamma_walk(const DataConst& d, const PointRec<Re
         const uint32_t pp0 = w0 + ps * run, pp = pp0 + it;
         if (pp < w1 && it < run) {
           char* out = reinterpret_cast<char*>(vecs + ((uint64_t)out_row[pp] * B + b0) * SC) + (q << sh);
-          if (wide)
-            __builtin_nontemporal_store(*reinterpret_cast<const piece_t*>(slice + ((uint64_t)c << 4)),
-                                        reinterpret_cast<piece_t*>(out));
-          else
-            *reinterpret_cast<half_t*>(out) = *reinterpret_cast<const half_t*>(slice + ((uint64_t)c << 3));
+          put_piece(out, slice + ((uint64_t)c << sh), wide);
         }
       }
       wave_lds_fence();
@@ -1613,9 +1646,9 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
       // rotation needs no exchange between lanes.  Points with a block in the
       // factor table take their antiphases there, the others form them.
       constexpr int SL = WSL;
-      C* lds = s_wide + wave * wide_atom_slice<Real>(SL);
+      C* lds = s_wide + wave * (node_order ? wide_walk_slice<Real>(SL) : wide_atom_slice<Real>(SL));
       const uint32_t na = d.sc / 3u, sc = d.sc, sv = d.sv;
-      const uint32_t mpw = 64u / na;
+      const uint32_t mpw = node_order ? wide_pass_modes(sc, sizeof(C)) : 64u / na;
       const uint32_t m = lane / na, a = lane - m * na;
       const uint32_t nmodes = b_end > b_lo ? b_end - b_lo : 0u;
       const uint32_t passes = (nmodes + mpw - 1) / mpw;
@@ -1673,9 +1706,18 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
       // phases the block first computes into LDS (once per point and atom
       // instead of once per mode); the rotation rows and atom map come from
       // per-operation LDS tables.
-      // (Staging a wave's rotated rows in LDS, to write them as one contiguous
-      // run per point instead of three 8-byte stores per lane at a permuted
-      // atom, saved no time: 64-grid batch of 1e7 points 140 -> 145 ms.)
+      // What bounds it: vector instructions (24 atoms FP32: 158 per lane, mode
+      // and point, of which 108 are the sums and the rotation; the vector units
+      // are 58 % busy at four waves per SIMD, the stores run at 2.4 TB/s).  A
+      // point's rotated rows go through the wave's LDS slice and out as one run
+      // of 16-byte stores, not as three 8-byte stores per lane at a permuted
+      // atom (300 007 points of 72 modes FP32 7.4 -> 7.0 ms), addresses are
+      // formed per wave and the rotation in fused steps (-> 6.8 ms); see
+      // sum_split for the rest (-> 5.2 ms).  Tried and slower: the weighted sums
+      // on v_mfma_f32_4x4x1_16b, four points at a time (same bits, 23 % fewer
+      // vector instructions, but runs of about six points fill the fours badly:
+      // 5.8 ms), two points in flight (5.2 ms, more registers), three or five
+      // waves per SIMD (5.7, 6.9 ms).
       const uint32_t chunk = wg.cap / na < npts ? wg.cap / na : npts;
       for (uint32_t c0 = 0; c0 < npts; c0 += chunk) {
         const uint32_t c1 = c0 + chunk < npts ? c0 + chunk : npts;
@@ -1689,36 +1731,59 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
         // fewer passes than waves: the chunk's points split too
         const uint32_t parts = passes < TB / 64 ? TB / 64 / passes : 1u;
         const uint32_t part_n = (c1 - c0 + parts - 1) / parts;
-        for (uint32_t u = wave; u < passes * parts; u += TB / 64) {
+        // (the wave's number, its points and their rows are read as scalars: the
+        // addresses they give are then formed once per wave, not per lane)
+        for (uint32_t u = uniform(wave); u < passes * parts; u += TB / 64) {
           const uint32_t part = u / passes, t = u - part * passes;
           const uint32_t b = b_lo + t * mpw + m;
           const bool on = m < mpw && b < b_end;
+          const uint32_t b0 = b_lo + t * mpw, nb = b_end - b0 < mpw ? b_end - b0 : mpw;
+          const uint32_t bytes = nb * sc * (uint32_t)sizeof(C);
+          const bool full = sizeof(Real) == 8 ||
+                            ((((uintptr_t)vecs | (B * sc * sizeof(C)) | (b0 * sc * sizeof(C)) | bytes) & 15u) == 0);
           uint32_t p0 = c0 + part * part_n;
           const uint32_t pe = p0 + part_n < c1 ? p0 + part_n : c1;
-          while (true) {
-            while (p0 < pe && s_rec[p0].nslot == 0) {
-              if (on) zero_rows(((out_row ? (uint64_t)out_row[p0] : row0 + p0)) * B, b);
-              ++p0;
-            }
-            if (p0 >= pe) break;
+          while (p0 < pe) {
+            // points from p0 on that share its block (none: outside the grid)
             const PointRec<Real>& rb = s_rec[p0];
-            uint32_t p1 = p0 + 1;
-            if (rb.trow != kNoCube)
-              while (p1 < pe && s_rec[p1].nslot != 0 && s_rec[p1].trow == rb.trow) ++p1;
+            const uint32_t left = pe - p0 < 64u ? pe - p0 : 64u;
+            const PointRec<Real>& rl = s_rec[p0 + (lane < left ? lane : 0u)];
+            const bool same = lane < left && (lane == 0 || (rb.trow != kNoCube && rl.trow == rb.trow)) && rl.nslot != 0;
+            const uint64_t other = ~__ballot(same);
+            const uint32_t run = other ? (uint32_t)__builtin_ctzll(other) : 64u;
+            if (run == 0) {
+              if (on) zero_rows((out_row ? (uint64_t)uniform(out_row[p0]) : row0 + p0) * B, b);
+              ++p0;
+              continue;
+            }
             C v[8][3];
             Real vv[8];
             wide_atom_load<Real>(d, rb, b, a, on, v, vv, pm_of(p0));
             wide_atom_phase<Real, SL>(d, rb, b, na, mpw, m, on, fac, v, lds);
+            const uint32_t p1 = p0 + run;
+            // a point's sums to its rows: rotation, LDS, one run of stores
+            auto finish = [&](uint32_t pl, const C* acc, Real va) {
+              const uint64_t row = (out_row ? (uint64_t)uniform(out_row[pl]) : row0 + pl) * B;
+              const uint32_t op = uniform(s_rec[pl].invrot);
+              if (on) {
+                if (a < sv) (vals + (row + b0) * sv)[m * sv + a] = va;
+                wide_atom_rotate<Real, true>(acc, wg.rot + 9u * op, wg.ph[(pl - c0) * na + a],
+                                             lds + m * sc + 3u * wg.dst[op * na + a]);
+              }
+              wave_lds_fence();
+              char* out = reinterpret_cast<char*>(vecs + (row + b0) * sc);
+              const char* from = reinterpret_cast<const char*>(lds);
+              if (full)
+                for (uint32_t k = 16u * lane; k < bytes; k += 1024u) put_piece(out + k, from + k, true);
+              else
+                for (uint32_t k = 8u * lane; k < bytes; k += 512u) put_piece(out + k, from + k, false);
+              wave_lds_fence();
+            };
             for (uint32_t pl = p0; pl < p1; ++pl) {
-              if (!on) continue;
-              const PointRec<Real>& r = s_rec[pl];
-              const uint64_t row = ((out_row ? (uint64_t)out_row[pl] : row0 + pl)) * B;
               C acc[3];
               Real va;
-              wide_atom_sum<Real>(r, v, vv, acc, &va);
-              if (a < sv) vals[row * sv + (uint64_t)b * sv + a] = va;
-              wide_atom_store<Real>(acc, wg.rot + 9u * r.invrot, wg.ph[(pl - c0) * na + a],
-                                    vecs + row * sc + (uint64_t)b * sc + 3u * wg.dst[r.invrot * na + a]);
+              wide_atom_sum<Real>(s_rec[pl], v, vv, acc, &va);
+              finish(pl, acc, va);
             }
             p0 = p1;
           }

@@ -103,9 +103,10 @@ bool wide_rows(const DataConst& d) {
   return (L == LAYOUT_GAMMA || L == LAYOUT_SCALAR) && d.sc > 12 && d.sc <= kWideMax && d.sv <= 64;
 }
 
-// wide Gamma rows of at most one value per atom: the sums go atom-major
+// wide Gamma rows of at most one value per atom, every operation mapping the
+// atoms one to one: the sums go atom-major (they write whole records)
 bool wide_by_atom(const DataConst& d) {
-  return wide_rows(d) && payload_layout(d) == LAYOUT_GAMMA && d.sv <= d.sc / 3u;
+  return wide_rows(d) && payload_layout(d) == LAYOUT_GAMMA && d.sv <= d.sc / 3u && d.gamma_maps;
 }
 
 // The instantiated specialisations: Gamma payloads of 1-4 atoms and scalar
