@@ -179,6 +179,13 @@ __global__ void k_batch_reset(BatchHeader* hdr, const BatchGrid* grids, uint32_t
   }
 }
 
+// the members' error records to pinned memory, one wait for all (a pageable copy
+// and wait per member: 16 grids 3.36 -> 3.15 ms in all)
+__global__ void k_batch_errors(const BatchGrid* grids, uint32_t n_grids, ErrRec* out) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n_grids) out[i] = *grids[i].err;
+}
+
 // a member grid as the batch kernel sees it
 static void describe_batch_grid(const brille_grid* G, BatchGrid& bg) {
   std::memset(&bg, 0, sizeof(bg));
@@ -208,6 +215,7 @@ struct brille_batch {
   BatchGrid* d_grids = nullptr;
   BatchSlot* d_slots = nullptr;
   BatchHeader* d_hdr = nullptr;
+  ErrRec* host_err = nullptr;  // the members' error records, pinned (null: copied one by one)
   uint32_t cap_slots = 0;
   uint32_t n_cu = 0;
   Schedule sched;
@@ -375,10 +383,16 @@ static int check_args(brille_batch* b, const double* Q, const uint64_t* offsets,
 
 // the first failing point of the lowest-numbered grid that has one
 static int batch_errors(brille_batch* b, const double* Q, const uint64_t* offsets, hipStream_t s) {
+  const uint32_t ng = (uint32_t)b->grids.size();
+  if (b->host_err) {
+    hipLaunchKernelGGL(k_batch_errors, dim3((ng + 63) / 64), dim3(64), 0, s, b->d_grids, ng, b->host_err);
+    BATCH_TRY(hipGetLastError());
+  }
   BATCH_TRY(hipStreamSynchronize(s));
   for (size_t g = 0; g < b->grids.size(); ++g) {
     ErrRec e;
-    BATCH_TRY(hipMemcpy(&e, b->grids[g]->err, sizeof(e), hipMemcpyDeviceToHost));
+    if (b->host_err) e = b->host_err[g];
+    else BATCH_TRY(hipMemcpy(&e, b->grids[g]->err, sizeof(e), hipMemcpyDeviceToHost));
     if (e.count) {
       const uint64_t n = offsets[g + 1] - offsets[g];
       int rc = report_point_error(e, Q + 3 * offsets[g], n, false);
@@ -547,6 +561,9 @@ int brille_batch_create(brille_grid* const* grids, uint32_t n_grids, brille_batc
   b->d_slots = static_cast<BatchSlot*>(ps);
   b->d_hdr = static_cast<BatchHeader*>(ph);
   b->cap_slots = n_grids;
+  void* pe = nullptr;
+  if (hipHostMalloc(&pe, n_grids * sizeof(ErrRec), hipHostMallocDefault) == hipSuccess) b->host_err = static_cast<ErrRec*>(pe);
+  else (void)hipGetLastError();
   *out = b;
   return BRILLE_OK;
 }
@@ -666,6 +683,7 @@ int brille_batch_destroy(brille_batch* b) {
   if (b->d_grids) (void)hipFree(b->d_grids);
   if (b->d_slots) (void)hipFree(b->d_slots);
   if (b->d_hdr) (void)hipFree(b->d_hdr);
+  if (b->host_err) (void)hipHostFree(b->host_err);
   if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
   if (b->cap_side) (void)hipStreamDestroy(b->cap_side);
   for (hipEvent_t e : b->cap_ev)

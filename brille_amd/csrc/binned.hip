@@ -730,7 +730,7 @@ static void sum_split(const brille_grid* G, uint32_t m, bool prop, int precision
 }
 
 // SC of the one-pass sums kernel pick_sums selects, or 0 for the general ones
-static int onepass_sc(const DataConst& d) {
+int onepass_sc(const DataConst& d) {
   const int L = payload_layout(d);
   if (d.sv != 1) return 0;
   if (L == LAYOUT_GAMMA && (d.sc == 3 || d.sc == 6 || d.sc == 9 || d.sc == 12)) return (int)d.sc;

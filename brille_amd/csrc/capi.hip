@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <limits>
 #include <string>
 #include <vector>
@@ -45,6 +46,34 @@ static int upload(const T* host, size_t n, const T** dev, std::vector<void*>& al
   *dev = static_cast<const T*>(p);
   return BRILLE_OK;
 }
+
+// The small tables of a handle in one allocation and one copy (about 14 us for
+// each of the twenty before); larger ones each by themselves.
+class Uploads {
+ public:
+  explicit Uploads(std::vector<void*>& allocs) : allocs_(allocs) {}
+  template <typename T>
+  int add(const T* host, size_t n, const T** dev) {
+    constexpr size_t kSmall = 64u << 10;
+    if (n == 0 || host == nullptr || n * sizeof(T) > kSmall) return upload(host, n, dev, allocs_);
+    const size_t off = (bytes_.size() + 255) & ~size_t(255);
+    bytes_.resize(off + n * sizeof(T));
+    std::memcpy(bytes_.data() + off, host, n * sizeof(T));
+    set_.push_back([dev, off](const char* base) { *dev = reinterpret_cast<const T*>(base + off); });
+    return BRILLE_OK;
+  }
+  int flush() {
+    const char* base = nullptr;
+    if (int rc = upload(bytes_.data(), bytes_.size(), &base, allocs_); rc != BRILLE_OK) return rc;
+    for (const auto& f : set_) f(base);
+    return BRILLE_OK;
+  }
+
+ private:
+  std::vector<void*>& allocs_;
+  std::vector<char> bytes_;
+  std::vector<std::function<void(const char*)>> set_;
+};
 
 static void free_all(std::vector<void*>& allocs) {
   for (void* p : allocs) (void)hipFree(p);
@@ -240,27 +269,28 @@ int brille_grid_create(const brille_grid_desc* desc, brille_grid** out) {
   make_tols(desc->float_tolerance, desc->approx_digits, &g.tol_bz_rel, &g.tol_bz_abs);
   make_tols(0.0, 1, &g.tol_def_rel, &g.tol_def_abs);
   auto& A = G->grid_allocs;
+  Uploads up(A);
   const size_t F3 = 3 * (size_t)desc->n_faces;
   int rc = BRILLE_OK;
   auto chk = [&](int r) { if (r != BRILLE_OK && rc == BRILLE_OK) rc = r; };
-  chk(upload(desc->prim_plane_a, F3, &g.prim_pa, A));
-  chk(upload(desc->prim_plane_b, F3, &g.prim_pb, A));
-  chk(upload(desc->prim_plane_c, F3, &g.prim_pc, A));
-  chk(upload(desc->prim_normals, F3, &g.prim_n, A));
-  chk(upload(desc->prim_taus, F3, &g.prim_taus, A));
-  chk(upload(desc->prim_tau_lens, (size_t)desc->n_faces, &g.prim_tau_lens, A));
-  chk(upload(desc->outer_plane_a, F3, &g.outer_pa, A));
-  chk(upload(desc->outer_plane_b, F3, &g.outer_pb, A));
-  chk(upload(desc->outer_plane_c, F3, &g.outer_pc, A));
-  chk(upload(desc->wedge_normals, 3 * (size_t)desc->n_wedge, &g.wedge_n, A));
-  chk(upload(desc->rotations, 9 * (size_t)desc->n_ops, &g.rot, A));
-  chk(upload(desc->inverse_index, (size_t)desc->n_ops, &g.inv_index, A));
+  chk(up.add(desc->prim_plane_a, F3, &g.prim_pa));
+  chk(up.add(desc->prim_plane_b, F3, &g.prim_pb));
+  chk(up.add(desc->prim_plane_c, F3, &g.prim_pc));
+  chk(up.add(desc->prim_normals, F3, &g.prim_n));
+  chk(up.add(desc->prim_taus, F3, &g.prim_taus));
+  chk(up.add(desc->prim_tau_lens, (size_t)desc->n_faces, &g.prim_tau_lens));
+  chk(up.add(desc->outer_plane_a, F3, &g.outer_pa));
+  chk(up.add(desc->outer_plane_b, F3, &g.outer_pb));
+  chk(up.add(desc->outer_plane_c, F3, &g.outer_pc));
+  chk(up.add(desc->wedge_normals, 3 * (size_t)desc->n_wedge, &g.wedge_n));
+  chk(up.add(desc->rotations, 9 * (size_t)desc->n_ops, &g.rot));
+  chk(up.add(desc->inverse_index, (size_t)desc->n_ops, &g.inv_index));
   // trellis (may be empty for a zone-only handle)
   uint64_t nodes = 1;
   for (int d = 0; d < 3; ++d) {
     g.nk[d] = desc->n_knots[d];
     if (desc->n_knots[d] >= 2) {
-      chk(upload(desc->knots[d], (size_t)desc->n_knots[d], &g.knots[d], A));
+      chk(up.add(desc->knots[d], (size_t)desc->n_knots[d], &g.knots[d]));
       g.knot_lo[d] = desc->knots[d][0];
       double step = (desc->knots[d][desc->n_knots[d] - 1] - desc->knots[d][0]) / (double)(desc->n_knots[d] - 1);
       g.knot_inv_step[d] = step > 0 ? 1.0 / step : 0.0;
@@ -275,17 +305,22 @@ int brille_grid_create(const brille_grid_desc* desc, brille_grid** out) {
     return fail(BRILLE_ERR_INVALID_ARGUMENT, "node count does not match the knots");
   }
   g.n_nodes = desc->n_nodes;
-  chk(upload(desc->node_type, (size_t)desc->n_nodes, &g.node_type, A));
-  chk(upload(desc->node_index, (size_t)desc->n_nodes, &g.node_index, A));
-  chk(upload(desc->cube_vertices, 8 * (size_t)desc->n_cubes, &g.cube_v, A));
-  if (desc->n_polys) chk(upload(desc->poly_tet_offset, (size_t)desc->n_polys + 1, &g.poly_off, A));
-  chk(upload(desc->tet_vertices, 4 * (size_t)desc->n_tets, &g.tet_v, A));
-  chk(upload(desc->tet_circumsphere, 4 * (size_t)desc->n_tets, &g.tet_c, A));
-  chk(upload(desc->tet_volume, (size_t)desc->n_tets, &g.tet_vol, A));
-  chk(upload(desc->vertices, 3 * (size_t)desc->n_vertices, &g.verts, A));
+  chk(up.add(desc->node_type, (size_t)desc->n_nodes, &g.node_type));
+  chk(up.add(desc->node_index, (size_t)desc->n_nodes, &g.node_index));
+  chk(up.add(desc->cube_vertices, 8 * (size_t)desc->n_cubes, &g.cube_v));
+  if (desc->n_polys) chk(up.add(desc->poly_tet_offset, (size_t)desc->n_polys + 1, &g.poly_off));
+  chk(up.add(desc->tet_vertices, 4 * (size_t)desc->n_tets, &g.tet_v));
+  chk(up.add(desc->tet_circumsphere, 4 * (size_t)desc->n_tets, &g.tet_c));
+  chk(up.add(desc->tet_volume, (size_t)desc->n_tets, &g.tet_vol));
+  chk(up.add(desc->vertices, 3 * (size_t)desc->n_vertices, &g.verts));
+  chk(up.flush());
+  void* r = nullptr;
+  if (hipHostMalloc(&r, sizeof(CallReport), hipHostMallocDefault) == hipSuccess) G->report = static_cast<CallReport*>(r);
+  else (void)hipGetLastError();
   if (rc == BRILLE_OK) rc = build_fast_tables(desc, G);
   if (rc != BRILLE_OK) {
     free_all(A);
+    if (G->report) (void)hipHostFree(G->report);
     delete G;
     return rc;
   }
@@ -302,6 +337,7 @@ int brille_grid_create(const brille_grid_desc* desc, brille_grid** out) {
   void* e = nullptr;
   if (hipMalloc(&e, sizeof(ErrRec)) != hipSuccess) {
     free_all(A);
+    if (G->report) (void)hipHostFree(G->report);
     delete G;
     return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the error record");
   }
@@ -323,6 +359,7 @@ int brille_grid_destroy(brille_grid* G) {
   free_staging(G);
   free_binned(G);
   if (G->err) (void)hipFree(G->err);
+  if (G->report) (void)hipHostFree(G->report);
   delete G;
   return BRILLE_OK;
 }

@@ -11,6 +11,15 @@
 #include "interp_kernels.hpp"
 #include "proposal.hpp"
 
+namespace brille_amd {
+struct CallReport {
+  ErrRec err;
+  unsigned long long tried, verified;  // by the learned proposal
+  uint32_t differ;  // 1: some cube's corners are not those of an aligned box
+};
+constexpr int kPinSlots = 8;
+constexpr size_t kPinChunk = 2ull << 20;
+}  // namespace brille_amd
 struct brille_grid {
   // Every entry point that uses the handle holds `mu` for the whole call: the
   // error record, staging and work buffers, side stream and proposal state are
@@ -38,6 +47,13 @@ struct brille_grid {
   // staging buffers for host-memory calls
   void* stage = nullptr;
   size_t stage_bytes = 0;
+  // what a checked call reads back, in pinned memory (null: copied instead)
+  brille_amd::CallReport* report = nullptr;
+  // pinned memory the results of host-memory calls pass through (null: pageable
+  // copies), at most kPinSlots * kPinChunk bytes, and an event per slot
+  void* pin = nullptr;
+  size_t pin_bytes = 0;
+  hipEvent_t pin_ev[brille_amd::kPinSlots] = {};
   // work space of the binned pipeline and the sort (grown on demand, kept)
   void* bin_ws = nullptr;
   size_t bin_ws_bytes = 0;
@@ -88,6 +104,9 @@ const char* g_last_error_text();  // the message of the last failure on this thr
 int build_fast_tables(const brille_grid_desc* desc, brille_grid* G);
 void free_proposal(brille_grid* G);
 void free_staging(brille_grid* G);
+// a stream's error record and proposal counts on the host; waits for the stream
+int read_report(brille_grid* G, hipStream_t s, CallReport* out);
+int onepass_sc(const DataConst& d);
 int check_rotation_modes(const brille_grid* G);
 int check_payload_precision(const brille_grid* G, int precision);
 // the fused tile kernel of one call (fast: tuned fold-in and sums; else the literal restatement)

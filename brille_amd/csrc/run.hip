@@ -3,8 +3,10 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "fast_tables.hpp"
@@ -31,6 +33,140 @@ void free_staging(brille_grid* G) {
   if (G->stage) (void)hipFree(G->stage);
   G->stage = nullptr;
   G->stage_bytes = 0;
+  if (G->pin) (void)hipHostFree(G->pin);
+  G->pin = nullptr;
+  G->pin_bytes = 0;
+  for (hipEvent_t& e : G->pin_ev) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
+  }
+}
+
+// Pinned memory of at least `bytes` for the handle's host-memory calls, kept
+// for the next; false where it cannot be had (the calls then copy pageable).
+static bool ensure_pin(brille_grid* G, size_t bytes) {
+  if (G->pin_bytes >= bytes) return true;
+  if (G->pin) (void)hipHostFree(G->pin);
+  G->pin = nullptr;
+  G->pin_bytes = 0;
+  if (hipHostMalloc(&G->pin, bytes, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    G->pin = nullptr;
+    return false;
+  }
+  G->pin_bytes = bytes;
+  return true;
+}
+
+// One result on its way to the caller's memory.
+struct OutPiece {
+  char* host;
+  const char* dev;
+  size_t bytes;
+};
+
+// Results in device memory to the caller's pageable memory, on stream s; waits.
+// What bounds it: a fresh array's pages are mapped and zeroed as they are first
+// written, 14 GB/s for one thread, against 57 GB/s of the link.  Chunks of
+// kPinChunk bytes come to a ring of pinned slots and go on to their place by
+// up to kPinWorkers threads, each of which sends its freed slot the next chunk.
+// Whole calls of 100 003 points of 6 modes and 2 atoms FP64 (62 MB), pageable
+// copies 6.0 ms: one thread 4.7, three 2.5, six 2.3 in 1 MB chunks; four threads
+// 2.0 in 2 MB chunks (eight the same), 2.0 in 4 MB, 2.2 in 8 MB, 3.2 in 512 KB
+// (each chunk costs about 10 us of launches and waits).  Below two chunks per
+// thread the caller's thread works with fewer or none; where a thread or the
+// ring cannot be had, the rest do the work.
+constexpr uint64_t kPinWorkers = 4;
+// bytes of a host-memory call up to which the kernels use pinned memory directly
+constexpr size_t kDirectBytes = 4ull << 20;
+static int copy_out(brille_grid* G, const std::vector<OutPiece>& out, hipStream_t s) {
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  std::vector<OutPiece> chunks;
+  for (const OutPiece& p : out)
+    for (size_t o = 0; o < p.bytes; o += kPinChunk)
+      chunks.push_back({p.host + o, p.dev + o, std::min(kPinChunk, p.bytes - o)});
+  bool ring = ensure_pin(G, kPinSlots * kPinChunk);
+  for (hipEvent_t& e : G->pin_ev)
+    if (ring && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+      (void)hipGetLastError();
+      e = nullptr;
+      ring = false;
+    }
+  if (!ring) {
+    for (const OutPiece& p : out) HIP_TRY(hipMemcpyAsync(p.host, p.dev, p.bytes, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    return BRILLE_OK;
+  }
+  char* pin = static_cast<char*>(G->pin);
+  std::atomic<uint64_t> next{0};
+  std::atomic<uint64_t> sent[kPinSlots];  // 1 + the chunk a slot was last sent
+  std::atomic<int> error{(int)hipSuccess};
+  auto send = [&](uint64_t k) {
+    const int slot = (int)(k % kPinSlots);
+    hipError_t e = hipMemcpyAsync(pin + slot * kPinChunk, chunks[k].dev, chunks[k].bytes, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipEventRecord(G->pin_ev[slot], s);
+    if (e != hipSuccess) error = (int)e;
+    sent[slot] = k + 1;
+  };
+  for (auto& x : sent) x = 0;
+  for (uint64_t k = 0; k < chunks.size() && k < (uint64_t)kPinSlots; ++k) send(k);
+  auto work = [&] {
+    for (uint64_t k; (k = next.fetch_add(1)) < chunks.size();) {
+      const int slot = (int)(k % kPinSlots);
+      // chunk k - kPinSlots was taken before and its worker sends this one
+      while (sent[slot] != k + 1 && error == (int)hipSuccess) std::this_thread::yield();
+      if (error != (int)hipSuccess) return;
+      const hipError_t e = hipEventSynchronize(G->pin_ev[slot]);
+      if (e != hipSuccess) {
+        error = (int)e;
+        return;
+      }
+      std::memcpy(chunks[k].host, pin + slot * kPinChunk, chunks[k].bytes);
+      if (k + kPinSlots < chunks.size()) send(k + kPinSlots);
+    }
+  };
+  std::vector<std::thread> helpers;
+  const uint64_t hw = std::max(1u, std::thread::hardware_concurrency());
+  const uint64_t n_help = std::min({kPinWorkers, (uint64_t)chunks.size() / 2, hw});
+  for (uint64_t i = 1; i < n_help; ++i) {
+    try {
+      helpers.emplace_back([&] {
+        if (hipSetDevice(dev) == hipSuccess) work();
+      });
+    } catch (const std::exception&) {
+      break;
+    }
+  }
+  work();
+  for (std::thread& t : helpers) t.join();
+  HIP_TRY(hipStreamSynchronize(s));
+  if (error != (int)hipSuccess)
+    return fail(BRILLE_ERR_DEVICE, std::string("copying results: ") + hipGetErrorString((hipError_t)error.load()));
+  return BRILLE_OK;
+}
+
+__global__ void k_report(const ErrRec* err, const unsigned long long* stats, CallReport* out) {
+  out->err = *err;
+  out->tried = stats ? stats[0] : 0ull;
+  out->verified = stats ? stats[1] : 0ull;
+}
+
+// A kernel writes the record to pinned memory, one wait instead of a pageable
+// copy's two (257 points of 6 scalar modes: whole call 54 -> 47 us).
+int read_report(brille_grid* G, hipStream_t s, CallReport* out) {
+  if (G->report) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(1), 0, s, G->err, G->prop_stats, G->report);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(s));
+    *out = *G->report;
+    return BRILLE_OK;
+  }
+  out->tried = out->verified = 0;
+  if (G->prop_stats) HIP_TRY(hipMemcpyAsync(&out->tried, G->prop_stats, 16, hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipMemcpyAsync(&out->err, G->err, sizeof(ErrRec), hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
+  return BRILLE_OK;
 }
 
 // Interpolator::rotate_in_place dispatch  src/interpolator.hpp:387-428
@@ -246,16 +382,6 @@ int report_point_error(const ErrRec& e, const double* Q, uint64_t n, bool host_m
   }
 }
 
-// proposals tried / verified by the call that just ran on stream s
-static int read_proposal_stats(brille_grid* G, hipStream_t s) {
-  unsigned long long st[2] = {0, 0};
-  HIP_TRY(hipMemcpyAsync(st, G->prop_stats, sizeof(st), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  G->last_tried = st[0];
-  G->last_hits = st[1];
-  return BRILLE_OK;
-}
-
 int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_run_opts* opts_in, void* values_out,
                     void* vectors_out, const brille_aux_out* aux_in, hipStream_t s, brille_kernel_times* times,
                     uint32_t iters, int fold) {
@@ -290,6 +416,15 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
   a.prop = G->prop;
   if (opts.use_proposal) zero_words(G->prop_stats, 4, s);  // tried, verified (two 64-bit counters)
   a.err = G->err;
+  CallReport rep{};
+  auto finish_call = [&] {
+    const int r = read_report(G, s, &rep);
+    if (r == BRILLE_OK && opts.use_proposal) {
+      G->last_tried = rep.tried;
+      G->last_hits = rep.verified;
+    }
+    return r;
+  };
   if (opts.memory == BRILLE_MEM_DEVICE) {
     a.Q = Q;
     a.n = n;
@@ -349,15 +484,11 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
       if (rc != BRILLE_OK) return rc;
     }
     HIP_TRY(hipGetLastError());
-    if (opts.use_proposal) {
-      rc = read_proposal_stats(G, s);
-      if (rc != BRILLE_OK) return rc;
-    }
-    if (!opts.check && !times) return BRILLE_OK;
-    ErrRec e;
-    HIP_TRY(hipMemcpyAsync(&e, G->err, sizeof(e), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (e.count) return report_point_error(e, Q, n, false);
+    const bool check = opts.check || times;
+    if (!check && !opts.use_proposal) return BRILLE_OK;
+    rc = finish_call();
+    if (rc != BRILLE_OK || !check) return rc;
+    if (rep.err.count) return report_point_error(rep.err, Q, n, false);
     return BRILLE_OK;
   }
   // host memory: stream through device staging in chunks
@@ -378,16 +509,26 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
   const size_t auxper[10] = {24, 12, 4, 4, 4, 4, 1, 32, 64, 1};
   for (int i = 0; i < 10; ++i)
     if (*auxp[i]) add(*auxp[i], auxper[i]);
-  if (G->stage_bytes < off) {
-    free_staging(G);
+  // A small call's kernels read Q from and write results to pinned memory
+  // themselves, one wait instead of a copy and wait per array (6 modes of 2
+  // atoms FP64: 101 points 84 -> 48 us, 1 001 points, 0.6 MB, 125 -> 70 us, 6 001
+  // points, 3.7 MB, 304 -> 247 us).  The general sums, which read back what they
+  // wrote, and the larger calls go through device memory.
+  const bool direct = off <= kDirectBytes && fast && !opts.use_proposal && (wide_rows(G->d) || onepass_sc(G->d)) &&
+                      ensure_pin(G, kDirectBytes);
+  if (!direct && G->stage_bytes < off) {
+    if (G->stage) (void)hipFree(G->stage);
+    G->stage = nullptr;
+    G->stage_bytes = 0;
     HIP_TRY(hipMalloc(&G->stage, off));
     G->stage_bytes = off;
   }
-  char* st = static_cast<char*>(G->stage);
+  char* st = static_cast<char*>(direct ? G->pin : G->stage);
   hipLaunchKernelGGL(k_err_init2, dim3(1), dim3(1), 0, s, G->err);
   for (uint64_t c0 = 0; c0 < n; c0 += chunk) {
     const uint64_t m = std::min(chunk, n - c0);
-    HIP_TRY(hipMemcpyAsync(st + slots[0].off, Q + 3 * c0, m * 3 * sizeof(double), hipMemcpyHostToDevice, s));
+    if (direct) std::memcpy(st + slots[0].off, Q + 3 * c0, m * 3 * sizeof(double));
+    else HIP_TRY(hipMemcpyAsync(st + slots[0].off, Q + 3 * c0, m * 3 * sizeof(double), hipMemcpyHostToDevice, s));
     a.Q = reinterpret_cast<const double*>(st + slots[0].off);
     a.n = m;
     a.base = c0;
@@ -402,21 +543,23 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
       if (*auxp[i]) *dauxp[i] = st + slots[k++].off;
     a.aux = da;
     rc = dispatch(G, a, opts, s);
-    if (rc != BRILLE_OK) return rc;
+    if (rc != BRILLE_OK) {
+      (void)hipStreamSynchronize(s);  // what was launched may still write to the buffers kept for the next call
+      return rc;
+    }
     HIP_TRY(hipGetLastError());
+    if (c0 + m == n && direct) rc = finish_call();
+    std::vector<OutPiece> out;
     for (size_t i = 1; i < slots.size(); ++i)
-      HIP_TRY(hipMemcpyAsync(static_cast<char*>(slots[i].host) + c0 * slots[i].per, st + slots[i].off, m * slots[i].per,
-                             hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-  }
-  if (opts.use_proposal) {
-    rc = read_proposal_stats(G, s);
+      out.push_back({static_cast<char*>(slots[i].host) + c0 * slots[i].per, st + slots[i].off, m * slots[i].per});
+    if (direct)
+      for (const OutPiece& p : out) std::memcpy(p.host, p.dev, p.bytes);
+    else rc = copy_out(G, out, s);
     if (rc != BRILLE_OK) return rc;
   }
-  ErrRec e;
-  HIP_TRY(hipMemcpyAsync(&e, G->err, sizeof(e), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  if (e.count) return report_point_error(e, Q, n, true);
+  if (!direct) rc = finish_call();
+  if (rc != BRILLE_OK) return rc;
+  if (rep.err.count) return report_point_error(rep.err, Q, n, true);
   return BRILLE_OK;
 }
 
@@ -436,7 +579,7 @@ __global__ __launch_bounds__(256) void k_cube_corners(GridConst g, uint64_t n_cu
            __double_as_longlong(p[1]) == __double_as_longlong(kCubeY[i] ? v7[1] : v0[1]) &&
            __double_as_longlong(p[2]) == __double_as_longlong(kCubeZ[i] ? v7[2] : v0[2]);
   }
-  if (!same) atomicOr(differ, 1u);
+  if (!same) *differ = 1u;
 }
 
 // FP32 affine forms of the barycentric weights of every tetrahedron (16 floats
@@ -495,17 +638,11 @@ static int build_cell_tables(const brille_grid_desc* d, brille_grid* G) {
   GridConst& g = G->g;
   g.cubes_aligned = 0;
   g.tet_bary = nullptr;
-  if (d->n_cubes) {
-    void* flag = nullptr;
-    uint32_t differ = 1;
-    if (hipMalloc(&flag, sizeof(differ)) != hipSuccess) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed");
-    G->grid_allocs.push_back(flag);
-    zero_words(flag, 1, nullptr);
+  const bool corners = d->n_cubes && G->report;
+  if (corners) {
+    G->report->differ = 0;
     hipLaunchKernelGGL(k_cube_corners, dim3((unsigned)((d->n_cubes + 255) / 256)), dim3(256), 0, nullptr, g, d->n_cubes,
-                       static_cast<uint32_t*>(flag));
-    if (hipMemcpy(&differ, flag, sizeof(differ), hipMemcpyDeviceToHost) != hipSuccess)
-      return fail(BRILLE_ERR_DEVICE, "checking the cubes failed");
-    g.cubes_aligned = differ ? 0 : 1;
+                       &G->report->differ);
   }
   if (d->n_tets) {
     double reach = 0;
@@ -517,9 +654,11 @@ static int build_cell_tables(const brille_grid_desc* d, brille_grid* G) {
     G->grid_allocs.push_back(forms);
     hipLaunchKernelGGL(k_tet_bary, dim3((unsigned)((d->n_tets + 255) / 256)), dim3(256), 0, nullptr, g, d->n_tets, reach,
                        static_cast<float*>(forms));
-    if (hipDeviceSynchronize() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "making the tetrahedron forms failed");
     g.tet_bary = static_cast<const float*>(forms);
   }
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
+    return fail(BRILLE_ERR_DEVICE, "making the cell tables failed");
+  if (corners) g.cubes_aligned = G->report->differ ? 0 : 1;
   return BRILLE_OK;
 }
 
