@@ -6,13 +6,16 @@
 // orders the points by trellis node range, so that the points one tile sums
 // share their vertices and the rows hit in cache:
 //   k_bin_fold     stage (a) + node subscript, one lane per point; a 32-byte
-//                  FoldRec per point in input order and a per-block histogram
-//                  of node-range buckets (failed points get the last bucket);
+//                  FoldRec and a 4-byte key per point in input order and a
+//                  per-block histogram of node-range buckets (failed points
+//                  get the last bucket);
 //   k_scan_*       exclusive scan of the block histograms (bucket-major);
-//   k_bin_scatter  each block moves its FoldRecs to its reserved slots of each
-//                  bucket (a SortRec adds the input index);
-//   k_bin_sums     the rest of stage (b) and stages (c1, c2) on bucket-ordered
-//                  tiles, writing output rows at the input index.
+//   k_bin_scatter  each block moves its keys and input indices to its reserved
+//                  slots of each bucket;
+//   k_bucket_perm  input indices in node order, bucket by bucket;
+//   k_bin_sums     the rest of stage (b) and stages (c1, c2) on node-ordered
+//                  tiles, reading FoldRecs and writing output rows at the
+//                  input index.
 // Within a bucket the order is whatever the LDS atomics give; every point is
 // computed independently, so the outputs do not depend on it.
 #include <algorithm>
@@ -49,16 +52,19 @@ constexpr uint32_t kNodePoly = 1u << 31;
 constexpr uint32_t kPermPoly = 1u << 31;
 constexpr uint32_t kPropMinCand = 8;
 __device__ __forceinline__ uint32_t meta_status(uint32_t meta) { return (meta >> 16) & 255u; }
-struct SortRec {
-  double q[3];
-  uint32_t node;
-  uint32_t meta;
-  uint32_t index;  // input index within the pass
-  uint32_t hint;   // proposed tetrahedron (kNoTet: none)
+// what the bucketing moves of a point: its node | kNodePoly (kNoKey: it failed)
+// and its input index within the pass.  The record stays where the fold wrote
+// it: moving 40 bytes of it cost more than the sums' reading it by index does
+// (1e7 points of 2 atoms FP32: bucketing 0.465 -> 0.225 ms, sums 1.75 -> 1.84;
+// FP64, 3e6: 0.124 -> 0.077, sums unchanged; a record padded to 64 bytes to
+// write whole granules was slower, 0.585).
+struct SortKey {
+  uint32_t key, index;
 };
+constexpr uint32_t kNoKey = 0xFFFFFFFFu;  // no node index: those stay below 2^31 - 1
 
-__device__ __forceinline__ uint32_t bucket_of(uint32_t node, uint32_t meta, uint32_t nb, uint64_t n_nodes) {
-  return meta_status(meta) != BRILLE_PT_OK ? nb : (uint32_t)(((uint64_t)node * nb) / n_nodes);
+__device__ __forceinline__ uint32_t bucket_of(uint32_t key, uint32_t nb, uint64_t n_nodes) {
+  return key == kNoKey ? nb : (uint32_t)(((uint64_t)(key & ~kNodePoly) * nb) / n_nodes);
 }
 
 // mark_poly: flag (kMetaPoly) the points for the learned proposal, those
@@ -68,7 +74,8 @@ __device__ __forceinline__ uint32_t bucket_of(uint32_t node, uint32_t meta, uint
 // than the four that 124 VGPRs allow: 9 % less time.
 template <bool Fast>
 __global__ __launch_bounds__(BIN_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_bin_fold(GridConst g, const double* Q, uint32_t n, int fold,
-                                                        FoldRec* __restrict__ rec, uint32_t* __restrict__ hist,
+                                                        FoldRec* __restrict__ rec, uint32_t* __restrict__ key,
+                                                        uint32_t* __restrict__ hist,
                                                         uint32_t nblk, uint32_t nb,
                                                         ErrRec* __restrict__ err, uint64_t base, int mark_poly) {
   extern __shared__ uint32_t h[];  // nb + 1 counters
@@ -92,7 +99,9 @@ __global__ __launch_bounds__(BIN_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) 
       r.node = L.node;
       r.meta = (L.rot & 255u) | ((L.invrot & 255u) << 8) | ((uint32_t)L.status << 16) | (poly ? kMetaPoly : 0u);
       rec[p] = r;
-      atomicAdd(&h[bucket_of(r.node, r.meta, nb, g.n_nodes)], 1u);
+      const uint32_t kp = L.status != BRILLE_PT_OK ? kNoKey : poly ? L.node | kNodePoly : L.node;
+      key[p] = kp;
+      atomicAdd(&h[bucket_of(kp, nb, g.n_nodes)], 1u);
     }
   }
   __syncthreads();
@@ -172,9 +181,9 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_scan_apply(uint32_t* a, uint64_t 
   }
 }
 
-__global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const FoldRec* rec, uint32_t n, const uint32_t* off,
-                                                           uint32_t nblk, uint32_t nb, uint64_t n_nodes, SortRec* out,
-                                                           uint32_t* out_node) {
+__global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const uint32_t* key, uint32_t n, const uint32_t* off,
+                                                           uint32_t nblk, uint32_t nb, uint64_t n_nodes,
+                                                           SortKey* out) {
   extern __shared__ uint32_t s[];  // base[nb + 1], count[nb + 1]
   uint32_t* base = s;
   uint32_t* cnt = s + nb + 1;
@@ -184,36 +193,24 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const FoldRec* rec, u
   }
   __syncthreads();
   const uint32_t b0 = blockIdx.x * BIN_SPAN;
-  constexpr int GRP = 8;  // records requested before any is placed
-  for (int i0 = 0; i0 < BIN_PPT; i0 += GRP) {
-    FoldRec rr[GRP];
+  uint32_t kk[BIN_PPT];  // requested before any is placed
 #pragma unroll
-    for (int i = 0; i < GRP; ++i) {
-      const uint32_t p = b0 + (i0 + i) * BIN_BLOCK + threadIdx.x;
-      if (p < n) rr[i] = rec[p];
-    }
+  for (int i = 0; i < BIN_PPT; ++i) {
+    const uint32_t p = b0 + i * BIN_BLOCK + threadIdx.x;
+    if (p < n) kk[i] = key[p];
+  }
 #pragma unroll
-    for (int i = 0; i < GRP; ++i) {
-    const uint32_t p = b0 + (i0 + i) * BIN_BLOCK + threadIdx.x;
+  for (int i = 0; i < BIN_PPT; ++i) {
+    const uint32_t p = b0 + i * BIN_BLOCK + threadIdx.x;
     if (p < n) {
-      const FoldRec& r = rr[i];
-      const uint32_t k = bucket_of(r.node, r.meta, nb, n_nodes);
-      const uint32_t j = atomicAdd(&cnt[k], 1u);
-      SortRec o;
-      o.q[0] = r.q[0]; o.q[1] = r.q[1]; o.q[2] = r.q[2];
-      o.node = r.node;
-      o.meta = r.meta;
-      o.index = p;
-      o.hint = kNoTet;
-      out[base[k] + j] = o;
-      out_node[base[k] + j] = r.node | ((r.meta & kMetaPoly) ? kNodePoly : 0u);
-    }
+      const uint32_t k = bucket_of(kk[i], nb, n_nodes);
+      out[base[k] + atomicAdd(&cnt[k], 1u)] = SortKey{kk[i], p};
     }
   }
 }
 
 // Node order inside each bucket: one block per bucket counts its points per
-// trellis node in LDS and writes perm, the positions of the bucket's records
+// trellis node in LDS and writes perm, the input indices of the bucket's points
 // in node order, so that the points of one cube are summed together and its
 // rows are read from L1.  Within a node the order is whatever the LDS atomics
 // give (the points are independent).  Buckets spanning more than kPermNodes
@@ -221,7 +218,7 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const FoldRec* rec, u
 // the record's proposal flag (kPermPoly, from kNodePoly).
 constexpr uint32_t kPermNodes = 4096;
 constexpr int PERM_BLOCK = 1024;
-__global__ __launch_bounds__(PERM_BLOCK) void k_bucket_perm(const uint32_t* node, uint32_t m, const uint32_t* off,
+__global__ __launch_bounds__(PERM_BLOCK) void k_bucket_perm(const SortKey* sk, uint32_t m, const uint32_t* off,
                                                            uint32_t nblk, uint32_t nb, uint64_t n_nodes,
                                                            uint32_t* perm) {
   __shared__ uint32_t cnt[kPermNodes];
@@ -232,12 +229,13 @@ __global__ __launch_bounds__(PERM_BLOCK) void k_bucket_perm(const uint32_t* node
   const uint64_t hi = b < nb ? ((uint64_t)(b + 1) * n_nodes + nb - 1) / nb : lo;
   const uint32_t nn = (uint32_t)(hi - lo);
   if (b == nb || nn == 0 || nn > kPermNodes) {
-    for (uint32_t i = s0 + threadIdx.x; i < s1; i += PERM_BLOCK) perm[i] = i | (node[i] & kNodePoly);
+    for (uint32_t i = s0 + threadIdx.x; i < s1; i += PERM_BLOCK)
+      perm[i] = sk[i].index | (sk[i].key == kNoKey ? 0u : sk[i].key & kNodePoly);
     return;
   }
   for (uint32_t k = threadIdx.x; k < nn; k += PERM_BLOCK) cnt[k] = 0;
   __syncthreads();
-  for (uint32_t i = s0 + threadIdx.x; i < s1; i += PERM_BLOCK) atomicAdd(&cnt[(node[i] & ~kNodePoly) - (uint32_t)lo], 1u);
+  for (uint32_t i = s0 + threadIdx.x; i < s1; i += PERM_BLOCK) atomicAdd(&cnt[(sk[i].key & ~kNodePoly) - (uint32_t)lo], 1u);
   __syncthreads();
   // exclusive scan of cnt[0, nn): each thread a contiguous run, then the runs
   const uint32_t per = (nn + PERM_BLOCK - 1) / PERM_BLOCK;
@@ -253,8 +251,8 @@ __global__ __launch_bounds__(PERM_BLOCK) void k_bucket_perm(const uint32_t* node
   }
   __syncthreads();
   for (uint32_t i = s0 + threadIdx.x; i < s1; i += PERM_BLOCK) {
-    const uint32_t nd = node[i];
-    perm[atomicAdd(&cnt[(nd & ~kNodePoly) - (uint32_t)lo], 1u)] = i | (nd & kNodePoly);
+    const SortKey e = sk[i];
+    perm[atomicAdd(&cnt[(e.key & ~kNodePoly) - (uint32_t)lo], 1u)] = e.index | (e.key & kNodePoly);
   }
 }
 
@@ -308,7 +306,7 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_poly_list(const uint32_t* perm, u
 // ranges in its LDS slice, runs the network and writes the proposed
 // tetrahedron to the record's hint.  Grid-stride over the list, whose length
 // is read on the device.
-__global__ __launch_bounds__(256) void k_bin_propose(GridConst g, ProposalConst pc, SortRec* srt,
+__global__ __launch_bounds__(256) void k_bin_propose(GridConst g, ProposalConst pc, const FoldRec* recs, uint32_t* hint,
                                                      const uint32_t* list, const uint32_t* count) {
   // chunks of 16 listed points per wave, four waves per block, grid-stride
   // over the list; blocks past the list's end leave before copying weights
@@ -335,7 +333,7 @@ __global__ __launch_bounds__(256) void k_bin_propose(GridConst g, ProposalConst 
   uint32_t rec = 0;
   if (lane < k) {
     rec = list[c0 + lane];
-    const SortRec& r = srt[rec];
+    const FoldRec& r = recs[rec];
     const double q[3] = {r.q[0], r.q[1], r.q[2]};
     const uint32_t nd = r.node;
     double x[3];
@@ -357,7 +355,7 @@ __global__ __launch_bounds__(256) void k_bin_propose(GridConst g, ProposalConst 
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if (lane < k) srt[rec].hint = s_out[wave][lane];
+  if (lane < k) hint[rec] = s_out[wave][lane];
   // the next chunk overwrites this wave's LDS slices
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -396,7 +394,7 @@ constexpr int sums_waves() {
 }
 template <typename Real, int L, int SC, int SV, bool Prop>
 __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(sums_waves<Real, L, SC>())))
-void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
+void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const FoldRec* recs, const uint32_t* hint,
                                                     const uint32_t* perm, uint32_t n, void* __restrict__ vals,
                                                     void* __restrict__ vecs, brille_aux_out aux,
                                                     ErrRec* __restrict__ err, uint64_t base, uint32_t tile_pts) {
@@ -459,12 +457,16 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
   __shared__ uint32_t s_wave_tab[TILE / 64];
   if (Prop) __syncthreads();
   const bool live = tid < tile_n && p < n;
-  SortRec sr;
+  FoldRec sr;
+  uint32_t index = 0, tet_hint = kNoTet;
   Located P;
   P.status = BRILLE_PT_OK;
   P.cube = kNoCube;
   if (live) {
-    sr = srt[perm[p] & ~kPermPoly];
+    const uint32_t e = perm[p];
+    index = e & ~kPermPoly;
+    sr = recs[index];
+    if (Prop) tet_hint = (e & kPermPoly) ? hint[index] : kNoTet;
     P.q[0] = sr.q[0]; P.q[1] = sr.q[1]; P.q[2] = sr.q[2];
     P.tau[0] = P.tau[1] = P.tau[2] = 0;
     P.node = sr.node;
@@ -477,8 +479,8 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
     if (P.status == BRILLE_PT_OK) {
       if constexpr (Prop) {
         bool verified = false;
-        node_slots(g, P, sr.hint, pc.margin, &verified);
-        if (sr.hint != kNoTet) {
+        node_slots(g, P, tet_hint, pc.margin, &verified);
+        if (tet_hint != kNoTet) {
           atomicAdd(&s_tried, 1u);
           if (verified) atomicAdd(&s_verified, 1u);
         }
@@ -486,7 +488,7 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
         node_slots(g, P);
       }
       // failed fold-ins were reported by k_bin_fold
-      if (P.status != BRILLE_PT_OK && lead) report_point(err, base + sr.index, P.status);
+      if (P.status != BRILLE_PT_OK && lead) report_point(err, base + index, P.status);
     }
   }
   // Stable partition of the tile: points the cube factor table serves first,
@@ -511,10 +513,10 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const SortRec* srt,
     PointRec<Real>& r = s_rec[slot];
     r.nslot = 0;
     if (live) {
-      s_out[slot] = sr.index;
+      s_out[slot] = index;
       if (P.status == BRILLE_PT_OK)
         store_record<Real, L, SC>(g, d, P, r, s_ph, s_q, slot, ph_in_lds, n_atoms, !kOpFrames);
-      if (lead) write_aux(aux, sr.index, P);
+      if (lead) write_aux(aux, index, P);
     }
   }
   __syncthreads();
@@ -659,7 +661,7 @@ __global__ __launch_bounds__(256) void k_wide_atom_factors(GridConst g, DataCons
   }
 }
 
-using SumsKernel = void (*)(GridConst, DataConst, ProposalConst, const SortRec*, const uint32_t*, uint32_t, void*,
+using SumsKernel = void (*)(GridConst, DataConst, ProposalConst, const FoldRec*, const uint32_t*, const uint32_t*, uint32_t, void*,
                            void*, brille_aux_out, ErrRec*, uint64_t, uint32_t);
 
 template <typename Real>
@@ -839,10 +841,9 @@ int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s) {
 
 // Buckets of at most kNodesPerBucket trellis nodes: k_bucket_perm orders each
 // bucket by node in LDS (kPermNodes counters), so the buckets only have to be
-// few enough that a bucketing block (BIN_SPAN points) puts runs of records
-// into each: the scatter writes a block's records of one bucket as one run,
-// and short runs cost partial-line writes.  Config 4 at 1e8 Q: 1024 nodes per
-// bucket 26.7 ms, 2048 26.6 ms, 4096 25.9 ms per call.  A grid of few nodes
+// few enough that a bucketing block (BIN_SPAN points) puts runs of keys into
+// each: the scatter writes a block's keys of one bucket as one run, and short
+// runs cost partial-line writes.  A grid of few nodes
 // still gets kMinBuckets of them (at most one per node): k_bucket_perm runs a
 // block per bucket, and sixteen blocks left the chip idle (1e7 points of a
 // 360-node grid: bucketing 1.24 ms with 16).
@@ -968,8 +969,10 @@ static int ensure_side_stream(brille_grid* G) {
 // One half of the work space: the buffers of one pass.
 struct PassBuffers {
   FoldRec* rec;
-  SortRec* srt;
-  uint32_t *hist, *part, *plist, *pcount, *perm, *snode;
+  SortKey* srt;
+  uint32_t* key;   // shares perm's memory (read before perm is written)
+  uint32_t* hint;  // shares srt's (written after srt is read)
+  uint32_t *hist, *part, *plist, *pcount, *perm;
 };
 
 // A call's passes (BIN_CHUNK points each) run as a two-stage pipeline when
@@ -990,7 +993,7 @@ struct PassBuffers {
 // Byte offsets of one pass's buffers (a half of the work space) for passes of
 // `chunk` points.
 struct PassLayout {
-  uint64_t rec, srt, hist, part, list, perm, node, cnt, half;
+  uint64_t rec, srt, hist, part, list, perm, cnt, half;
   uint64_t scan_blocks;  // segments of the histogram scan (k_scan_top handles at most 256 Ki)
 };
 static PassLayout pass_layout(uint64_t chunk, uint32_t nb) {
@@ -1001,12 +1004,11 @@ static PassLayout pass_layout(uint64_t chunk, uint32_t nb) {
   PassLayout L;
   L.rec = 0;
   L.srt = al(chunk * sizeof(FoldRec));
-  L.hist = L.srt + al(chunk * sizeof(SortRec));
+  L.hist = L.srt + al(chunk * sizeof(SortKey));
   L.part = L.hist + al(m_max * 4);
   L.list = L.part + al(np_max * 4);
   L.perm = L.list + al(chunk * 4);
-  L.node = L.perm + al(chunk * 4);
-  L.cnt = L.node + al(chunk * 4);
+  L.cnt = L.perm + al(chunk * 4);
   L.half = L.cnt + 256;
   L.scan_blocks = np_max;
   return L;
@@ -1046,20 +1048,21 @@ int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStr
   if (Lo.scan_blocks > 256ull * 1024) return fail(BRILLE_ERR_INVALID_ARGUMENT, "binned pass too large");
   if (G->g.n_nodes >= kNodePoly) return fail(BRILLE_ERR_INVALID_ARGUMENT, "the binned kernel takes grids of fewer than 2^31 nodes");
   const uint64_t o_rec = Lo.rec, o_srt = Lo.srt, o_hist = Lo.hist, o_part = Lo.part, o_list = Lo.list,
-                 o_perm = Lo.perm, o_node = Lo.node, o_cnt = Lo.cnt, half = Lo.half;
+                 o_perm = Lo.perm, o_cnt = Lo.cnt, half = Lo.half;
   const bool prop = a.use_proposal != 0;
   PassBuffers buf[2];
   for (int h = 0; h < halves; ++h) {
     char* ws = static_cast<char*>(ws_base) + h * half;
     PassBuffers& b = buf[h];
     b.rec = reinterpret_cast<FoldRec*>(ws + o_rec);
-    b.srt = reinterpret_cast<SortRec*>(ws + o_srt);
+    b.srt = reinterpret_cast<SortKey*>(ws + o_srt);
+    b.hint = reinterpret_cast<uint32_t*>(ws + o_srt);
+    b.key = reinterpret_cast<uint32_t*>(ws + o_perm);
     b.hist = reinterpret_cast<uint32_t*>(ws + o_hist);
     b.part = reinterpret_cast<uint32_t*>(ws + o_part);
     b.plist = reinterpret_cast<uint32_t*>(ws + o_list);
     b.pcount = reinterpret_cast<uint32_t*>(ws + o_cnt);
     b.perm = reinterpret_cast<uint32_t*>(ws + o_perm);
-    b.snode = reinterpret_cast<uint32_t*>(ws + o_node);
   }
   // timing: five events per pass (fold start, fold end, bucket end on the
   // preparing stream; sums start and end on the call stream)
@@ -1103,20 +1106,20 @@ int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStr
     if (prop) zero_words(b.pcount, 1, side);
     mark(k, 0, side);
     hipLaunchKernelGGL(k_bin_fold<true>, dim3(nblk), dim3(BIN_BLOCK), lds1, side, G->g, a.Q + 3 * c0, m, a.fold,
-                       b.rec, b.hist, nblk, nb, a.err, a.base + c0, prop ? 1 : 0);
+                       b.rec, b.key, b.hist, nblk, nb, a.err, a.base + c0, prop ? 1 : 0);
     mark(k, 1, side);
     hipLaunchKernelGGL(k_scan_reduce, dim3(np), dim3(BIN_BLOCK), 0, side, b.hist, M, b.part);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(BIN_BLOCK), 0, side, b.part, np);
     hipLaunchKernelGGL(k_scan_apply, dim3(np), dim3(BIN_BLOCK), 0, side, b.hist, M, b.part);
-    hipLaunchKernelGGL(k_bin_scatter, dim3(nblk), dim3(BIN_BLOCK), 2 * lds1, side, b.rec, m, b.hist, nblk, nb,
-                       G->g.n_nodes, b.srt, b.snode);
-    hipLaunchKernelGGL(k_bucket_perm, dim3(nb + 1), dim3(PERM_BLOCK), 0, side, b.snode, m, b.hist, nblk, nb,
+    hipLaunchKernelGGL(k_bin_scatter, dim3(nblk), dim3(BIN_BLOCK), 2 * lds1, side, b.key, m, b.hist, nblk, nb,
+                       G->g.n_nodes, b.srt);
+    hipLaunchKernelGGL(k_bucket_perm, dim3(nb + 1), dim3(PERM_BLOCK), 0, side, b.srt, m, b.hist, nblk, nb,
                        G->g.n_nodes, b.perm);
     if (prop) {
       hipLaunchKernelGGL(k_poly_list, dim3((m + LIST_SPAN - 1) / LIST_SPAN), dim3(BIN_BLOCK), 0, side, b.perm, m,
                          b.plist, b.pcount);
       hipLaunchKernelGGL(k_bin_propose, dim3(std::min<uint32_t>((m + 63) / 64, std::max<uint32_t>(G->n_cu, 1) * 4)),
-                         dim3(256), 0, side, G->g, a.prop, b.srt, b.plist, b.pcount);
+                         dim3(256), 0, side, G->g, a.prop, b.rec, b.hint, b.plist, b.pcount);
     }
     mark(k, 2, side);
     if (halves > 1) {
@@ -1128,7 +1131,7 @@ int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStr
     uint32_t tile_pts, groups;
     sum_split(G, m, prop, precision, &tile_pts, &groups);
     const dim3 sgrid((m + tile_pts - 1) / tile_pts, groups);
-    hipLaunchKernelGGL(sums, sgrid, dim3(TILE), G->d.n_keys ? 32u * TILE : 0u, s, G->g, G->d, a.prop, b.srt, b.perm, m,
+    hipLaunchKernelGGL(sums, sgrid, dim3(TILE), G->d.n_keys ? 32u * TILE : 0u, s, G->g, G->d, a.prop, b.rec, b.hint, b.perm, m,
                        static_cast<char*>(a.vals) + c0 * vb, static_cast<char*>(a.vecs) + c0 * cb,
                        offset_aux(a.aux, c0), a.err, a.base + c0, tile_pts);
     mark(k, 4, s);
