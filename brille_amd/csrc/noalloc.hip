@@ -3,13 +3,13 @@
 // tight serving loops, harnesses that forbid hipMalloc).
 //
 // Everything brille_ir_interpolate_at keeps in device memory of its own for
-// a call -- the error record, and for the binned pipeline the fold and sort
-// records, bucket histograms, scans, node-order permutation and proposal list
+// a call -- the error record, and for the binned pipeline the fold
+// records and keys, bucket histograms, scans, node-order permutation and proposal list
 // of a pass -- lives here in one file-scope device array, `scratch`, of
 // kScratchBytes.  Each GPU holds its own copy at its own address from module
 // load until the process ends; the first call on a device looks that address
 // up (hipGetSymbolAddress) and keeps it.  The binned pipeline runs in passes
-// sized to fit (2^19 points) on the caller's stream alone, with the row table
+// sized to fit (2^20 points) on the caller's stream alone, with the row table
 // only if an earlier call built it.  Inputs and outputs are caller device
 // memory, as in brille_ir_interpolate_at with BRILLE_MEM_DEVICE.
 //

@@ -127,6 +127,7 @@ static int copy_out(brille_grid* G, const std::vector<OutPiece>& out, hipStream_
     }
   };
   std::vector<std::thread> helpers;
+  helpers.reserve(kPinWorkers);
   const uint64_t hw = std::max(1u, std::thread::hardware_concurrency());
   const uint64_t n_help = std::min({kPinWorkers, (uint64_t)chunks.size() / 2, hw});
   for (uint64_t i = 1; i < n_help; ++i) {

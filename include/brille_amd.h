@@ -185,8 +185,9 @@ typedef struct brille_perm_desc {
 
 enum brille_precision { BRILLE_FP64 = 0, BRILLE_FP32 = 1 };
 enum brille_memory { BRILLE_MEM_DEVICE = 0, BRILLE_MEM_HOST = 1 };
-/* AUTO and TUNED pick TILE or BINNED by size (TILE when any aux output is
- * requested); PLAIN is the literal FP64 restatement (exact fold-in, atan2
+/* AUTO and TUNED pick TILE or BINNED by the work and the payload (TILE when any
+ * aux output is requested, and under stream capture unless an earlier call has
+ * left what BINNED would allocate); PLAIN is the literal FP64 restatement (exact fold-in, atan2
  * antiphases); TILE is the fused one-launch kernel; BINNED buckets points by
  * trellis node range first so the payload gathers hit in cache (device work
  * space; reports every aux output but tau). */
@@ -304,7 +305,7 @@ int brille_interpolate_at(brille_grid* grid, const double* Q, uint64_t n,
  * loops, harnesses that forbid hipMalloc): it allocates nothing.  Its error
  * record and the binned pipeline's work space live in one static device array
  * of 64 MiB per GPU (held from module load until the process ends); passes
- * are sized to fit it (2^19 points) and run on `stream` alone, and the row
+ * are sized to fit it (2^20 points) and run on `stream` alone, and the row
  * table is used only if an earlier call built it.  Q, the outputs and aux must
  * be device memory (opts->memory = BRILLE_MEM_DEVICE); everything else is as
  * brille_ir_interpolate_at, results bit for bit the same.  Calls share their
@@ -319,10 +320,10 @@ int brille_ir_moveinto(brille_grid* grid, const double* Q, uint64_t n, int32_t m
                        uint32_t* invrot_out, uint8_t* status_out, void* stream);
 
 /* ---- many grids in one persistent launch (no reference counterpart) ---- */
-/* A batch holds filled grids (not owned; they must outlive it).  A run is one
- * persistent kernel whose blocks take tiles of points from a work counter
- * across all grids, captured once into a HIP graph per precision and schedule
- * and replayed, followed on the same stream by one binned call per grid
+/* A batch holds filled grids (not owned; they must outlive it).  A run is two
+ * persistent kernels side by side (grids of wide rows, and the others) whose
+ * blocks take tiles of points from a work counter across their grids, captured
+ * once into a HIP graph per precision and schedule and replayed, followed on the same stream by one binned call per grid
  * given at least `binned_min` points; the tile shape, block count, tiles per
  * grab, grid order and binned_min come from brille_batch_autotune (defaults
  * before it runs: no binned grids). */
@@ -338,8 +339,8 @@ int brille_batch_run(brille_batch* batch, const double* Q, const uint64_t* offse
 int brille_batch_autotune(brille_batch* batch, const double* Q, const uint64_t* offsets,
                           const brille_run_opts* opts, void* const* values_out,
                           void* const* vectors_out, void* stream);
-/* the schedule in use: points per tile (= threads per block), persistent
- * blocks, tiles per grab, grid order (0 as given, 1 costliest first), and
+/* the schedule in use: threads per block (and the most points of a tile; they
+ * hold fewer where a list's work is small), persistent blocks of each kernel, tiles per grab, grid order (0 as given, 1 costliest first), and
  * the point count from which a grid runs its own binned pipeline after the
  * persistent kernel instead (UINT64_MAX: none) */
 int brille_batch_schedule(const brille_batch* batch, uint32_t* tile_points, uint32_t* blocks,
