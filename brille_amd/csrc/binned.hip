@@ -870,8 +870,10 @@ static bool has_table(const DataConst& d, int precision) {
 //   2 atoms FP32: 300 007 points 140 / 160, 600 011 256 / 218 (46 MB payload
 //     330 / 328); FP64: 100 003 128 / 125, 200 003 239 / 160 (93 MB: 299 / 286)
 //   4 atoms FP32: 60 013 138 / 150, 100 003 235 / 152; FP64: 60 013 157 / 155
-//   8 atoms FP32: 10 007 128 / 126, 30 001 277 / 168; FP64: 3001 97 / 120
-//   24 atoms FP32: 3001 266 / 272, 10 001 799 / 547; FP64: 1001 290 / 226
+//   10 atoms FP32: 10 007 129 / 130, 30 001 270 / 164; FP64: 3001 96 / 130
+//   24 atoms FP32: 3001 263 / 261, 10 001 796 / 482; FP64: 1001 290 / 233
+// (a lower line for wide FP32 rows gained 3 % at 3001 points of a coarser grid
+// and cost the table's 0.4 ms on each first call).
 // A first call also builds the table, whose rows it would mostly compute for
 // itself anyway once there is a point for every four cells; a call that may
 // not build it (`build` false) is binned from the size where node order alone
