@@ -696,11 +696,11 @@ __device__ __forceinline__ void unit_onepass(const DataConst& d, const PointRec<
 // element and slot.  Every output element gets unit_onepass's arithmetic in
 // the same order, so both give the same bits.
 
-// lanes per unit: the row stride in 16-byte chunks (1 = no cooperation)
+// lanes per unit: the row stride in 16-byte chunks
 template <typename Real, int SC, int SV>
 constexpr int coop_lanes() {
-  const int bytes = ((2 * SC + SV) * (int)sizeof(Real) + 15) / 16 * 16;
-  if (bytes > 128) return 1;
+  constexpr int bytes = ((2 * SC + SV) * (int)sizeof(Real) + 15) / 16 * 16;
+  static_assert(bytes <= 128, "longer rows are not padded to a power of two");
   int p = 16;
   while (p < bytes) p <<= 1;
   return p / 16;
@@ -1896,8 +1896,9 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
       u0 = n_coop * B;
     }
   }
-  constexpr bool kCoop = L == LAYOUT_SCALAR && coop_lanes<Real, SC, SV>() > 1;
-  if constexpr (kCoop) {
+  if constexpr (L == LAYOUT_SCALAR) {
+    // (rows of one chunk too: tile_perms has no entry for the points the table
+    // serves, so none of them may reach unit_onepass below)
     constexpr uint32_t G = coop_lanes<Real, SC, SV>();
     if (table) {
       u0 = n_coop * B;

@@ -1,0 +1,46 @@
+"""Scalar rows of one to four elements with a PermutationTable in the binned sums:
+every point the row table serves is summed from it, also where a row is a single
+16-byte chunk (one element FP32), so that no point follows a slot permutation
+that was never looked up.  Needs an MI355X.
+"""
+import numpy as np
+import pytest
+
+from brille_amd import capi
+from brille_amd import synthetic as S
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+# modes: one, the usual, more than the block has lanes
+@pytest.mark.parametrize("elements", [1, 2, 3, 4])
+@pytest.mark.parametrize("modes", [1, 6, 300])
+def test_permuted_scalar_rows_in_the_binned_sums(elements, modes):
+    print(f"sorted rows: {elements} elements, {modes} modes", flush=True)
+    sp = dict(S.batch_specs(16)[3], v_target=400.0)
+    g = S.batch_grid(sp)
+    t = S.batch_layout_tables(g, sp)
+    V = len(t["vertices"])
+    r = np.random.default_rng(10 * modes + elements)
+    t.update(values=r.normal(size=(V, modes, 1)), values_elements=[1, 0, 0], branches=modes,
+             vectors=r.normal(size=(V, modes, elements)) + 1j * r.normal(size=(V, modes, elements)),
+             vectors_elements=[elements, 0, 0], vectors_rotates_like=0)
+    Q = r.uniform(-3, 3, size=(1500, 3))
+    rc, _, _, aux, _ = O.ir_interpolate_at(t, Q, nthreads=8)
+    assert rc == 0
+    used = [aux["iw_index"][:, 0].astype(np.uint64) * V + aux["iw_index"][:, k] for k in range(1, 8)]
+    keys = np.unique(np.concatenate(used))
+    perms = np.array([r.permutation(modes) for _ in range(9)], np.uint32)
+    perm = (keys, r.integers(0, 9, size=len(keys)).astype(np.uint32), perms)
+    rc, ov, oc, _, _ = O.ir_interpolate_at(t, Q, nthreads=8, perm=perm)
+    assert rc == 0
+    dev = capi.Grid(t, perm=perm)
+    for prec, tol in ((capi.FP64, 1e-12), (capi.FP32, 1e-5)):
+        bv, bc = dev.ir_interpolate_at(Q, precision=prec, kernel=capi.KERNEL_BINNED)
+        tv, tc = dev.ir_interpolate_at(Q, precision=prec, kernel=capi.KERNEL_TILE)
+        np.testing.assert_array_equal(bv, tv)
+        np.testing.assert_array_equal(bc, tc)
+        assert np.max(np.abs(bv - ov)) <= tol * np.abs(ov).max()
+        if elements == 1:  # one element's antiphase turns it onto the pivot: no cancelling overlap
+            assert np.max(np.abs(bc - oc)) <= tol * np.abs(oc).max()
