@@ -766,7 +766,8 @@ static int build_cube_rows(brille_grid* G, hipStream_t s, Real** out) {
     case 12: hipLaunchKernelGGL((k_table_rows<Real, 12>), grid, dim3(256), 0, s, G->g, d, cube_units, units, t); break;
     default: return fail(BRILLE_ERR_UNSUPPORTED, "no cube row kernel for this payload");
   }
-  if (hipGetLastError() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "cube row table launch failed");
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
+    return fail(BRILLE_ERR_DEVICE, "building the cube row table failed");
   *out = t;
   return BRILLE_OK;
 }
@@ -791,7 +792,8 @@ static int build_wide_factors(brille_grid* G, hipStream_t s, typename Cplx<Real>
   else
     hipLaunchKernelGGL((k_wide_factors<Real>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, G->g, d, cube_units,
                        units, t);
-  if (hipGetLastError() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "wide factor table launch failed");
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
+    return fail(BRILLE_ERR_DEVICE, "building the wide factor table failed");
   *out = t;
   return BRILLE_OK;
 }
@@ -950,6 +952,8 @@ void free_binned(brille_grid* G) {
     if (e) (void)hipEventDestroy(e);
     e = nullptr;
   }
+  if (G->bin_used) (void)hipEventDestroy(G->bin_used);
+  G->bin_used = nullptr;
   if (G->bin_side) (void)hipStreamDestroy(G->bin_side);
   G->bin_side = nullptr;
 }
@@ -1025,8 +1029,39 @@ uint64_t binned_pass_for(const brille_grid* G, uint64_t bytes) {
   return binned_pass_bytes(G, c) <= bytes ? c : 0;
 }
 
+bool recording(hipStream_t s) {
+  if (!s) return false;  // the null stream cannot
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+// The handle's lock covers the enqueueing of a call alone, so calls on two
+// streams would meet in the work space: each waits for the event the call
+// before it recorded.  (A call that records a graph cannot wait for an event
+// from outside it, nor leave one.)
+static int begin_work_space(brille_grid* G, hipStream_t s) {
+  if (G->bin_used && hipStreamWaitEvent(s, G->bin_used, 0) != hipSuccess)
+    return fail(BRILLE_ERR_DEVICE, "waiting for the work space failed");
+  return BRILLE_OK;
+}
+static int end_work_space(brille_grid* G, hipStream_t s) {
+  if (!G->bin_used && hipEventCreateWithFlags(&G->bin_used, hipEventDisableTiming) != hipSuccess) {
+    (void)hipGetLastError();
+    G->bin_used = nullptr;
+  }
+  const hipError_t e = G->bin_used ? hipEventRecord(G->bin_used, s) : hipStreamSynchronize(s);
+  return e == hipSuccess ? BRILLE_OK : fail(BRILLE_ERR_DEVICE, "recording the work space's use failed");
+}
+
 int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms) {
-  if (int rc = ensure_cube_rows(G, precision, s); rc != BRILLE_OK) return rc;
+  const bool rec = recording(s);
+  // (a table built while a graph records would be complete only after a replay)
+  if (!rec)
+    if (int rc = ensure_cube_rows(G, precision, s); rc != BRILLE_OK) return rc;
   const uint64_t chunk = std::min<uint64_t>(a.n, BIN_CHUNK);
   if (chunk == 0) return BRILLE_OK;
   const uint64_t passes = (a.n + chunk - 1) / chunk;
@@ -1035,7 +1070,12 @@ int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_
   if (int rc = ensure_work_space(G, need); rc != BRILLE_OK) return rc;
   if (halves > 1)
     if (int rc = ensure_side_stream(G); rc != BRILLE_OK) return rc;
-  return run_binned_passes(G, a, precision, s, stage_ms, G->bin_ws, chunk, halves);
+  if (!rec)
+    if (int rc = begin_work_space(G, s); rc != BRILLE_OK) return rc;
+  const int rc = run_binned_passes(G, a, precision, s, stage_ms, G->bin_ws, chunk, halves);
+  if (rec) return rc;
+  const int end = end_work_space(G, s);
+  return rc != BRILLE_OK ? rc : end;
 }
 
 // The pipeline over work space `ws` in passes of `chunk` points; with two

@@ -57,6 +57,9 @@ struct brille_grid {
   // work space of the binned pipeline and the sort (grown on demand, kept)
   void* bin_ws = nullptr;
   size_t bin_ws_bytes = 0;
+  // recorded after each binned call's last kernel: the next call, on whatever
+  // stream, waits for it before it writes the work space
+  hipEvent_t bin_used = nullptr;
   // side stream of the binned pipeline (preparation of the next pass) and its
   // events: call start, prepared[2], summed[2]
   hipStream_t bin_side = nullptr;
@@ -134,6 +137,8 @@ inline brille_aux_out offset_aux(const brille_aux_out& x, uint64_t c0) {
 bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool build = true);
 bool binned_ready(const brille_grid* G, uint64_t n, int precision);
 int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms);
+// whether stream s is recording a graph
+bool recording(hipStream_t s);
 // the pipeline on a given work space: passes of `chunk` points, `halves` = 2
 // overlaps preparation and sums (grid side stream), 1 runs all on `s`
 int run_binned_passes(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms, void* ws,
@@ -155,6 +160,7 @@ int exclusive_scan_u32(uint32_t* a, uint64_t m, uint32_t* part, hipStream_t s);
 // set), kept in `allocs`
 int install_permutations(brille_grid* G, std::vector<void*>& allocs, hipStream_t s);
 // the cube row table of the bucketed sums, built on first use (derived_allocs)
+// and complete when the function returns: later calls read it from any stream
 int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s);
 // the first failing point of a call as the reference's error text
 int report_point_error(const ErrRec& e, const double* Q, uint64_t n, bool host_mem);

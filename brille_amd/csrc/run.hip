@@ -339,9 +339,7 @@ void launch_tile(const brille_grid* G, const LaunchArgs& a, int precision, bool 
 // an AUTO call under graph capture stays with the fused kernel until an earlier
 // binned call has left the work space and the tables it would need
 static bool must_not_allocate(const brille_grid* G, const LaunchArgs& a, const brille_run_opts& o, hipStream_t s) {
-  if (o.kernel == BRILLE_KERNEL_BINNED || a.use_proposal || !s || binned_ready(G, a.n, o.precision)) return false;
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+  return o.kernel != BRILLE_KERNEL_BINNED && !a.use_proposal && !binned_ready(G, a.n, o.precision) && recording(s);
 }
 
 // every kernel of one call on device buffers

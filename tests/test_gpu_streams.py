@@ -1,0 +1,72 @@
+"""Calls of one handle on several streams, unchecked, so that nothing waits on the host
+between them: the binned calls share the handle's work space and its derived tables, and each
+must still get exactly what it gets alone.  Needs an MI355X.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from brille_amd import capi
+from brille_amd import synthetic as S
+from test_gpu_small_calls import device_call, points
+
+pytestmark = pytest.mark.gpu
+
+
+class Stream:
+    def __init__(self):
+        self.p = C.c_void_p()
+        capi.check(capi.lib().brille_stream_create(C.byref(self.p)))
+
+    def __del__(self):
+        capi.lib().brille_stream_destroy(self.p)
+
+
+class Call:
+    """Q and outputs in device memory, allocated beforehand."""
+
+    def __init__(self, dev, Q, precision):
+        vs, cs = dev.out_shapes(len(Q))
+        f32 = precision == capi.FP32
+        self.dev, self.n, self.precision = dev, len(Q), precision
+        self.Q = capi.DeviceArray.from_host(Q)
+        self.out = (capi.DeviceArray(vs, np.float32 if f32 else np.float64),
+                    capi.DeviceArray(cs, np.complex64 if f32 else np.complex128))
+
+    def run(self, stream, kernel):
+        o = capi.RunOpts(0, self.precision, 0, capi.MEM_DEVICE, kernel, 0)
+        capi.check(capi.lib().brille_ir_interpolate_at(self.dev.h, self.Q.ptr, self.n, C.byref(o), self.out[0].ptr,
+                                                       self.out[1].ptr, None, stream.p if stream else None))
+
+
+def grid_tables(spec, v_target=600.0):
+    sp = dict(S.batch_specs(16)[spec], v_target=v_target)
+    g = S.batch_grid(sp)
+    vals, vecs = S.batch_payload(g, sp)
+    return g, dict(S.batch_layout_tables(g, sp), values=vals, vectors=vecs)
+
+
+# 4 and 24 atoms; sizes AUTO gives to the pipeline
+@pytest.mark.parametrize("spec,precision,sizes,kernel", [
+    (7, capi.FP64, (60_000, 75_000), capi.KERNEL_AUTO), (7, capi.FP32, (120_000, 100_000), capi.KERNEL_AUTO),
+    (5, capi.FP64, (2_000, 3_000), capi.KERNEL_AUTO), (3, capi.FP32, (50_000, 400_000), capi.KERNEL_BINNED)])
+def test_unchecked_calls_on_two_streams_and_the_null_stream(spec, precision, sizes, kernel):
+    print(f"streams: grid {spec} {precision} {sizes}", flush=True)
+    g, t = grid_tables(spec)
+    r = np.random.default_rng(5)
+    Qs = [points(g, r, n) for n in sizes * 3]
+    ref = capi.Grid(t)
+    want = [[x.to_host() for x in device_call(ref, Q, precision, capi.KERNEL_TILE)[1:]] for Q in Qs]
+    for _ in range(3):  # a fresh handle each time: its first call also builds the table
+        dev = capi.Grid(t)
+        calls = [Call(dev, Q, precision) for Q in Qs]
+        streams = [Stream(), Stream(), None]
+        capi.check(capi.lib().brille_device_sync())
+        for _ in range(2):
+            for k, c in enumerate(calls):
+                c.run(streams[k % 3], kernel)
+        capi.check(capi.lib().brille_device_sync())
+        for c, w in zip(calls, want):
+            for a, b in zip(c.out, w):
+                np.testing.assert_array_equal(a.to_host(), b)
