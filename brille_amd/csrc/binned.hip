@@ -877,12 +877,13 @@ static bool has_table(const DataConst& d, int precision) {
 // (a lower line for wide FP32 rows gained 3 % at 3001 points of a coarser grid
 // and cost the table's 0.4 ms on each first call).
 // A first call also builds the table, whose rows it would mostly compute for
-// itself anyway once there is a point for every four cells; a call that may
-// not build it (`build` false) is binned from the size where node order alone
-// pays.  Scalar rows are so short that bucketing them costs more than it saves
-// (6 modes, 556 830 vertices, 1 000 003 points: 274 / 370) until the payload
-// is far beyond the caches.
-bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool build) {
+// itself anyway once there is a point for every four cells.  Scalar rows are
+// so short that bucketing them costs more than it saves (6 modes, 556 830
+// vertices, 1 000 003 points: 274 / 370) until the payload is far beyond the
+// caches.
+// A call whose work space is not ordered after its other users' (`shared`
+// false) is binned only on payloads beyond the L2 and from 2^18 points on.
+bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool shared) {
   if (kernel == BRILLE_KERNEL_PLAIN || kernel == BRILLE_KERNEL_TILE) return false;
   const brille_aux_out& x = a.aux;
   // the records carry no tau; the sums keep a Gamma frame per point-group
@@ -896,8 +897,8 @@ bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int p
   const bool scalars = payload_layout(d) == LAYOUT_SCALAR && !wide_rows(d);
   // large calls on payloads that do not fit the L2 of one XCD
   if (a.n >= (1ull << 18) && payload > (scalars ? 512ull << 20 : 8ull << 20)) return true;
-  if (payload_layout(d) != LAYOUT_GAMMA || !(wide_rows(d) || onepass_sc(d))) return false;
-  if (!has_table(d, precision) && !(build && 4 * a.n >= G->n_cubes + G->n_tets / 2)) return false;
+  if (!shared || payload_layout(d) != LAYOUT_GAMMA || !(wide_rows(d) || onepass_sc(d))) return false;
+  if (!has_table(d, precision) && 4 * a.n < G->n_cubes + G->n_tets / 2) return false;
   const uint64_t work = a.n * d.B * d.sc;
   if (wide_rows(d)) return work >= (precision == BRILLE_FP32 ? 20000000ull : 4000000ull);
   return work >= (precision == BRILLE_FP32 ? 13000000ull : 7000000ull);

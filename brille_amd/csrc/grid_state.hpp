@@ -133,8 +133,9 @@ inline brille_aux_out offset_aux(const brille_aux_out& x, uint64_t c0) {
   return o;
 }
 // binned pipeline (binned.hip)
-// (build: the call may build the derived table)
-bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool build = true);
+// (shared: the call may take a work space that other calls use, ordered after
+// them; otherwise AUTO keeps to the line for large calls)
+bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool shared = true);
 bool binned_ready(const brille_grid* G, uint64_t n, int precision);
 int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms);
 // whether stream s is recording a graph

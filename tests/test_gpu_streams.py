@@ -34,10 +34,10 @@ class Call:
         self.out = (capi.DeviceArray(vs, np.float32 if f32 else np.float64),
                     capi.DeviceArray(cs, np.complex64 if f32 else np.complex128))
 
-    def run(self, stream, kernel):
+    def run(self, stream, kernel, entry="brille_ir_interpolate_at"):
         o = capi.RunOpts(0, self.precision, 0, capi.MEM_DEVICE, kernel, 0)
-        capi.check(capi.lib().brille_ir_interpolate_at(self.dev.h, self.Q.ptr, self.n, C.byref(o), self.out[0].ptr,
-                                                       self.out[1].ptr, None, stream.p if stream else None))
+        capi.check(getattr(capi.lib(), entry)(self.dev.h, self.Q.ptr, self.n, C.byref(o), self.out[0].ptr,
+                                              self.out[1].ptr, None, stream.p if stream else None))
 
 
 def grid_tables(spec, v_target=600.0):
@@ -70,3 +70,25 @@ def test_unchecked_calls_on_two_streams_and_the_null_stream(spec, precision, siz
         for c, w in zip(calls, want):
             for a, b in zip(c.out, w):
                 np.testing.assert_array_equal(a.to_host(), b)
+
+
+def test_unchecked_allocation_free_calls_of_two_handles():
+    """They share one array per GPU, which only large calls work in: two ordinary ones (here with
+    their tables built) may run side by side."""
+    print("streams: allocation-free calls", flush=True)
+    g, t = grid_tables(7)
+    r = np.random.default_rng(6)
+    devs, streams = [capi.Grid(t), capi.Grid(t)], [Stream(), Stream()]
+    Qs = [points(g, r, n) for n in (60_000, 70_000)]
+    want = [[x.to_host() for x in device_call(d, Q, capi.FP64, capi.KERNEL_TILE)[1:]] for d, Q in zip(devs, Qs)]
+    for d in devs:
+        device_call(d, Qs[0], capi.FP64, capi.KERNEL_BINNED)
+    calls = [Call(d, Q, capi.FP64) for d, Q in zip(devs, Qs)]
+    capi.check(capi.lib().brille_device_sync())
+    for _ in range(5):
+        for c, s in zip(calls, streams):
+            c.run(s, capi.KERNEL_AUTO, "brille_ir_interpolate_at_noalloc")
+    capi.check(capi.lib().brille_device_sync())
+    for c, w in zip(calls, want):
+        for a, b in zip(c.out, w):
+            np.testing.assert_array_equal(a.to_host(), b)
