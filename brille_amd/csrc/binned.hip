@@ -882,7 +882,9 @@ static bool has_table(const DataConst& d, int precision) {
 // vertices, 1 000 003 points: 274 / 370) until the payload is far beyond the
 // caches.
 // A call whose work space is not ordered after its other users' (`shared`
-// false) is binned only on payloads beyond the L2 and from 2^18 points on.
+// false: allocation-free calls, and calls that a graph records, which may not
+// build the table either) is binned only on payloads beyond the L2 and from
+// 2^18 points on.
 bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool shared) {
   if (kernel == BRILLE_KERNEL_PLAIN || kernel == BRILLE_KERNEL_TILE) return false;
   const brille_aux_out& x = a.aux;
@@ -902,15 +904,6 @@ bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int p
   const uint64_t work = a.n * d.B * d.sc;
   if (wide_rows(d)) return work >= (precision == BRILLE_FP32 ? 20000000ull : 4000000ull);
   return work >= (precision == BRILLE_FP32 ? 13000000ull : 7000000ull);
-}
-
-// whether a binned call of n points would allocate or build nothing, so that
-// it can be captured in a graph
-bool binned_ready(const brille_grid* G, uint64_t n, int precision) {
-  const uint64_t chunk = std::min<uint64_t>(n, BIN_CHUNK);
-  const int halves = n > chunk ? 2 : 1;
-  return has_table(G->d, precision) && G->bin_ws_bytes >= binned_pass_bytes(G, chunk) * (uint64_t)halves &&
-         (halves == 1 || G->bin_side);
 }
 
 __global__ void k_zero_words(uint32_t* p, uint32_t n) {
@@ -949,6 +942,8 @@ int ensure_work_space(brille_grid* G, uint64_t bytes) {
 
 void free_binned(brille_grid* G) {
   free_work_space(G);
+  if (G->rec_ws) (void)hipFree(G->rec_ws);
+  for (void* p : G->rec_old) (void)hipFree(p);
   for (auto& e : G->bin_ev) {
     if (e) (void)hipEventDestroy(e);
     e = nullptr;
@@ -1030,6 +1025,26 @@ uint64_t binned_pass_for(const brille_grid* G, uint64_t bytes) {
   return binned_pass_bytes(G, c) <= bytes ? c : 0;
 }
 
+// the passes of a call of n points
+struct Passes {
+  uint64_t chunk;  // points of each
+  int halves;      // buffers: one, or two that take turns
+  uint64_t bytes;  // of work space
+};
+static Passes passes_of(const brille_grid* G, uint64_t n) {
+  Passes p;
+  p.chunk = std::min<uint64_t>(n, BIN_CHUNK);
+  p.halves = n > p.chunk ? 2 : 1;
+  p.bytes = binned_pass_bytes(G, p.chunk) * (uint64_t)p.halves;
+  return p;
+}
+
+// whether a graph can record a binned call of n points without an allocation
+bool binned_recordable(const brille_grid* G, uint64_t n) {
+  const Passes p = passes_of(G, n);
+  return std::max(G->rec_ws_bytes, G->bin_ws_bytes) >= p.bytes && (p.halves == 1 || G->bin_side);
+}
+
 bool recording(hipStream_t s) {
   if (!s) return false;  // the null stream cannot
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -1058,23 +1073,46 @@ static int end_work_space(brille_grid* G, hipStream_t s) {
   return e == hipSuccess ? BRILLE_OK : fail(BRILLE_ERR_DEVICE, "recording the work space's use failed");
 }
 
+// The work space of a call that a graph records.  The graph keeps the address,
+// so the memory is never freed before the handle, and no call that runs at once
+// works in it: a replay may run beside any of those.  It is the handle's
+// present work space where that is large enough (the next call gets another).
+// All recorded calls share it, one graph's in their order; replays of two
+// graphs of one handle must not overlap.
+static int recorded_work_space(brille_grid* G, uint64_t bytes) {
+  if (G->rec_ws_bytes >= bytes) return BRILLE_OK;
+  void* ws = nullptr;
+  uint64_t held = bytes;
+  if (G->bin_ws_bytes >= bytes) {
+    // its last user is done before a replay can start
+    if (G->bin_used && hipEventSynchronize(G->bin_used) != hipSuccess)
+      return fail(BRILLE_ERR_DEVICE, "waiting for the work space failed");
+    ws = G->bin_ws;
+    held = G->bin_ws_bytes;
+    G->bin_ws = nullptr;
+    G->bin_ws_bytes = 0;
+  } else if (hipMalloc(&ws, bytes) != hipSuccess) {
+    return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the work space");
+  }
+  if (G->rec_ws) G->rec_old.push_back(G->rec_ws);
+  G->rec_ws = ws;
+  G->rec_ws_bytes = held;
+  return BRILLE_OK;
+}
+
 int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms) {
   const bool rec = recording(s);
   // (a table built while a graph records would be complete only after a replay)
   if (!rec)
     if (int rc = ensure_cube_rows(G, precision, s); rc != BRILLE_OK) return rc;
-  const uint64_t chunk = std::min<uint64_t>(a.n, BIN_CHUNK);
-  if (chunk == 0) return BRILLE_OK;
-  const uint64_t passes = (a.n + chunk - 1) / chunk;
-  const int halves = passes > 1 ? 2 : 1;
-  const uint64_t need = binned_pass_bytes(G, chunk) * (uint64_t)halves;
-  if (int rc = ensure_work_space(G, need); rc != BRILLE_OK) return rc;
-  if (halves > 1)
+  if (a.n == 0) return BRILLE_OK;
+  const Passes p = passes_of(G, a.n);
+  if (int rc = rec ? recorded_work_space(G, p.bytes) : ensure_work_space(G, p.bytes); rc != BRILLE_OK) return rc;
+  if (p.halves > 1)
     if (int rc = ensure_side_stream(G); rc != BRILLE_OK) return rc;
-  if (!rec)
-    if (int rc = begin_work_space(G, s); rc != BRILLE_OK) return rc;
-  const int rc = run_binned_passes(G, a, precision, s, stage_ms, G->bin_ws, chunk, halves);
-  if (rec) return rc;
+  if (rec) return run_binned_passes(G, a, precision, s, stage_ms, G->rec_ws, p.chunk, p.halves);
+  if (int rc = begin_work_space(G, s); rc != BRILLE_OK) return rc;
+  const int rc = run_binned_passes(G, a, precision, s, stage_ms, G->bin_ws, p.chunk, p.halves);
   const int end = end_work_space(G, s);
   return rc != BRILLE_OK ? rc : end;
 }

@@ -57,6 +57,11 @@ struct brille_grid {
   // work space of the binned pipeline and the sort (grown on demand, kept)
   void* bin_ws = nullptr;
   size_t bin_ws_bytes = 0;
+  // the work space of the binned calls that graphs have recorded: no call that
+  // runs at once uses it, and what a graph holds lives as long as the handle
+  void* rec_ws = nullptr;
+  size_t rec_ws_bytes = 0;
+  std::vector<void*> rec_old;
   // recorded after each binned call's last kernel: the next call, on whatever
   // stream, waits for it before it writes the work space
   hipEvent_t bin_used = nullptr;
@@ -136,7 +141,7 @@ inline brille_aux_out offset_aux(const brille_aux_out& x, uint64_t c0) {
 // (shared: the call may take a work space that other calls use, ordered after
 // them; otherwise AUTO keeps to the line for large calls)
 bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool shared = true);
-bool binned_ready(const brille_grid* G, uint64_t n, int precision);
+bool binned_recordable(const brille_grid* G, uint64_t n);
 int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms);
 // whether stream s is recording a graph
 bool recording(hipStream_t s);

@@ -336,16 +336,19 @@ void launch_tile(const brille_grid* G, const LaunchArgs& a, int precision, bool 
   launch_sel(G, a, precision, fast, s);
 }
 
-// an AUTO call under graph capture stays with the fused kernel until an earlier
-// binned call has left the work space and the tables it would need
-static bool must_not_allocate(const brille_grid* G, const LaunchArgs& a, const brille_run_opts& o, hipStream_t s) {
-  return o.kernel != BRILLE_KERNEL_BINNED && !a.use_proposal && !binned_ready(G, a.n, o.precision) && recording(s);
+// A graph records an AUTO call as the fused kernel, which holds nothing of the
+// handle's that another call writes; a large one as the pipeline if an earlier
+// call has left a work space it can take over.
+static bool takes_pipeline(const brille_grid* G, const LaunchArgs& a, const brille_run_opts& o, hipStream_t s) {
+  if (!binned_applies(G, a, o.kernel, o.precision)) return false;
+  if (o.kernel == BRILLE_KERNEL_BINNED || a.use_proposal || !recording(s)) return true;
+  return binned_applies(G, a, o.kernel, o.precision, false) && binned_recordable(G, a.n);
 }
 
 // every kernel of one call on device buffers
 static int dispatch(brille_grid* G, const LaunchArgs& a, const brille_run_opts& o, hipStream_t s) {
   const bool fast = o.kernel != BRILLE_KERNEL_PLAIN;
-  if (fast && binned_applies(G, a, o.kernel, o.precision) && !(must_not_allocate(G, a, o, s)))
+  if (takes_pipeline(G, a, o, s))
     return launch_binned(G, a, o.precision, s, nullptr);
   launch_sel(G, a, o.precision, fast, s);
   return BRILLE_OK;

@@ -92,3 +92,64 @@ def test_unchecked_allocation_free_calls_of_two_handles():
     for c, w in zip(calls, want):
         for a, b in zip(c.out, w):
             np.testing.assert_array_equal(a.to_host(), b)
+
+
+def hip_runtime():
+    maps = open("/proc/self/maps").read().split()
+    return C.CDLL(next(m for m in maps if "libamdhip64" in m))  # the one the library itself uses
+
+
+class Graph:
+    """Calls recorded on a stream of their own (mode 0: global, 1: thread-local)."""
+
+    def __init__(self, mode, record):
+        self.hip, self.s, graph = hip_runtime(), Stream(), C.c_void_p()
+        self.exec = C.c_void_p()
+        capi.check(capi.lib().brille_device_sync())
+        assert self.hip.hipStreamBeginCapture(self.s.p, mode) == 0
+        try:
+            record(self.s)
+        finally:
+            assert self.hip.hipStreamEndCapture(self.s.p, C.byref(graph)) == 0
+        assert self.hip.hipGraphInstantiate(C.byref(self.exec), graph, None, None, C.c_size_t(0)) == 0
+        assert self.hip.hipGraphDestroy(graph) == 0
+
+    def replay(self):
+        assert self.hip.hipGraphLaunch(self.exec, self.s.p) == 0
+
+    def __del__(self):
+        self.hip.hipGraphExecDestroy(self.exec)
+
+
+def clobber(call):
+    for x in call.out:
+        junk = np.full(x.shape, 7, x.dtype)
+        capi.check(capi.lib().brille_memcpy_h2d(x.ptr, junk.ctypes.data_as(C.c_void_p), x.nbytes))
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("kernel", [capi.KERNEL_AUTO, capi.KERNEL_BINNED])
+def test_a_recorded_call_keeps_its_work_space(mode, kernel):
+    """Larger calls after the recording get a work space of their own, also where they run while
+    the graph replays."""
+    print(f"streams: recorded call, mode {mode}, kernel {kernel}", flush=True)
+    g, t = grid_tables(7)
+    r = np.random.default_rng(7)
+    dev = capi.Grid(t)
+    Qs = [points(g, r, n) for n in (60_000, 20_000, 300_000, 900_000)]
+    want = [[x.to_host() for x in device_call(dev, Q, capi.FP64, capi.KERNEL_TILE)[1:]] for Q in Qs]
+    calls = [Call(dev, Q, capi.FP64) for Q in Qs]
+    calls[0].run(None, kernel)  # leaves a work space and the tables
+    graph = Graph(mode, lambda s: [calls[0].run(s, kernel), calls[1].run(s, kernel)])
+    other = Stream()
+    for big in (2, 3, 2):
+        for c in calls:
+            clobber(c)
+        calls[big].run(other, capi.KERNEL_BINNED)
+        graph.replay()
+        calls[big].run(other, capi.KERNEL_BINNED)
+        graph.replay()
+        capi.check(capi.lib().brille_device_sync())
+        for k in (0, 1, big):
+            for a, b in zip(calls[k].out, want[k]):
+                np.testing.assert_array_equal(a.to_host(), b, err_msg=f"call {k}")
