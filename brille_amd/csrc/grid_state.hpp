@@ -39,6 +39,9 @@ struct brille_grid {
   // the row and factor tables built from the payload and its permutations
   // (freed by the next fill or sort)
   std::vector<void*> derived_allocs;
+  // a graph has recorded a call, and so the present tables: a sort then keeps
+  // those it replaces until the next fill, like the payload
+  bool recorded = false;
   uint32_t n_perms = 0;  // permutations of the installed table
   bool filled = false;
   uint64_t n_vertices = 0, n_cubes = 0, n_polys = 0, n_tets = 0;

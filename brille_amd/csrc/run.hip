@@ -428,6 +428,7 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
     return r;
   };
   if (opts.memory == BRILLE_MEM_DEVICE) {
+    if (!opts.check && !times && recording(s)) G->recorded = true;
     a.Q = Q;
     a.n = n;
     a.base = 0;

@@ -920,11 +920,15 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   // install: the previous sorted table goes, and the tables derived from the
   // payload and the permutations with it (the calls queued before this one have
   // ended, and others wait for the handle's lock); a fill-given table stays in
-  // the payload allocations until the next fill
+  // the payload allocations until the next fill, and so do tables whose
+  // addresses a graph has recorded
   for (std::vector<void*>* old : {&G->sort_allocs, &G->derived_allocs}) {
-    for (void* p : *old) (void)hipFree(p);
+    if (G->recorded) G->data_allocs.insert(G->data_allocs.end(), old->begin(), old->end());
+    else
+      for (void* p : *old) (void)hipFree(p);
     old->clear();
   }
+  G->recorded = false;
   for (void* p : {(void*)keys, (void*)pidx, (void*)perms_fit}) {
     buf.release(p);
     G->sort_allocs.push_back(p);

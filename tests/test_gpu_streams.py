@@ -153,3 +153,29 @@ def test_a_recorded_call_keeps_its_work_space(mode, kernel):
         for k in (0, 1, big):
             for a, b in zip(calls[k].out, want[k]):
                 np.testing.assert_array_equal(a.to_host(), b, err_msg=f"call {k}")
+
+
+@pytest.mark.parametrize("spec,kernel,entry", [
+    (5, capi.KERNEL_TILE, "brille_ir_interpolate_at"), (5, capi.KERNEL_BINNED, "brille_ir_interpolate_at"),
+    (3, capi.KERNEL_BINNED, "brille_ir_interpolate_at"), (3, capi.KERNEL_BINNED, "brille_ir_interpolate_at_noalloc")])
+def test_a_recorded_call_keeps_its_tables_over_a_sort(spec, kernel, entry):
+    """The graph goes on giving what its handle gave when it was recorded: unsorted, then sorted."""
+    print(f"streams: recorded before a sort, grid {spec}, kernel {kernel}, {entry}", flush=True)
+    g, t = grid_tables(spec, 300.0)
+    t["values"], t["vectors"], _ = S.shuffled_modes(t, seed=4)
+    dev = capi.Grid(t)
+    Q = points(g, np.random.default_rng(8), 3_000)
+    graphs = []
+    for _ in range(2):
+        want = [x.to_host() for x in device_call(dev, Q, capi.FP64, capi.KERNEL_BINNED)[1:]]
+        call = Call(dev, Q, capi.FP64)
+        graphs.append((Graph(1, lambda s: call.run(s, kernel, entry)), call, want))
+        dev.sort()
+        device_call(dev, Q, capi.FP64, capi.KERNEL_BINNED)  # its tables anew
+        for graph, c, w in graphs * 2:
+            clobber(c)
+            graph.replay()
+            capi.check(capi.lib().brille_device_sync())
+            for a, b in zip(c.out, w):
+                np.testing.assert_array_equal(a.to_host(), b)
+    assert not np.array_equal(graphs[0][2][1], graphs[1][2][1])
