@@ -1100,17 +1100,21 @@ static int recorded_work_space(brille_grid* G, uint64_t bytes) {
   return BRILLE_OK;
 }
 
-int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms) {
+int prepare_binned(brille_grid* G, uint64_t n, int precision, hipStream_t s) {
   const bool rec = recording(s);
   // (a table built while a graph records would be complete only after a replay)
   if (!rec)
     if (int rc = ensure_cube_rows(G, precision, s); rc != BRILLE_OK) return rc;
+  if (n == 0) return BRILLE_OK;
+  const Passes p = passes_of(G, n);
+  if (int rc = rec ? recorded_work_space(G, p.bytes) : ensure_work_space(G, p.bytes); rc != BRILLE_OK) return rc;
+  return p.halves > 1 ? ensure_side_stream(G) : BRILLE_OK;
+}
+
+int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms) {
   if (a.n == 0) return BRILLE_OK;
   const Passes p = passes_of(G, a.n);
-  if (int rc = rec ? recorded_work_space(G, p.bytes) : ensure_work_space(G, p.bytes); rc != BRILLE_OK) return rc;
-  if (p.halves > 1)
-    if (int rc = ensure_side_stream(G); rc != BRILLE_OK) return rc;
-  if (rec) return run_binned_passes(G, a, precision, s, stage_ms, G->rec_ws, p.chunk, p.halves);
+  if (recording(s)) return run_binned_passes(G, a, precision, s, stage_ms, G->rec_ws, p.chunk, p.halves);
   if (int rc = begin_work_space(G, s); rc != BRILLE_OK) return rc;
   const int rc = run_binned_passes(G, a, precision, s, stage_ms, G->bin_ws, p.chunk, p.halves);
   const int end = end_work_space(G, s);

@@ -145,6 +145,9 @@ inline brille_aux_out offset_aux(const brille_aux_out& x, uint64_t c0) {
 // them; otherwise AUTO keeps to the line for large calls)
 bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool shared = true);
 bool binned_recordable(const brille_grid* G, uint64_t n);
+// the derived table, work space and side stream of a binned call of n points;
+// launch_binned needs them
+int prepare_binned(brille_grid* G, uint64_t n, int precision, hipStream_t s);
 int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms);
 // whether stream s is recording a graph
 bool recording(hipStream_t s);

@@ -345,12 +345,25 @@ static bool takes_pipeline(const brille_grid* G, const LaunchArgs& a, const bril
   return binned_applies(G, a, o.kernel, o.precision, false) && binned_recordable(G, a.n);
 }
 
+// Whether the call runs in the pipeline, which is then ready for it.  A call that
+// only AUTO gave to it needs none of the memory the pipeline allocates: where
+// that cannot be had, the fused kernel serves it.
+static int choose_pipeline(brille_grid* G, const LaunchArgs& a, const brille_run_opts& o, hipStream_t s, bool* binned) {
+  *binned = takes_pipeline(G, a, o, s);
+  if (!*binned) return BRILLE_OK;
+  const int rc = prepare_binned(G, a.n, o.precision, s);
+  if (rc == BRILLE_OK || o.kernel == BRILLE_KERNEL_BINNED || a.use_proposal) return rc;
+  (void)hipGetLastError();
+  *binned = false;
+  return BRILLE_OK;
+}
+
 // every kernel of one call on device buffers
 static int dispatch(brille_grid* G, const LaunchArgs& a, const brille_run_opts& o, hipStream_t s) {
-  const bool fast = o.kernel != BRILLE_KERNEL_PLAIN;
-  if (takes_pipeline(G, a, o, s))
-    return launch_binned(G, a, o.precision, s, nullptr);
-  launch_sel(G, a, o.precision, fast, s);
+  bool binned;
+  if (int rc = choose_pipeline(G, a, o, s, &binned); rc != BRILLE_OK) return rc;
+  if (binned) return launch_binned(G, a, o.precision, s, nullptr);
+  launch_sel(G, a, o.precision, o.kernel != BRILLE_KERNEL_PLAIN, s);
   return BRILLE_OK;
 }
 
@@ -439,7 +452,9 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
     if (times) {
       std::memset(times, 0, sizeof(*times));
       const uint32_t it_n = std::max(iters, 1u);
-      if (fast && binned_applies(G, a, opts.kernel, opts.precision)) {
+      bool binned;
+      if (rc = choose_pipeline(G, a, opts, s, &binned); rc != BRILLE_OK) return rc;
+      if (binned) {
         // stages from events on the streams that ran them; the call from
         // events on `s` around all of it
         float st[3] = {0.f, 0.f, 0.f};
