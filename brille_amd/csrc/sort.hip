@@ -380,8 +380,9 @@ __device__ __forceinline__ void wave_argmin(double& v, uint32_t& j) {
 // sin^2 of the Hermitian angle) the cost needs no phase and no angle:
 // sin^2 = 1 - |a.b|^2 / (|a|^2 |b|^2), some eighty operations against seven
 // hundred, whose value agrees with the literal one to rounding (~1e-14 of the
-// terms); a row whose lead is within kLead of that scale, a norm near zero, or a
-// value that is not finite sends the pair to the literal costs.  Memory: the rows
+// terms); a row whose lead is within kLead of that scale, a norm near zero or
+// near overflow, or a value that is not finite sends the pair to the literal
+// costs.  Memory: the rows
 // alone (one wave reads each pair's from the cache); 1.4e6 pairs of 6 modes,
 // FP64: 4.1 ms for the stored matrices and their row minima, 0.3 ms here.
 // asg[p * B + a]: the column of row a; hard[p], moved[p]: 0 or 1.
@@ -410,7 +411,7 @@ __global__ __launch_bounds__(256) void k_pair_easy(CostArgs c, const Real* __res
       aa += x[k] * x[k];
     }
     double best = __builtin_huge_val(), second = __builtin_huge_val();
-    bool fine = true;
+    bool fine = aa > 1e-140 && aa < 1e140;
     for (uint32_t b = 0; b < B; ++b, rb += c.stride) {
       double s = 0, hr = 0, hi = 0, bb = 0;
       for (uint32_t z = 0; z < c.ev[0]; ++z) s += fabs((double)ra[2 * SC + z] - (double)rb[2 * SC + z]);
@@ -422,7 +423,8 @@ __global__ __launch_bounds__(256) void k_pair_easy(CostArgs c, const Real* __res
         bb += br * br + bi * bi;
       }
       const double cost = c.vw[0] * s + c.cw[1] * (1.0 - (hr * hr + hi * hi) / (aa * bb));
-      fine = fine && aa * bb > 1e-280 && fabs(cost) < 1e300;  // false for NaN
+      // (norms whose products neither overflow nor underflow; false for NaN)
+      fine = fine && bb > 1e-140 && bb < 1e140 && fabs(cost) < 1e300;
       if (cost < best) {
         second = best;
         best = cost;
