@@ -20,6 +20,7 @@
 // The assignment goes to key (i, j), its inverse to (j, i)
 // (src/interpolatordual.hpp:422-432); identity assignments share permutation 0.
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "grid_state.hpp"
@@ -719,6 +720,10 @@ static bool launch_easy(const brille_grid* G, const CostArgs& c, const uint32_t*
   const DataConst& d = G->d;
   const bool vectors = c.ec[0] == 0 && c.ec[2] == 0 && (c.cv < 1 || c.cv > 4);
   if (d.B > 64 || c.ev[1] || c.ev[2] || !vectors) return false;
+  // (the literal sum has the terms of absent elements too: an infinite weight of
+  // one is a NaN there)
+  for (int q = 0; q < 3; ++q)
+    if (!std::isfinite(c.vw[q]) || !std::isfinite(c.cw[q])) return false;
   const unsigned blocks = (unsigned)((n_pairs + 256 / d.B - 1) / (256 / d.B));
   auto go = [&](auto k64, auto k32) {
     if (d.rows64) hipLaunchKernelGGL(k64, dim3(blocks), dim3(256), 0, s, c, d.rows64, pi, pj, rev, n_pairs, asg, hard, moved);

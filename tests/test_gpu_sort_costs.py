@@ -27,3 +27,15 @@ def test_sort_of_vectors_whose_norms_product_overflows(scale):
     gk, gp = device_table(dev)
     np.testing.assert_array_equal(gk, keys)
     np.testing.assert_array_equal(gp, perms)
+
+
+@pytest.mark.parametrize("which,at", [("values", 1), ("values", 2), ("vectors", 0), ("vectors", 2)])
+def test_sort_refuses_weights_that_are_not_finite(which, at):
+    """An infinite weight of an absent term makes every cost a NaN, as in the reference's sum."""
+    print(f"sort with an infinite weight: {which} {at}", flush=True)
+    t, _ = small_tables("a2")
+    dev = capi.Grid(t)
+    w = [1.0, 1.0, 1.0]
+    w[at] = np.inf
+    with pytest.raises(capi.BrilleError):
+        dev.sort(**{which + "_cost": capi.cost_info(weights=w)})
