@@ -11,6 +11,7 @@
 
 #include "fast_tables.hpp"
 #include "grid_state.hpp"
+#include "launch_pieces.hpp"
 
 using namespace brille_amd;
 
@@ -315,21 +316,17 @@ static void launch_sel(const brille_grid* G, LaunchArgs a, int precision, bool f
   TileKernel k;
   if (precision == BRILLE_FP32) k = fast ? pick_tuned<float>(G->d) : k_ir_interpolate<float, false, LAYOUT_GENERIC, 0, 0>;
   else k = fast ? pick_tuned<double>(G->d) : k_ir_interpolate<double, false, LAYOUT_GENERIC, 0, 0>;
-  // a launch holds fewer than 2^32 threads along x
-  constexpr uint64_t kMostBlocks = (1ull << 24) - 1;
   const size_t rs = precision == BRILLE_FP32 ? 4 : 8;
-  const uint64_t n = a.n, piece = kMostBlocks * a.tile;
-  for (uint64_t c0 = 0; c0 < n; c0 += piece) {
+  in_pieces(a.n, a.tile, [&](uint64_t c0, uint64_t count, unsigned blocks) {
     LaunchArgs c = a;
     c.Q = a.Q + 3 * c0;
-    c.n = std::min(piece, n - c0);
+    c.n = count;
     c.base = a.base + c0;
     c.vals = static_cast<char*>(a.vals) + c0 * G->d.B * G->d.sv * rs;
     c.vecs = static_cast<char*>(a.vecs) + c0 * G->d.B * G->d.sc * 2 * rs;
     c.aux = offset_aux(a.aux, c0);
-    hipLaunchKernelGGL(k, dim3((unsigned)((c.n + a.tile - 1) / a.tile), groups), dim3(TILE), G->d.n_keys ? 32u * a.tile : 0u, s,
-                       G->g, G->d, c);
-  }
+    hipLaunchKernelGGL(k, dim3(blocks, groups), dim3(TILE), G->d.n_keys ? 32u * a.tile : 0u, s, G->g, G->d, c);
+  });
 }
 
 void launch_tile(const brille_grid* G, const LaunchArgs& a, int precision, bool fast, hipStream_t s) {

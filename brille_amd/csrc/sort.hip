@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "grid_state.hpp"
+#include "launch_pieces.hpp"
 
 namespace brille_amd {
 
@@ -64,18 +65,18 @@ __global__ __launch_bounds__(256) void k_pair_emit(const uint32_t* cube_v, uint6
   }
 }
 
-// Each vertex's list sorted and de-duplicated in place, one wave per vertex;
+// Each list of the vertices [v0, V) sorted and de-duplicated in place, one wave per vertex;
 // uniq[v] = its length, fwd[v] = its entries beyond v.  Lists of up to kListMax
 // entries go through the wave's LDS slice (a bitonic sort over the next power
 // of two: an insertion sort by one thread in memory took 1.1 ms for the 121 200
 // lists of the hexagonal grid of 318 472 nodes, this 0.06 ms); longer ones are
 // sorted by one lane.
 constexpr uint32_t kListMax = 512;
-__global__ __launch_bounds__(256) void k_pair_unique(uint64_t V, const uint32_t* __restrict__ off,
+__global__ __launch_bounds__(256) void k_pair_unique(uint64_t v0, uint64_t V, const uint32_t* __restrict__ off,
                                                      const uint32_t* __restrict__ cnt, uint32_t* __restrict__ adj,
                                                      uint32_t* __restrict__ uniq, uint32_t* __restrict__ fwd) {
   __shared__ uint32_t s_list[4][kListMax];
-  const uint64_t v = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const uint64_t v = v0 + (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (v >= V) return;  // wave-uniform; no block-wide barrier follows
   const uint32_t lane = threadIdx.x & 63u;
   uint32_t* a = adj + off[v];
@@ -132,15 +133,15 @@ __global__ __launch_bounds__(256) void k_pair_unique(uint64_t V, const uint32_t*
   }
 }
 
-// One wave per vertex: its keys i * V + j in list order, the neighbour j of
-// each key, and its forward pairs (j > i, the end of the sorted list) with
-// the key each came from.
-__global__ __launch_bounds__(256) void k_pair_keys(uint64_t V, const uint32_t* __restrict__ off,
+// One wave per vertex, from v0 on: its keys i * V + j in list order, the
+// neighbour j of each key, and its forward pairs (j > i, the end of the sorted
+// list) with the key each came from.
+__global__ __launch_bounds__(256) void k_pair_keys(uint64_t v0, uint64_t V, const uint32_t* __restrict__ off,
                                                    const uint32_t* __restrict__ adj, const uint32_t* __restrict__ koff,
                                                    const uint32_t* __restrict__ poff, uint64_t* __restrict__ keys,
                                                    uint32_t* __restrict__ nbr, uint32_t* __restrict__ pi,
                                                    uint32_t* __restrict__ pj, uint32_t* __restrict__ pk) {
-  const uint64_t v = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const uint64_t v = v0 + (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (v >= V) return;
   const uint32_t* a = adj + off[v];
   const uint32_t k0 = koff[v], n = koff[v + 1] - k0, p0 = poff[v], nf = poff[v + 1] - p0;
@@ -724,10 +725,13 @@ static bool launch_easy(const brille_grid* G, const CostArgs& c, const uint32_t*
   // one is a NaN there)
   for (int q = 0; q < 3; ++q)
     if (!std::isfinite(c.vw[q]) || !std::isfinite(c.cw[q])) return false;
-  const unsigned blocks = (unsigned)((n_pairs + 256 / d.B - 1) / (256 / d.B));
   auto go = [&](auto k64, auto k32) {
-    if (d.rows64) hipLaunchKernelGGL(k64, dim3(blocks), dim3(256), 0, s, c, d.rows64, pi, pj, rev, n_pairs, asg, hard, moved);
-    else hipLaunchKernelGGL(k32, dim3(blocks), dim3(256), 0, s, c, d.rows32, pi, pj, rev, n_pairs, asg, hard, moved);
+    in_pieces(n_pairs, 256 / d.B, [&](uint64_t p, uint64_t n, unsigned blocks) {
+      if (d.rows64)
+        hipLaunchKernelGGL(k64, dim3(blocks), dim3(256), 0, s, c, d.rows64, pi + p, pj + p, rev + p, n, asg + p * d.B, hard + p, moved + p);
+      else
+        hipLaunchKernelGGL(k32, dim3(blocks), dim3(256), 0, s, c, d.rows32, pi + p, pj + p, rev + p, n, asg + p * d.B, hard + p, moved + p);
+    });
     return true;
   };
   switch (c.sc) {
@@ -805,13 +809,15 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   uint32_t* counter = part + scan_words;
   uint32_t* adj = counter + 4;
   zero_words(ws0, (uint32_t)(5 * (V + 1) + scan_words + 4), s);
-  const unsigned ub = (unsigned)((units + 255) / 256), wb = (unsigned)((V + 3) / 4);
+  const unsigned ub = (unsigned)((units + 255) / 256);
   if (units) hipLaunchKernelGGL(k_pair_emit<0>, dim3(ub), dim3(256), 0, s, G->g.cube_v, G->n_cubes, G->g.tet_v, G->n_tets, cnt, off, nullptr);
   if (hipMemcpyAsync(off, cnt, (V + 1) * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
     return fail(BRILLE_ERR_DEVICE, "hipMemcpyAsync failed");
   if (int rc = exclusive_scan_u32(off, V + 1, part, s); rc != BRILLE_OK) return rc;
   if (units) hipLaunchKernelGGL(k_pair_emit<1>, dim3(ub), dim3(256), 0, s, G->g.cube_v, G->n_cubes, G->g.tet_v, G->n_tets, cursor, off, adj);
-  hipLaunchKernelGGL(k_pair_unique, dim3(wb), dim3(256), 0, s, V, off, cnt, adj, koff, poff);
+  in_pieces(V, 4, [&](uint64_t v0, uint64_t, unsigned blocks) {
+    hipLaunchKernelGGL(k_pair_unique, dim3(blocks), dim3(256), 0, s, v0, V, off, cnt, adj, koff, poff);
+  });
   if (int rc = exclusive_scan_u32(koff, V + 1, part, s); rc != BRILLE_OK) return rc;
   if (int rc = exclusive_scan_u32(poff, V + 1, part, s); rc != BRILLE_OK) return rc;
   uint32_t n32[2] = {0, 0};
@@ -842,7 +848,9 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   uint32_t* keep = moved + (n_pairs + 1);  // the moved flags, kept while hard pairs are left
   uint32_t* hpart = keep + (n_pairs + 1);
   uint16_t* asg = reinterpret_cast<uint16_t*>(hpart + hwords);
-  hipLaunchKernelGGL(k_pair_keys, dim3(wb), dim3(256), 0, s, V, off, adj, koff, poff, keys, nbr, pi, pj, pk);
+  in_pieces(V, 4, [&](uint64_t v0, uint64_t, unsigned blocks) {
+    hipLaunchKernelGGL(k_pair_keys, dim3(blocks), dim3(256), 0, s, v0, V, off, adj, koff, poff, keys, nbr, pi, pj, pk);
+  });
   CostArgs ca{};
   ca.B = d.B;
   ca.sv = d.sv;
@@ -916,9 +924,13 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   uint32_t* perms_fit = buf.get<uint32_t>((uint64_t)n_perms * d.B);
   if (!perms_fit) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the permutation table");
   hipLaunchKernelGGL(k_identity_perm, dim3(1), dim3(256), 0, s, perms_fit, d.B);
-  if (n_pairs)
-    hipLaunchKernelGGL(k_perm_write, dim3((unsigned)((n_pairs * d.B + 255) / 256)), dim3(256), 0, s, n_pairs, d.B, asg,
-                       moved, pk, rev, pidx, perms_fit);
+  // (whole pairs in each launch, a lane per pair and row)
+  const uint64_t most_pairs = kMostBlocks * 256 / d.B;
+  for (uint64_t p = 0; p < n_pairs; p += most_pairs) {
+    const uint64_t n = std::min(most_pairs, n_pairs - p);
+    hipLaunchKernelGGL(k_perm_write, dim3((unsigned)((n * d.B + 255) / 256)), dim3(256), 0, s, n, d.B, asg + p * d.B,
+                       moved + p, pk + p, rev + p, pidx, perms_fit);
+  }
   if (hipGetLastError() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "sort launch failed");
   uint32_t hc[2] = {0, 0};
   if (hipMemcpyAsync(hc, counter, 8, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
