@@ -31,6 +31,7 @@ namespace brille_amd {
 namespace {
 
 constexpr int SORT_BLOCK = 64;  // one wave per pair
+constexpr uint64_t kSortKeep = 128ull << 20;  // bytes of work space a sort may leave with the handle
 
 // ---- pairs ----------------------------------------------------------------
 
@@ -833,12 +834,19 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   // the rest of the work space is the binned pipeline's, grown when it is
   // smaller (its calls and this one hold the handle's lock in turn, and the
   // device was synchronised above): allocating and freeing as much anew took a
-  // third of a sort of 1.4e6 pairs
+  // third of a sort of 1.4e6 pairs.  Beyond kSortKeep bytes the handle does not
+  // keep it.
   const uint64_t hwords = (n_pairs + 1 + 4095) / 4096 + 1;
   const uint64_t words = n_keys + 4 * n_pairs + 3 * (n_pairs + 1) + hwords;
   const uint64_t ws_bytes = words * 4 + n_pairs * d.B * 2 + 16;
-  if (int rc = ensure_work_space(G, ws_bytes); rc != BRILLE_OK) return rc;
-  uint32_t* nbr = static_cast<uint32_t*>(G->bin_ws);
+  uint32_t* nbr = nullptr;
+  if (ws_bytes > std::max<uint64_t>(kSortKeep, G->bin_ws_bytes)) {
+    nbr = reinterpret_cast<uint32_t*>(buf.get<char>(ws_bytes));
+    if (!nbr) return fail(BRILLE_ERR_DEVICE, "hipMalloc failed for the sort work space");
+  } else {
+    if (int rc = ensure_work_space(G, ws_bytes); rc != BRILLE_OK) return rc;
+    nbr = static_cast<uint32_t*>(G->bin_ws);
+  }
   uint32_t* pi = nbr + n_keys;
   uint32_t* pj = pi + n_pairs;
   uint32_t* pk = pj + n_pairs;

@@ -67,3 +67,28 @@ def test_auto_without_memory_for_the_table():
     capi.check(capi.lib().brille_device_sync())
     for a, b in zip(call.out, want):
         np.testing.assert_array_equal(a.to_host(), b)
+
+
+def test_a_large_sort_gives_its_work_space_back():
+    print("memory after a sort", flush=True)
+    sp = dict(S.batch_specs(16)[7], v_target=120_000.0)
+    g = S.batch_grid(sp)
+    t = S.batch_layout_tables(g, sp)
+    V, B, sc = len(t["vertices"]), 60, int(sum(t["vectors_elements"]))
+    r = np.random.default_rng(2)
+    values = np.tile(2.0 * np.arange(B)[:, None], (V, 1, 1))  # far apart: every pair keeps its order
+    vectors = np.broadcast_to(r.normal(size=(1, B, sc)) + 1j * r.normal(size=(1, B, sc)), (V, B, sc))
+    t.update(values=values, vectors=vectors, branches=B)
+    dev = capi.Grid(t)
+    hip = hip_runtime()
+    before = free_bytes(hip)
+    dev.sort()
+    left = before - free_bytes(hip)
+    keys, index, perms = dev.permutations()
+    assert len(perms) == 1 and len(keys) > 1_500_000
+    work = len(keys) // 2 * (36 + 2 * B)
+    print(f"  {len(keys)} keys, work space {work >> 20} MB, {left >> 20} MB left with the handle", flush=True)
+    # what stays: keys, their indices, the first key of every vertex, a word per cell slot
+    cells = 8 * len(t["cube_vertices"]) + 4 * len(t["tet_vertices"])
+    assert work > 128 << 20
+    assert left <= 12 * len(keys) + 4 * (V + cells) + (16 << 20)
