@@ -877,10 +877,17 @@ static bool has_table(const DataConst& d, int precision) {
 // (a lower line for wide FP32 rows gained 3 % at 3001 points of a coarser grid
 // and cost the table's 0.4 ms on each first call).
 // A first call also builds the table, whose rows it would mostly compute for
-// itself anyway once there is a point for every four cells.  Scalar rows are
-// so short that bucketing them costs more than it saves (6 modes, 556 830
-// vertices, 1 000 003 points: 274 / 370) until the payload is far beyond the
-// caches.
+// itself anyway once there is a point for every four cells.
+// Rows of one to four scalars are so short that bucketing them costs more than
+// it saves until a call sums many: payloads of 12 to 420 MB, tile / binned (us),
+//   FP64: 1 element 2 000 003 points 598 / 546 (1 000 003: 310 / 343), 2 elements
+//     1 000 003 492 / 405 (600 011: 305 / 317), on a grid of a million cells
+//     578 / 707 (2 000 003: 1107 / 1044); 4 elements 300 007 336 / 330
+//   FP32: 1 element 4 000 037 810 / 754 (2 000 003: 415 / 431), 2 elements
+//     2 000 003 596 / 512 (1 000 003: 311 / 320), 4 elements 1 000 003 493 / 400
+//     (600 011: 307 / 313), on the million cells 576 / 694 (2 000 003: 1107 / 1026)
+// Longer rows, which the general sums read twice, take the pipeline like any
+// other: 8 elements FP64, 49 MB, 300 007 points 3656 / 991.
 // A call whose work space is not ordered after its other users' (`shared`
 // false: allocation-free calls, and calls that a graph records, which may not
 // build the table either) is binned only on payloads beyond the L2 and from
@@ -896,12 +903,16 @@ bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int p
     return false;
   const DataConst& d = G->d;
   const uint64_t payload = (uint64_t)d.V * d.B * d.stride32 * 4;
-  const bool scalars = payload_layout(d) == LAYOUT_SCALAR && !wide_rows(d);
+  const uint64_t work = a.n * d.B * d.sc, cells = G->n_cubes + G->n_tets / 2;
   // large calls on payloads that do not fit the L2 of one XCD
-  if (a.n >= (1ull << 18) && payload > (scalars ? 512ull << 20 : 8ull << 20)) return true;
+  if (a.n >= (1ull << 18) && payload > (8ull << 20)) {
+    const bool short_rows = payload_layout(d) == LAYOUT_SCALAR && onepass_sc(d) != 0;
+    if (!short_rows || payload > (512ull << 20)) return true;
+    if (precision == BRILLE_FP32) return work >= 26000000ull && a.n >= cells;
+    return d.sc >= 4 ? work >= 7000000ull : work >= 14000000ull && 2 * a.n >= cells;
+  }
   if (!shared || payload_layout(d) != LAYOUT_GAMMA || !(wide_rows(d) || onepass_sc(d))) return false;
-  if (!has_table(d, precision) && 4 * a.n < G->n_cubes + G->n_tets / 2) return false;
-  const uint64_t work = a.n * d.B * d.sc;
+  if (!has_table(d, precision) && 4 * a.n < cells) return false;
   if (wide_rows(d)) return work >= (precision == BRILLE_FP32 ? 20000000ull : 4000000ull);
   return work >= (precision == BRILLE_FP32 ? 13000000ull : 7000000ull);
 }
