@@ -746,7 +746,7 @@ static uint64_t payload_stride_host(const DataConst& d) {
 }
 
 template <typename Real>
-static int build_cube_rows(brille_grid* G, hipStream_t s, Real** out) {
+static int build_cube_rows(brille_grid* G, hipStream_t s, const Real** out) {
   const DataConst& d = G->d;
   const uint64_t cube_units = G->n_cubes * 8 * d.B;
   const uint64_t units = cube_units + G->n_tets * 4 * d.B;
@@ -773,7 +773,7 @@ static int build_cube_rows(brille_grid* G, hipStream_t s, Real** out) {
 }
 
 template <typename Real>
-static int build_wide_factors(brille_grid* G, hipStream_t s, typename Cplx<Real>::T** out) {
+static int build_wide_factors(brille_grid* G, hipStream_t s, const typename Cplx<Real>::T** out) {
   using C = typename Cplx<Real>::T;
   const DataConst& d = G->d;
   const bool atom = wide_by_atom(d);
@@ -798,47 +798,40 @@ static int build_wide_factors(brille_grid* G, hipStream_t s, typename Cplx<Real>
   return BRILLE_OK;
 }
 
-// Builds the payload's derived table of the given precision once (freed with
-// the payload, or when a sort replaces the permutations it follows): the antiphased rows (8 per cube, 4 per tetrahedron and mode)
-// for the one-pass layouts, the antiphase factors alone for wide rows.  The
-// general layout, grids without cells and tables beyond kCubeRowsMax go
-// without, and their sums compute every antiphase on the fly.
+// Bytes of the payload's derived table of a precision: the antiphased rows (8 per
+// cube, 4 per tetrahedron and mode) for the one-pass layouts, the antiphase
+// factors alone for wide rows.  The general layout, grids without cells and
+// tables beyond kCubeRowsMax go without (0), and their sums compute every
+// antiphase on the fly.
 constexpr uint64_t kCubeRowsMax = (4ull << 30) - 1;  // the sums address the table with 32-bit offsets
+static uint64_t table_bytes(const brille_grid* G, int precision) {
+  const DataConst& d = G->d;
+  if (!d.has_blocks) return 0;
+  const bool f32 = precision == BRILLE_FP32;
+  const uint64_t row = wide_rows(d)          ? (f32 ? 8 : 16)
+                       : onepass_sc(d) == 0 ? 0
+                       : f32                ? d.stride32 * 4ull
+                                            : d.stride64 * 8ull;
+  const uint64_t bytes = (G->n_cubes * 8 + G->n_tets * 4) * d.B * row;
+  return bytes > kCubeRowsMax ? 0 : bytes;
+}
+
+// the derived table of a precision exists (or the payload has none)
+static bool has_table(const DataConst& d, int precision) {
+  if (wide_rows(d)) return precision == BRILLE_FP32 ? d.wide_fac32 != nullptr : d.wide_fac64 != nullptr;
+  if (onepass_sc(d) == 0) return true;
+  return precision == BRILLE_FP32 ? d.cube_rows32 != nullptr : d.cube_rows64 != nullptr;
+}
+
+// Builds that table once (freed with the payload, or when a sort replaces the
+// permutations it follows).
 int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s) {
   DataConst& d = G->d;
-  if (G->n_cubes + G->n_tets == 0 || d.B == 0 || !d.has_blocks) return BRILLE_OK;
-  if (wide_rows(d)) {
-    // wide rows: the antiphases only (one complex per slot row)
-    const uint64_t fac_bytes = (G->n_cubes * 8 + G->n_tets * 4) * d.B * (precision == BRILLE_FP32 ? 8ull : 16ull);
-    if (fac_bytes > kCubeRowsMax) return BRILLE_OK;
-    if (precision == BRILLE_FP32) {
-      if (d.wide_fac32) return BRILLE_OK;
-      float2* t = nullptr;
-      const int rc = build_wide_factors<float>(G, s, &t);
-      if (rc == BRILLE_OK) d.wide_fac32 = t;
-      return rc;
-    }
-    if (d.wide_fac64) return BRILLE_OK;
-    double2* t = nullptr;
-    const int rc = build_wide_factors<double>(G, s, &t);
-    if (rc == BRILLE_OK) d.wide_fac64 = t;
-    return rc;
-  }
-  if (onepass_sc(d) == 0) return BRILLE_OK;
-  const uint64_t row_bytes = precision == BRILLE_FP32 ? d.stride32 * 4ull : d.stride64 * 8ull;
-  if ((G->n_cubes * 8 + G->n_tets * 4) * d.B * row_bytes > kCubeRowsMax) return BRILLE_OK;
-  if (precision == BRILLE_FP32) {
-    if (d.cube_rows32) return BRILLE_OK;
-    float* t = nullptr;
-    const int rc = build_cube_rows<float>(G, s, &t);
-    if (rc == BRILLE_OK) d.cube_rows32 = t;
-    return rc;
-  }
-  if (d.cube_rows64) return BRILLE_OK;
-  double* t = nullptr;
-  const int rc = build_cube_rows<double>(G, s, &t);
-  if (rc == BRILLE_OK) d.cube_rows64 = t;
-  return rc;
+  if (table_bytes(G, precision) == 0 || has_table(d, precision)) return BRILLE_OK;
+  const bool wide = wide_rows(d);
+  if (precision == BRILLE_FP32)
+    return wide ? build_wide_factors<float>(G, s, &d.wide_fac32) : build_cube_rows<float>(G, s, &d.cube_rows32);
+  return wide ? build_wide_factors<double>(G, s, &d.wide_fac64) : build_cube_rows<double>(G, s, &d.cube_rows64);
 }
 
 // Buckets of at most kNodesPerBucket trellis nodes: k_bucket_perm orders each
@@ -858,13 +851,6 @@ static uint32_t bucket_count(const brille_grid* G) {
   return (uint32_t)std::min<uint64_t>(nb, n_nodes);
 }
 
-// the derived table of a precision exists (or the payload has none)
-static bool has_table(const DataConst& d, int precision) {
-  if (wide_rows(d)) return precision == BRILLE_FP32 ? d.wide_fac32 != nullptr : d.wide_fac64 != nullptr;
-  if (onepass_sc(d) == 0) return true;
-  return precision == BRILLE_FP32 ? d.cube_rows32 != nullptr : d.cube_rows64 != nullptr;
-}
-
 // AUTO's choice between the fused tile kernel and the binned pipeline, on the
 // complex elements summed (n B sc) of Gamma rows.  The pipeline's fixed cost is
 // nine launches; its sums read antiphased rows and reuse them over a node's
@@ -876,8 +862,9 @@ static bool has_table(const DataConst& d, int precision) {
 //   24 atoms FP32: 3001 263 / 261, 10 001 796 / 482; FP64: 1001 290 / 233
 // (a lower line for wide FP32 rows gained 3 % at 3001 points of a coarser grid
 // and cost the table's 0.4 ms on each first call).
-// A first call also builds the table, whose rows it would mostly compute for
-// itself anyway once there is a point for every four cells.
+// With fewer than two points a cell the narrow rows are reused too little
+// (4 atoms FP64, 49 583 points of 34 973 cells: 213 / 236).  A table that is not
+// there yet: see table_due.
 // Rows of one to four scalars are so short that bucketing them costs more than
 // it saves until a call sums many: payloads of 12 to 420 MB, tile / binned (us),
 //   FP64: 1 element 2 000 003 points 598 / 546 (1 000 003: 310 / 343), 2 elements
@@ -912,9 +899,27 @@ bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int p
     return d.sc >= 4 ? work >= 7000000ull : work >= 14000000ull && 2 * a.n >= cells;
   }
   if (!shared || payload_layout(d) != LAYOUT_GAMMA || !(wide_rows(d) || onepass_sc(d))) return false;
-  if (!has_table(d, precision) && 4 * a.n < cells) return false;
   if (wide_rows(d)) return work >= (precision == BRILLE_FP32 ? 20000000ull : 4000000ull);
-  return work >= (precision == BRILLE_FP32 ? 13000000ull : 7000000ull);
+  return a.n >= 2 * cells && work >= (precision == BRILLE_FP32 ? 13000000ull : 7000000ull);
+}
+
+// Whether an ordinary call of n points may build the table it is to be summed
+// from.  Building costs what the fused kernel takes for so many points a cell:
+// narrow rows FP64 14, FP32 24, wide rows 1.5 and 2.5 (a first call of 4 atoms
+// FP64, 10 757 cells, 99 166 points, 9 a cell: 431 us against 362 fused, 18 a
+// cell 480 against 720; 2 atoms FP32, 20 a cell 249 against 188, 40 a cell 320
+// against 353; 24 atoms FP64, 1 a cell 1738 against 1633, 2 a cell 1952 against
+// 3129).  A call of so many builds it at once; shorter ones take the fused
+// kernel until they have come to so many since the last fill or sort, so that
+// a payload used for a call or two never pays for its table.
+bool table_due(brille_grid* G, uint64_t n, int precision) {
+  if (has_table(G->d, precision)) return true;
+  if (table_bytes(G, precision) == 0) return false;
+  uint64_t& points = G->untabled[precision == BRILLE_FP32];
+  points += n;
+  const bool f32 = precision == BRILLE_FP32;
+  const uint64_t halves = wide_rows(G->d) ? (f32 ? 5 : 3) : (f32 ? 48 : 28);
+  return 2 * points >= halves * (G->n_cubes + G->n_tets / 2);
 }
 
 __global__ void k_zero_words(uint32_t* p, uint32_t n) {

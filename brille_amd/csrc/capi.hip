@@ -474,6 +474,7 @@ static int grid_fill(brille_grid* G, const brille_data_desc* vals, const brille_
   free_all(G->sort_allocs);
   free_all(G->derived_allocs);
   G->recorded = false;
+  G->untabled[0] = G->untabled[1] = 0;
   G->n_perms = 0;
   ++G->fill_gen;  // the payload tables are replaced from here on (batches re-read them)
   G->filled = false;

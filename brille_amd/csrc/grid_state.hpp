@@ -39,6 +39,8 @@ struct brille_grid {
   // the row and factor tables built from the payload and its permutations
   // (freed by the next fill or sort)
   std::vector<void*> derived_allocs;
+  // points AUTO has given to the fused kernel for want of those tables, FP64 and FP32
+  uint64_t untabled[2] = {0, 0};
   // a graph has recorded a call, and so the present tables: a sort then keeps
   // those it replaces until the next fill, like the payload
   bool recorded = false;
@@ -145,6 +147,7 @@ inline brille_aux_out offset_aux(const brille_aux_out& x, uint64_t c0) {
 // them; otherwise AUTO keeps to the line for large calls)
 bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int precision, bool shared = true);
 bool binned_recordable(const brille_grid* G, uint64_t n);
+bool table_due(brille_grid* G, uint64_t n, int precision);
 // the derived table, work space and side stream of a binned call of n points;
 // launch_binned needs them
 int prepare_binned(brille_grid* G, uint64_t n, int precision, hipStream_t s);

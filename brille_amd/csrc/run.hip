@@ -348,8 +348,13 @@ static bool takes_pipeline(const brille_grid* G, const LaunchArgs& a, const bril
 static int choose_pipeline(brille_grid* G, const LaunchArgs& a, const brille_run_opts& o, hipStream_t s, bool* binned) {
   *binned = takes_pipeline(G, a, o, s);
   if (!*binned) return BRILLE_OK;
+  const bool asked = o.kernel == BRILLE_KERNEL_BINNED || a.use_proposal;
+  if (!asked && !binned_applies(G, a, o.kernel, o.precision, false) && !table_due(G, a.n, o.precision)) {
+    *binned = false;
+    return BRILLE_OK;
+  }
   const int rc = prepare_binned(G, a.n, o.precision, s);
-  if (rc == BRILLE_OK || o.kernel == BRILLE_KERNEL_BINNED || a.use_proposal) return rc;
+  if (rc == BRILLE_OK || asked) return rc;
   (void)hipGetLastError();
   *binned = false;
   return BRILLE_OK;

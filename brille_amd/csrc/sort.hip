@@ -956,6 +956,7 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
     old->clear();
   }
   G->recorded = false;
+  G->untabled[0] = G->untabled[1] = 0;
   for (void* p : {(void*)keys, (void*)pidx, (void*)perms_fit}) {
     buf.release(p);
     G->sort_allocs.push_back(p);

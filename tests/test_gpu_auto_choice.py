@@ -56,3 +56,32 @@ def test_scalar_rows(elements, values, precision, n, binned):
     tile = device_call(dev, Q, precision, capi.KERNEL_TILE)
     for a, b in zip(auto[1:], tile[1:]):
         np.testing.assert_array_equal(a.to_host(), b.to_host())
+
+
+# grid, precision, points of a call above the line of work, points a cell that pay for the table
+@pytest.mark.parametrize("spec,v_target,precision,n,per_cell", [
+    (7, 30_000, capi.FP64, 60_000, 14), (7, 30_000, capi.FP32, 110_000, 24), (5, 1_000, capi.FP64, 1_000, 1.5),
+    (5, 12_000, capi.FP32, 4_500, 2.5)])
+def test_ordinary_calls_until_they_have_paid_for_the_table(spec, v_target, precision, n, per_cell):
+    print(f"auto choice: table of grid {spec}, {precision}, {n} points", flush=True)
+    sp = dict(S.batch_specs(16)[spec], v_target=float(v_target))
+    g = S.batch_grid(sp)
+    vals, vecs = S.batch_payload(g, sp)
+    t = dict(S.batch_layout_tables(g, sp), values=vals, vectors=vecs)
+    cells = len(t["cube_vertices"]) + len(t["tet_vertices"]) // 2
+    due = int(np.ceil(per_cell * cells / n))  # the call that builds it
+    assert 1 < due < 60
+    dev = capi.Grid(t)
+    Q = points(g, np.random.default_rng(4), n)
+    want = [x.to_host() for x in device_call(dev, Q, precision, capi.KERNEL_TILE)[1:]]
+    for k in range(1, due + 2):
+        assert takes_pipeline(dev, Q, precision) == (k >= due), k
+        if k in (1, due):
+            for a, b in zip(device_call(dev, Q[:n // 9], precision, capi.KERNEL_AUTO)[1:], want):
+                np.testing.assert_array_equal(a.to_host(), b[:n // 9])
+    for a, b in zip(device_call(dev, Q, precision, capi.KERNEL_AUTO)[1:], want):
+        np.testing.assert_array_equal(a.to_host(), b)
+    dev.fill(t)  # a new payload counts anew
+    assert not takes_pipeline(dev, Q, precision)
+    device_call(dev, Q, precision, capi.KERNEL_BINNED)  # a call that asks for the table
+    assert takes_pipeline(dev, Q, precision)
