@@ -44,3 +44,37 @@ def test_permuted_scalar_rows_in_the_binned_sums(elements, modes):
         assert np.max(np.abs(bv - ov)) <= tol * np.abs(ov).max()
         if elements == 1:  # one element's antiphase turns it onto the pivot: no cancelling overlap
             assert np.max(np.abs(bc - oc)) <= tol * np.abs(oc).max()
+
+
+# either side of the longest sorted row a lane sums, and rows of more values than atoms
+@pytest.mark.parametrize("elements,values,atoms", [(13, 1, False), (24, 1, False), (25, 1, False), (15, 6, True), (24, 9, True), (27, 10, True)])
+def test_sorted_rows_around_the_longest_a_lane_sums(elements, values, atoms):
+    print(f"sorted rows: {elements} elements, {values} values, atoms {atoms}", flush=True)
+    sp = dict(S.batch_specs(16)[3], v_target=400.0)
+    g = S.batch_grid(sp)
+    t = S.batch_layout_tables(g, sp)
+    V, G = len(t["vertices"]), np.asarray(t["gamma_F0"]).shape[1]
+    r = np.random.default_rng(elements)
+    modes, A = 7, elements // 3
+    t.update(values=r.normal(size=(V, modes, values)), values_elements=[values, 0, 0], branches=modes,
+             vectors=r.normal(size=(V, modes, elements)) + 1j * r.normal(size=(V, modes, elements)))
+    if atoms:
+        t.update(vectors_elements=[0, elements, 0], gamma_F0=np.stack([r.permutation(A) for _ in range(G)], 1).astype(np.uint32),
+                 gamma_vector_index=r.integers(0, 7, size=(A, G)).astype(np.uint32), gamma_vectors=r.normal(size=(7, 3)))
+    else:
+        t.update(vectors_elements=[elements, 0, 0], vectors_rotates_like=0)
+    dev = capi.Grid(t)
+    dev.sort()
+    perm = dev.permutations()
+    for n in (1, 300, 20_000):
+        Q = r.uniform(-3, 3, size=(n, 3))
+        rc, ov, oc, _, _ = O.ir_interpolate_at(t, Q, nthreads=8, perm=perm)
+        assert rc == 0
+        for prec, tol in ((capi.FP64, 1e-12), (capi.FP32, 1e-5)):
+            bv, bc = dev.ir_interpolate_at(Q, precision=prec, kernel=capi.KERNEL_BINNED)
+            tv, tc = dev.ir_interpolate_at(Q, precision=prec, kernel=capi.KERNEL_TILE)
+            np.testing.assert_array_equal(bv, tv)
+            np.testing.assert_array_equal(bc, tc)
+            assert np.max(np.abs(bv - ov)) <= tol * np.abs(ov).max(), (n, prec)
+            # an assigned pair's overlap can still be small, and the antiphase then carries the products' rounding
+            assert np.max(np.abs(bc - oc)) <= 10 * tol * np.abs(oc).max(), (n, prec)
