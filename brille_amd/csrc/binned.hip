@@ -1071,22 +1071,25 @@ bool recording(hipStream_t s) {
   return st != hipStreamCaptureStatusNone;
 }
 
-// The handle's lock covers the enqueueing of a call alone, so calls on two
-// streams would meet in the work space: each waits for the event the call
-// before it recorded.  (A call that records a graph cannot wait for an event
-// from outside it, nor leave one.)
+// The handle's lock covers the enqueueing of an unchecked call alone, so such
+// calls on two streams would meet in the work space: each waits for the event
+// the one before it recorded.  (A call that records a graph cannot wait for an
+// event from outside it, nor leave one; one that the host waits for leaves
+// nothing to wait for, which spares a call of 50 us some 10 of them.)
 static int begin_work_space(brille_grid* G, hipStream_t s) {
-  if (G->bin_used && hipStreamWaitEvent(s, G->bin_used, 0) != hipSuccess)
+  if (G->bin_pending && hipStreamWaitEvent(s, G->bin_used, 0) != hipSuccess)
     return fail(BRILLE_ERR_DEVICE, "waiting for the work space failed");
+  G->bin_touched = true;
   return BRILLE_OK;
 }
-static int end_work_space(brille_grid* G, hipStream_t s) {
-  if (!G->bin_used && hipEventCreateWithFlags(&G->bin_used, hipEventDisableTiming) != hipSuccess) {
-    (void)hipGetLastError();
-    G->bin_used = nullptr;
-  }
-  const hipError_t e = G->bin_used ? hipEventRecord(G->bin_used, s) : hipStreamSynchronize(s);
-  return e == hipSuccess ? BRILLE_OK : fail(BRILLE_ERR_DEVICE, "recording the work space's use failed");
+void end_binned(brille_grid* G, hipStream_t s, bool waited) {
+  if (!G->bin_touched) return;
+  G->bin_touched = false;
+  G->bin_pending = false;
+  if (waited) return;
+  if (!G->bin_used && hipEventCreateWithFlags(&G->bin_used, hipEventDisableTiming) != hipSuccess) G->bin_used = nullptr;
+  if (G->bin_used && hipEventRecord(G->bin_used, s) == hipSuccess) G->bin_pending = true;
+  else (void)hipStreamSynchronize(s);
 }
 
 // The work space of a call that a graph records.  The graph keeps the address,
@@ -1101,8 +1104,9 @@ static int recorded_work_space(brille_grid* G, uint64_t bytes) {
   uint64_t held = bytes;
   if (G->bin_ws_bytes >= bytes) {
     // its last user is done before a replay can start
-    if (G->bin_used && hipEventSynchronize(G->bin_used) != hipSuccess)
+    if (G->bin_pending && hipEventSynchronize(G->bin_used) != hipSuccess)
       return fail(BRILLE_ERR_DEVICE, "waiting for the work space failed");
+    G->bin_pending = false;
     ws = G->bin_ws;
     held = G->bin_ws_bytes;
     G->bin_ws = nullptr;
@@ -1132,9 +1136,7 @@ int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_
   const Passes p = passes_of(G, a.n);
   if (recording(s)) return run_binned_passes(G, a, precision, s, stage_ms, G->rec_ws, p.chunk, p.halves);
   if (int rc = begin_work_space(G, s); rc != BRILLE_OK) return rc;
-  const int rc = run_binned_passes(G, a, precision, s, stage_ms, G->bin_ws, p.chunk, p.halves);
-  const int end = end_work_space(G, s);
-  return rc != BRILLE_OK ? rc : end;
+  return run_binned_passes(G, a, precision, s, stage_ms, G->bin_ws, p.chunk, p.halves);
 }
 
 // The pipeline over work space `ws` in passes of `chunk` points; with two

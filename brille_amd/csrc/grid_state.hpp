@@ -67,9 +67,11 @@ struct brille_grid {
   void* rec_ws = nullptr;
   size_t rec_ws_bytes = 0;
   std::vector<void*> rec_old;
-  // recorded after each binned call's last kernel: the next call, on whatever
-  // stream, waits for it before it writes the work space
+  // bin_pending: kernels of a call that nothing has waited for may still work in
+  // bin_ws; bin_used is recorded after them, and the next call, on whatever
+  // stream, waits for it.  bin_touched: the present call's kernels do
   hipEvent_t bin_used = nullptr;
+  bool bin_pending = false, bin_touched = false;
   // side stream of the binned pipeline (preparation of the next pass) and its
   // events: call start, prepared[2], summed[2]
   hipStream_t bin_side = nullptr;
@@ -151,6 +153,9 @@ bool table_due(brille_grid* G, uint64_t n, int precision);
 // the derived table, work space and side stream of a binned call of n points;
 // launch_binned needs them
 int prepare_binned(brille_grid* G, uint64_t n, int precision, hipStream_t s);
+// ends a call on stream s that may have launched the pipeline; waited: the host
+// has waited for the stream since
+void end_binned(brille_grid* G, hipStream_t s, bool waited);
 int launch_binned(brille_grid* G, const LaunchArgs& a, int precision, hipStream_t s, float* stage_ms);
 // whether stream s is recording a graph
 bool recording(hipStream_t s);

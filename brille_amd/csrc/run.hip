@@ -442,8 +442,15 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
   if (opts.use_proposal) zero_words(G->prop_stats, 4, s);  // tried, verified (two 64-bit counters)
   a.err = G->err;
   CallReport rep{};
+  struct End {  // however the call returns
+    brille_grid* G;
+    hipStream_t s;
+    bool waited = false;
+    ~End() { end_binned(G, s, waited); }
+  } end{G, s};
   auto finish_call = [&] {
     const int r = read_report(G, s, &rep);
+    end.waited = r == BRILLE_OK;
     if (r == BRILLE_OK && opts.use_proposal) {
       G->last_tried = rep.tried;
       G->last_hits = rep.verified;

@@ -34,8 +34,8 @@ class Call:
         self.out = (capi.DeviceArray(vs, np.float32 if f32 else np.float64),
                     capi.DeviceArray(cs, np.complex64 if f32 else np.complex128))
 
-    def run(self, stream, kernel, entry="brille_ir_interpolate_at"):
-        o = capi.RunOpts(0, self.precision, 0, capi.MEM_DEVICE, kernel, 0)
+    def run(self, stream, kernel, entry="brille_ir_interpolate_at", check=0):
+        o = capi.RunOpts(0, self.precision, 0, capi.MEM_DEVICE, kernel, check)
         capi.check(getattr(capi.lib(), entry)(self.dev.h, self.Q.ptr, self.n, C.byref(o), self.out[0].ptr,
                                               self.out[1].ptr, None, stream.p if stream else None))
 
@@ -48,6 +48,7 @@ def grid_tables(spec, v_target=600.0):
 
 
 # 4 and 24 atoms; sizes AUTO gives to the pipeline
+# (every seventh call is checked: the host waits for it, and the next ones need not)
 @pytest.mark.parametrize("spec,precision,sizes,kernel", [
     (7, capi.FP64, (60_000, 75_000), capi.KERNEL_AUTO), (7, capi.FP32, (120_000, 100_000), capi.KERNEL_AUTO),
     (5, capi.FP64, (2_000, 3_000), capi.KERNEL_AUTO), (3, capi.FP32, (50_000, 400_000), capi.KERNEL_BINNED)])
@@ -63,9 +64,8 @@ def test_unchecked_calls_on_two_streams_and_the_null_stream(spec, precision, siz
         calls = [Call(dev, Q, precision) for Q in Qs]
         streams = [Stream(), Stream(), None]
         capi.check(capi.lib().brille_device_sync())
-        for _ in range(2):
-            for k, c in enumerate(calls):
-                c.run(streams[k % 3], kernel)
+        for k in range(2 * len(calls)):
+            calls[k % len(calls)].run(streams[k % 3], kernel, check=int(k % 7 == 3))
         capi.check(capi.lib().brille_device_sync())
         for c, w in zip(calls, want):
             for a, b in zip(c.out, w):
