@@ -74,9 +74,12 @@ struct OutPiece {
 // Whole calls of 100 003 points of 6 modes and 2 atoms FP64 (62 MB), pageable
 // copies 6.0 ms: one thread 4.7, three 2.5, six 2.3 in 1 MB chunks; four threads
 // 2.0 in 2 MB chunks (eight the same), 2.0 in 4 MB, 2.2 in 8 MB, 3.2 in 512 KB
-// (each chunk costs about 10 us of launches and waits).  Below two chunks per
-// thread the caller's thread works with fewer or none; where a thread or the
-// ring cannot be had, the rest do the work.
+// (each chunk costs about 10 us of launches and waits).  Below one and a quarter
+// chunks' bytes per thread the caller's thread works with fewer or none (by the
+// number of chunks the dozen arrays of a call with every aux output, 4.5 to 6 MB,
+// started threads that cost more than they copied: 20 011 points of 6 scalars
+// FP32 506 us against 478 of pageable copies, 463 with one thread); where a
+// thread or the ring cannot be had, the rest do the work.
 constexpr uint64_t kPinWorkers = 4;
 // bytes of a host-memory call up to which the kernels use pinned memory directly
 constexpr size_t kDirectBytes = 4ull << 20;
@@ -130,7 +133,9 @@ static int copy_out(brille_grid* G, const std::vector<OutPiece>& out, hipStream_
   std::vector<std::thread> helpers;
   helpers.reserve(kPinWorkers);
   const uint64_t hw = std::max(1u, std::thread::hardware_concurrency());
-  const uint64_t n_help = std::min({kPinWorkers, (uint64_t)chunks.size() / 2, hw});
+  uint64_t bytes = 0;
+  for (const OutPiece& p : out) bytes += p.bytes;
+  const uint64_t n_help = std::min({kPinWorkers, bytes / (kPinChunk + kPinChunk / 4), hw});
   for (uint64_t i = 1; i < n_help; ++i) {
     try {
       helpers.emplace_back([&] {
