@@ -85,14 +85,12 @@ struct PointRec {
 // Per-point constants of the Gamma rotation (rip_gamma_complex,
 // src/interpolator_gamma.tpp:100-114), kept in LDS by phase 1 so that the sums
 // read no tables: R is invRidx (integer, or Cartesian for angstrom units) as
-// the sums' scale factors, to[a] the output atom of source atom a (GammaTable
-// F0) and from[o] the source atom written to output atom o (255: none; the
-// last source atom wins, as in a loop over source atoms).
+// the sums' scale factors and to[a] the output atom of source atom a (GammaTable
+// F0).
 template <typename Real>
 struct GammaFrame {
   Real R[9];
   uint8_t to[4];
-  uint8_t from[4];
 };
 template <typename Real>
 constexpr int frame_words() {
@@ -1562,20 +1560,8 @@ __device__ __forceinline__ void fill_frame(const GridConst& g, const DataConst& 
 #pragma unroll
     for (int k = 0; k < 9; ++k) f.R[k] = (Real)g.rot[9 * (uint64_t)invrot + k];
   }
-  uint8_t to[4] = {255, 255, 255, 255}, from[4] = {255, 255, 255, 255};
 #pragma unroll
-  for (int a = 0; a < SC / 3; ++a) {
-    const uint32_t l = d.F0[a * d.gamma_ops + invrot];
-    to[a] = (uint8_t)l;
-#pragma unroll
-    for (int o = 0; o < SC / 3; ++o)
-      if ((uint32_t)o == l) from[o] = (uint8_t)a;
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    f.to[a] = to[a];
-    f.from[a] = from[a];
-  }
+  for (int a = 0; a < SC / 3; ++a) f.to[a] = (uint8_t)d.F0[a * d.gamma_ops + invrot];
 }
 
 // a located point's phase-2 record (plus phases, and q for the general
