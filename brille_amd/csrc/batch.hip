@@ -426,6 +426,7 @@ static int ensure_batch_tables(brille_batch* b, int precision, hipStream_t s) {
       b->fill_gen[g] = G->fill_gen;
       changed = true;
     }
+    if (const int rc = await_tables(G, s); rc != BRILLE_OK) return rc;
     if (!wide_rows(G->d)) continue;
     const void* before = precision == BRILLE_FP32 ? (const void*)G->d.wide_fac32 : (const void*)G->d.wide_fac64;
     const int rc = ensure_cube_rows(G, precision, s);
@@ -438,6 +439,7 @@ static int ensure_batch_tables(brille_batch* b, int precision, hipStream_t s) {
   }
   if (changed) {
     BATCH_TRY(hipStreamSynchronize(s));
+    for (brille_grid* G : b->grids) G->tables_pending = false;  // the stream waited for each
     BATCH_TRY(hipMemcpy(b->d_grids, b->host_grids.data(), b->host_grids.size() * sizeof(BatchGrid),
                         hipMemcpyHostToDevice));
   }

@@ -475,6 +475,7 @@ static int grid_fill(brille_grid* G, const brille_data_desc* vals, const brille_
   free_all(G->derived_allocs);
   G->recorded = false;
   G->untabled[0] = G->untabled[1] = 0;
+  G->tables_pending = false;
   G->n_perms = 0;
   ++G->fill_gen;  // the payload tables are replaced from here on (batches re-read them)
   G->filled = false;

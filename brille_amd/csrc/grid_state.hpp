@@ -39,6 +39,10 @@ struct brille_grid {
   // the row and factor tables built from the payload and its permutations
   // (freed by the next fill or sort)
   std::vector<void*> derived_allocs;
+  // tables_pending: a build of such a table that nothing has waited for may still
+  // run; tables_built is recorded after it, and calls on any stream wait for it
+  hipEvent_t tables_built = nullptr;
+  bool tables_pending = false;
   // points AUTO has given to the fused kernel for want of those tables, FP64 and FP32
   uint64_t untabled[2] = {0, 0};
   // a graph has recorded a call, and so the present tables: a sort then keeps
@@ -179,8 +183,9 @@ int exclusive_scan_u32(uint32_t* a, uint64_t m, uint32_t* part, hipStream_t s);
 // the lookup tables of an installed PermutationTable (d.keys and d.perm_index
 // set), kept in `allocs`
 int install_permutations(brille_grid* G, std::vector<void*>& allocs, hipStream_t s);
+// work queued on stream s from here on finds the handle's derived tables built
+int await_tables(brille_grid* G, hipStream_t s);
 // the cube row table of the bucketed sums, built on first use (derived_allocs)
-// and complete when the function returns: later calls read it from any stream
 int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s);
 // the first failing point of a call as the reference's error text
 int report_point_error(const ErrRec& e, const double* Q, uint64_t n, bool host_mem);

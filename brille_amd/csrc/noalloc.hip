@@ -105,6 +105,7 @@ extern "C" int brille_ir_interpolate_at_noalloc(brille_grid* G, const double* Q,
   a.use_proposal = o.use_proposal;
   a.prop = G->prop;
   if (!o.check && recording(s)) G->recorded = true;
+  if ((rc = await_tables(G, s)) != BRILLE_OK) return rc;
   const bool fast = o.kernel != BRILLE_KERNEL_PLAIN;
   const bool binned = fast && binned_applies(G, a, o.kernel, o.precision, false);
   uint64_t chunk = 0;

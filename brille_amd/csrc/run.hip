@@ -462,6 +462,7 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
     }
     return r;
   };
+  if (rc = await_tables(G, s); rc != BRILLE_OK) return rc;
   if (opts.memory == BRILLE_MEM_DEVICE) {
     if (!opts.check && !times && recording(s)) G->recorded = true;
     a.Q = Q;

@@ -957,6 +957,7 @@ extern "C" int brille_grid_sort(brille_grid* G, const brille_cost_info* values_c
   }
   G->recorded = false;
   G->untabled[0] = G->untabled[1] = 0;
+  G->tables_pending = false;
   for (void* p : {(void*)keys, (void*)pidx, (void*)perms_fit}) {
     buf.release(p);
     G->sort_allocs.push_back(p);
