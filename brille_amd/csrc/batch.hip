@@ -439,7 +439,7 @@ static int ensure_batch_tables(brille_batch* b, int precision, hipStream_t s) {
   }
   if (changed) {
     BATCH_TRY(hipStreamSynchronize(s));
-    for (brille_grid* G : b->grids) G->tables_pending = false;  // the stream waited for each
+    for (brille_grid* G : b->grids) G->tables_pending = G->tables_touched = false;  // the stream waited for each
     BATCH_TRY(hipMemcpy(b->d_grids, b->host_grids.data(), b->host_grids.size() * sizeof(BatchGrid),
                         hipMemcpyHostToDevice));
   }

@@ -747,17 +747,12 @@ static uint64_t payload_stride_host(const DataConst& d) {
 
 // The build of a table is queued on one stream and its address published at
 // once, so that the call that builds it need not wait on the host (two atoms
-// FP64, 3 000 017 points: first call 2090 us, 2170 with a wait); calls on other
-// streams wait for this event.
-static int end_build(brille_grid* G, hipStream_t s) {
+// FP64, 3 000 017 points: first call 2090 us, 2170 with a wait).  Where the call
+// returns without a wait, calls on other streams wait for an event (end_binned).
+static int end_build(brille_grid* G) {
   if (hipGetLastError() != hipSuccess) return fail(BRILLE_ERR_DEVICE, "building a derived table failed");
-  if (!G->tables_built && hipEventCreateWithFlags(&G->tables_built, hipEventDisableTiming) != hipSuccess) G->tables_built = nullptr;
-  if (G->tables_built && hipEventRecord(G->tables_built, s) == hipSuccess) {
-    G->tables_pending = true;
-    return BRILLE_OK;
-  }
-  (void)hipGetLastError();
-  return hipStreamSynchronize(s) == hipSuccess ? BRILLE_OK : fail(BRILLE_ERR_DEVICE, "building a derived table failed");
+  G->tables_touched = true;
+  return BRILLE_OK;
 }
 
 int await_tables(brille_grid* G, hipStream_t s) {
@@ -795,7 +790,7 @@ static int build_cube_rows(brille_grid* G, hipStream_t s, const Real** out) {
     case 12: hipLaunchKernelGGL((k_table_rows<Real, 12>), grid, dim3(256), 0, s, G->g, d, cube_units, units, t); break;
     default: return fail(BRILLE_ERR_UNSUPPORTED, "no cube row kernel for this payload");
   }
-  if (int rc = end_build(G, s); rc != BRILLE_OK) return rc;
+  if (int rc = end_build(G); rc != BRILLE_OK) return rc;
   *out = t;
   return BRILLE_OK;
 }
@@ -820,7 +815,7 @@ static int build_wide_factors(brille_grid* G, hipStream_t s, const typename Cplx
   else
     hipLaunchKernelGGL((k_wide_factors<Real>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, G->g, d, cube_units,
                        units, t);
-  if (int rc = end_build(G, s); rc != BRILLE_OK) return rc;
+  if (int rc = end_build(G); rc != BRILLE_OK) return rc;
   *out = t;
   return BRILLE_OK;
 }
@@ -1113,14 +1108,19 @@ static int begin_work_space(brille_grid* G, hipStream_t s) {
   return BRILLE_OK;
 }
 void end_binned(brille_grid* G, hipStream_t s, bool waited) {
-  if (waited) G->tables_pending = false;  // the stream waited for them, or built them
-  if (!G->bin_touched) return;
-  G->bin_touched = false;
-  G->bin_pending = false;
-  if (waited) return;
-  if (!G->bin_used && hipEventCreateWithFlags(&G->bin_used, hipEventDisableTiming) != hipSuccess) G->bin_used = nullptr;
-  if (G->bin_used && hipEventRecord(G->bin_used, s) == hipSuccess) G->bin_pending = true;
-  else (void)hipStreamSynchronize(s);
+  // records *e after what the stream holds, or waits for it here
+  auto leave = [s](hipEvent_t* e) {
+    if (!*e && hipEventCreateWithFlags(e, hipEventDisableTiming) != hipSuccess) *e = nullptr;
+    if (*e && hipEventRecord(*e, s) == hipSuccess) return true;
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(s);
+    return false;
+  };
+  // (a call waits for what is pending before it adds to it)
+  if (waited) G->tables_pending = false;
+  else if (G->tables_touched) G->tables_pending = leave(&G->tables_built);
+  if (G->bin_touched) G->bin_pending = !waited && leave(&G->bin_used);
+  G->tables_touched = G->bin_touched = false;
 }
 
 // The work space of a call that a graph records.  The graph keeps the address,

@@ -39,10 +39,11 @@ struct brille_grid {
   // the row and factor tables built from the payload and its permutations
   // (freed by the next fill or sort)
   std::vector<void*> derived_allocs;
-  // tables_pending: a build of such a table that nothing has waited for may still
-  // run; tables_built is recorded after it, and calls on any stream wait for it
+  // tables_pending: the build of such a table by a call that nothing has waited for
+  // may still run; tables_built is recorded after it, and calls on any stream
+  // wait for it.  tables_touched: the present call builds one
   hipEvent_t tables_built = nullptr;
-  bool tables_pending = false;
+  bool tables_pending = false, tables_touched = false;
   // points AUTO has given to the fused kernel for want of those tables, FP64 and FP32
   uint64_t untabled[2] = {0, 0};
   // a graph has recorded a call, and so the present tables: a sort then keeps
