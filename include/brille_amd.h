@@ -186,8 +186,9 @@ typedef struct brille_perm_desc {
 enum brille_precision { BRILLE_FP64 = 0, BRILLE_FP32 = 1 };
 enum brille_memory { BRILLE_MEM_DEVICE = 0, BRILLE_MEM_HOST = 1 };
 /* AUTO and TUNED pick TILE or BINNED by the work and the payload (TILE when any
- * aux output is requested, and under stream capture unless an earlier call has
- * left what BINNED would allocate); PLAIN is the literal FP64 restatement (exact fold-in, atan2
+ * aux output is requested, when the memory BINNED needs cannot be had, and under
+ * stream capture except for large calls after an eager one has left a work
+ * space); PLAIN is the literal FP64 restatement (exact fold-in, atan2
  * antiphases); TILE is the fused one-launch kernel; BINNED buckets points by
  * trellis node range first so the payload gathers hit in cache (device work
  * space; reports every aux output but tau). */
@@ -288,6 +289,13 @@ int brille_grid_permutations(const brille_grid* grid, uint64_t* n_keys, uint32_t
 uint64_t brille_bytes_per_point(const brille_grid* grid, int32_t precision);
 
 /* ---- the hot path ---- */
+/* An unchecked call (opts->check = 0) on device memory returns while its kernels
+ * run.  Calls of one handle on several streams each get their own results: those
+ * that share its work space follow each other on the device.  A graph that has
+ * recorded a call holds addresses of the handle's tables and work space; they
+ * stay valid until the next fill or the handle's end, over larger calls and
+ * sorts, and no eager call works in them.  Replays of two graphs of one handle
+ * must not overlap. */
 int brille_ir_interpolate_at(brille_grid* grid, const double* Q, uint64_t n,
                              const brille_run_opts* opts, void* values_out,
                              void* vectors_out, const brille_aux_out* aux,
