@@ -48,10 +48,9 @@ struct BatchGrid {
   GridConst g;
   DataConst d;
   ErrRec* err;
-  int32_t kind;
+  int32_t kind[2];  // BatchKind in FP64 and FP32
   int32_t ph_in_lds;
   uint32_t n_atoms;
-  uint32_t pad;
 };
 
 struct BatchSlot {
@@ -76,13 +75,13 @@ struct BatchHeader {
 };
 
 // the specialised phase 2 a grid's payload takes inside the batch kernel
-static int32_t batch_kind(const DataConst& d) {
+static int32_t batch_kind(const DataConst& d, int precision) {
   const int L = payload_layout(d);
   if (L == LAYOUT_GAMMA && d.sv == 1 && d.sc == 3) return BK_GAMMA3;
   if (L == LAYOUT_GAMMA && d.sv == 1 && d.sc == 6) return BK_GAMMA6;
   if (L == LAYOUT_SCALAR && d.sv == 1 && d.sc >= 1 && d.sc <= 4) return BK_SCALAR1 + (int32_t)d.sc - 1;
   if (wide_by_atom(d)) return BK_WIDE_ATOM;
-  if (wide_rows(d)) return BK_WIDE;
+  if (wide_rows(d, precision)) return BK_WIDE;
   return BK_GENERIC;
 }
 
@@ -151,12 +150,12 @@ void k_batch(const BatchGrid* grids, const BatchSlot* all_slots, BatchHeader* hd
       const uint64_t left = sl.n - p0;
       const uint32_t npts = left < (uint64_t)sl.pts ? (uint32_t)left : sl.pts;
       if constexpr (kWide) {
-        if (bg.kind == BK_WIDE_ATOM)
+        if (bg.kind[sizeof(Real) == 4] == BK_WIDE_ATOM)
           batch_tile<Real, LAYOUT_WIDE, kWideAtom, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold);
         else
           batch_tile<Real, LAYOUT_WIDE, kWideAll, 0, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold);
         continue;
-      } else switch (bg.kind) {
+      } else switch (bg.kind[sizeof(Real) == 4]) {
         case BK_GAMMA3: batch_tile<Real, LAYOUT_GAMMA, 3, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
         case BK_GAMMA6: batch_tile<Real, LAYOUT_GAMMA, 6, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
         case BK_SCALAR1: batch_tile<Real, LAYOUT_SCALAR, 1, 1, TB>(bg, sl, p0, npts, s_rec, s_ph, s_q, s_wide, s_pm, fold); break;
@@ -192,10 +191,11 @@ static void describe_batch_grid(const brille_grid* G, BatchGrid& bg) {
   bg.g = G->g;
   bg.d = G->d;
   bg.err = G->err;
-  bg.kind = batch_kind(G->d);
+  bg.kind[0] = batch_kind(G->d, BRILLE_FP64);
+  bg.kind[1] = batch_kind(G->d, BRILLE_FP32);
   const bool want_phase = G->d.vec_rot == BRILLE_ROT_GAMMA && G->d.ec[1] > 0;
   bg.n_atoms = G->d.ec[1] / 3u;
-  bg.ph_in_lds = (bg.kind == BK_GAMMA3 || bg.kind == BK_GAMMA6 || (want_phase && bg.n_atoms <= 4)) ? 1 : 0;
+  bg.ph_in_lds = (bg.kind[0] == BK_GAMMA3 || bg.kind[0] == BK_GAMMA6 || (want_phase && bg.n_atoms <= 4)) ? 1 : 0;
 }
 
 struct Schedule {
@@ -304,7 +304,7 @@ static double point_cost(const brille_grid* G) {
 
 // slots of one run (empty grids take no slot) and their upload
 static int stage_slots(brille_batch* b, const double* Q, const uint64_t* offsets, void* const* vals,
-                       void* const* vecs, const Schedule& sc, int fold, hipStream_t s) {
+                       void* const* vecs, const Schedule& sc, int precision, int fold, hipStream_t s) {
   const uint32_t ng = (uint32_t)b->grids.size();
   std::vector<uint32_t> order(ng);
   for (uint32_t g = 0; g < ng; ++g) order[g] = g;
@@ -319,14 +319,14 @@ static int stage_slots(brille_batch* b, const double* Q, const uint64_t* offsets
   constexpr double kTilesPerBlock = 4.0;
   auto units = [&](const brille_grid* G) {
     const DataConst& d = G->d;
-    if (!wide_rows(d)) return (double)d.B / 64.0;
+    if (!wide_rows(d, precision)) return (double)d.B / 64.0;
     const uint32_t mpw = wide_by_atom(d) ? 64u / (d.sc / 3u) : 1u;
     return (double)((d.B + mpw - 1) / mpw);
   };
   double work[kLists] = {0.0, 0.0};
   for (uint32_t g : order) {
     const uint64_t n = offsets[g + 1] - offsets[g];
-    if (n && n < sc.binned_min) work[wide_rows(b->grids[g]->d)] += (double)n * units(b->grids[g]);
+    if (n && n < sc.binned_min) work[wide_rows(b->grids[g]->d, precision)] += (double)n * units(b->grids[g]);
   }
   std::vector<BatchSlot> slots;
   BatchHeader h{};
@@ -335,7 +335,7 @@ static int stage_slots(brille_batch* b, const double* Q, const uint64_t* offsets
     h.slot0[list] = (uint32_t)slots.size();
     for (uint32_t g : order) {
       const uint64_t n = offsets[g + 1] - offsets[g];
-      if (n == 0 || n >= sc.binned_min || (int)wide_rows(b->grids[g]->d) != list) continue;
+      if (n == 0 || n >= sc.binned_min || (int)wide_rows(b->grids[g]->d, precision) != list) continue;
       const double per = work[list] / (blocks * kTilesPerBlock) / units(b->grids[g]);
       BatchSlot sl{};
       sl.Q = Q + 3 * offsets[g];
@@ -427,7 +427,7 @@ static int ensure_batch_tables(brille_batch* b, int precision, hipStream_t s) {
       changed = true;
     }
     if (const int rc = await_tables(G, s); rc != BRILLE_OK) return rc;
-    if (!wide_rows(G->d)) continue;
+    if (!wide_rows(G->d, precision)) continue;
     const void* before = precision == BRILLE_FP32 ? (const void*)G->d.wide_fac32 : (const void*)G->d.wide_fac64;
     const int rc = ensure_cube_rows(G, precision, s);
     if (rc != BRILLE_OK) return rc;
@@ -453,7 +453,7 @@ static int run_with(brille_batch* b, const double* Q, const uint64_t* offsets, c
                     void* const* vals, void* const* vecs, hipStream_t s, const Schedule& sc) {
   int rc = ensure_batch_tables(b, o.precision, s);
   if (rc != BRILLE_OK) return rc;
-  rc = stage_slots(b, Q, offsets, vals, vecs, sc, o.no_move ? FOLD_NONE : FOLD_IR, s);
+  rc = stage_slots(b, Q, offsets, vals, vecs, sc, o.precision, o.no_move ? FOLD_NONE : FOLD_IR, s);
   if (rc != BRILLE_OK) return rc;
   hipGraphExec_t exec;
   rc = graph_for(b, o.precision, sc, &exec);

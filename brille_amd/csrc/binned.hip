@@ -691,7 +691,7 @@ static SumsKernel pick_sums(const DataConst& d, bool prop) {
     }
   }
   if (wide_by_atom(d)) return k_bin_sums<Real, LAYOUT_WIDE, kWideAtom, 0, false>;
-  if (wide_rows(d)) return k_bin_sums<Real, LAYOUT_WIDE, kWideAll, 0, false>;
+  if (wide_rows(d, sizeof(Real) == 4 ? BRILLE_FP32 : BRILLE_FP64)) return k_bin_sums<Real, LAYOUT_WIDE, kWideAll, 0, false>;
   return k_bin_sums<Real, LAYOUT_GENERIC, 0, 0, false>;
 }
 
@@ -714,7 +714,7 @@ static void sum_split(const brille_grid* G, uint32_t m, bool prop, int precision
   *tile = TILE;
   *groups = 1;
   const DataConst& d = G->d;
-  if (prop || !wide_rows(d)) return;
+  if (prop || !wide_rows(d, precision)) return;
   const bool atoms = wide_by_atom(d);
   if (atoms) *tile = sums_points(LAYOUT_WIDE, kWideAtom);
   const uint64_t want = 8ull * std::max<uint32_t>(G->n_cu, 1);
@@ -830,17 +830,17 @@ static uint64_t table_bytes(const brille_grid* G, int precision) {
   const DataConst& d = G->d;
   if (!d.has_blocks) return 0;
   const bool f32 = precision == BRILLE_FP32;
-  const uint64_t row = wide_rows(d)          ? (f32 ? 8 : 16)
-                       : onepass_sc(d) == 0 ? 0
-                       : f32                ? d.stride32 * 4ull
-                                            : d.stride64 * 8ull;
+  const uint64_t row = wide_rows(d, precision) ? (f32 ? 8 : 16)
+                       : onepass_sc(d) == 0   ? 0
+                       : f32                  ? d.stride32 * 4ull
+                                              : d.stride64 * 8ull;
   const uint64_t bytes = (G->n_cubes * 8 + G->n_tets * 4) * d.B * row;
   return bytes > kCubeRowsMax ? 0 : bytes;
 }
 
 // the derived table of a precision exists (or the payload has none)
 static bool has_table(const DataConst& d, int precision) {
-  if (wide_rows(d)) return precision == BRILLE_FP32 ? d.wide_fac32 != nullptr : d.wide_fac64 != nullptr;
+  if (wide_rows(d, precision)) return precision == BRILLE_FP32 ? d.wide_fac32 != nullptr : d.wide_fac64 != nullptr;
   if (onepass_sc(d) == 0) return true;
   return precision == BRILLE_FP32 ? d.cube_rows32 != nullptr : d.cube_rows64 != nullptr;
 }
@@ -851,7 +851,7 @@ static bool has_table(const DataConst& d, int precision) {
 int ensure_cube_rows(brille_grid* G, int precision, hipStream_t s) {
   DataConst& d = G->d;
   if (table_bytes(G, precision) == 0 || has_table(d, precision)) return BRILLE_OK;
-  const bool wide = wide_rows(d);
+  const bool wide = wide_rows(d, precision);
   if (precision == BRILLE_FP32)
     return wide ? build_wide_factors<float>(G, s, &d.wide_fac32) : build_cube_rows<float>(G, s, &d.cube_rows32);
   return wide ? build_wide_factors<double>(G, s, &d.wide_fac64) : build_cube_rows<double>(G, s, &d.cube_rows64);
@@ -921,8 +921,8 @@ bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int p
     if (precision == BRILLE_FP32) return work >= 26000000ull && a.n >= cells;
     return d.sc >= 4 ? work >= 7000000ull : work >= 14000000ull && 2 * a.n >= cells;
   }
-  if (!shared || payload_layout(d) != LAYOUT_GAMMA || !(wide_rows(d) || onepass_sc(d))) return false;
-  if (wide_rows(d)) return work >= (precision == BRILLE_FP32 ? 20000000ull : 4000000ull);
+  if (!shared || payload_layout(d) != LAYOUT_GAMMA || !(wide_rows(d, precision) || onepass_sc(d))) return false;
+  if (wide_rows(d, precision)) return work >= (precision == BRILLE_FP32 ? 20000000ull : 4000000ull);
   return a.n >= 2 * cells && work >= (precision == BRILLE_FP32 ? 13000000ull : 7000000ull);
 }
 
@@ -941,7 +941,7 @@ bool table_due(brille_grid* G, uint64_t n, int precision) {
   uint64_t& points = G->untabled[precision == BRILLE_FP32];
   points += n;
   const bool f32 = precision == BRILLE_FP32;
-  const uint64_t halves = wide_rows(G->d) ? (f32 ? 5 : 3) : (f32 ? 48 : 28);
+  const uint64_t halves = wide_rows(G->d, precision) ? (f32 ? 5 : 3) : (f32 ? 48 : 28);
   return 2 * points >= halves * (G->n_cubes + G->n_tets / 2);
 }
 

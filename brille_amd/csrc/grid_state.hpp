@@ -132,7 +132,7 @@ int check_payload_precision(const brille_grid* G, int precision);
 // the fused tile kernel of one call (fast: tuned fold-in and sums; else the literal restatement)
 void launch_tile(const brille_grid* G, const LaunchArgs& a, int precision, bool fast, hipStream_t s);
 int payload_layout(const DataConst& d);
-bool wide_rows(const DataConst& d);
+bool wide_rows(const DataConst& d, int precision);
 bool wide_by_atom(const DataConst& d);
 // the aux outputs of a part of a call that starts at point c0
 inline brille_aux_out offset_aux(const brille_aux_out& x, uint64_t c0) {

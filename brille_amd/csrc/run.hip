@@ -247,18 +247,19 @@ static bool by_atom(const DataConst& d) {
 
 // Gamma or scalar payloads whose rows are too long for one lane (more than 12
 // and at most kWideMax complex elements, at most 64 values): one wave per row.
-// With a PermutationTable the rows of up to kSortedLaneMax elements that are not
-// summed atom by atom keep to the general sums, a lane per row, which leave
-// fewer of a wave's lanes without an element (20 scalars of 6 modes FP64,
-// 300 007 points binned: 342 vertices 4.49 ms a wave per row, 1.14 a lane, 14 513
-// vertices 3.09 / 1.64; 48 elements there 3.11 / 4.11).
+// With a PermutationTable the FP64 rows of up to kSortedLaneMax elements that are
+// not summed atom by atom keep to the general sums, a lane per row, which leave
+// fewer of a wave's lanes without an element (20 scalars of 6 modes, 300 007
+// points binned: 342 vertices 4.49 ms a wave per row, 1.14 a lane, 14 513 vertices
+// 3.09 / 1.64; 48 elements there 3.11 / 4.11; FP32, 20 elements: binned 1.58 /
+// 1.22, fused 3.24 / 6.64).
 constexpr uint32_t kSortedLaneMax = 24;
-bool wide_rows(const DataConst& d) {
+bool wide_rows(const DataConst& d, int precision) {
   const int L = payload_layout(d);
   if (!(L == LAYOUT_GAMMA || L == LAYOUT_SCALAR) || d.sc <= 12 || d.sc > kWideMax || d.sv > 64) return false;
-  return d.n_keys == 0 || d.sc > kSortedLaneMax || by_atom(d);
+  return d.n_keys == 0 || precision == BRILLE_FP32 || d.sc > kSortedLaneMax || by_atom(d);
 }
-bool wide_by_atom(const DataConst& d) { return wide_rows(d) && by_atom(d); }
+bool wide_by_atom(const DataConst& d) { return wide_rows(d, BRILLE_FP32) && by_atom(d); }
 
 // The instantiated specialisations: Gamma payloads of 1-4 atoms and scalar
 // payloads of 1-4 complex elements, each with one value per mode; anything
@@ -285,7 +286,7 @@ static TileKernel pick_tuned(const DataConst& d) {
     }
   }
   if (wide_by_atom(d)) return k_ir_interpolate<Real, true, LAYOUT_WIDE, kWideAtom, 0>;
-  if (wide_rows(d)) return k_ir_interpolate<Real, true, LAYOUT_WIDE, kWideAll, 0>;
+  if (wide_rows(d, sizeof(Real) == 4 ? BRILLE_FP32 : BRILLE_FP64)) return k_ir_interpolate<Real, true, LAYOUT_WIDE, kWideAll, 0>;
   return k_ir_interpolate<Real, true, LAYOUT_GENERIC, 0, 0>;
 }
 
@@ -304,12 +305,12 @@ static TileKernel pick_tuned(const DataConst& d) {
 //     idle, the modes split too, to three blocks per CU (301 points of 72
 //     modes: 64 us whole, 50 us in two groups, 68 us in six, each of which
 //     repeats phase 1).
-static void tile_split(const brille_grid* G, uint64_t n, bool fast, uint32_t* tile, uint32_t* groups) {
+static void tile_split(const brille_grid* G, uint64_t n, int precision, bool fast, uint32_t* tile, uint32_t* groups) {
   const DataConst& d = G->d;
   const uint64_t cu = std::max<uint32_t>(G->n_cu, 1);
   uint32_t t = TILE;
   *groups = 1;
-  if (fast && wide_rows(d)) {
+  if (fast && wide_rows(d, precision)) {
     const uint32_t mpw = wide_by_atom(d) ? 64u / (d.sc / 3u) : 1u;
     const uint32_t passes = (d.B + mpw - 1) / mpw;
     t = tile_capacity(LAYOUT_WIDE);
@@ -325,7 +326,7 @@ static void tile_split(const brille_grid* G, uint64_t n, bool fast, uint32_t* ti
 // plain: the literal FP64 restatement; tuned: fast fold-in and specialised sums
 static void launch_sel(const brille_grid* G, LaunchArgs a, int precision, bool fast, hipStream_t s) {
   uint32_t groups;
-  tile_split(G, a.n, fast, &a.tile, &groups);
+  tile_split(G, a.n, precision, fast, &a.tile, &groups);
   TileKernel k;
   if (precision == BRILLE_FP32) k = fast ? pick_tuned<float>(G->d) : k_ir_interpolate<float, false, LAYOUT_GENERIC, 0, 0>;
   else k = fast ? pick_tuned<double>(G->d) : k_ir_interpolate<double, false, LAYOUT_GENERIC, 0, 0>;
@@ -555,7 +556,7 @@ int run_interpolate(brille_grid* G, const double* Q, uint64_t n, const brille_ru
   // atoms FP64: 101 points 84 -> 48 us, 1 001 points, 0.6 MB, 125 -> 70 us, 6 001
   // points, 3.7 MB, 304 -> 247 us).  The general sums, which read back what they
   // wrote, and the larger calls go through device memory.
-  const bool direct = off <= kDirectBytes && fast && !opts.use_proposal && (wide_rows(G->d) || onepass_sc(G->d)) &&
+  const bool direct = off <= kDirectBytes && fast && !opts.use_proposal && (wide_rows(G->d, opts.precision) || onepass_sc(G->d)) &&
                       ensure_pin(G, kDirectBytes);
   if (!direct && G->stage_bytes < off) {
     if (G->stage) (void)hipFree(G->stage);

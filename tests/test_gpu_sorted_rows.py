@@ -46,10 +46,7 @@ def test_permuted_scalar_rows_in_the_binned_sums(elements, modes):
             assert np.max(np.abs(bc - oc)) <= tol * np.abs(oc).max()
 
 
-# either side of the longest sorted row a lane sums, and rows of more values than atoms
-@pytest.mark.parametrize("elements,values,atoms", [(13, 1, False), (24, 1, False), (25, 1, False), (15, 6, True), (24, 9, True), (27, 10, True)])
-def test_sorted_rows_around_the_longest_a_lane_sums(elements, values, atoms):
-    print(f"sorted rows: {elements} elements, {values} values, atoms {atoms}", flush=True)
+def sorted_grid(elements, values, atoms):
     sp = dict(S.batch_specs(16)[3], v_target=400.0)
     g = S.batch_grid(sp)
     t = S.batch_layout_tables(g, sp)
@@ -66,6 +63,14 @@ def test_sorted_rows_around_the_longest_a_lane_sums(elements, values, atoms):
     dev = capi.Grid(t)
     dev.sort()
     perm = dev.permutations()
+    return dev, t, perm, r
+
+
+# either side of the longest sorted row a lane sums, and rows of more values than atoms
+@pytest.mark.parametrize("elements,values,atoms", [(13, 1, False), (24, 1, False), (25, 1, False), (15, 6, True), (24, 9, True), (27, 10, True)])
+def test_sorted_rows_around_the_longest_a_lane_sums(elements, values, atoms):
+    print(f"sorted rows: {elements} elements, {values} values, atoms {atoms}", flush=True)
+    dev, t, perm, r = sorted_grid(elements, values, atoms)
     for n in (1, 300, 20_000):
         Q = r.uniform(-3, 3, size=(n, 3))
         rc, ov, oc, _, _ = O.ir_interpolate_at(t, Q, nthreads=8, perm=perm)
@@ -78,3 +83,21 @@ def test_sorted_rows_around_the_longest_a_lane_sums(elements, values, atoms):
             assert np.max(np.abs(bv - ov)) <= tol * np.abs(ov).max(), (n, prec)
             # an assigned pair's overlap can still be small, and the antiphase then carries the products' rounding
             assert np.max(np.abs(bc - oc)) <= 10 * tol * np.abs(oc).max(), (n, prec)
+
+
+def test_a_batch_of_sorted_rows_around_the_longest_a_lane_sums():
+    print("sorted rows: batch", flush=True)
+    devs = [sorted_grid(*form)[0] for form in ((13, 1, False), (24, 1, False), (25, 1, False), (15, 6, True))]
+    Qs = [np.random.default_rng(k).uniform(-3, 3, size=(600 + 100 * k, 3)) for k in range(len(devs))]
+    off = np.concatenate([[0], np.cumsum([len(q) for q in Qs])]).astype(np.uint64)
+    dQ = capi.DeviceArray.from_host(np.vstack(Qs))
+    b = capi.Batch(devs)
+    for binned_min in (None, 1):
+        b.set_schedule(tile_points=128, binned_min=binned_min)
+        for prec in (capi.FP64, capi.FP32):
+            vals, vecs = b.outputs(off, prec)
+            capi.check(b.run(dQ, off, vals, vecs, precision=prec))
+            for d, Q, v, c in zip(devs, Qs, vals, vecs):
+                tv, tc = d.ir_interpolate_at(Q, precision=prec, kernel=capi.KERNEL_TILE)
+                np.testing.assert_array_equal(v.to_host(), tv.reshape(v.shape))
+                np.testing.assert_array_equal(c.to_host(), tc.reshape(c.shape))
