@@ -378,7 +378,7 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nb) {
 // points a block of the sums holds: the atom-major wide sums run as fast with 64
 // as with 128 or 256 (24 atoms, 300 007 points of 72 modes FP32 5.2 ms), which
 // leaves the LDS to the records being assembled
-constexpr uint32_t sums_points(int L, int SC) { return L == LAYOUT_WIDE && SC == kWideAtom ? 64u : (uint32_t)TILE; }
+constexpr uint32_t sums_points(int L, int SC) { return L == LAYOUT_WIDE && wide_atom_major(SC) ? 64u : (uint32_t)TILE; }
 
 // waves per SIMD asked of the compiler: the atom-major wide sums run best at
 // four (FP32) and two (FP64), a few registers below what it would take for
@@ -388,7 +388,7 @@ constexpr uint32_t sums_points(int L, int SC) { return L == LAYOUT_WIDE && SC ==
 // of scratch in the walk, 3 000 017 points 1.03 -> 1.92 ms.)
 template <typename Real, int L, int SC>
 constexpr int sums_waves() {
-  if (L == LAYOUT_WIDE && SC == kWideAtom) return sizeof(Real) == 4 ? 4 : 2;
+  if (L == LAYOUT_WIDE && wide_atom_major(SC)) return sizeof(Real) == 4 ? 4 : 2;
   if (L == LAYOUT_GAMMA) return sizeof(Real) == 4 ? 4 : 2;
   return 1;
 }
@@ -406,7 +406,7 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const FoldRec* recs,
   __shared__ PointRec<Real> s_rec[TP];
   // wide rows: the phase table of the node-ordered Gamma sums instead
   constexpr uint32_t kPh =
-      kWide ? (SC == kWideAtom ? kWideAtomPhaseBytes : kWidePhaseBytes) / sizeof(C) : TILE * S::NPH;
+      kWide ? (wide_atom_major(SC) ? kWideAtomPhaseBytes : kWidePhaseBytes) / sizeof(C) : TILE * S::NPH;
   __shared__ C s_ph[kPh];
   __shared__ Real s_wrot[kWide ? 9 * kMaxOps : 1];
   __shared__ uint8_t s_wdst[kWide ? kWideAtoms * kMaxOps : 1];
@@ -418,7 +418,7 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const FoldRec* recs,
   if (kOpFrames && threadIdx.x < g.G) fill_frame<Real, SC>(g, d, threadIdx.x, s_frames[threadIdx.x]);
   __shared__ uint32_t s_out[TP];
   // wide rows' slices, or the atom lanes' records
-  constexpr bool kAtoms = kWide && SC == kWideAtom;
+  constexpr bool kAtoms = kWide && wide_atom_major(SC);
   constexpr uint32_t kWalk = kOpFrames ? TILE / 64 * walk_slice<Real>() / sizeof(C)
                              : kAtoms  ? TILE / 64 * wide_walk_slice<Real>(WSL)
                                        : 1;
@@ -438,7 +438,7 @@ void k_bin_sums(GridConst g, DataConst d, ProposalConst pc, const FoldRec* recs,
   // first one reports the points' errors and aux outputs)
   const bool lead = blockIdx.y == 0;
   uint32_t per_group = (d.B + gridDim.y - 1) / gridDim.y;
-  if (L == LAYOUT_WIDE && SC == kWideAtom) {  // whole passes of the atom-major walk
+  if (L == LAYOUT_WIDE && wide_atom_major(SC)) {  // whole passes of the atom-major walk
     const uint32_t mpw = wide_pass_modes(d.sc, sizeof(C));
     per_group = (per_group + mpw - 1) / mpw * mpw;
   }
@@ -690,7 +690,8 @@ static SumsKernel pick_sums(const DataConst& d, bool prop) {
       default: break;
     }
   }
-  if (wide_by_atom(d)) return k_bin_sums<Real, LAYOUT_WIDE, kWideAtom, 0, false>;
+  if (wide_by_atom(d))
+    return d.gamma_maps ? k_bin_sums<Real, LAYOUT_WIDE, kWideAtom, 0, false> : k_bin_sums<Real, LAYOUT_WIDE, kWideLoose, 0, false>;
   if (wide_rows(d, sizeof(Real) == 4 ? BRILLE_FP32 : BRILLE_FP64)) return k_bin_sums<Real, LAYOUT_WIDE, kWideAll, 0, false>;
   return k_bin_sums<Real, LAYOUT_GENERIC, 0, 0, false>;
 }

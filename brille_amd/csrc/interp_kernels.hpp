@@ -783,8 +783,11 @@ constexpr uint32_t kWideMax = 128;  // complex elements per row the wide phase 2
 constexpr uint32_t kWideAtoms = kWideMax / 3;  // atoms of the longest wide Gamma row
 // SC of the wide sums (LAYOUT_WIDE): rows summed a wave per (point, mode)
 // (kWideAll: scalar rows, or more values than atoms), or atom-major
-// (kWideAtom: Gamma rows of at most one value per atom)
-constexpr int kWideAll = 0, kWideAtom = 1;
+// (kWideAtom: Gamma rows of at most one value per atom; kWideLoose: the same where
+// an operation maps two atoms to one, so that the node-ordered sums have no
+// whole record to assemble and store atom by atom)
+constexpr int kWideAll = 0, kWideAtom = 1, kWideLoose = 2;
+constexpr bool wide_atom_major(int SC) { return SC != kWideAll; }
 // LDS of the node-ordered wide sums' Gamma table: per-point phases of a chunk
 // of the tile's points, every atom (FP32: 4608 complex, 192 points of 24
 // atoms).  Those sums hold over 200 VGPRs, so two blocks per CU is their
@@ -1536,7 +1539,7 @@ struct TileShape {
                             : (L == LAYOUT_GAMMA ? frame_words<Real>() * TB : 1);
   // wide-row slices, one per wave
   static constexpr int NW =
-      L == LAYOUT_WIDE ? (TB / 64) * (int)(SC == kWideAtom ? wide_atom_slice<Real>(WSL) : kWideMax) : 1;
+      L == LAYOUT_WIDE ? (TB / 64) * (int)(wide_atom_major(SC) ? wide_atom_slice<Real>(WSL) : kWideMax) : 1;
 };
 
 // The row-table block of a point: cube c's eight slots at rows c * 8 * B, the
@@ -1625,7 +1628,7 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
     const bool gamma = d.vec_rot == BRILLE_ROT_GAMMA && d.ec[1] > 0;
     const bool tab = wide_factors<Real>(d) != nullptr;
     const uint32_t b_end = b_hi < B ? b_hi : B;
-    if constexpr (SC == kWideAtom) {
+    if constexpr (wide_atom_major(SC)) {
       // Atom-major (Gamma rows of at most one value per atom): lane l takes
       // atom a = l % na of mode l / na, so a wave sums mpw = 64 / na modes of a
       // point at once (a "pass"), each lane its atom's three elements: the
@@ -1751,6 +1754,13 @@ __device__ __forceinline__ void tile_sums(const GridConst& g, const DataConst& d
             auto finish = [&](uint32_t pl, const C* acc, Real va) {
               const uint64_t row = (out_row ? (uint64_t)uniform(out_row[pl]) : row0 + pl) * B;
               const uint32_t op = uniform(s_rec[pl].invrot);
+              if constexpr (SC == kWideLoose) {
+                if (!on) return;
+                if (a < sv) vals[row * sv + (uint64_t)b * sv + a] = va;
+                wide_atom_store<Real>(acc, wg.rot + 9u * op, wg.ph[(pl - c0) * na + a],
+                                      vecs + row * sc + (uint64_t)b * sc + 3u * wg.dst[op * na + a]);
+                return;
+              }
               if (on) {
                 if (a < sv) (vals + (row + b0) * sv)[m * sv + a] = va;
                 wide_atom_rotate<Real, true>(acc, wg.rot + 9u * op, wg.ph[(pl - c0) * na + a],

@@ -239,11 +239,8 @@ int payload_layout(const DataConst& d) {
   return LAYOUT_GENERIC;
 }
 
-// wide Gamma rows of at most one value per atom, every operation mapping the
-// atoms one to one: the sums go atom-major (they write whole records)
-static bool by_atom(const DataConst& d) {
-  return payload_layout(d) == LAYOUT_GAMMA && d.sv <= d.sc / 3u && d.gamma_maps;
-}
+// wide Gamma rows of at most one value per atom: the sums go atom-major
+static bool by_atom(const DataConst& d) { return payload_layout(d) == LAYOUT_GAMMA && d.sv <= d.sc / 3u; }
 
 // Gamma or scalar payloads whose rows are too long for one lane (more than 12
 // and at most kWideMax complex elements, at most 64 values): one wave per row.

@@ -101,3 +101,31 @@ def test_batch_members_whose_operations_map_two_atoms_to_one():
                 for p, op in enumerate(aux["invrot"]):
                     once = [a for a in range(A) if np.count_nonzero(F0[:, op] == a) == 1]
                     np.testing.assert_array_equal(got[p][:, once], ref[p][:, once])
+
+
+@pytest.mark.parametrize("atoms,modes", [(5, 13), (12, 9), (24, 41), (42, 3)])
+def test_wide_tables_that_are_not_one_to_one(atoms, modes):
+    """Element for element the fused kernel's results in every pipeline, and the elements no atom is
+    mapped to are left as they were."""
+    print(f"call edges: {atoms} atoms, {modes} modes, not one to one", flush=True)
+    t, F0 = payload(atoms, modes, False, 10 * atoms + modes)
+    dev = capi.Grid(t)
+    for n in (1, 700):
+        Q = np.random.default_rng(n).uniform(-3, 3, size=(n, 3))
+        dQ = capi.DeviceArray.from_host(Q)
+        for prec in (capi.FP64, capi.FP32):
+            got = []
+            for kernel in (capi.KERNEL_TILE, capi.KERNEL_BINNED, capi.KERNEL_TILE):  # without and with the table
+                dv = capi.DeviceArray((n, modes), np.float32 if prec == capi.FP32 else np.float64)
+                dc = capi.DeviceArray.from_host(np.full((n, modes, atoms, 3), 7, np.complex64 if prec == capi.FP32 else np.complex128))
+                o = capi.RunOpts(0, prec, 0, capi.MEM_DEVICE, kernel, 1)
+                capi.check(capi.lib().brille_ir_interpolate_at(dev.h, dQ.ptr, n, C.byref(o), dv.ptr, dc.ptr, None, None))
+                got.append((dv.to_host(), dc.to_host()))
+            rc, _, _, aux = dev.run_device(Q, precision=prec, aux=("invrot",))
+            assert rc == 0
+            for v, c in got[1:]:
+                np.testing.assert_array_equal(v, got[0][0])
+                for p, op in enumerate(aux["invrot"]):
+                    count = np.bincount(F0[:, op], minlength=atoms)
+                    np.testing.assert_array_equal(c[p][:, count == 1], got[0][1][p][:, count == 1])
+                    assert (c[p][:, count == 0] == 7).all()
