@@ -912,6 +912,7 @@ bool binned_applies(const brille_grid* G, const LaunchArgs& a, int kernel, int p
   if (a.use_proposal || kernel == BRILLE_KERNEL_BINNED) return true;
   if (x.ir_q || x.rot || x.invrot || x.node || x.tet || x.n_iw || x.iw_index || x.iw_weight || x.status)
     return false;
+  if (G->g.n_nodes >= kNodePoly) return false;  // the pipeline refuses such grids, the fused kernel takes them
   const DataConst& d = G->d;
   const uint64_t payload = (uint64_t)d.V * d.B * d.stride32 * 4;
   const uint64_t work = a.n * d.B * d.sc, cells = G->n_cubes + G->n_tets / 2;
